@@ -20,6 +20,7 @@ SYMBOLS = [
     "gelib_hip_gather_map_destroy", "gelib_hip_part_gather", "gelib_hip_part_mix_channels",
     "gelib_hip_part_mix_channels_static", "gelib_hip_part_mix_channels_wgrad", "gelib_hip_part_mix_workspace_bytes",
     "gelib_hip_so3vec_cg_linear_fwd", "gelib_hip_so3vec_cg_linear_workspace_bytes",
+    "gelib_hip_so3vec_cg_linear_workspace_bytes_shared",
     "gelib_hip_so3vec_cg_linear_bwd", "gelib_hip_so3vec_cg_linear_bwd_workspace_bytes",
     "gelib_hip_set_option", "gelib_hip_set_stream_workspace",
     "gelib_hip_last_path",
@@ -92,8 +93,9 @@ def lib():
         L.gelib_hip_so3vec_cg_linear_bwd_workspace_bytes.restype = ctypes.c_uint64
         L.gelib_hip_so3vec_cg_linear_bwd_workspace_bytes.argtypes = [ctypes.c_int, P, ctypes.c_int, P, ctypes.c_int, P,
                                                                      ctypes.c_int64]
-        L.gelib_hip_so3vec_cg_linear_workspace_bytes.restype = ctypes.c_uint64
-        L.gelib_hip_so3vec_cg_linear_workspace_bytes.argtypes = [ctypes.c_int, P, ctypes.c_int, P, ctypes.c_int, P]
+        for name in ("gelib_hip_so3vec_cg_linear_workspace_bytes", "gelib_hip_so3vec_cg_linear_workspace_bytes_shared"):
+            getattr(L, name).restype = ctypes.c_uint64
+            getattr(L, name).argtypes = [ctypes.c_int, P, ctypes.c_int, P, ctypes.c_int, P]
         L.gelib_hip_part_mix_workspace_bytes.restype = ctypes.c_uint64
         L.gelib_hip_part_mix_workspace_bytes.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
         L.gelib_hip_set_option.argtypes = [ctypes.c_char_p, ctypes.c_int]
@@ -213,7 +215,7 @@ def so3vec_cg_linear_fwd(rparts, xparts, yparts, wparts, accumulate=False):
     import torch
     L = lib()
     ra, xa, ya = _arr(rparts), _arr(xparts), _arr(yparts)
-    nbytes = int(L.gelib_hip_so3vec_cg_linear_workspace_bytes(len(rparts), ra, len(xparts), xa, len(yparts), ya))
+    nbytes = int(L.gelib_hip_so3vec_cg_linear_workspace_bytes_shared(len(rparts), ra, len(xparts), xa, len(yparts), ya))
     if nbytes == 0:
         return False
     ws = torch.empty(nbytes, dtype=torch.uint8, device=rparts[0].device)

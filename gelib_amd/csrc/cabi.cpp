@@ -1229,8 +1229,9 @@ uint64_t gelib_hip_so3vec_cg_linear_bwd_workspace_bytes(int ng, const gelib_part
   if (cb <= 0) return 0;
   return (uint64_t)lin_bwd_bytes(sh, cb, nullptr, nullptr, nullptr, nullptr);
 }
-uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes(int nr, const gelib_part_desc *r, int nx, const gelib_part_desc *x,
-                                                    int ny, const gelib_part_desc *y) {
+namespace {
+uint64_t linear_workspace_bytes(int nr, const gelib_part_desc *r, int nx, const gelib_part_desc *x, int ny,
+                                const gelib_part_desc *y, bool shared) {
   std::vector<View> R, X, Y;
   if (sort_parts(nr, r, kMaxOutParts, R) || sort_parts(nx, x, kMaxParts, X) || sort_parts(ny, y, kMaxParts, Y)) return 0;
   VecPlan plan;
@@ -1243,8 +1244,21 @@ uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes(int nr, const gelib_part_des
     t5[l] = tau[l];
   }
   long long x_elems = 0;
-  for (auto &v : X) x_elems += (long long)(2 * v.l + 1) * v.n;
-  return (uint64_t)cg_linear_workspace_bytes(t5, x_elems, plan.E[0] * plan.E[1] * plan.E[2]);
+  int x_channels = shared ? 1 : 0;
+  for (auto &v : X) {
+    x_elems += (long long)(2 * v.l + 1) * v.n;
+    if (shared) x_channels = std::max(x_channels, v.n);
+  }
+  return (uint64_t)cg_linear_workspace_bytes(t5, x_elems, x_channels, plan.E[0] * plan.E[1] * plan.E[2]);
+}
+}  // namespace
+uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes(int nr, const gelib_part_desc *r, int nx, const gelib_part_desc *x,
+                                                    int ny, const gelib_part_desc *y) {
+  return linear_workspace_bytes(nr, r, nx, x, ny, y, false);
+}
+uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes_shared(int nr, const gelib_part_desc *r, int nx,
+                                                           const gelib_part_desc *x, int ny, const gelib_part_desc *y) {
+  return linear_workspace_bytes(nr, r, nx, x, ny, y, true);
 }
 
 int gelib_hip_so3part_spharm(const gelib_part_desc *r, const float *x, const int64_t xdims[5],

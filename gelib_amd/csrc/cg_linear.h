@@ -13,8 +13,10 @@ constexpr int kLinMaxOut = 16;   // most output channels of a product part
 constexpr int kLinCells = 32;    // cells per block: the rows of one matrix-core tile
 
 // Bytes of workspace: the re-packed matrices of a product with tau[l] channels in part l (l = 0..kLinL) and a copy of
-// the first operand (x_elems_per_cell complex numbers per cell) transposed per group of kLinCells cells.
-size_t cg_linear_workspace_bytes(const long long tau[kLinL + 1], long long x_elems_per_cell, long long ncells);
+// the first operand (x_elems_per_cell complex numbers per cell) transposed per group of kLinCells cells.  With
+// x_channels > 0 (the most channels of a part of the first operand) also room for the partial sums of the waves that
+// share a group in launches with few of them; without that room one wave takes a whole group.
+size_t cg_linear_workspace_bytes(const long long tau[kLinL + 1], long long x_elems_per_cell, int x_channels, long long ncells);
 
 // out_l[cell, m, :] (+)= P_l[cell, m, :] W_l with P = CGproduct(x, y) never stored.  w[k] belongs to r[k] (both l-sorted):
 // (tau_l, n_out_l) complex, row-major, device memory.  *used = 0 when the shapes are not ones the kernel takes (nothing

@@ -1,6 +1,7 @@
 // Host side and helper kernels of the fused SO3vec CGproduct -> channel mixing forward pass (the kernel itself:
 // cg_linear_impl.h): the matrices re-packed for the matrix cores, the first operand transposed per group of cells, the
 // two launches.
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -43,15 +44,94 @@ __global__ void pack_linear_kernel(float *wp, const float2 *w, long long tau, in
   wp[idx] = val;
 }
 
+// out_l[cell, m, o] (+)= sum over the shares of partial[share][group][l^2 + l + m][cell of the group][2 o, 2 o + 1], in the
+// order of the shares; one thread per complex number.  Memory-bound (8192 cells, 4 shares: 105 MB read, 26 MB written).
+__global__ void __launch_bounds__(256) sum_shares_kernel(const LinArgs a, int shares, long long groups) {
+  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;   // (group, row, cell of the group, o)
+  const int o = idx & 15, c = (idx >> 4) & 31;
+  const long long gr = idx >> 9;
+  const long long g = gr / kLinRows;
+  if (g >= groups) return;
+  const int lm = (int)(gr - g * kLinRows);
+  const long long cell = g * kLinCells + c;
+  if (cell >= a.ncells) return;
+  static_for<kNL>([&](auto lc) __attribute__((always_inline)) {
+    constexpr int l = decltype(lc)::value;
+    if (lm >= l * l && lm < (l + 1) * (l + 1)) {
+      const FastPart O = a.out[l];
+      if (o < O.n) {
+        const float2 *p = (const float2 *)a.partial + (gr * kLinCells + c) * 16 + o;
+        float2 s = make_float2(0.f, 0.f);
+        for (int k = 0; k < shares; k++) {
+          const float2 v = p[(long long)k * groups * (kLinGroupFloats / 2)];
+          s.x += v.x;
+          s.y += v.y;
+        }
+        float2 *q = O.ptr + cell * O.sb + (long long)(lm - l * l) * O.sm + o;
+        if (a.accumulate) {
+          s.x += q->x;
+          s.y += q->y;
+        }
+        *q = s;
+      }
+    }
+  });
+}
+
 size_t packed_bytes(long long tau) { return (size_t)(tau + kBAhead) * 256; }  // padding behind the last channel
+
+// Waves that share a group of cells: split_a shares of the channels of x, times kLinSets sets of parts of y.
+// A wave takes most of a SIMD's registers, so a launch fills the GPU with 1024 waves, and one of G groups takes
+// ceil(G * shares / 1024) rounds of what one wave has to do: the channels of its share, plus about 3 % of a whole group's
+// work for the pairs' coefficients, plus the writing and summing of the partial results (a 50000th of a whole group's time
+// per wave).  The cheapest choice is taken; with 1024 groups (32768 cells) that is one wave per group, as it is for whole
+// multiples of it.  One wave per group / shared, microseconds: L=4, 16 x 16 -> 16 channels, 64 cells 5340 / 187,
+// 1024 cells 5380 / 306, 5003 cells 5430 / 1210, 8192 cells 5440 / 1570, 20000 cells 5470 / 4100, 32768 cells 5570 / (not
+// shared) 5610, 40000 cells 11340 / 8700; 7 x 3 -> 12 channels, 8192 cells 896 / 327.
+struct LinSplit {
+  int a = 1, l2 = 0;
+  int shares() const { return a * (l2 ? kLinSets : 1); }
+};
+constexpr long long kLinWaves = 1024;       // waves that run at once
+constexpr long long kLinMaxPartial = 4096;  // most (share, group) pairs: 420 MB of partial sums
+
+LinSplit choose_split(long long groups, int nmax) {
+  LinSplit best;
+  double least = 0;
+  for (int l2 = 0; l2 < 2; l2++)
+    for (int sa = 1; sa <= nmax; sa++) {
+      LinSplit t;
+      t.a = sa;
+      t.l2 = l2;
+      const long long waves = groups * t.shares();
+      if (t.shares() > 1 && waves > kLinMaxPartial) continue;
+      const double mine = ((double)((nmax + sa - 1) / sa) / nmax + 0.03) * (l2 ? 0.27 : 1.0);
+      const double cost = (double)((waves + kLinWaves - 1) / kLinWaves) * mine + (t.shares() > 1 ? 2e-5 * (double)waves : 0.0);
+      if (t.shares() == 1 || cost < least) {
+        least = cost;
+        best = t;
+      }
+    }
+  return best;
+}
+
+size_t plain_workspace_bytes(const long long tau[kLinL + 1], long long x_elems_per_cell, long long groups) {
+  size_t total = 0;
+  for (int l = 0; l <= kLinL; l++) total += packed_bytes(tau[l]);
+  return total + (size_t)groups * kLinCells * (size_t)x_elems_per_cell * sizeof(float2);
+}
+
+size_t partial_bytes(const LinSplit &t, long long groups) {
+  return t.shares() > 1 ? (size_t)t.shares() * groups * kLinGroupFloats * sizeof(float) : 0;
+}
 
 }  // namespace
 
-size_t cg_linear_workspace_bytes(const long long tau[kLinL + 1], long long x_elems_per_cell, long long ncells) {
-  size_t total = 0;
-  for (int l = 0; l <= kLinL; l++) total += packed_bytes(tau[l]);
+size_t cg_linear_workspace_bytes(const long long tau[kLinL + 1], long long x_elems_per_cell, int x_channels, long long ncells) {
   const long long groups = (ncells + kLinCells - 1) / kLinCells;
-  return total + (size_t)groups * kLinCells * (size_t)x_elems_per_cell * sizeof(float2);
+  const size_t plain = plain_workspace_bytes(tau, x_elems_per_cell, groups);
+  if (x_channels <= 0) return plain;
+  return plain + partial_bytes(choose_split(groups, std::min(x_channels, kLinMaxN)), groups);
 }
 
 int cg_linear_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *> &r,
@@ -95,8 +175,12 @@ int cg_linear_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
       if (have != std::min(p.first + q.first, kLinL) - std::abs(p.first - q.first) + 1) return GELIB_HIP_OK;
     }
   long long x_elems = 0;
-  for (auto &p : lx) x_elems += (long long)(2 * p.first + 1) * p.second;
-  if (!ws || ((uintptr_t)ws & 15) || ws_bytes < cg_linear_workspace_bytes(tau, x_elems, ncells)) return GELIB_HIP_ERR_WORKSPACE;
+  int x_channels = 1;
+  for (auto &p : lx) x_elems += (long long)(2 * p.first + 1) * p.second, x_channels = std::max(x_channels, p.second);
+  const size_t plain = plain_workspace_bytes(tau, x_elems, nblocks);
+  if (!ws || ((uintptr_t)ws & 15) || ws_bytes < plain) return GELIB_HIP_ERR_WORKSPACE;
+  LinSplit split = choose_split(nblocks, x_channels);
+  if (ws_bytes - plain < partial_bytes(split, nblocks)) split = LinSplit();   // no room for partial sums: one wave per group
   int rc = cg_table_bank(&a.bank);
   if (rc) return rc;
   a.ncells = ncells;
@@ -116,8 +200,16 @@ int cg_linear_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
     GELIB_HIP_TRY(hipGetLastError());
     cursor += (size_t)nblocks * kLinCells * elems * sizeof(float2);
   }
+  a.split_a = split.a;
+  a.split_l2 = split.l2;
+  a.partial = split.shares() > 1 ? (float *)cursor : nullptr;
   if ((rc = launch_cg_linear_pass0(a, nblocks, s))) return rc;
   if ((rc = launch_cg_linear_pass1(a, nblocks, s))) return rc;
+  if (a.partial) {
+    const long long threads = nblocks * kLinRows * kLinCells * 16;
+    sum_shares_kernel<<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s>>>(a, split.shares(), nblocks);
+    GELIB_HIP_TRY(hipGetLastError());
+  }
   *used = 1;
   return GELIB_HIP_OK;
 }

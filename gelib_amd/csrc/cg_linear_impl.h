@@ -45,7 +45,20 @@ struct LinArgs {
   const float *bank;                  // coefficient tables, table_off(l1, l2, l)
   long long ncells;
   int accumulate;
+  // Launches with few groups of cells: gridDim.y = split_a * (split_l2 ? kLinSets : 1) waves share a group, each with a
+  // share of the channels of the first operand and, with split_l2, one of kLinSets sets of parts of the second.  Their
+  // sums go to partial[share][group][row of the product][cell of the group][32 floats], and sum_shares_kernel adds them
+  // in the order of the shares.  partial == nullptr: one wave per group, straight into the result.
+  int split_a, split_l2;
+  float *partial;
 };
+
+// The sets of l2 of a launch with split_l2: matrix instructions per channel pair with every l1 = 0..4 there, both
+// passes: {0, 1} 89, {2} 90, {3} 101, {4} 95 of 375.
+constexpr int kLinSets = 4;
+constexpr int set_of(int l2) { return l2 < 2 ? 0 : l2 - 1; }
+constexpr int kLinRows = kNL * kNL;                              // rows (l, m) of the product, row l * l + l + m
+constexpr int kLinGroupFloats = kLinRows * kLinCells * 32;       // floats of one share's sums of one group
 
 constexpr int kBAhead = 16;  // most channel pairs between the load of a B operand and its use
 
@@ -88,12 +101,15 @@ constexpr bool pair_needed(int pass, int l1, int l2) {
 
 template <int L1, int L2, int PASS, int U>
 __device__ __forceinline__ void pair_body(const LinArgs &a, f16v (&acc)[kTiles], const v2f *ys, long long cell,
-                                          int slot, int h, int lane, int zero) {
+                                          int slot, int h, int lane, int zero, int share_a) {
   constexpr int lmin = iabs(L1 - L2), lmax = imin(L1 + L2, kLinL);
   constexpr int R1 = 2 * L1 + 1, R2 = 2 * L2 + 1, NLP = lmax - lmin + 1;
   if constexpr (!pair_needed(PASS, L1, L2)) return;
   const FastPart X = a.x[L1];
   const int n1 = X.n, n2 = a.y[L2].n;
+  // the wave's channels of x (at most kLinMaxN * kLinMaxN fits an int)
+  const int ia0 = n1 * share_a / a.split_a, ia1 = n1 * (share_a + 1) / a.split_a;
+  if (ia0 == ia1) return;
   // x from its transposed copy: the 32 cells of the block side by side, so a load touches two lines, not 32 (read from
   // the part itself -- eight bytes per cell, a cell's row apart -- the gathers of the waves of an XCD kept more lines
   // alive than its L2 cache holds and pushed the matrices out of it)
@@ -101,7 +117,7 @@ __device__ __forceinline__ void pair_body(const LinArgs &a, f16v (&acc)[kTiles],
   GlobalF wl[NLP];
   static_for<NLP>([&](auto dc) __attribute__((always_inline)) {
     constexpr int l = lmin + decltype(dc)::value;
-    if constexpr (l_in_pass(PASS, l)) wl[dc.value] = (GlobalF)(a.wp[l] + (long long)a.offs[L1][L2][l] * 64 + lane);
+    if constexpr (l_in_pass(PASS, l)) wl[dc.value] = (GlobalF)(a.wp[l] + (long long)(a.offs[L1][L2][l] + ia0 * n2) * 64 + lane);
   });
 
   // The coefficients of the pair's l of this pass, one register each (the same value in every lane): the scalar
@@ -133,7 +149,7 @@ __device__ __forceinline__ void pair_body(const LinArgs &a, f16v (&acc)[kTiles],
   v2f xn[R1], yq[2][R2];
   float bq[U][NLP];
 #pragma unroll
-  for (int k = 0; k < R1; k++) xn[k] = xp[(k * n1) * kLinCells];
+  for (int k = 0; k < R1; k++) xn[k] = xp[(k * n1 + ia0) * kLinCells];
 #pragma unroll
   for (int k = 0; k < R2; k++) yq[0][k] = ys[(k * n2) * kLinCells + slot];
   static_for<U>([&](auto ac) __attribute__((always_inline)) {
@@ -143,8 +159,8 @@ __device__ __forceinline__ void pair_body(const LinArgs &a, f16v (&acc)[kTiles],
     });
   });
 
-  int t = 0;  // channel of the block: a n2 + j
-  for (int ia = 0; ia < n1; ia++) {
+  int t = 0;  // channel of the block behind the wave's first: (a - ia0) n2 + j
+  for (int ia = ia0; ia < ia1; ia++) {
     // component h of x y is u yr + v yi with (u, v) = (xr, -xi) for the real part, (xi, xr) for the imaginary part
     float u[R1], v[R1];
 #pragma unroll
@@ -152,7 +168,7 @@ __device__ __forceinline__ void pair_body(const LinArgs &a, f16v (&acc)[kTiles],
       u[k] = h ? xn[k].y : xn[k].x;
       v[k] = h ? xn[k].x : -xn[k].y;
     }
-    const int ian = ia + 1 < n1 ? ia + 1 : ia;
+    const int ian = ia + 1 < ia1 ? ia + 1 : ia;
 #pragma unroll
     for (int k = 0; k < R1; k++) xn[k] = xp[(k * n1 + ian) * kLinCells];
     for (int j = 0; j < n2; j += U, t += U) {
@@ -225,10 +241,11 @@ __global__ void __launch_bounds__(64) cg_linear_fwd_kernel(const LinArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; e++) acc[k][e] = 0.f;
 
+  const int share_a = (int)blockIdx.y % a.split_a, share_l2 = a.split_l2 ? (int)blockIdx.y / a.split_a : -1;
   static_for<kNL>([&](auto l2c) __attribute__((always_inline)) {
     constexpr int L2 = decltype(l2c)::value;
     const FastPart Y = a.y[L2];
-    if (Y.ptr != nullptr) {
+    if (Y.ptr != nullptr && (share_l2 < 0 || share_l2 == set_of(L2))) {
       __syncthreads();
       const GlobalC yp = (GlobalC)(Y.ptr + cell * Y.sb);
       for (int row = 0; row < 2 * L2 + 1; row++)
@@ -240,13 +257,29 @@ __global__ void __launch_bounds__(64) cg_linear_fwd_kernel(const LinArgs a) {
           constexpr int UW = wide_u(PASS, L1, L2);
           // the second operand's channel count must be a multiple of the ring length; any other count takes one
           // channel pair per trip and waits for every load (correct, slow)
-          if ((Y.n & (UW - 1)) == 0) pair_body<L1, L2, PASS, UW>(a, acc, ys, cell, slot, h, lane, zero);
-          else pair_body<L1, L2, PASS, 1>(a, acc, ys, cell, slot, h, lane, zero);
+          if ((Y.n & (UW - 1)) == 0) pair_body<L1, L2, PASS, UW>(a, acc, ys, cell, slot, h, lane, zero, share_a);
+          else pair_body<L1, L2, PASS, 1>(a, acc, ys, cell, slot, h, lane, zero, share_a);
         }
       });
     }
   });
 
+  if (a.partial != nullptr) {
+    float *pp = a.partial + ((long long)blockIdx.y * gridDim.x + blockIdx.x) * kLinGroupFloats + slot;
+    static_for<kNL>([&](auto lc) __attribute__((always_inline)) {
+      constexpr int l = decltype(lc)::value;
+      static_for<2 * l + 1>([&](auto rc) __attribute__((always_inline)) {
+        constexpr int row = decltype(rc)::value;
+        if constexpr (in_pass(PASS, l, row - l)) {
+          constexpr int tile = tile_of(PASS, l, row - l);
+#pragma unroll
+          for (int v = 0; v < 16; v++)
+            pp[((l * l + row) * kLinCells + 8 * (v / 4) + 4 * h + (v % 4)) * 32] = acc[tile][v];
+        }
+      });
+    });
+    return;
+  }
   // register v of a tile: row (cell) 8 (v / 4) + 4 h + v % 4, column (float of the output row) = lane % 32
   static_for<kNL>([&](auto lc) __attribute__((always_inline)) {
     constexpr int l = decltype(lc)::value;
@@ -269,9 +302,11 @@ __global__ void __launch_bounds__(64) cg_linear_fwd_kernel(const LinArgs a) {
   });
 }
 
+inline int lin_shares(const LinArgs &a) { return a.split_a * (a.split_l2 ? kLinSets : 1); }
+
 template <int PASS>
 int launch_cg_linear_pass_impl(const LinArgs &a, long long nblocks, hipStream_t s) {
-  cg_linear_fwd_kernel<PASS><<<dim3((unsigned)nblocks), dim3(64), 0, s>>>(a);
+  cg_linear_fwd_kernel<PASS><<<dim3((unsigned)nblocks, (unsigned)lin_shares(a)), dim3(64), 0, s>>>(a);
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
 }

@@ -299,3 +299,44 @@ def test_linear_backward_declines_and_workspace_rules(cabi):
     assert call(base + 16, one) == 13        # 256-byte alignment
     assert call(0, one) == 13
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("B,tx,ty", [
+    (32 * 33 + 5, {l: 6 for l in range(5)}, {l: 4 for l in range(5)}),        # uneven shares of the channels of x
+    (32 * 9, {0: 5, 1: 1, 2: 2, 3: 7, 4: 3}, {0: 4, 1: 2, 2: 3, 4: 1}),       # parts with fewer channels than shares, l2 = 3 absent
+    (70, {4: 16}, {0: 1, 1: 1, 2: 1, 3: 1, 4: 16}),                           # a set of l2 without work for some shares
+])
+def test_waves_that_share_a_group(cabi, B, tx, ty):
+    """With the larger workspace several waves share a group of cells; with the smaller one a wave takes the group by
+    itself.  Both add the same float32 terms in different orders: each lies within a few roundings of the sum of the moduli
+    of the terms (oracle_linear's S) from the exact result, 8 eps32 S for the two together."""
+    import ctypes
+    xs = [U.seeded(5 + l, B, 2 * l + 1, n) for l, n in sorted(tx.items())]
+    ys = [U.seeded(60 + l, B, 2 * l + 1, n) for l, n in sorted(ty.items())]
+    O = U.VecOracle(xs, ys, 4, False)
+    taus = [p.shape[2] for p in O.r32]
+    ws = weights(900, taus, [6] * 5)
+    S = oracle_linear(O, ws)[2]
+    dxs, dys, dws = [U.dev(a) for a in xs], [U.dev(a) for a in ys], [U.dev(a) for a in ws]
+    outs = [torch.zeros((B, 2 * l + 1, 6), dtype=torch.complex64, device="cuda") for l in range(5)]
+    L = cabi.lib()
+    ra, xa, ya = cabi._arr(outs), cabi._arr(dxs), cabi._arr(dys)
+    n = (5, ra, len(dxs), xa, len(dys), ya)
+    small = int(L.gelib_hip_so3vec_cg_linear_workspace_bytes(*n))
+    large = int(L.gelib_hip_so3vec_cg_linear_workspace_bytes_shared(*n))
+    assert 0 < small < large
+    wp = (ctypes.c_void_p * 5)(*[w.data_ptr() for w in dws])
+    buf = torch.empty(large, dtype=torch.uint8, device="cuda")
+    got = []
+    for nbytes in (small, large, large):
+        for o in outs:
+            o.fill_(3.0)
+        cabi.check(L.gelib_hip_so3vec_cg_linear_fwd(*n, wp, 0, ctypes.c_void_p(buf.data_ptr()), nbytes, cabi._stream(outs[0])))
+        torch.cuda.synchronize()
+        got.append([U.host(o) for o in outs])
+    eps = 2.0 ** -24
+    for l in range(5):
+        assert np.array_equal(got[1][l], got[2][l])
+        d = np.abs((got[0][l] - got[1][l]).view(np.float32))
+        bound = 4 * 2 * eps * np.repeat(S[l][..., None], 2, -1).reshape(d.shape) + 1e-7
+        assert (d <= bound).all(), "l=%d: %g" % (l, float((d / bound).max()))
