@@ -3,7 +3,7 @@ of python/src/gelib/SO3partArr.py:18-234 for the CG product path.  The grid dime
 as the grid dimensions of the part descriptor (core/Gpart.hpp:416-432, 495-531); nothing is reshaped or copied."""
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch
+from gelib_amd.gelib_common import backend, common_batch, output
 from gelib_amd.SO3element import SO3element, SO3irrep
 from gelib_amd.SO3part import SO3part
 
@@ -101,8 +101,8 @@ def _part_fn(diag):
             a = x.get_adims() if isinstance(x, SO3partArr) else list(x.size()[1:x.dim() - 2])
             if diag:
                 assert x.size(-1) == y.size(-1)
-            r = SO3partArr.zeros(b, a, l, x.size(-1) if diag else x.size(-1) * y.size(-1), device=x.device)
-            getattr(_view(r), "add_" + name)(_view(x), _view(y))
+            r = SO3partArr(output([b] + list(a) + [2 * l + 1, x.size(-1) if diag else x.size(-1) * y.size(-1)], x, y))
+            getattr(_view(r), "set_" + name)(_view(x), _view(y))
             return r
 
         @staticmethod

@@ -58,6 +58,19 @@ static SO3vec<float> vec_of(const std::vector<at::Tensor> &parts) {
   return R;
 }
 
+static void spharm(SO3part<float> &r, const at::Tensor &X, const int accumulate) {
+  TORCH_CHECK(X.scalar_type() == at::kFloat, "GElib: add_spharm takes a float32 tensor of (x, y, z) vectors");
+  cnine::Gdims dims;
+  std::vector<size_t> strides;
+  for (int i = 0; i < X.dim(); i++) {
+    dims.push_back((int)X.size(i));
+    TORCH_CHECK(X.stride(i) >= 0, "GElib: negative strides are not supported");
+    strides.push_back((size_t)X.stride(i));
+  }
+  StreamGuard sg(accumulate);
+  r.add_spharm(cnine::TensorView<float>(X.data_ptr<float>(), dims, cnine::GstridesB(strides), X.is_cuda() ? 1 : 0));
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("version", []() { return std::string(_GELIB_VERSION); });
 
@@ -145,20 +158,21 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
              Gpart_add_DiagCGproduct_back1(r, g, x, offs);
            },
            py::arg("g"), py::arg("x"), py::arg("offs") = 0)
-      .def("add_spharm",
-           [](SO3part<float> &r, at::Tensor &X) {
-             TORCH_CHECK(X.scalar_type() == at::kFloat, "GElib: add_spharm takes a float32 tensor of (x, y, z) vectors");
-             cnine::Gdims dims;
-             std::vector<size_t> strides;
-             for (int i = 0; i < X.dim(); i++) {
-               dims.push_back((int)X.size(i));
-               TORCH_CHECK(X.stride(i) >= 0, "GElib: negative strides are not supported");
-               strides.push_back((size_t)X.stride(i));
-             }
-             StreamGuard sg;
-             r.add_spharm(cnine::TensorView<float>(X.data_ptr<float>(), dims, cnine::GstridesB(strides), X.is_cuda() ? 1 : 0));
+      // Written into an uninitialised part (no zero-fill, no read of r); no counterpart in the reference.
+      .def("set_CGproduct",
+           [](SO3part<float> &r, const SO3part<float> &x, const SO3part<float> &y) {
+             StreamGuard g(0);
+             Gpart_add_CGproduct(r, x, y, 0);
            },
-           py::arg("X"))
+           py::arg("x"), py::arg("y"))
+      .def("set_DiagCGproduct",
+           [](SO3part<float> &r, const SO3part<float> &x, const SO3part<float> &y) {
+             StreamGuard g(0);
+             Gpart_add_DiagCGproduct(r, x, y, 0);
+           },
+           py::arg("x"), py::arg("y"))
+      .def("add_spharm", [](SO3part<float> &r, at::Tensor &X) { spharm(r, X, 1); }, py::arg("X"))
+      .def("set_spharm", [](SO3part<float> &r, at::Tensor &X) { spharm(r, X, 0); }, py::arg("X"))
       .def("add_gather",
            [](SO3part<float> &r, at::Tensor &x, const cnine::GatherMapB &gmap, int d) {
              StreamGuard sg;

@@ -1,4 +1,13 @@
 """Helpers shared by the SO3part / SO3vec classes (python/src/gelib/gelib_common.py:15-20 in the reference)."""
+import torch
+
+
+def output(shape, x, y):
+    """The complex64 tensor that receives a product of parts x and y, on the device of x.  Every element is written by one launch, so
+    it starts uninitialised: at 65536 cells of (2, 32 channels) x (3, 32 channels) -> 4 the zero-fill and the reading of
+    what it wrote made the forward pass 3.0 ms instead of 0.9.  A product with an empty operand launches nothing."""
+    make = torch.empty if x.numel() and y.numel() else torch.zeros
+    return make(shape, dtype=torch.complex64, device=x.device)
 
 
 def common_batch(x, y):

@@ -424,7 +424,7 @@ class SO3part : public cnine::BatchedTensor<std::complex<TYPE>>, public GpartBas
         xstr[1] = (int64_t)x.strides[ng];
       }
     }
-    gelib_check(gelib_hip_so3part_spharm(&R, x.arr, xdims, xstr, 1, gelib_stream()));
+    gelib_check(gelib_hip_so3part_spharm(&R, x.arr, xdims, xstr, accumulate_mode(), gelib_stream()));
   }
 
   // ---- sums of slices along grid dimension d (core/Gpart.hpp:556-562) ----
@@ -474,7 +474,7 @@ inline void skip_on(const int rc) {
   void NAME(GPART dest, GPART a, GPART b, const int offs = 0) {                                   \
     detail::check_devices(dest, a, b);                                                            \
     auto D = dest.descriptor(), A = a.descriptor(), B = b.descriptor();                           \
-    detail::skip_on(ENTRY(&D, &A, &B, offs, 1, gelib_stream()));                                         \
+    detail::skip_on(ENTRY(&D, &A, &B, offs, accumulate_mode(), gelib_stream()));                         \
   }
 GELIB_PART_DISPATCH(Gpart_add_CGproduct, gelib_hip_so3part_cg_fwd)              // (r, x, y, offs)
 GELIB_PART_DISPATCH(Gpart_add_CGproduct_back0, gelib_hip_so3part_cg_back0)      // (xg, g, y, offs)
