@@ -75,7 +75,7 @@ class SO3partArr(torch.Tensor):
     def gather(self, gmap, dim=0):
         """Sums of cells along grid dimension dim: cell t of the result = sum of the cells s of self over the pairs
         (s, t) of gmap (python/src/gelib/SO3partArr.py:142-146)."""
-        return SO3partArr_GatherFn.apply(self, gmap, dim)
+        return SO3partArr_GatherFn.apply(gmap, dim, self)[0]
 
     def CGproduct(self, y, l):
         return SO3partArr_CGproductFn.apply(self, y, l)
@@ -124,23 +124,33 @@ SO3partArr_DiagCGproductFn = _part_fn(True)
 
 
 class SO3partArr_GatherFn(torch.autograd.Function):
-    """python/src/gelib/SO3partArr.py:236-254: forward add_gather, backward add_gather_back with the same map."""
+    """python/src/gelib/SO3partArr.py:236-254: forward add_gather, backward add_gather_back with the same map; here of all
+    parts of a vector at once (SO3vecArr.gather), each result written by the launch that sums it."""
 
     @staticmethod
-    def forward(ctx, x, gmap, d):
+    def forward(ctx, gmap, d, *xs):
         from gelib_amd.gather_map import gather_map
         assert isinstance(gmap, gather_map)
-        adims = list(x.size()[1:x.dim() - 2])
-        assert 0 <= d < len(adims) and len(adims) <= 2, "gather runs along one of at most two grid dimensions"
-        assert adims[d] == gmap.d_in()
-        ctx.gmap, ctx.d, ctx.adims = gmap, d, list(adims)
-        adims[d] = gmap.d_out()
-        r = SO3partArr.zeros(x.size(0), adims, (x.size(-2) - 1) // 2, x.size(-1), device=x.device)
-        _view(r).add_gather(x, gmap.obj, d)
-        return r
+        ctx.gmap, ctx.d, ctx.shapes = gmap, d, [list(x.size()) for x in xs]
+        ctx.set_materialize_grads(False)
+        rs = []
+        for x in xs:
+            shape = list(x.size())
+            adims = shape[1:-2]
+            assert 0 <= d < len(adims) and len(adims) <= 2, "gather runs along one of at most two grid dimensions"
+            assert adims[d] == gmap.d_in()
+            shape[1 + d] = gmap.d_out()
+            rs.append(SO3partArr(torch.empty(shape, dtype=torch.complex64, device=x.device)))
+        backend().SO3part.set_gather(rs, list(xs), gmap.obj, d, False)
+        return tuple(rs)
 
     @staticmethod
-    def backward(ctx, rg):
-        xg = SO3partArr.zeros(rg.size(0), ctx.adims, (rg.size(-2) - 1) // 2, rg.size(-1), device=rg.device)
-        _view(xg).add_gather_back(rg.contiguous(), ctx.gmap.obj, ctx.d)
-        return xg, None, None
+    def backward(ctx, *rgs):
+        used = [i for i, g in enumerate(rgs) if g is not None]
+        xgs = [None] * len(rgs)
+        for i in used:
+            shape = [rgs[i].size(0)] + ctx.shapes[i][1:]
+            xgs[i] = SO3partArr(torch.empty(shape, dtype=torch.complex64, device=rgs[i].device))
+        if used:
+            backend().SO3part.set_gather([xgs[i] for i in used], [rgs[i].contiguous() for i in used], ctx.gmap.obj, ctx.d, True)
+        return tuple([None, None] + xgs)

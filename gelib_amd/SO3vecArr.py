@@ -5,7 +5,7 @@ import torch
 
 from gelib_amd.SO3weights import mix_channels
 from gelib_amd.gelib_common import backend
-from gelib_amd.SO3partArr import SO3partArr
+from gelib_amd.SO3partArr import SO3partArr, SO3partArr_GatherFn
 from gelib_amd.SO3vec import _product_fn
 
 
@@ -91,8 +91,12 @@ class SO3vecArr:
         return r
 
     def gather(self, gmap, dim=0):
-        """Part by part (python/src/gelib/SO3vecArr.py:230-234)."""
-        return SO3vecArr(*[SO3partArr(p).gather(gmap, dim) for p in self.parts.values()])
+        """Every part (python/src/gelib/SO3vecArr.py:230-234), all of them in one launch where they either all need a gradient
+        or none does."""
+        parts = [SO3partArr(p) for p in self.parts.values()]
+        if parts and len({(p.requires_grad, p.device) for p in parts}) == 1:
+            return SO3vecArr(*SO3partArr_GatherFn.apply(gmap, dim, *parts))
+        return SO3vecArr(*[p.gather(gmap, dim) for p in parts])
 
     def odot(self, y):
         assert list(self.parts.keys()) == list(y.parts.keys())

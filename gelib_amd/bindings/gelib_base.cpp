@@ -185,6 +185,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
              xg.add_gather_back(SO3part<float>(view_of(rg)), gmap, d);
            },
            py::arg("rg"), py::arg("gmap"), py::arg("d") = 0)
+      // r[i] = x[i] gathered along grid dimension d, for all parts of a vector; back: with the map read backwards
+      .def_static("set_gather",
+                  [](const std::vector<at::Tensor> &r, const std::vector<at::Tensor> &x, const cnine::GatherMapB &gmap, int d,
+                     bool back) {
+                    std::vector<SO3part<float>> R, X;
+                    for (auto &t : r) R.push_back(SO3part<float>(view_of(t)));
+                    for (auto &t : x) X.push_back(SO3part<float>(view_of(t)));
+                    gmap.device_handle();  // made on the caller's map, which the reversed copy below shares
+                    StreamGuard sg(0);
+                    SO3part<float>::gather_parts(R, X, back ? gmap.inv() : gmap, d);
+                  },
+                  py::arg("r"), py::arg("x"), py::arg("gmap"), py::arg("d"), py::arg("back"))
       .def("getl", &SO3part<float>::getl)
       .def("getn", &SO3part<float>::getn)
       .def("str", &SO3part<float>::str, py::arg("indent") = "")

@@ -20,7 +20,7 @@ SYMBOLS = [
     "gelib_hip_gather_map_destroy", "gelib_hip_part_gather", "gelib_hip_part_mix_channels",
     "gelib_hip_part_mix_channels_static", "gelib_hip_part_mix_channels_wgrad", "gelib_hip_part_mix_workspace_bytes",
     "gelib_hip_so3vec_cg_linear_fwd", "gelib_hip_so3vec_cg_linear_workspace_bytes",
-    "gelib_hip_so3vec_cg_linear_workspace_bytes_shared",
+    "gelib_hip_so3vec_cg_linear_workspace_bytes_shared", "gelib_hip_vec_gather",
     "gelib_hip_so3vec_cg_linear_bwd", "gelib_hip_so3vec_cg_linear_bwd_workspace_bytes",
     "gelib_hip_set_option", "gelib_hip_set_stream_workspace",
     "gelib_hip_last_path",
@@ -74,6 +74,8 @@ def lib():
         L.gelib_hip_gather_map_destroy.argtypes = [ctypes.c_void_p]
         L.gelib_hip_part_gather.argtypes = [P, P, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                             ctypes.c_void_p]
+        L.gelib_hip_vec_gather.argtypes = [ctypes.c_int, P, P, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                           ctypes.c_void_p]
         L.gelib_hip_part_mix_channels.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
                                                   ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int64,
                                                   ctypes.c_int, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p]
@@ -307,6 +309,12 @@ def part_gather(r, x, gmap, dim, inverse=False, accumulate=True):
     5-D views; inverse swaps the roles of sources and targets."""
     check(lib().gelib_hip_part_gather(ctypes.byref(desc(r)), ctypes.byref(desc(x)), gmap.handle, int(dim), int(inverse),
                                       int(accumulate), _stream(r)))
+
+
+def vec_gather(rs, xs, gmap, dim, inverse=False, accumulate=True):
+    """part_gather of every x in xs into the r of rs at its place, in one launch where the layouts allow."""
+    check(lib().gelib_hip_vec_gather(len(rs), _arr(rs), _arr(xs), gmap.handle, int(dim), int(inverse), int(accumulate),
+                                     _stream(rs[0])))
 
 
 def mix_channels_ok(x):

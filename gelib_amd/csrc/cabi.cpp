@@ -1348,40 +1348,54 @@ int gelib_hip_gather_map_destroy(void *map) {
   return GELIB_HIP_OK;
 }
 
-int gelib_hip_part_gather(const gelib_part_desc *r, const gelib_part_desc *x, const void *map, int dim, int inverse,
-                          int accumulate, void *stream) {
+int gelib_hip_vec_gather(int nparts, const gelib_part_desc *r, const gelib_part_desc *x, const void *map, int dim,
+                         int inverse, int accumulate, void *stream) {
   t_last_path = kPathNone;
   const GatherMap *m = (const GatherMap *)map;
   if (!m) return GELIB_HIP_ERR_NULL;
-  View R, X;
-  int rc;
-  if ((rc = check_desc(r, R)) || (rc = check_desc(x, X))) return rc;
-  if (dim < 0 || dim > 2) return GELIB_HIP_ERR_ARG;
+  if (nparts < 0) return GELIB_HIP_ERR_ARG;
+  if (nparts > 0 && (!r || !x)) return GELIB_HIP_ERR_NULL;
   const int dir = inverse ? 1 : 0;
   const int n_from = inverse ? m->n_out : m->n_in, n_to = inverse ? m->n_in : m->n_out;
-  for (int k = 0; k < 5; k++) {
-    if (k == dim) {
-      if (x->dims[k] != n_from || r->dims[k] != n_to) return k == 0 ? GELIB_HIP_ERR_BATCH : GELIB_HIP_ERR_GRID;
-    } else if (x->dims[k] != r->dims[k]) {
-      return k == 0 ? GELIB_HIP_ERR_BATCH : (k < 3 ? GELIB_HIP_ERR_GRID : GELIB_HIP_ERR_CHANNELS);
+  std::vector<GatherJob> jobs;
+  for (int i = 0; i < nparts; i++) {
+    View R, X;
+    int rc;
+    if ((rc = check_desc(&r[i], R)) || (rc = check_desc(&x[i], X))) return rc;
+    if (dim < 0 || dim > 2) return GELIB_HIP_ERR_ARG;
+    for (int k = 0; k < 5; k++) {
+      if (k == dim) {
+        if (x[i].dims[k] != n_from || r[i].dims[k] != n_to) return k == 0 ? GELIB_HIP_ERR_BATCH : GELIB_HIP_ERR_GRID;
+      } else if (x[i].dims[k] != r[i].dims[k]) {
+        return k == 0 ? GELIB_HIP_ERR_BATCH : (k < 3 ? GELIB_HIP_ERR_GRID : GELIB_HIP_ERR_CHANNELS);
+      }
     }
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev != m->device) return GELIB_HIP_ERR_DEVICE;
+    GatherJob j;
+    long long total = 1;
+    for (int k = 0; k < 5; k++) {
+      j.D[k] = r[i].dims[k];
+      j.rs[k] = r[i].strides[k];
+      j.xs[k] = x[i].strides[k];
+      total *= j.D[k];
+      if (r[i].dims[k] > 1 && r[i].strides[k] == 0) return GELIB_HIP_ERR_BROADCAST_DEST;
+    }
+    if (total == 0) continue;
+    if (!r[i].ptr || (!x[i].ptr && n_from > 0)) return GELIB_HIP_ERR_NULL;
+    if ((rc = check_pointer(&r[i])) || (rc = check_pointer(&x[i]))) return rc;
+    j.r = (float2 *)r[i].ptr;
+    j.x = (const float2 *)x[i].ptr;
+    jobs.push_back(j);
   }
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev != m->device) return GELIB_HIP_ERR_DEVICE;
-  long long D[5], rs[5], xs[5], total = 1;
-  for (int k = 0; k < 5; k++) {
-    D[k] = r->dims[k];
-    rs[k] = r->strides[k];
-    xs[k] = x->strides[k];
-    total *= D[k];
-    if (r->dims[k] > 1 && r->strides[k] == 0) return GELIB_HIP_ERR_BROADCAST_DEST;
-  }
-  if (total == 0) return GELIB_HIP_OK;
-  if (!r->ptr || (!x->ptr && n_from > 0)) return GELIB_HIP_ERR_NULL;
-  if ((rc = check_pointer(r)) || (rc = check_pointer(x))) return rc;
+  if (jobs.empty()) return GELIB_HIP_OK;
   t_last_path = kPathGeneric;
-  return launch_gather((float2 *)r->ptr, (const float2 *)x->ptr, rs, xs, D, dim, m->rows[dir], m->cols[dir],
-                       accumulate != 0, (hipStream_t)stream);
+  return launch_gather(jobs, dim, m->rows[dir], m->cols[dir], accumulate != 0, (hipStream_t)stream);
+}
+
+int gelib_hip_part_gather(const gelib_part_desc *r, const gelib_part_desc *x, const void *map, int dim, int inverse,
+                          int accumulate, void *stream) {
+  return gelib_hip_vec_gather(1, r, x, map, dim, inverse, accumulate, stream);
 }
 
 // ---- channel mixing (the linear layer that consumes a product) ------------------------------------------------------

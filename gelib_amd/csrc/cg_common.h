@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <mutex>
+#include <vector>
 
 #include "gelib_hip.h"
 
@@ -75,8 +76,13 @@ int launch_spharm(const PartDev &r, const float *x, const long long xs[5], const
                   bool accumulate, hipStream_t s);
 
 // ---- sum of slices along one leading dimension (gather.hip): r[.., t, ..] (+)= sum_{k in row t} x[.., sources[k], ..] ----
-int launch_gather(float2 *r, const float2 *x, const long long rs[5], const long long xs[5], const long long D[5], int dim,
-                  const int *row_ptr, const int *sources, bool accumulate, hipStream_t s);
+struct GatherJob {   // one part: strides in complex elements over (batch, grid0, grid1, m, channel), extents of r (none 0)
+  float2 *r;
+  const float2 *x;
+  long long rs[5], xs[5], D[5];
+};
+int launch_gather(const std::vector<GatherJob> &jobs, int dim, const int *row_ptr, const int *sources, bool accumulate,
+                  hipStream_t s);
 
 // ---- channel mixing on the matrix cores (mix.hip): r[row, :] = x[row, :] V, V = W (n_in, n_out) or W^H for W (n_out, n_in);
 // strides in complex elements.  Returns 0, 10 (a HIP call failed), 11 (n_in odd or rows of x not 16-byte aligned) or 13

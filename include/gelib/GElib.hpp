@@ -428,15 +428,23 @@ class SO3part : public cnine::BatchedTensor<std::complex<TYPE>>, public GpartBas
   }
 
   // ---- sums of slices along grid dimension d (core/Gpart.hpp:556-562) ----
-  void add_gather(const SO3part &x, const cnine::GatherMapB &gmap, const int d = 0) const {
-    GELIB_ASSRT(x.dev == dev);
-    if (dev != 1) GELIB_ERROR("SO3part::add_gather: the operands must be on GPU");
-    GELIB_ASSRT(ndims() <= 5 && x.ndims() == ndims());
-    GELIB_ASSRT(d >= 0 && d < ndims() - 3);
-    GELIB_ASSRT(gmap.d_in() == x.dims[d + 1]);
-    GELIB_ASSRT(gmap.d_out() == dims[d + 1]);
-    auto R = descriptor(), X = x.descriptor();
-    gelib_check(gelib_hip_part_gather(&R, &X, gmap.device_handle(), d + 1, gmap.inverted ? 1 : 0, 1, gelib_stream()));
+  void add_gather(const SO3part &x, const cnine::GatherMapB &gmap, const int d = 0) const { gather_parts({*this}, {x}, gmap, d); }
+  // r[i] (+)= x[i] gathered, for several parts in one call (parts of ordinary layout share a launch)
+  static void gather_parts(const std::vector<SO3part> &r, const std::vector<SO3part> &x, const cnine::GatherMapB &gmap, const int d) {
+    GELIB_ASSRT(r.size() == x.size());
+    std::vector<gelib_part_desc> R, X;
+    for (size_t i = 0; i < r.size(); i++) {
+      GELIB_ASSRT(x[i].dev == r[i].dev);
+      if (r[i].dev != 1) GELIB_ERROR("SO3part::add_gather: the operands must be on GPU");
+      GELIB_ASSRT(r[i].ndims() <= 5 && x[i].ndims() == r[i].ndims());
+      GELIB_ASSRT(d >= 0 && d < r[i].ndims() - 3);
+      GELIB_ASSRT(gmap.d_in() == x[i].dims[d + 1]);
+      GELIB_ASSRT(gmap.d_out() == r[i].dims[d + 1]);
+      R.push_back(r[i].descriptor());
+      X.push_back(x[i].descriptor());
+    }
+    gelib_check(gelib_hip_vec_gather((int)R.size(), R.data(), X.data(), gmap.device_handle(), d + 1, gmap.inverted ? 1 : 0,
+                                     accumulate_mode(), gelib_stream()));
   }
   void add_gather_back(const SO3part &r, const cnine::GatherMapB &gmap, const int d = 0) const {
     gmap.device_handle();  // made on the caller's map, so the reversed copy below shares it instead of uploading,

@@ -261,6 +261,10 @@ int gelib_hip_gather_map_destroy(void *map);
  */
 int gelib_hip_part_gather(const gelib_part_desc *r, const gelib_part_desc *x, const void *map, int dim, int inverse,
                           int accumulate, void *stream);
+/* The same for nparts parts along the same dimension of the same map, in one launch for up to eight parts of ordinary
+ * layout (r[i] from x[i]); nothing is launched when one of them is refused. */
+int gelib_hip_vec_gather(int nparts, const gelib_part_desc *r, const gelib_part_desc *x, const void *map, int dim,
+                         int inverse, int accumulate, void *stream);
 
 /*
  * Device memory helpers for host code that does not include the HIP headers itself (the C++ mirror of the

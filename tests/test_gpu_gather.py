@@ -124,3 +124,50 @@ def test_python_gather_and_its_gradient(G):
     wr = u.apply(R).gather(G.gather_map.random(3, 5, 0.5, seed=9), 1)
     for l in w.parts:
         assert torch.allclose(w.apply(R).parts[l], wr.parts[l], rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("shape,dim,n_out,k", [
+    ((1, 70, 5, 8), 1, 33, 300),       # 16 bytes a thread
+    ((1, 70, 5, 3), 1, 33, 300),       # an odd slice: 8 bytes a thread
+    ((3, 50, 3, 1), 1, 41, 200),       # an outer dimension, short slices
+    ((2, 3, 20, 1, 2), 2, 31, 90),     # two outer dimensions that nest
+    ((33, 1, 64), 0, 257, 1100),       # along the batch, several blocks
+])
+def test_vec_gather_of_parts_with_other_layouts(G, shape, dim, n_out, k):
+    """One call for three parts: as it is, 8 bytes past 16-byte alignment, and with strides that nest in no slice."""
+    from gelib_amd import cabi
+    src, tgt = random_pairs(shape[dim], n_out, k, 12)
+    gm = cabi.GatherMap(src, tgt, shape[dim], n_out)
+    rshape = list(shape)
+    rshape[dim] = n_out
+    x = cplx(*shape, seed=7)
+    n = x.numel()
+    odd = torch.empty(n + 1, dtype=torch.complex64, device="cuda")[1:].reshape(shape)
+    odd.copy_(x)
+    strided = torch.empty(list(shape[:-1]) + [2 * shape[-1]], dtype=torch.complex64, device="cuda")[..., ::2]
+    strided.copy_(x)
+    xs = [x.cuda(), odd, strided]
+    rs = [torch.full(rshape, 5.0, dtype=torch.complex64, device="cuda") for _ in xs]
+    cabi.vec_gather(rs, xs, gm, dim, accumulate=False)
+    want = ora.gather(x.numpy(), src, tgt, n_out, dim)
+    for r in rs:
+        assert np.array_equal(U.host(r), want)
+    many = [torch.full(rshape, 5.0, dtype=torch.complex64, device="cuda") for _ in range(11)]   # more parts than a launch takes
+    cabi.vec_gather(many, [xs[0]] * 11, gm, dim, accumulate=True)
+    for r in many:
+        assert np.array_equal(U.host(r), ora.gather(x.numpy(), src, tgt, n_out, dim, r=np.full(rshape, 5.0, np.complex64)))
+
+
+def test_vec_gather_gradients_of_some_parts(G):
+    """Gradients arrive for the parts that are used, as when every part was gathered by itself."""
+    x = [cplx(1, 9, 2 * l + 1, 4, seed=l).cuda().requires_grad_(l != 1) for l in range(3)]
+    gm = G.gather_map.sources_targets([0, 3, 3, 8], [1, 1, 0, 2], 9, 5)
+    for sel in (slice(0, 3), slice(0, 3, 2)):
+        v = G.SO3vecArr(*x[sel]).gather(gm)
+        assert [p.requires_grad for p in v.parts.values()] == [t.requires_grad for t in x[sel]]
+        got = torch.autograd.grad(torch.view_as_real(v.parts[2].as_subclass(torch.Tensor)).sum(), [x[0], x[2]], allow_unused=True)
+        assert got[0] is None
+        want = torch.zeros(9)
+        for s in (0, 3, 3, 8):
+            want[s] += 1
+        assert torch.equal(got[1].as_subclass(torch.Tensor).real.cpu(), want.reshape(1, 9, 1, 1).expand(1, 9, 5, 4))
