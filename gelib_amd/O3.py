@@ -5,8 +5,8 @@ O(3) adds nothing to the arithmetic: a product of parts with parities p1, p2 is 
 (O3/O3group.hpp:38-53, O3/O3part.hpp:214-269 forward every kernel to SO3part).  So these classes only keep the labels,
 check the parity rule and enumerate the (mu1, mu2, mu) triples of a vector product in the reference's order -- parts
 sorted by the index 2l + (p == -1) (O3/O3index.hpp:28-31), then l ascending, each block at the running channel offset
-of its output part (core/Gvec.hpp:311-321) -- and call the part-level HIP entry points with those offsets.  There is
-one launch per triple, as in the reference; the fused single-launch kernels take one part per l and are not used here.
+of its output part (core/Gvec.hpp:311-321) -- which the library does (gelib_hip_o3vec_cg_fwd / _bwd): one launch of the
+fused kernels per pair of parities.
 """
 import torch
 
@@ -154,23 +154,6 @@ def _part_product(x, y, mu, diag):
     return O3part(fn.apply(_plain(x), _plain(y), mu[0]), mu)
 
 
-def _triples(xmus, ymus, rmus, ns_x, ns_y, diag):
-    """(xi, yi, ri, offs) in the reference's order; offs = running channel offset inside output part ri."""
-    offs = [0] * len(rmus)
-    where = {mu: k for k, mu in enumerate(rmus)}
-    out = []
-    for xi, mu1 in enumerate(xmus):
-        for yi, mu2 in enumerate(ymus):
-            for l in range(abs(mu1[0] - mu2[0]), mu1[0] + mu2[0] + 1):
-                mu = (l, mu1[1] * mu2[1])
-                if mu not in where:
-                    continue
-                ri = where[mu]
-                out.append((xi, yi, ri, offs[ri]))
-                offs[ri] += ns_x[xi] if diag else ns_x[xi] * ns_y[yi]
-    return out
-
-
 def _vec_fn(diag):
     name = "DiagCGproduct" if diag else "CGproduct"
 
@@ -184,13 +167,15 @@ def _vec_fn(diag):
             tau = getattr(O3type({mu: t.size(-1) for mu, t in zip(xmus, xs)}), name)(
                 O3type({mu: t.size(-1) for mu, t in zip(ymus, ys)}), maxl)
             b = common_batch(xs[0], ys[0])
-            rmus = list(tau)
-            rs = [torch.zeros([b, 2 * mu[0] + 1, n], dtype=torch.complex64, device=xs[0].device) for mu, n in tau.items()]
-            ctx.triples = _triples(xmus, ymus, rmus, [t.size(-1) for t in xs], [t.size(-1) for t in ys], diag)
-            ctx.k1, ctx.rmus = k1, rmus
+            # every channel of every part is written by one launch; a product with an empty operand launches nothing
+            make = torch.empty if all(t.numel() for t in args) else torch.zeros
+            rs = [make([b, 2 * mu[0] + 1, n], dtype=torch.complex64, device=xs[0].device) for mu, n in tau.items()]
+            ctx.k1 = k1
+            ctx.ps = [[mu[1] for mu in mus] for mus in (tau, xmus, ymus)]
             ctx.save_for_backward(*args)
-            for xi, yi, ri, offs in ctx.triples:
-                getattr(gb.SO3part.view(rs[ri]), "add_" + name)(gb.SO3part.view(xs[xi]), gb.SO3part.view(ys[yi]), offs)
+            if rs:
+                rp, xp, yp = ctx.ps
+                gb.o3vec_product(diag, rs, rp, list(xs), xp, list(ys), yp)
             return tuple(rs)
 
         @staticmethod
@@ -198,13 +183,11 @@ def _vec_fn(diag):
             gb = backend()
             saved = ctx.saved_tensors
             xs, ys = saved[:ctx.k1], saved[ctx.k1:]
-            gs = [g.contiguous() for g in gs]
-            xgs = [torch.zeros_like(t) for t in xs]
-            ygs = [torch.zeros_like(t) for t in ys]
-            for xi, yi, ri, offs in ctx.triples:
-                G = gb.SO3part.view(gs[ri])
-                getattr(gb.SO3part.view(xgs[xi]), "add_%s_back0" % name)(G, gb.SO3part.view(ys[yi]), offs)
-                getattr(gb.SO3part.view(ygs[yi]), "add_%s_back1" % name)(G, gb.SO3part.view(xs[xi]), offs)
+            make = torch.empty_like if all(t.numel() for t in saved) else torch.zeros_like
+            xgs = [make(t, memory_format=torch.contiguous_format) for t in xs]
+            ygs = [make(t, memory_format=torch.contiguous_format) for t in ys]
+            gp, xp, yp = ctx.ps
+            gb.o3vec_product_back(diag, xgs, ygs, [g.contiguous() for g in gs], gp, list(xs), xp, list(ys), yp)
             return tuple([None, None, None] + xgs + ygs)
 
     Fn.__name__ = "O3vec_%sFn" % name

@@ -71,6 +71,16 @@ static void spharm(SO3part<float> &r, const at::Tensor &X, const int accumulate)
   r.add_spharm(cnine::TensorView<float>(X.data_ptr<float>(), dims, cnine::GstridesB(strides), X.is_cuda() ? 1 : 0));
 }
 
+static std::vector<gelib_part_desc> parts_on_gpu(const std::vector<at::Tensor> &v) {
+  std::vector<gelib_part_desc> d;
+  for (auto &t : v) {
+    SO3part<float> P(view_of(t));
+    if (P.get_dev() != 1) GELIB_ERROR("SO3part must be on GPU: products of host parts are not part of this build");
+    d.push_back(P.descriptor());
+  }
+  return d;
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("version", []() { return std::string(_GELIB_VERSION); });
 
@@ -217,6 +227,29 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     Gpart_add_CGproduct(SO3part<float>(view_of(r)), X, Y, 0);
     return r;
   });
+
+  // Products of parts labelled (l, p), p = +1 / -1, written into uninitialised parts, and both gradients of them
+  m.def("o3vec_product",
+        [](bool diag, const std::vector<at::Tensor> &r, const std::vector<int> &rp, const std::vector<at::Tensor> &x,
+           const std::vector<int> &xp, const std::vector<at::Tensor> &y, const std::vector<int> &yp) {
+          GELIB_ASSRT(r.size() == rp.size() && x.size() == xp.size() && y.size() == yp.size());
+          auto R = parts_on_gpu(r), X = parts_on_gpu(x), Y = parts_on_gpu(y);
+          StreamGuard g(0);
+          GElib::detail::skip_on(gelib_hip_o3vec_cg_fwd(diag, (int)R.size(), R.data(), rp.data(), (int)X.size(), X.data(), xp.data(),
+                                                 (int)Y.size(), Y.data(), yp.data(), accumulate_mode(), gelib_stream()));
+        });
+  m.def("o3vec_product_back",
+        [](bool diag, const std::vector<at::Tensor> &xg, const std::vector<at::Tensor> &yg, const std::vector<at::Tensor> &gr,
+           const std::vector<int> &gp, const std::vector<at::Tensor> &x, const std::vector<int> &xp,
+           const std::vector<at::Tensor> &y, const std::vector<int> &yp) {
+          GELIB_ASSRT(gr.size() == gp.size() && x.size() == xp.size() && y.size() == yp.size() && xg.size() == x.size() &&
+                      yg.size() == y.size());
+          auto XG = parts_on_gpu(xg), YG = parts_on_gpu(yg), G = parts_on_gpu(gr), X = parts_on_gpu(x), Y = parts_on_gpu(y);
+          StreamGuard g(0);
+          GElib::detail::skip_on(gelib_hip_o3vec_cg_bwd(diag, XG.data(), YG.data(), (int)G.size(), G.data(), gp.data(), (int)X.size(),
+                                                 X.data(), xp.data(), (int)Y.size(), Y.data(), yp.data(), accumulate_mode(),
+                                                 gelib_stream()));
+        });
 
   py::class_<SO3vec<float>>(m, "SO3vec", "Class to store an SO(3)-covariant vector")
       .def_static("view",

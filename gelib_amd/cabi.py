@@ -21,6 +21,7 @@ SYMBOLS = [
     "gelib_hip_part_mix_channels_static", "gelib_hip_part_mix_channels_wgrad", "gelib_hip_part_mix_workspace_bytes",
     "gelib_hip_so3vec_cg_linear_fwd", "gelib_hip_so3vec_cg_linear_workspace_bytes",
     "gelib_hip_so3vec_cg_linear_workspace_bytes_shared", "gelib_hip_vec_gather",
+    "gelib_hip_o3vec_cg_fwd", "gelib_hip_o3vec_cg_bwd",
     "gelib_hip_so3vec_cg_linear_bwd", "gelib_hip_so3vec_cg_linear_bwd_workspace_bytes",
     "gelib_hip_set_option", "gelib_hip_set_stream_workspace",
     "gelib_hip_last_path",
@@ -74,6 +75,9 @@ def lib():
         L.gelib_hip_gather_map_destroy.argtypes = [ctypes.c_void_p]
         L.gelib_hip_part_gather.argtypes = [P, P, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                             ctypes.c_void_p]
+        I = ctypes.POINTER(ctypes.c_int)
+        L.gelib_hip_o3vec_cg_fwd.argtypes = [ctypes.c_int] + [ctypes.c_int, P, I] * 3 + [ctypes.c_int, ctypes.c_void_p]
+        L.gelib_hip_o3vec_cg_bwd.argtypes = [ctypes.c_int, P, P] + [ctypes.c_int, P, I] * 3 + [ctypes.c_int, ctypes.c_void_p]
         L.gelib_hip_vec_gather.argtypes = [ctypes.c_int, P, P, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                            ctypes.c_void_p]
         L.gelib_hip_part_mix_channels.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
@@ -206,6 +210,24 @@ def so3vec_bwd(xgparts, ygparts, gparts, xparts, yparts, accumulate=True, diag=F
     fn = lib().gelib_hip_so3vec_diagcg_bwd if diag else lib().gelib_hip_so3vec_cg_bwd
     check(fn(_arr(xgparts), _arr(ygparts), len(gparts), _arr(gparts), len(xparts), _arr(xparts), len(yparts),
              _arr(yparts), int(accumulate), _stream(gparts[0])))
+
+
+def _parities(ps):
+    return (ctypes.c_int * max(len(ps), 1))(*ps)
+
+
+def o3vec_fwd(rparts, rp, xparts, xp, yparts, yp, accumulate=True, diag=False):
+    """The product of parts labelled by parities xp, yp (+1 / -1) into those of rparts labelled rp."""
+    check(lib().gelib_hip_o3vec_cg_fwd(int(diag), len(rparts), _arr(rparts), _parities(rp), len(xparts), _arr(xparts),
+                                       _parities(xp), len(yparts), _arr(yparts), _parities(yp), int(accumulate),
+                                       _stream(rparts[0])))
+
+
+def o3vec_bwd(xgparts, ygparts, gparts, gp, xparts, xp, yparts, yp, accumulate=True, diag=False):
+    """Its gradients; either gradient list may be None to skip it."""
+    check(lib().gelib_hip_o3vec_cg_bwd(int(diag), _arr(xgparts), _arr(ygparts), len(gparts), _arr(gparts), _parities(gp),
+                                       len(xparts), _arr(xparts), _parities(xp), len(yparts), _arr(yparts), _parities(yp),
+                                       int(accumulate), _stream(gparts[0])))
 
 
 UNSUPPORTED = 15

@@ -622,6 +622,30 @@ int fwd_dispatch(const VecPlan &plan, const std::vector<View> &R, const std::vec
   return GELIB_HIP_OK;
 }
 
+// A validated product: Diag products that reach above l = 6 are split, everything else goes to the families in order.
+int fwd_planned(const VecPlan &plan, const std::vector<View> &R, const std::vector<View> &X, const std::vector<View> &Y,
+                int accumulate, hipStream_t s) {
+  int rc;
+  if (!g_force_generic) {
+    VecPlan A, B;
+    std::vector<View> RA, RB;
+    if (split_diag(plan, R, X, Y, A, B, RA, RB, true)) {
+      std::vector<const gelib_part_desc *> rd, xd, yd;
+      for (auto &v : RA) rd.push_back(v.d);
+      for (auto &v : X) xd.push_back(v.d);
+      for (auto &v : Y) yd.push_back(v.d);
+      int used = 0;
+      if ((rc = diag6_vec_fwd(A, rd, xd, yd, accumulate != 0, s, &used))) return rc;
+      if (used) {
+        rc = fwd_dispatch(B, RB, X, Y, accumulate, s);
+        t_last_path = kPathDiag6;
+        return rc;
+      }
+    }
+  }
+  return fwd_dispatch(plan, R, X, Y, accumulate, s);
+}
+
 int vec_fwd_entry(bool diag, int nr, const gelib_part_desc *r, int nx, const gelib_part_desc *x, int ny,
                   const gelib_part_desc *y, int accumulate, void *stream) {
   t_last_path = kPathNone;
@@ -642,25 +666,7 @@ int vec_fwd_entry(bool diag, int nr, const gelib_part_desc *r, int nx, const gel
   for (auto &v : Y)
     if ((rc = check_pointer(v.d))) return rc;
   if (plan.E[0] * plan.E[1] * plan.E[2] == 0 || plan.triples.empty()) return GELIB_HIP_OK;
-  hipStream_t s = (hipStream_t)stream;
-  if (!g_force_generic) {
-    VecPlan A, B;
-    std::vector<View> RA, RB;
-    if (split_diag(plan, R, X, Y, A, B, RA, RB, true)) {
-      std::vector<const gelib_part_desc *> rd, xd, yd;
-      for (auto &v : RA) rd.push_back(v.d);
-      for (auto &v : X) xd.push_back(v.d);
-      for (auto &v : Y) yd.push_back(v.d);
-      int used = 0;
-      if ((rc = diag6_vec_fwd(A, rd, xd, yd, accumulate != 0, s, &used))) return rc;
-      if (used) {
-        rc = fwd_dispatch(B, RB, X, Y, accumulate, s);
-        t_last_path = kPathDiag6;
-        return rc;
-      }
-    }
-  }
-  return fwd_dispatch(plan, R, X, Y, accumulate, s);
+  return fwd_planned(plan, R, X, Y, accumulate, (hipStream_t)stream);
 }
 
 // Vectors of several parts with l above 7: one launch of the single-pair kernels per (x part, y part) pair, each adding
@@ -798,6 +804,35 @@ int bwd_dispatch(const VecPlan &plan, const std::vector<View> &G, const std::vec
   return GELIB_HIP_OK;
 }
 
+int bwd_planned(const VecPlan &plan, const std::vector<View> &G, const std::vector<View> &X, const std::vector<View> &Y,
+                const std::vector<View> &XG, const std::vector<View> &YG, bool want_x, bool want_y, int accumulate,
+                hipStream_t s) {
+  int rc;
+  if (!g_force_generic) {
+    VecPlan A, B;
+    std::vector<View> GA, GB;
+    if (split_diag(plan, G, X, Y, A, B, GA, GB)) {
+      std::vector<const gelib_part_desc *> gd, xd, yd, xgd, ygd;
+      for (auto &v : GA) gd.push_back(v.d);
+      for (auto &v : X) xd.push_back(v.d);
+      for (auto &v : Y) yd.push_back(v.d);
+      for (auto &v : XG) xgd.push_back(v.d);
+      for (auto &v : YG) ygd.push_back(v.d);
+      int used = 0;
+      if ((rc = diag6_vec_bwd(A, gd, xd, yd, xgd, ygd, accumulate != 0, s, &used))) return rc;
+      if (used) {
+        // The rest adds on top of what the first part wrote.  It is a few triples of a vector with many parts: the
+        // unrolled backward kernels stage and flush the images of all parts per cell whatever the number of triples
+        // (39 ms against 18 ms on Diag L=4, 64 channels, 131072 cells, uncapped), so they are passed over here.
+        rc = bwd_dispatch(B, GB, X, Y, XG, YG, want_x, want_y, 1, s, true);
+        t_last_path = kPathDiag6;
+        return rc;
+      }
+    }
+  }
+  return bwd_dispatch(plan, G, X, Y, XG, YG, want_x, want_y, accumulate, s);
+}
+
 int vec_bwd_entry(bool diag, const gelib_part_desc *xg, const gelib_part_desc *yg, int ng, const gelib_part_desc *g,
                   int nx, const gelib_part_desc *x, int ny, const gelib_part_desc *y, int accumulate, void *stream) {
   t_last_path = kPathNone;
@@ -859,29 +894,191 @@ int vec_bwd_entry(bool diag, const gelib_part_desc *xg, const gelib_part_desc *y
       // broadcasts, and the shape-agnostic kernels sum it serially
     }
   }
-  if (!g_force_generic) {
-    VecPlan A, B;
-    std::vector<View> GA, GB;
-    if (split_diag(plan, G, X, Y, A, B, GA, GB)) {
-      std::vector<const gelib_part_desc *> gd, xd, yd, xgd, ygd;
-      for (auto &v : GA) gd.push_back(v.d);
-      for (auto &v : X) xd.push_back(v.d);
-      for (auto &v : Y) yd.push_back(v.d);
-      for (auto &v : XG) xgd.push_back(v.d);
-      for (auto &v : YG) ygd.push_back(v.d);
-      int used = 0;
-      if ((rc = diag6_vec_bwd(A, gd, xd, yd, xgd, ygd, accumulate != 0, s, &used))) return rc;
-      if (used) {
-        // The rest adds on top of what the first part wrote.  It is a few triples of a vector with many parts: the
-        // unrolled backward kernels stage and flush the images of all parts per cell whatever the number of triples
-        // (39 ms against 18 ms on Diag L=4, 64 channels, 131072 cells, uncapped), so they are passed over here.
-        rc = bwd_dispatch(B, GB, X, Y, XG, YG, xg != nullptr, yg != nullptr, 1, s, true);
-        t_last_path = kPathDiag6;
-        return rc;
-      }
+  return bwd_planned(plan, G, X, Y, XG, YG, xg != nullptr, yg != nullptr, accumulate, s);
+}
+
+// ---- vectors with two parts per l, told apart by a parity ---------------------------------------------------------
+// A part (l, p), p = +1 or -1; a product of parities p1, p2 has parity p1 p2 (O3/O3group.hpp:38-53).  Blocks lie in the
+// product parts in the order of x parts by 2l + (p == -1), then y parts in that order, then l (O3/O3index.hpp:28-31,
+// core/Gvec.hpp:311-321).  For each of the four pairs of parities the parts are vectors with one part per l, and the
+// kernels for those take their product as it stands, the blocks at the offsets counted here: four launches where the
+// reference has one per (mu1, mu2, mu).
+struct ParityViews {
+  std::vector<View> p[2];           // [0]: parity +1, [1]: -1, each sorted by l
+  std::vector<std::pair<int, int>> order;   // (parity index, position in p[..]) of every part by 2l + (p == -1)
+};
+
+int split_parities(int n, const gelib_part_desc *parts, const int *parity, int max_parts, ParityViews &out) {
+  if (n < 0) return GELIB_HIP_ERR_PARTS;
+  if (n > 0 && (!parts || !parity)) return GELIB_HIP_ERR_NULL;
+  for (int i = 0; i < n; i++) {
+    if (parity[i] != 1 && parity[i] != -1) return GELIB_HIP_ERR_ARG;
+    View v;
+    int rc = check_desc(&parts[i], v);
+    if (rc) return rc;
+    out.p[parity[i] < 0].push_back(v);
+  }
+  for (int q = 0; q < 2; q++) {
+    auto &L = out.p[q];
+    if ((int)L.size() > max_parts) return GELIB_HIP_ERR_PARTS;
+    std::sort(L.begin(), L.end(), [](const View &a, const View &b) { return a.l < b.l; });
+    for (size_t i = 1; i < L.size(); i++)
+      if (L[i].l == L[i - 1].l) return GELIB_HIP_ERR_PARTS;
+    for (size_t i = 0; i < L.size(); i++) out.order.push_back({q, (int)i});
+  }
+  std::sort(out.order.begin(), out.order.end(), [&](const std::pair<int, int> &a, const std::pair<int, int> &b) {
+    return 2 * out.p[a.first][a.second].l + a.first < 2 * out.p[b.first][b.second].l + b.first;
+  });
+  return GELIB_HIP_OK;
+}
+
+// The four products [p1][p2] with the offsets of the whole one.
+int build_parity_plans(bool diag, const ParityViews &R, const ParityViews &X, const ParityViews &Y, const long long E[3],
+                       VecPlan plans[2][2]) {
+  for (int k = 0; k < 4; k++) {
+    plans[k >> 1][k & 1].diag = diag;
+    for (int d = 0; d < 3; d++) plans[k >> 1][k & 1].E[d] = E[d];
+  }
+  std::vector<long long> offset[2];
+  for (int q = 0; q < 2; q++) offset[q].assign(R.p[q].size(), 0);
+  for (auto &ox : X.order)
+    for (auto &oy : Y.order) {
+      const View &x = X.p[ox.first][ox.second], &y = Y.p[oy.first][oy.second];
+      if (x.l > kMaxL || y.l > kMaxL) return GELIB_HIP_ERR_PARTS;
+      const int q = ox.first ^ oy.first;
+      for (int l = std::abs(x.l - y.l); l <= x.l + y.l; l++)
+        for (size_t k = 0; k < R.p[q].size(); k++) {
+          if (R.p[q][k].l != l) continue;
+          if (diag && x.n != y.n) return GELIB_HIP_ERR_DIAG_CHANNELS;
+          const long long nout = diag ? x.n : (long long)x.n * y.n;
+          if (offset[q][k] + nout > R.p[q][k].n) return GELIB_HIP_ERR_CHANNELS;
+          plans[ox.first][oy.first].triples.push_back(
+              {ox.second, oy.second, (int)k, x.l, y.l, l, (int)offset[q][k], (int)nout});
+          offset[q][k] += nout;
+        }
+    }
+  return GELIB_HIP_OK;
+}
+
+int reconcile_views(std::initializer_list<const ParityViews *> lists, long long E[3]) {
+  std::vector<const gelib_part_desc *> all;
+  for (auto *v : lists)
+    for (auto &L : v->p)
+      for (auto &w : L) all.push_back(w.d);
+  return reconcile(all.data(), (int)all.size(), E);
+}
+
+int check_views(std::initializer_list<const ParityViews *> lists, bool dest) {
+  int rc;
+  for (auto *v : lists)
+    for (auto &L : v->p)
+      for (auto &w : L)
+        if ((rc = dest ? check_dest(w.d) : check_pointer(w.d))) return rc;
+  return GELIB_HIP_OK;
+}
+
+int o3vec_fwd_entry(bool diag, int nr, const gelib_part_desc *r, const int *rp, int nx, const gelib_part_desc *x,
+                    const int *xp, int ny, const gelib_part_desc *y, const int *yp, int accumulate, void *stream) {
+  t_last_path = kPathNone;
+  ParityViews R, X, Y;
+  int rc;
+  if ((rc = split_parities(nr, r, rp, kMaxOutParts, R)) || (rc = split_parities(nx, x, xp, kMaxParts, X)) ||
+      (rc = split_parities(ny, y, yp, kMaxParts, Y)))
+    return rc;
+  if (nr == 0 || nx == 0 || ny == 0) return GELIB_HIP_OK;
+  long long E[3];
+  if ((rc = reconcile_views({&R, &X, &Y}, E))) return rc;
+  VecPlan plans[2][2];
+  if ((rc = build_parity_plans(diag, R, X, Y, E, plans))) return rc;
+  if ((rc = check_views({&R}, true)) || (rc = check_views({&R, &X, &Y}, false))) return rc;
+  if (E[0] * E[1] * E[2] == 0) return GELIB_HIP_OK;
+  for (int k = 0; k < 4; k++) {
+    const int p1 = k >> 1, p2 = k & 1;
+    if (plans[p1][p2].triples.empty()) continue;
+    if ((rc = fwd_planned(plans[p1][p2], R.p[p1 ^ p2], X.p[p1], Y.p[p2], accumulate, (hipStream_t)stream))) return rc;
+  }
+  return GELIB_HIP_OK;
+}
+
+int o3vec_bwd_entry(bool diag, const gelib_part_desc *xg, const gelib_part_desc *yg, int ng, const gelib_part_desc *g,
+                    const int *gp, int nx, const gelib_part_desc *x, const int *xp, int ny, const gelib_part_desc *y,
+                    const int *yp, int accumulate, void *stream) {
+  t_last_path = kPathNone;
+  if (!xg && !yg) return GELIB_HIP_OK;
+  ParityViews G, X, Y, XG, YG;
+  int rc;
+  if ((rc = split_parities(ng, g, gp, kMaxOutParts, G)) || (rc = split_parities(nx, x, xp, kMaxParts, X)) ||
+      (rc = split_parities(ny, y, yp, kMaxParts, Y)) || (xg && (rc = split_parities(nx, xg, xp, kMaxParts, XG))) ||
+      (yg && (rc = split_parities(ny, yg, yp, kMaxParts, YG))))
+    return rc;
+  for (int q = 0; q < 2; q++) {
+    for (size_t i = 0; i < XG.p[q].size(); i++)
+      if (XG.p[q][i].l != X.p[q][i].l || XG.p[q][i].n != X.p[q][i].n) return GELIB_HIP_ERR_PARTS;
+    for (size_t i = 0; i < YG.p[q].size(); i++)
+      if (YG.p[q][i].l != Y.p[q][i].l || YG.p[q][i].n != Y.p[q][i].n) return GELIB_HIP_ERR_PARTS;
+  }
+  if (ng == 0 || nx == 0 || ny == 0) return GELIB_HIP_OK;
+  long long E[3];
+  if ((rc = reconcile_views({&G, &X, &Y, &XG, &YG}, E))) return rc;
+  VecPlan plans[2][2];
+  if ((rc = build_parity_plans(diag, G, X, Y, E, plans))) return rc;
+  if ((rc = check_views({&XG, &YG}, true)) || (rc = check_views({&G, &X, &Y, &XG, &YG}, false))) return rc;
+  if (E[0] * E[1] * E[2] == 0) return GELIB_HIP_OK;
+  hipStream_t s = (hipStream_t)stream;
+  if (!g_force_generic && g_bcast_reduce) {
+    std::vector<gelib_part_desc> d;
+    d.insert(d.end(), g, g + ng);
+    d.insert(d.end(), x, x + nx);
+    d.insert(d.end(), y, y + ny);
+    const int ixg = (int)d.size();
+    if (xg) d.insert(d.end(), xg, xg + nx);
+    const int iyg = (int)d.size();
+    if (yg) d.insert(d.end(), yg, yg + ny);
+    std::vector<int> dests;
+    bool bcast = false;
+    for (int i = ixg; i < (int)d.size(); i++) {
+      dests.push_back(i);
+      bcast = bcast || dest_broadcasts(&d[i], E);
+    }
+    if (bcast) {
+      rc = with_bcast_dests(d, dests, E, accumulate, s, [&](int acc) {
+        return o3vec_bwd_entry(diag, xg ? &d[ixg] : nullptr, yg ? &d[iyg] : nullptr, ng, &d[0], gp, nx, &d[ng], xp, ny,
+                               &d[ng + nx], yp, acc, stream);
+      });
+      if (rc != GELIB_HIP_ERR_UNSUPPORTED) return rc;   // otherwise no scratch (recorded into a graph): summed serially below
     }
   }
-  return bwd_dispatch(plan, G, X, Y, XG, YG, xg != nullptr, yg != nullptr, accumulate, s);
+  // The first product that feeds a destination writes it, later ones add: (+,+) and (-,-) touch every destination once
+  // where both operands have both parities, (+,-) and (-,+) add.
+  bool done_x[2] = {accumulate != 0, accumulate != 0}, done_y[2] = {accumulate != 0, accumulate != 0};
+  auto zero = [&](const std::vector<View> &L) -> int {
+    for (auto &v : L) {
+      long long own[3];
+      PartDev pd = to_dev(v.d, E, own);
+      int rc2 = launch_zero_fill(pd, own, 2 * v.l + 1, v.n, s);
+      if (rc2) return rc2;
+    }
+    return GELIB_HIP_OK;
+  };
+  const int turn[4][2] = {{0, 0}, {1, 1}, {0, 1}, {1, 0}};
+  for (auto &t : turn) {
+    const int p1 = t[0], p2 = t[1];
+    if (plans[p1][p2].triples.empty()) continue;
+    const bool fresh = (!xg || !done_x[p1]) && (!yg || !done_y[p2]);   // every wanted destination is still unwritten
+    if (!fresh) {
+      if (xg && !done_x[p1] && (rc = zero(XG.p[p1]))) return rc;
+      if (yg && !done_y[p2] && (rc = zero(YG.p[p2]))) return rc;
+    }
+    rc = bwd_planned(plans[p1][p2], G.p[p1 ^ p2], X.p[p1], Y.p[p2], XG.p[p1], YG.p[p2], xg != nullptr, yg != nullptr,
+                     fresh ? 0 : 1, s);
+    if (rc) return rc;
+    done_x[p1] = done_y[p2] = true;
+  }
+  for (int q = 0; q < 2; q++) {   // parts that no product feeds
+    if (xg && !done_x[q] && (rc = zero(XG.p[q]))) return rc;
+    if (yg && !done_y[q] && (rc = zero(YG.p[q]))) return rc;
+  }
+  return GELIB_HIP_OK;
 }
 
 // Channels of the product's parts (indexed like R) for a plan built with check_channels = false.
@@ -1208,6 +1405,16 @@ int gelib_hip_so3vec_diagcg_bwd(const gelib_part_desc *xg, const gelib_part_desc
                                 const gelib_part_desc *g, int nx, const gelib_part_desc *x, int ny,
                                 const gelib_part_desc *y, int accumulate, void *stream) {
   return vec_bwd_entry(true, xg, yg, ng, g, nx, x, ny, y, accumulate, stream);
+}
+
+int gelib_hip_o3vec_cg_fwd(int diag, int nr, const gelib_part_desc *r, const int *rp, int nx, const gelib_part_desc *x,
+                           const int *xp, int ny, const gelib_part_desc *y, const int *yp, int accumulate, void *stream) {
+  return o3vec_fwd_entry(diag != 0, nr, r, rp, nx, x, xp, ny, y, yp, accumulate, stream);
+}
+int gelib_hip_o3vec_cg_bwd(int diag, const gelib_part_desc *xg, const gelib_part_desc *yg, int ng,
+                           const gelib_part_desc *g, const int *gp, int nx, const gelib_part_desc *x, const int *xp, int ny,
+                           const gelib_part_desc *y, const int *yp, int accumulate, void *stream) {
+  return o3vec_bwd_entry(diag != 0, xg, yg, ng, g, gp, nx, x, xp, ny, y, yp, accumulate, stream);
 }
 
 int gelib_hip_so3vec_cg_linear_fwd(int nr, const gelib_part_desc *r, int nx, const gelib_part_desc *x, int ny,

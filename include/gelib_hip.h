@@ -185,6 +185,18 @@ int gelib_hip_part_mix_channels_wgrad(void *wg, const void *x, const void *g, in
  * n_out as passed to that call), kind 1 for gelib_hip_part_mix_channels_wgrad.  0 for empty shapes or an unknown kind. */
 uint64_t gelib_hip_part_mix_workspace_bytes(int kind, int64_t rows, int n_in, int n_out);
 
+/* ---- vectors with two parts per l, told apart by a parity (O(3)) ------------------------------------------------------------
+ * The product (diag: the Diag product) of vectors whose parts carry a label (l, p), p = +1 or -1, given in rp / xp / yp; a
+ * product of parities p1, p2 has parity p1 p2 (O3/O3group.hpp:38-53).  Blocks lie in a product part in the order of the x
+ * parts by 2l + (p == -1), then of the y parts, at the running channel offset (O3/O3index.hpp:28-31, core/Gvec.hpp:311-321);
+ * product parts that are absent are skipped.  One launch of the so3vec kernels per pair of parities.  The backward call
+ * computes both gradients (either may be NULL); xg and yg are labelled like x and y. */
+int gelib_hip_o3vec_cg_fwd(int diag, int nr, const gelib_part_desc *r, const int *rp, int nx, const gelib_part_desc *x,
+                           const int *xp, int ny, const gelib_part_desc *y, const int *yp, int accumulate, void *stream);
+int gelib_hip_o3vec_cg_bwd(int diag, const gelib_part_desc *xg, const gelib_part_desc *yg, int ng,
+                           const gelib_part_desc *g, const int *gp, int nx, const gelib_part_desc *x, const int *xp, int ny,
+                           const gelib_part_desc *y, const int *yp, int accumulate, void *stream);
+
 /* ---- CGproduct followed by the weight matrices, in one pass ---------------------------------------------------------------
  * out_l[.., m, o] (+)= sum over c of P_l[.., m, c] w_l[c, o] with P = CGproduct(x, y) restricted to the l of the parts of
  * r, its channels c in the order of core/Gvec.hpp:311-321 -- what the model code of the reference writes as

@@ -132,3 +132,58 @@ def test_vec_backprop(G, diag):
     assert torch.allclose(fn(x + xeps, y).odot(t) - loss, xeps.odot(x.get_grad()), rtol=1e-3, atol=1e-3)
     yeps = G.O3vec.randn_like(y)
     assert torch.allclose(fn(x, y + yeps).odot(t) - loss, yeps.odot(y.get_grad()), rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("diag", [False, True])
+@pytest.mark.parametrize("xmus,ymus", [
+    ([(0, 1), (1, -1), (2, 1)], [(1, -1), (1, 1)]),      # every pair of parities somewhere
+    ([(1, 1), (2, 1)], [(0, -1), (1, -1), (2, -1)]),     # one parity on each side
+    ([(1, -1)], [(0, 1), (1, 1), (1, -1)]),              # a destination first touched by a later product
+    ([(7, 1), (2, -1)], [(1, -1), (7, -1)]),             # operands above what the small-l kernels take
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_o3vec_entry_points_match_part_level_calls(G, xmus, ymus, diag, accumulate):
+    """The vector calls against one part-level call per (mu1, mu2, mu) at the running channel offset.  Products are bit for
+    bit single sums in both (compared to rounding: the families differ); a gradient adds up to a few hundred terms in
+    another order, each order within 2^-24 times the terms' moduli per addition of a running sum: 1e-5 of the largest."""
+    from gelib_amd import cabi
+    from gelib_amd.O3 import _index
+    n = 3
+    B = 5
+    xmus, ymus = sorted(xmus, key=_index), sorted(ymus, key=_index)
+    mk = lambda mus, seed: [U.dev(U.seeded(seed + i, B, 2 * mu[0] + 1, n)) for i, mu in enumerate(mus)]
+    x, y = mk(xmus, 1), mk(ymus, 30)
+    tx, ty = G.O3type({mu: n for mu in xmus}), G.O3type({mu: n for mu in ymus})
+    tau = tx.DiagCGproduct(ty, 8) if diag else tx.CGproduct(ty, 8)
+    rmus = list(tau)
+    start = [U.dev(U.seeded(60 + i, B, 2 * mu[0] + 1, tau[mu])) for i, mu in enumerate(rmus)]
+    g = [U.dev(U.seeded(90 + i, B, 2 * mu[0] + 1, tau[mu])) for i, mu in enumerate(rmus)]
+    base = (lambda ts: [t.clone() for t in ts]) if accumulate else (lambda ts: [torch.zeros_like(t) for t in ts])
+    r0, xg0, yg0 = base(start), base(x), base(y)
+    name = "so3part_diagcg_%s" if diag else "so3part_cg_%s"
+    fwd, b0, b1 = (getattr(cabi, name % k) for k in ("fwd", "back0", "back1"))
+    offs = {mu: 0 for mu in rmus}
+    for i, mu1 in enumerate(xmus):
+        for j, mu2 in enumerate(ymus):
+            for l in range(abs(mu1[0] - mu2[0]), mu1[0] + mu2[0] + 1):
+                mu = (l, mu1[1] * mu2[1])
+                if mu not in offs:
+                    continue
+                k = rmus.index(mu)
+                fwd(r0[k], x[i], y[j], offs[mu])
+                b0(xg0[i], g[k], y[j], offs[mu])
+                b1(yg0[j], g[k], x[i], offs[mu])
+                offs[mu] += n if diag else n * n
+    ps = lambda mus: [mu[1] for mu in mus]
+    new = (lambda ts: [t.clone() for t in ts]) if accumulate else (lambda ts: [torch.full_like(t, 7.0) for t in ts])
+    r, xg, yg = new(start), new(x), new(y)
+    cabi.o3vec_fwd(r, ps(rmus), x, ps(xmus), y, ps(ymus), accumulate=accumulate, diag=diag)
+    cabi.o3vec_bwd(xg, yg, g, ps(rmus), x, ps(xmus), y, ps(ymus), accumulate=accumulate, diag=diag)
+    only = new(y)
+    cabi.o3vec_bwd(None, only, g, ps(rmus), x, ps(xmus), y, ps(ymus), accumulate=accumulate, diag=diag)
+    for a, b in list(zip(r, r0)) + list(zip(xg, xg0)) + list(zip(yg, yg0)) + list(zip(only, yg0)):
+        assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max())
+    # any order of the parts in the call
+    r2 = new(start)
+    cabi.o3vec_fwd(r2[::-1], ps(rmus)[::-1], x[::-1], ps(xmus)[::-1], y, ps(ymus), accumulate=accumulate, diag=diag)
+    assert all(torch.equal(torch.view_as_real(a), torch.view_as_real(b)) for a, b in zip(r, r2))
