@@ -23,6 +23,8 @@ struct FwdArgs {
   int accumulate;
   long long tile;                  // cells per tile; the blocks of one tile are consecutive
   int blocks_per_tile;
+  int tile_per_xcd;                // consecutive blocks go round the eight XCDs; 1: blocks are numbered so that those of a
+                                   // tile run on one XCD (eight tiles at a time), 0: a tile's blocks go round all of them
   int first_block[kMaxPairs + 1];  // inside a tile, blocks [first_block[p], first_block[p+1]) work on pair p
   int cpb[kMaxPairs];              // cells per block of pair p
 };
@@ -94,10 +96,10 @@ __device__ __forceinline__ int pick_int(const int (&arr)[N], int i) {
   return (int)r;
 }
 
-// ti: channels of the first operand handled per thread (1, 2 or 4); must divide every n1.
+// ti: channels of the first operand handled per thread (1, 2 or 4); divides every n1 unless ragged.
 // lop: largest l of an operand (above kLT: the kernel for l up to kLTMax -- unrolled_fwd_takes says when it exists)
 bool unrolled_fwd_takes(bool diag, int ti, int lcap, int lop);
-int launch_unrolled_fwd(const FwdArgs &a, bool diag, int ti, int lcap, int lop, int nblocks, size_t lds_bytes, hipStream_t s);
+int launch_unrolled_fwd(const FwdArgs &a, bool diag, int ti, bool ragged, int lcap, int lop, int nblocks, size_t lds_bytes, hipStream_t s);
 // lcap: largest l present in the gradient; lop: largest l of an operand (above kLT: the kernel for l up to kLTMax, which
 // exists for CGproduct with power-of-two channel counts and lcap <= kLTMax only -- unrolled_bwd_takes says so)
 bool unrolled_bwd_takes(bool diag, bool padded, int lcap, int lop, int llo);

@@ -27,10 +27,11 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(1))) v2f *GlobalOut;  // product rows: global_store, not flat_store
 
 // One (l1,l2,l) triple for one thread: rows m = -L..L of the block, TI channels each.
-template <int L1, int L2, int L, int TI>
+// last: the thread's channels 0..last exist (RAGGED; otherwise all TI do).
+template <int L1, int L2, int L, int TI, bool RAGGED>
 __device__ __forceinline__ void triple_fwd(const float2 (&xv)[TI][2 * L1 + 1], const float2 (&yv)[2 * L2 + 1],
                                            CoeffPtr C, GlobalOut rp, int sm, int kstride, bool accumulate,
-                                           bool live) {
+                                           bool live, int last) {
 #pragma unroll
   for (int m = -L; m <= L; m++) {
     float2 acc[TI];
@@ -56,6 +57,7 @@ __device__ __forceinline__ void triple_fwd(const float2 (&xv)[TI][2 * L1 + 1], c
       GlobalOut row = rp + (m + L) * sm;
 #pragma unroll
       for (int k = 0; k < TI; k++) {
+        if (RAGGED && k > last) break;
         v2f v;
         v.x = acc[k].x;
         v.y = acc[k].y;
@@ -73,7 +75,7 @@ struct RParts {
   FastPart R[LCAP + 1];
 };
 
-template <int L1, int L2, int LCAP, int TI, bool DIAG>
+template <int L1, int L2, int LCAP, int TI, bool DIAG, bool RAGGED>
 __device__ __forceinline__ void pair_fwd(const RParts<LCAP> &rp_all, PairPtr pr, CoeffPtr Cs, const float2 *xs,
                                          const float2 *ys, int offs_add, bool accumulate, long long cell, int dc,
                                          int u, bool live) {
@@ -87,14 +89,19 @@ __device__ __forceinline__ void pair_fwd(const RParts<LCAP> &rp_all, PairPtr pr,
     i0 = u / N2;
     j = u - i0 * N2;
   }
-  const int istep = N1 / TI;  // the thread's k-th channel of x is i0 + k*istep
+  const int istep = RAGGED ? (N1 + TI - 1) / TI : N1 / TI;  // the thread's k-th channel of x is i0 + k*istep
+  int last = 0;   // RAGGED: the last k whose channel exists
+  if (RAGGED) {
+#pragma unroll
+    for (int k = 1; k < TI; k++) last += i0 + k * istep < N1 ? 1 : 0;
+  }
   const float2 *xp = xs + dc * (2 * L1 + 1) * N1 + i0;
   const float2 *yp = ys + dc * (2 * L2 + 1) * N2 + j;
   float2 xv[TI][2 * L1 + 1], yv[2 * L2 + 1];
 #pragma unroll
   for (int m1 = 0; m1 <= 2 * L1; m1++)
 #pragma unroll
-    for (int k = 0; k < TI; k++) xv[k][m1] = xp[m1 * N1 + k * istep];
+    for (int k = 0; k < TI; k++) xv[k][m1] = xp[m1 * N1 + (RAGGED && k > last ? last : k) * istep];
 #pragma unroll
   for (int m2 = 0; m2 <= 2 * L2; m2++) yv[m2] = yp[m2 * N2];
 
@@ -108,7 +115,7 @@ __device__ __forceinline__ void pair_fwd(const RParts<LCAP> &rp_all, PairPtr pr,
       if (p.ri[dl] >= 0) {
         const FastPart R = rp_all.R[L];
         GlobalOut rp = (GlobalOut)R.ptr + cell * R.sb + (p.offs[dl] + offs_add + u);
-        triple_fwd<L1, L2, L, TI>(xv, yv, Cs + p.cg[dl], rp, R.sm, kstride, accumulate, live);
+        triple_fwd<L1, L2, L, TI, RAGGED>(xv, yv, Cs + p.cg[dl], rp, R.sm, kstride, accumulate, live, last);
       }
     }
   });
@@ -128,13 +135,17 @@ __device__ __forceinline__ void stage_part(float2 *dst, const FastPart P, int ro
   }
 }
 
-// LT: largest operand l of the pairs the kernel has code for.
-template <int LCAP, bool DIAG, int TI, int LT>
+// LT: largest operand l of the pairs the kernel has code for.  RAGGED: channel counts of x that TI does not divide -- the
+// slots then are ceil(n1 / TI) * n2, and the threads of the last channels leave out those beyond n1.
+template <int LCAP, bool DIAG, int TI, int LT, bool RAGGED>
 __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
   extern __shared__ float2 lds_ops[];
   int pidx = 0, first = 0;
   const int per_tile = a.blocks_per_tile;
-  const int tile_idx = (int)blockIdx.x / per_tile, in_tile = (int)blockIdx.x - tile_idx * per_tile;
+  // (with tile_per_xcd the grid is whole groups of eight tiles; the blocks of a tile beyond the last have no cells)
+  const int seq = a.tile_per_xcd ? (int)blockIdx.x >> 3 : (int)blockIdx.x;
+  const int turn = seq / per_tile, in_tile = seq - turn * per_tile;
+  const int tile_idx = a.tile_per_xcd ? 8 * turn + ((int)blockIdx.x & 7) : turn;
   static_for<(LT + 1) * (LT + 1)>([&](auto k) __attribute__((always_inline)) {
     if (k.value > 0 && k.value < a.npairs && in_tile >= a.first_block[k.value]) {
       pidx = k.value;
@@ -159,7 +170,7 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
   const bool accumulate = a.accumulate != 0;
   __syncthreads();
 
-  const int U = DIAG ? n1 : (n1 / TI) * n2;
+  const int U = DIAG ? n1 : (RAGGED ? (n1 + TI - 1) / TI : n1 / TI) * n2;
   const int slots = ncell * U;
   const CoeffPtr C = (CoeffPtr)(a.bank + p->cg_base);
   const int code = l1 * (kLTMax + 1) + l2;
@@ -174,7 +185,7 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
 #define GELIB_CASE(A, B)                                                                                      \
   case A * (kLTMax + 1) + B:                                                                                  \
     if constexpr (A <= LT && B <= LT)                                                                         \
-      pair_fwd<A, B, LCAP, TI, DIAG>(rp_all, p, C, xs, ys, offs_add, accumulate, cell, dc, u, live);          \
+      pair_fwd<A, B, LCAP, TI, DIAG, RAGGED>(rp_all, p, C, xs, ys, offs_add, accumulate, cell, dc, u, live);          \
     break;
 #define GELIB_ROW(A) \
   GELIB_CASE(A, 0) GELIB_CASE(A, 1) GELIB_CASE(A, 2) GELIB_CASE(A, 3) GELIB_CASE(A, 4) GELIB_CASE(A, 5) GELIB_CASE(A, 6)
@@ -186,10 +197,10 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
   }
 }
 
-template <int LCAP, bool DIAG, int TI, int LT = kLT>
+template <int LCAP, bool DIAG, int TI, int LT = kLT, bool RAGGED = false>
 int launch_fwd_variant(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s) {
   static_assert(kLTMax == 6 && LT <= kLTMax, "the case table above lists l1, l2 = 0..6");
-  hipLaunchKernelGGL((unrolled_fwd_kernel<LCAP, DIAG, TI, LT>), dim3(nblocks), dim3(kBlock), lds_bytes, s, a);
+  hipLaunchKernelGGL((unrolled_fwd_kernel<LCAP, DIAG, TI, LT, RAGGED>), dim3(nblocks), dim3(kBlock), lds_bytes, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
 }

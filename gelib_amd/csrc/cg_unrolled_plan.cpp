@@ -16,6 +16,7 @@ int g_fwd_block_bytes = 0;           // product bytes one forward block aims to 
 int g_fwd_lds_bytes = 16 * 1024;     // LDS one forward block may use for its staged operands
 int g_fwd_cell_tile = -1;            // cells per tile of the forward launch (0 = all cells in one tile, -1 = by channels)
 int g_fwd_narrow_decline = 1;  // leave products with at most four channel pairs per block to the any-l forward kernel
+int g_fwd_tile_per_xcd = -1;          // blocks of a tile on one XCD (-1 = by the alignment of the blocks, 0 no, 1 yes)
 int g_fwd_ti = 0;                    // 0 = widest tile that divides every n1, else force 1 / 2 / 4
 int g_bwd_enable = 1;
 int g_bwd_one_enable = 1; // the backward kernel for calls with one triple
@@ -283,7 +284,10 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   }
   // which kernel would run is decided from the type alone, before any table is built: a product this family declines
   // (e.g. operands of l = 6 uncapped) must not cost a device allocation, and its l range does not fit a PairRec
+  int lcap_all = 0, lop = 0;
+  for (auto &t : triples) lcap_all = std::max(lcap_all, t.l), lop = std::max(lop, std::max(t.l1, t.l2));
   int ti = 1;
+  bool ragged = false;
   if (!diag) {
     ti = 4;
     for (auto &t : triples) {
@@ -296,10 +300,23 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
       // L=4 x L=2, B=1M 9.85 -> 8.5 ms; 32 x 1 channels 8.6 -> 7.5 ms)
       if (ti > 2 && (n1 / ti) * n2 < 16) ti = 2;
     }
+    // An odd channel count leaves one channel per thread, and the kernel is then bound by its scalar loads: a coefficient
+    // serves 64 results.  Four channels per thread with the last ones of a part idle are faster up to about twice the work (one
+    // channel / four, microseconds: L=4, 9 channels, 16384 cells 1830 / 1195; 13 x 7 channels uncapped 3796 / 2153; 5
+    // channels, L=3, 100000 cells 1700 / 1431; 3 channels, 200000 cells 1696 / 1622; 25 channels, L=2 2151 / 1399; 20, 12, 9,
+    // 6, 3 x 10, 7, 6, 5 channels, every l, 5003 cells 354 / 251; 5, 3, 1 channels, 2.1 times the work, 636 / 366; two channels per thread lie between or equal).
+    if (ti == 1 && lcap_all <= 2 * kLT && lop <= kLT) {
+      double useful = 0, padded = 0;
+      for (auto &t : triples) {
+        const double terms = (2.0 * t.l1 + 1) * (2 * t.l2 + 1) * ys[t.yi].second;
+        useful += terms * xs[t.xi].second;
+        padded += terms * ((xs[t.xi].second + 3) / 4 * 4);
+      }
+      if (padded <= 2.5 * useful) ti = 4;
+    }
     if (g_fwd_ti == 1 || g_fwd_ti == 2 || g_fwd_ti == 4) ti = std::min(ti, g_fwd_ti);
+    for (auto &t : triples) ragged = ragged || xs[t.xi].second % ti;
   }
-  int lcap_all = 0, lop = 0;
-  for (auto &t : triples) lcap_all = std::max(lcap_all, t.l), lop = std::max(lop, std::max(t.l1, t.l2));
   if (lop > kLT && ti == 4) ti = 2;  // the kernel for operands above kLT is built for two channels per thread
   if (!unrolled_fwd_takes(diag, ti, lcap_all, lop) || (lop > kLT && !g_fwd_l6_enable)) return GELIB_HIP_OK;
   const DevicePlan *plan = nullptr;
@@ -325,9 +342,24 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   // Measured in one process, forward pass: L=4 with 16 channels 4.41 ms at 64 cells per tile, 4.30 at 32, 4.56 at 128;
   // 8 channels 4.34 at 32 and 64, 4.89 at 4096; 4 channels (128-byte pieces per pair and row) 7.0 at 64, 6.7 at 1024,
   // 5.85 at 4096, 7.9 with all cells in one tile.
+  // Blocks of a row that are not whole 128-byte lines share a line with the next pair's: the two halves meet in one L2 cache
+  // only if both blocks run on the same XCD, and otherwise reach memory as two partial lines.  There the blocks of a tile
+  // go to one XCD, eight tiles at a time, in tiles small enough that a part's neighbouring blocks are written close
+  // together in time (tiles over all XCDs / one each, microseconds: 9 channels, L=4, 16384 cells 1195 / 983; 13 x 7 uncapped
+  // 2139 / 1883; 5 channels, L=3, 100000 cells 1434 / 1110; 3 channels, 200000 cells 1622 / 977; 6 channels, L=4, 50000 cells
+  // 1944 / 1673; 6 channels, L=5, 10000 cells 846 / 709; 17 x 2 channels 526 / 541).  Whole lines go round the XCDs: 12
+  // channels, L=4 1328 / 1486, 4 channels 578 / 660.  Fewer than 32 tiles would leave XCDs without work.
   long long auto_tile = 4096;
-  for (auto &p : plan->pairs)
-    if ((long long)p.n1 * (diag ? 1 : p.n2) >= 64) auto_tile = 32;
+  bool unaligned = false;
+  for (auto &p : plan->pairs) {
+    const long long n = (long long)p.n1 * (diag ? 1 : p.n2);
+    if (n >= 64) auto_tile = 32;
+    unaligned = unaligned || n % 16;
+  }
+  const long long xcd_tile = auto_tile == 32 ? 16 : 64;
+  const bool want_xcd = g_fwd_tile_per_xcd < 0 ? unaligned && !diag && a.npairs > 1 && ncells >= 32 * xcd_tile
+                                               : g_fwd_tile_per_xcd == 1;
+  if (want_xcd) auto_tile = xcd_tile;
   const long long want_tile = g_fwd_cell_tile < 0 ? auto_tile : g_fwd_cell_tile;
   const long long tile = want_tile > 0 ? std::min<long long>(want_tile, ncells) : ncells;
   // product bytes a block aims at: 96 KB; 128 KB for products that reach above l = 4 (measured in one process on L=4,
@@ -341,7 +373,7 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
       if (p.ri[d] >= 0) rows += 2 * (std::abs(p.l1 - p.l2) + d) + 1;
     const long long nout = diag ? p.n1 : (long long)p.n1 * p.n2;
     const long long bytes_per_cell = rows * nout * 8;
-    const long long U = diag ? p.n1 : (long long)(p.n1 / ti) * p.n2;
+    const long long U = diag ? p.n1 : (long long)((p.n1 + ti - 1) / ti) * p.n2;
     long long cpb = std::max<long long>(1, block_bytes / std::max<long long>(1, bytes_per_cell));
     const long long op_bytes = 8LL * ((2 * p.l1 + 1) * (long long)p.n1 + (2 * p.l2 + 1) * (long long)p.n2);
     cpb = std::min(cpb, std::max<long long>(1, g_fwd_lds_bytes / op_bytes));
@@ -357,9 +389,11 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   a.first_block[a.npairs] = (int)nblocks;  // blocks of one tile
   a.tile = tile;
   a.blocks_per_tile = (int)nblocks;
-  nblocks *= (ncells + tile - 1) / tile;
+  a.tile_per_xcd = want_xcd ? 1 : 0;
+  const long long ntiles = (ncells + tile - 1) / tile;
+  nblocks *= a.tile_per_xcd ? (ntiles + 7) / 8 * 8 : ntiles;
   if (nblocks > 0x7fffffffLL) return GELIB_HIP_ERR_ARG;
-  rc = launch_unrolled_fwd(a, diag, ti, lcap, lop, (int)nblocks, lds_bytes, s);
+  rc = launch_unrolled_fwd(a, diag, ti, ragged, lcap, lop, (int)nblocks, lds_bytes, s);
   if (rc) return rc;
   *used = 1;
   return GELIB_HIP_OK;
@@ -629,6 +663,11 @@ int unrolled_set_option(const char *name, int value) {
   if (!std::strcmp(name, "fwd_cell_tile")) {
     if (value < -1) return GELIB_HIP_ERR_ARG;
     g_fwd_cell_tile = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "fwd_tile_per_xcd")) {
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_fwd_tile_per_xcd = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "fwd_narrow_decline")) {
