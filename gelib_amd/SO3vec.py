@@ -156,21 +156,30 @@ def _product_fn(diag, part_cls=SO3part, prefix="SO3vec"):
             gb = backend()
             k1, k2 = ctx.k1, ctx.k2
             saved = ctx.saved_tensors
-            grads = [torch.empty_like(t, memory_format=torch.contiguous_format) for t in saved]
+            # An operand none of whose parts needs a gradient (harmonics of edge directions, say) gets none where the kernels
+            # gain by that: products without sums over channels of operands up to l = 6.  The kernels for large l compute
+            # both gradients faster than one.
+            need = ctx.needs_input_grad[3:]
+            want = [True] * len(saved)
+            if diag or all(t.size(-1) == 1 for t in saved[:k1]) != all(t.size(-1) == 1 for t in saved[k1:]):
+                if max(t.size(-2) for t in saved) <= 13:
+                    want = [any(need[:k1])] * k1 + [any(need[k1:])] * k2
+            grads = [torch.empty_like(t, memory_format=torch.contiguous_format) if w else None for t, w in zip(saved, want)]
             x = gb.SO3vec.view(list(saved[0:k1]))
             y = gb.SO3vec.view(list(saved[k1:k1 + k2]))
             g = gb.SO3vec.view([t.contiguous() for t in gargs])
-            xg = gb.SO3vec.view(grads[0:k1])
-            yg = gb.SO3vec.view(grads[k1:k1 + k2])
+            xg = gb.SO3vec.view([t for t in grads[0:k1] if t is not None])
+            yg = gb.SO3vec.view([t for t in grads[k1:k1 + k2] if t is not None])
             lead = gargs[0].shape[:-2]
             if any(t.shape[:-2] != lead for t in saved) and (len(lead) > 3 or any(t.dim() not in (3, len(lead) + 2) for t in saved)):
                 # Broadcast operands among more than two grid dimensions: the library sees those fused into one, which
                 # an extent of 1 inside them prevents.  The operand enters as a view with stride 0, the fused backward
                 # writes one gradient per cell and torch sums them over the cells the operand is shared by.
                 wide = [t.expand(*lead, *t.shape[-2:]) for t in saved]
-                full = [torch.empty(list(lead) + list(t.shape[-2:]), dtype=t.dtype, device=t.device) if t.shape[:-2] != lead
-                        else grads[i] for i, t in enumerate(saved)]
-                getattr(gb.SO3vec, "set%s_back" % gb_type)(gb.SO3vec.view(full[0:k1]), gb.SO3vec.view(full[k1:k1 + k2]), g,
+                full = [torch.empty(list(lead) + list(t.shape[-2:]), dtype=t.dtype, device=t.device)
+                        if t.shape[:-2] != lead and grads[i] is not None else grads[i] for i, t in enumerate(saved)]
+                getattr(gb.SO3vec, "set%s_back" % gb_type)(gb.SO3vec.view([f for f in full[0:k1] if f is not None]),
+                                                           gb.SO3vec.view([f for f in full[k1:k1 + k2] if f is not None]), g,
                                                            gb.SO3vec.view(wide[0:k1]), gb.SO3vec.view(wide[k1:k1 + k2]))
                 grads = [f if f is grads[i] else f.sum_to_size(saved[i].shape) for i, f in enumerate(full)]
             else:

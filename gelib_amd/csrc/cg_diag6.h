@@ -48,6 +48,12 @@ struct Diag6Args {
   const float *bank;  // device, kBankFloats coefficients followed by kZeroFloats zeros
   long long nwaves;   // cells * groups, or cells / (64 >> lg_npad) rounded up
   long long ncells;
+  // tight: the (cell, channel) pairs follow each other without gaps, 64 per wave, so that a channel count that is no power
+  // of two (or no multiple of 64) leaves no lane idle; kernels of the packed form only, and no sums over the lanes of a
+  // cell (lg_npad is 0 then).  nwaves = cells * n / 64 rounded up.
+  int tight;
+  unsigned long long magic64;  // ceil(2^64 / n): quotients of pair numbers below 2^50
+  unsigned magic32;            // ceil(2^32 / n): quotients of numbers below n + 64
   int groups;         // 64-channel groups per cell (more than 32 channels)
   int lg_npad;        // log2 of the channel count rounded up to a power of two, at most 6
   int n;              // channels of every part (of every part of the wider operand when xbc or ybc is set)
@@ -64,6 +70,7 @@ int launch_diag6_bwd_l6_sets(const Diag6Args &a, hipStream_t s);  // every part 
 // operand parts up to l = 2, product up to l = 4: a wave per cell and channel group, no barriers
 int launch_diag6_small_fwd(const Diag6Args &a, hipStream_t s);
 int launch_diag6_small_bwd(const Diag6Args &a, hipStream_t s);
+int launch_diag6_small4_fwd(const Diag6Args &a, hipStream_t s);     // forward, operand parts up to l = 4, product parts up to l = 6
 int launch_diag6_small4_bwd(const Diag6Args &a, hipStream_t s);     // backward, operand parts up to l = 4, gradient parts up to l = 6
 int launch_diag6_small4_hi_bwd(const Diag6Args &a, hipStream_t s);  // ... gradient parts l = 7, 8 only
 // product parts l = 7..12 only

@@ -66,7 +66,14 @@ struct WavePos {
 __device__ __forceinline__ WavePos wave_pos(const Diag6Args &a, long long w) {
   WavePos q;
   const int lane = (int)(threadIdx.x & 63);
-  if (a.lg_npad < 6) {
+  if (a.tight) {
+    const unsigned long long first = (unsigned long long)w << 6;
+    q.cell = (long long)__umul64hi(a.magic64, first);
+    const unsigned at = (unsigned)(first - (unsigned long long)q.cell * (unsigned)a.n) + (unsigned)lane;
+    q.cell_local = (int)__umulhi(a.magic32, at);
+    q.ch = (int)at - q.cell_local * a.n;
+    q.live = q.cell + q.cell_local < a.ncells;
+  } else if (a.lg_npad < 6) {
     q.cell = w << (6 - a.lg_npad);
     q.cell_local = lane >> a.lg_npad;
     q.ch = lane & ((1 << a.lg_npad) - 1);
@@ -233,8 +240,9 @@ __global__ void __launch_bounds__(256) diag6_fwd_kernel(const Diag6Args a) {
   });
 }
 
-// One pair of the backward pass: every l of the pair together, one row number m = m1 + m2 at a time.
-template <int L1, int L2, int LCAP, bool PACKED, int LLO = 0>
+// One pair of the backward pass: every l of the pair together, one row number m = m1 + m2 at a time.  WY = false: the
+// y-gradient is not wanted (no sums, no image).
+template <int L1, int L2, int LCAP, bool PACKED, int LLO = 0, bool WY = true>
 __device__ __forceinline__ void bwd_pair(const Diag6Args &a, const float2 (&xv)[2 * L1 + 1],
                                          const float2 (&yv)[2 * L2 + 1], float2 (&ax)[2 * L1 + 1], float2 *yimg,
                                          const WavePos q) {
@@ -305,22 +313,26 @@ __device__ __forceinline__ void bwd_pair(const Diag6Args &a, const float2 (&xv)[
         ax[m1 + L1].x = fmaf(qi, yc.y, ax[m1 + L1].x);
         ax[m1 + L1].y = fmaf(qi, yc.x, ax[m1 + L1].y);
         ax[m1 + L1].y = fmaf(-qr, yc.y, ax[m1 + L1].y);
-        ay[m2 + L2].x = fmaf(qr, xc.x, ay[m2 + L2].x);
-        ay[m2 + L2].x = fmaf(qi, xc.y, ay[m2 + L2].x);
-        ay[m2 + L2].y = fmaf(qi, xc.x, ay[m2 + L2].y);
-        ay[m2 + L2].y = fmaf(-qr, xc.y, ay[m2 + L2].y);
+        if constexpr (WY) {
+          ay[m2 + L2].x = fmaf(qr, xc.x, ay[m2 + L2].x);
+          ay[m2 + L2].x = fmaf(qi, xc.y, ay[m2 + L2].x);
+          ay[m2 + L2].y = fmaf(qi, xc.x, ay[m2 + L2].y);
+          ay[m2 + L2].y = fmaf(-qr, xc.y, ay[m2 + L2].y);
+        }
       });
       __builtin_amdgcn_sched_barrier(0);
     });
 #pragma unroll
     for (int m1 = 0; m1 <= 2 * L1; m1++) asm volatile("" : "+v"(ax[m1].x), "+v"(ax[m1].y));
-    float2 *col = yimg + (L2 * L2) * 64 + (threadIdx.x & 63);
+    if constexpr (WY) {
+      float2 *col = yimg + (L2 * L2) * 64 + (threadIdx.x & 63);
 #pragma unroll
-    for (int m2 = 0; m2 <= 2 * L2; m2++) {
-      float2 o = col[m2 * 64];
-      o.x += ay[m2].x;
-      o.y += ay[m2].y;
-      col[m2 * 64] = o;
+      for (int m2 = 0; m2 <= 2 * L2; m2++) {
+        float2 o = col[m2 * 64];
+        o.x += ay[m2].x;
+        o.y += ay[m2].y;
+        col[m2 * 64] = o;
+      }
     }
   }
 }

@@ -23,6 +23,8 @@ int g_sets_enable = 1;  // backward: the kernel with the waves' sets of l2 fixed
 int g_small_enable = 1;  // operands up to l = 2, and backward up to l = 4: the kernels that give a wave, not a block, a cell and
                          // channel group
 int g_hi_enable = 1;    // the kernels for the part l = 7..12 of a product by itself
+int g_tight = -1;        // (cell, channel) pairs without gaps between the cells: -1 where enough lanes would idle, 0 never, 1 always
+int g_small4_fwd = -1;   // forward, operands up to l = 4: the kernel that gives a wave a cell and channel group (-1 = by the shape)
 int g_one_channel = 1;  // CGproduct with a one-channel operand runs here as the Diag product with the channel repeated
 
 int device_bank(const float **out) {
@@ -160,7 +162,32 @@ int make_args(const VecPlan &plan, const std::vector<const gelib_part_desc *> &r
   int lg = 0;
   while ((1 << lg) < n && lg < 6) lg++;
   a->lg_npad = lg;
-  if (lg < 6) {
+  // Sums over the lanes of a cell (the gradient of a one-channel operand) need the cells in aligned groups of lanes.
+  // Otherwise the cells follow each other without gaps where enough lanes would idle.  Measured, aligned groups / without gaps,
+  // microseconds: features x harmonics up to l = 2, 24 channels, L = 3, 60013 cells forward 460 / 440, x-gradient 358 / 340;
+  // 48 channels, L = 2 528 / 496, 544 / 455; Diag L = 6, 72 channels, 8000 cells 2617 / 2045, 2242 / 1684; L = 4, 100 channels
+  // 1153 / 976, 943 / 909.  Forward, rows that are no multiple of 64 bytes then lie across more cache lines per store
+  // (Diag L = 6, 20 channels 1943 / 2097, 50 channels 1967 / 2795); backward that is less (1611 / 1298, 1516 / 1575).
+  const double busy = n <= 64 ? (double)n / (1 << lg) : (double)n / (64 * ((n + 63) / 64));
+  const bool lane_sums = (xbc && xg) || (ybc && yg);
+  const bool gaps = n >= 16 && (r_is_dest ? busy < 0.79 && (n % 8 == 0 || n > 64) : busy < 0.77);
+  const bool want_tight = g_tight < 0 ? gaps : g_tight != 0 && busy < 1;
+  if (want_tight && !lane_sums) {
+    const long long reach = (n + 62) / n;   // cells behind the wave's first that its lanes reach
+    auto fits = [&](const std::vector<FastPart> &v) {
+      for (auto &p : v)
+        if (p.sb < 0 || (reach * p.sb + n) * 8 >= (1LL << 31)) return false;
+      return true;
+    };
+    a->tight = fits(fx) && fits(fy) && fits(fr) && fits(fxg) && fits(fyg) && ncells < (1LL << 36);
+  }
+  if (a->tight) {
+    a->lg_npad = 0;
+    a->groups = 1;
+    a->nwaves = (ncells * n + 63) / 64;
+    a->magic64 = ~0ull / (unsigned long long)n + 1;
+    a->magic32 = ~0u / (unsigned)n + 1;
+  } else if (lg < 6) {
     // several cells per wave: the lane's offset from the wave's first cell must fit 32 bits in every part
     const long long cpw = 64 >> lg;
     auto fits = [&](const std::vector<FastPart> &v) {
@@ -208,7 +235,16 @@ int diag6_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
   const bool l8 = lcap > kL6 && !hi;
   if (l8 && !(lcap <= 8 && operands_up_to(a, 4) && g_l8_enable)) return GELIB_HIP_OK;
   a.accumulate = accumulate ? 1 : 0;
+  // A one-channel operand up to l = 2 (harmonics) leaves few pairs per part of the other one, and the block form's staging
+  // and barrier cost more than its waves' neighbouring stores gain, from 24 channels on (block / wave form, microseconds:
+  // L = 3, 24 channels, 60013 cells 440 / 371; 40 channels 470 / 388; 64 channels 441 / 352; L = 2, 48 channels, harmonics
+  // up to l = 3 496 / 356 -- but 17 channels 319 / 399, and up to l = 4 at L = 4, 16 channels 640 / 676).
+  int narrow_l = kNP;
+  for (int l = 0; l < kNP; l++)
+    if ((a.xbc && a.x[l].ptr) || (a.ybc && a.y[l].ptr)) narrow_l = l;
+  const bool small4 = g_small_enable && (g_small4_fwd < 0 ? narrow_l <= 2 && a.n >= 24 : g_small4_fwd != 0);
   if (g_small_enable && lcap <= 4 && operands_up_to(a, 2)) rc = launch_diag6_small_fwd(a, s);
+  else if (small4 && lcap <= 6 && operands_up_to(a, 4)) rc = launch_diag6_small4_fwd(a, s);
   else if (hi) rc = a.lg_npad < 6 ? launch_diag6_fwd_hi_packed(a, s) : launch_diag6_fwd_hi(a, s);
   else if (l8) rc = a.lg_npad < 6 ? launch_diag6_fwd_l8_packed(a, s) : launch_diag6_fwd_l8(a, s);
   else rc = a.lg_npad < 6 ? launch_diag6_fwd_l6_packed(a, s) : launch_diag6_fwd_l6(a, s);
@@ -278,6 +314,16 @@ int diag6_part(int kind, const long long E[3], const gelib_part_desc *r, const g
 int diag6_set_option(const char *name, int value) {
   if (!std::strcmp(name, "diag6")) {
     g_enable = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "diag6_tight")) {
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_tight = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "diag6_small4_fwd")) {
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_small4_fwd = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "diag6_small")) {

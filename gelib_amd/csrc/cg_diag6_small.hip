@@ -37,20 +37,24 @@ __global__ void __launch_bounds__(256) diag6_small_fwd_kernel(const Diag6Args a)
   });
 }
 
-template <int kSmallLop, int kSmallCap, bool PACKED, int LLO = 0>
+// WY = false: only the x-gradient is wanted -- half the multiply-adds behind the contraction, and without the image of the
+// y-gradient (51 KB a block for operands up to l = 4) the registers alone say how many waves a compute unit holds.
+template <int kSmallLop, int kSmallCap, bool PACKED, int LLO, bool WY>
 __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a) {
   constexpr int kYRows = (kSmallLop + 1) * (kSmallLop + 1);
-  __shared__ float2 yimg_all[4 * kYRows * 64];  // [wave][row][lane]
+  __shared__ float2 yimg_all[WY ? 4 * kYRows * 64 : 1];  // [wave][row][lane]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const long long w = (long long)blockIdx.x * 4 + wave;
   if (w >= a.nwaves) return;  // uniform for the wave; the kernel has no barrier
   const WavePos q = wave_pos(a, w);
   const bool accumulate = a.accumulate != 0;
-  const bool wx = a.want_x != 0, wy = a.want_y != 0;
+  const bool wx = a.want_x != 0, wy = WY && a.want_y != 0;
   // the wave's own image: only this wave touches it, and a wave's LDS operations execute in order
-  float2 *yimg = yimg_all + wave * kYRows * 64;
+  float2 *yimg = yimg_all + (WY ? wave * kYRows * 64 : 0);
+  if constexpr (WY) {
 #pragma unroll
-  for (int r = 0; r < kYRows; r++) yimg[r * 64 + lane] = make_float2(0.f, 0.f);
+    for (int r = 0; r < kYRows; r++) yimg[r * 64 + lane] = make_float2(0.f, 0.f);
+  }
   static_for<kSmallLop + 1>([&](auto l1c) __attribute__((always_inline)) {
     constexpr int L1 = decltype(l1c)::value;
     if constexpr (L1 + kSmallLop < LLO) return;  // no pair of this l1 reaches an l the launch takes
@@ -74,7 +78,7 @@ __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a)
 #pragma unroll
             for (int m2 = 0; m2 <= 2 * L2; m2++) yv[m2] = make_float2(0.f, 0.f);
           }
-          if constexpr (L1 + L2 >= LLO) bwd_pair<L1, L2, kSmallCap, PACKED, LLO>(a, xv, yv, ax, yimg, q);
+          if constexpr (L1 + L2 >= LLO) bwd_pair<L1, L2, kSmallCap, PACKED, LLO, WY>(a, xv, yv, ax, yimg, q);
         }
       });
       if (wx && a.xg[L1].ptr != nullptr) store_rows<L1, PACKED>(ax, 1, a.xg[L1], q, accumulate, a.xbc != 0, a.lg_npad);
@@ -83,7 +87,7 @@ __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a)
   static_for<kSmallLop + 1>([&](auto l2c) __attribute__((always_inline)) {
     constexpr int L2 = decltype(l2c)::value;
     const FastPart YG = a.yg[L2];
-    if constexpr (L2 + kSmallLop >= LLO) {
+    if constexpr (WY && L2 + kSmallLop >= LLO) {
       if (wy && YG.ptr != nullptr)
         store_rows<L2, PACKED>(yimg + (L2 * L2) * 64 + lane, 64, YG, q, accumulate, a.ybc != 0, a.lg_npad);
     }
@@ -91,24 +95,35 @@ __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a)
 }
 
 template <int LOP, int LCAP, int LLO = 0>
-int launch_small(bool bwd, const Diag6Args &a, hipStream_t s) {
+int launch_small_bwd(const Diag6Args &a, hipStream_t s) {
   const unsigned nblocks = (unsigned)((a.nwaves + 3) / 4);
-  if (bwd) {
-    if (a.lg_npad < 6) hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, true, LLO>), dim3(nblocks), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, false, LLO>), dim3(nblocks), dim3(256), 0, s, a);
+  const bool packed = a.lg_npad < 6;
+  if (LLO == 0 && !a.want_y) {
+    if (packed) hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, true, 0, false>), dim3(nblocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, false, 0, false>), dim3(nblocks), dim3(256), 0, s, a);
   } else {
-    if (a.lg_npad < 6) hipLaunchKernelGGL((diag6_small_fwd_kernel<LOP, LCAP, true>), dim3(nblocks), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((diag6_small_fwd_kernel<LOP, LCAP, false>), dim3(nblocks), dim3(256), 0, s, a);
+    if (packed) hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, true, LLO, true>), dim3(nblocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, false, LLO, true>), dim3(nblocks), dim3(256), 0, s, a);
   }
+  GELIB_HIP_TRY(hipGetLastError());
+  return GELIB_HIP_OK;
+}
+
+template <int LOP, int LCAP>
+int launch_small_fwd(const Diag6Args &a, hipStream_t s) {
+  const unsigned nblocks = (unsigned)((a.nwaves + 3) / 4);
+  if (a.lg_npad < 6) hipLaunchKernelGGL((diag6_small_fwd_kernel<LOP, LCAP, true>), dim3(nblocks), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((diag6_small_fwd_kernel<LOP, LCAP, false>), dim3(nblocks), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
 }
 
 }  // namespace
 
-int launch_diag6_small_fwd(const Diag6Args &a, hipStream_t s) { return launch_small<2, 4>(false, a, s); }
-int launch_diag6_small_bwd(const Diag6Args &a, hipStream_t s) { return launch_small<2, 4>(true, a, s); }
-int launch_diag6_small4_bwd(const Diag6Args &a, hipStream_t s) { return launch_small<4, 6>(true, a, s); }
-int launch_diag6_small4_hi_bwd(const Diag6Args &a, hipStream_t s) { return launch_small<4, 8, 7>(true, a, s); }
+int launch_diag6_small_fwd(const Diag6Args &a, hipStream_t s) { return launch_small_fwd<2, 4>(a, s); }
+int launch_diag6_small4_fwd(const Diag6Args &a, hipStream_t s) { return launch_small_fwd<4, 6>(a, s); }
+int launch_diag6_small_bwd(const Diag6Args &a, hipStream_t s) { return launch_small_bwd<2, 4>(a, s); }
+int launch_diag6_small4_bwd(const Diag6Args &a, hipStream_t s) { return launch_small_bwd<4, 6>(a, s); }
+int launch_diag6_small4_hi_bwd(const Diag6Args &a, hipStream_t s) { return launch_small_bwd<4, 8, 7>(a, s); }
 
 }  // namespace gelib_hip

@@ -573,12 +573,13 @@ class SO3vec : public GvecBase {
   void add_DiagCGproduct(const SO3vec &x, const SO3vec &y) { fwd(true, x, y); }
   void add_DiagCGproduct_back0(const SO3vec &g, const SO3vec &y) { bwd(true, this, nullptr, g, *this, y); }
   void add_DiagCGproduct_back1(const SO3vec &g, const SO3vec &x) { bwd(true, nullptr, this, g, x, *this); }
-  // both gradients from one pass over g (no counterpart in the reference, which reads g twice)
+  // both gradients from one pass over g (no counterpart in the reference, which reads g twice); an empty vector in the
+  // place of a gradient leaves that one out
   static void add_CGproduct_back(SO3vec &xg, SO3vec &yg, const SO3vec &g, const SO3vec &x, const SO3vec &y) {
-    bwd(false, &xg, &yg, g, x, y);
+    bwd(false, xg.parts.empty() ? nullptr : &xg, yg.parts.empty() ? nullptr : &yg, g, x, y);
   }
   static void add_DiagCGproduct_back(SO3vec &xg, SO3vec &yg, const SO3vec &g, const SO3vec &x, const SO3vec &y) {
-    bwd(true, &xg, &yg, g, x, y);
+    bwd(true, xg.parts.empty() ? nullptr : &xg, yg.parts.empty() ? nullptr : &yg, g, x, y);
   }
 
   std::string classname() const { return "GElib::SO3vec"; }

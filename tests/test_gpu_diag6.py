@@ -278,3 +278,60 @@ def test_cgproduct_of_one_channel_vectors_goes_forward_on_the_diag_kernels(cabi,
     assert cabi.last_path() != DIAG6
     torch.cuda.synchronize()
     O.check_bwd([U.host(a) for a in dxg], [U.host(a) for a in dyg], "one channel on both sides, backward")
+
+
+TIGHT = [
+    # (B, tau_x, tau_y, maxl, diag): 64 (cell, channel) pairs a wave, cells starting anywhere in it
+    (7, {l: 24 for l in range(5)}, {l: 24 for l in range(5)}, 4, True),      # 2 2/3 cells a wave
+    (5, {l: 72 for l in range(7)}, {l: 72 for l in range(7)}, 6, True),      # a cell and its neighbours' ends
+    (3, {1: 200, 3: 200}, {2: 200, 4: 200}, -1, True),                       # up to l = 7: two launches
+    (64, {0: 48, 1: 48}, {0: 48, 2: 48}, 2, True),                           # whole waves at the end
+    (1, {l: 17 for l in range(3)}, {l: 17 for l in range(3)}, 2, True),      # less than a wave
+    (9, {l: 24 for l in range(4)}, {0: 1, 1: 1, 2: 1}, 3, False),            # features x harmonics
+    (5, {0: 1, 2: 1}, {l: 40 for l in range(4)}, -1, False),                 # ... harmonics first, up to l = 5
+    (11, {l: 64 for l in range(4)}, {2: 1}, 3, False),                       # no gaps to close: the wave form alone
+    (6, {3: 17, 6: 17}, {1: 1}, 6, False),
+]
+
+
+@pytest.mark.parametrize("B,tx,ty,maxl,diag", TIGHT)
+@pytest.mark.parametrize("tight", [-1, 1])
+def test_pairs_without_gaps_and_one_gradient(cabi, B, tx, ty, maxl, diag, tight):
+    """Both gradients, and each by itself: the kernels that compute one leave the other's sums out."""
+    seed = 1300 + B
+    xs = [U.seeded(seed + l, B, 2 * l + 1, n) for l, n in sorted(tx.items())]
+    ys = [U.seeded(seed + 50 + l, B, 2 * l + 1, n) for l, n in sorted(ty.items())]
+    O = U.VecOracle(xs, ys, maxl, diag, gseed=seed + 100)
+    dxs, dys, dgs = [U.dev(a) for a in xs], [U.dev(a) for a in ys], [U.dev(a) for a in O.gs]
+    drs = [torch.full(p.shape, 7.0 + 1j, dtype=torch.complex64, device="cuda") for p in O.r32]
+    new = lambda L: [torch.full(a.shape, 3.0 - 2j, dtype=torch.complex64, device="cuda") for a in L]
+    cabi.set_option("diag6_tight", tight)
+    try:
+        cabi.so3vec_fwd(drs, dxs, dys, accumulate=False, diag=diag)
+        assert cabi.last_path() == DIAG6
+        xg, yg, xg1, yg1 = new(xs), new(ys), new(xs), new(ys)
+        cabi.so3vec_bwd(xg, yg, dgs, dxs, dys, accumulate=False, diag=diag)
+        cabi.so3vec_bwd(xg1, None, dgs, dxs, dys, accumulate=False, diag=diag)
+        cabi.so3vec_bwd(None, yg1, dgs, dxs, dys, accumulate=False, diag=diag)
+        torch.cuda.synchronize()
+    finally:
+        cabi.set_option("diag6_tight", -1)
+    tag = "B%d %s x %s maxl %d" % (B, tx, ty, maxl)
+    O.check_fwd([U.host(a) for a in drs], tag)
+    O.check_bwd([U.host(a) for a in xg], [U.host(a) for a in yg], tag)
+    O.check_bwd([U.host(a) for a in xg1], [U.host(a) for a in yg1], tag + " one at a time")
+
+
+def test_no_gradient_for_harmonics(cabi):
+    """An operand that needs no gradient gets none, and the other's is the same as with it."""
+    import gelib_amd as G
+    x = [U.dev(U.seeded(3 + l, 7, 2 * l + 1, 24)).requires_grad_() for l in range(4)]
+    y = [U.dev(U.seeded(30 + l, 7, 2 * l + 1, 1)) for l in range(3)]
+    out = list(G.CGproduct(G.SO3vec(*x), G.SO3vec(*y), 3).parts.values())
+    gs = [U.dev(U.seeded(60 + i, *p.shape)) for i, p in enumerate(out)]
+    got = torch.autograd.grad(out, x, gs)
+    for t in y:
+        t.requires_grad_()
+    both = torch.autograd.grad(list(G.CGproduct(G.SO3vec(*x), G.SO3vec(*y), 3).parts.values()), x + y, gs)
+    for a, b in zip(got, both):
+        assert float((a - b).abs().max()) <= 1e-6 * float(b.abs().max())
