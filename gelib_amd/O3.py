@@ -10,7 +10,7 @@ fused kernels per pair of parities.
 """
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch
+from gelib_amd.gelib_common import backend, common_batch, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 
 
@@ -160,6 +160,7 @@ def _vec_fn(diag):
     class Fn(torch.autograd.Function):
 
         @staticmethod
+        @without_torch_function
         def forward(ctx, xmus, ymus, maxl, *args):
             gb = backend()
             k1 = len(xmus)

@@ -3,7 +3,7 @@ of python/src/gelib/SO3partArr.py:18-234 for the CG product path.  The grid dime
 as the grid dimensions of the part descriptor (core/Gpart.hpp:416-432, 495-531); nothing is reshaped or copied."""
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch, output
+from gelib_amd.gelib_common import backend, common_batch, output, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 from gelib_amd.SO3part import SO3part
 
@@ -128,6 +128,7 @@ class SO3partArr_GatherFn(torch.autograd.Function):
     parts of a vector at once (SO3vecArr.gather), each result written by the launch that sums it."""
 
     @staticmethod
+    @without_torch_function
     def forward(ctx, gmap, d, *xs):
         from gelib_amd.gather_map import gather_map
         assert isinstance(gmap, gather_map)
@@ -145,6 +146,7 @@ class SO3partArr_GatherFn(torch.autograd.Function):
         return tuple(rs)
 
     @staticmethod
+    @without_torch_function
     def backward(ctx, *rgs):
         used = [i for i, g in enumerate(rgs) if g is not None]
         xgs = [None] * len(rgs)

@@ -4,7 +4,7 @@ forward writes into uninitialised parts and the backward computes both gradients
 import torch
 
 from gelib_amd.SO3weights import mix_channels
-from gelib_amd.gelib_common import backend, common_batch
+from gelib_amd.gelib_common import backend, common_batch, without_torch_function
 from gelib_amd.SO3part import SO3part
 
 
@@ -12,10 +12,10 @@ class SO3vec:
 
     def __init__(self, *args):
         self.parts = {}
-        for x in args:
-            assert isinstance(x, torch.Tensor)
-            p = SO3part(x)
-            self.parts[p.getl()] = x
+        with torch._C.DisableTorchFunctionSubclass():   # x may be an SO3part: reading its shape would go through Python
+            for x in args:
+                assert isinstance(x, torch.Tensor)
+                self.parts[(x.shape[-2] - 1) // 2] = x
 
     @classmethod
     def zeros(cls, b, tau, device='cpu'):
@@ -135,6 +135,7 @@ def _product_fn(diag, part_cls=SO3part, prefix="SO3vec"):
     class Fn(torch.autograd.Function):
 
         @staticmethod
+        @without_torch_function
         def forward(ctx, k1, k2, maxl, *args):
             gb = backend()
             ctx.k1, ctx.k2 = k1, k2
@@ -153,7 +154,6 @@ def _product_fn(diag, part_cls=SO3part, prefix="SO3vec"):
 
         @staticmethod
         def backward(ctx, *gargs):
-            gb = backend()
             k1, k2 = ctx.k1, ctx.k2
             saved = ctx.saved_tensors
             # An operand none of whose parts needs a gradient (harmonics of edge directions, say) gets none where the kernels
@@ -165,6 +165,12 @@ def _product_fn(diag, part_cls=SO3part, prefix="SO3vec"):
                 if max(t.size(-2) for t in saved) <= 13:
                     want = [any(need[:k1])] * k1 + [any(need[k1:])] * k2
             grads = [torch.empty_like(t, memory_format=torch.contiguous_format) if w else None for t, w in zip(saved, want)]
+            return tuple([None, None, None] + Fn.fill(k1, k2, saved, grads, gargs))
+
+        @staticmethod
+        @without_torch_function
+        def fill(k1, k2, saved, grads, gargs):
+            gb = backend()
             x = gb.SO3vec.view(list(saved[0:k1]))
             y = gb.SO3vec.view(list(saved[k1:k1 + k2]))
             g = gb.SO3vec.view([t.contiguous() for t in gargs])
@@ -186,7 +192,7 @@ def _product_fn(diag, part_cls=SO3part, prefix="SO3vec"):
                 # a gradient shaped like an operand that is shared by the batch or the grid (extent 1 there) is summed
                 # over the cells inside the library, in a fixed order
                 getattr(gb.SO3vec, "set%s_back" % gb_type)(xg, yg, g, x, y)
-            return tuple([None, None, None] + grads)
+            return grads
 
     Fn.__name__ = "%s_%sFn" % (prefix, gb_type)
     return Fn

@@ -15,10 +15,10 @@ class SO3vecArr:
         self.parts = {}
         if len(args) == 1 and not isinstance(args[0], torch.Tensor) and hasattr(args[0], '__iter__'):
             args = list(args[0])
-        for x in args:
-            assert isinstance(x, torch.Tensor)
-            p = SO3partArr(x)
-            self.parts[p.getl()] = x
+        with torch._C.DisableTorchFunctionSubclass():   # x may be an SO3partArr: reading its shape would go through Python
+            for x in args:
+                assert isinstance(x, torch.Tensor)
+                self.parts[(x.shape[-2] - 1) // 2] = x
 
     @classmethod
     def _filled(cls, maker, b, adims, tau, device):
@@ -93,10 +93,12 @@ class SO3vecArr:
     def gather(self, gmap, dim=0):
         """Every part (python/src/gelib/SO3vecArr.py:230-234), all of them in one launch where they either all need a gradient
         or none does."""
-        parts = [SO3partArr(p) for p in self.parts.values()]
-        if parts and len({(p.requires_grad, p.device) for p in parts}) == 1:
+        parts = list(self.parts.values())
+        with torch._C.DisableTorchFunctionSubclass():
+            alike = len({(p.requires_grad, p.device) for p in parts}) == 1
+        if alike:
             return SO3vecArr(*SO3partArr_GatherFn.apply(gmap, dim, *parts))
-        return SO3vecArr(*[p.gather(gmap, dim) for p in parts])
+        return SO3vecArr(*[SO3partArr(p).gather(gmap, dim) for p in parts])
 
     def odot(self, y):
         assert list(self.parts.keys()) == list(y.parts.keys())

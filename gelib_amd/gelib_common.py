@@ -1,5 +1,18 @@
 """Helpers shared by the SO3part / SO3vec classes (python/src/gelib/gelib_common.py:15-20 in the reference)."""
+import functools
+
 import torch
+
+
+def without_torch_function(f):
+    """f with the __torch_function__ hooks of the tensor subclasses off while it runs: the parts are torch.Tensor
+    subclasses whose every size, shape or dtype would otherwise take a detour through Python (3 us each; a gather of three
+    parts and its gradient spent more time there than on the GPU)."""
+    @functools.wraps(f)
+    def g(*args):
+        with torch._C.DisableTorchFunctionSubclass():
+            return f(*args)
+    return g
 
 
 def output(shape, x, y):
