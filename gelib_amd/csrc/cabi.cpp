@@ -1275,21 +1275,32 @@ int linear_bwd_entry(const gelib_part_desc *xg, const gelib_part_desc *yg, void 
       d.strides[0] = sh.G01 * rows_cell * n;
       off += (((size_t)cb * sh.G01 * rows_cell * n * sizeof(float2)) + 255) & ~(size_t)255;
     }
-    // 1. the chunk's product
-    if ((rc = vec_fwd_entry(false, (int)P.size(), P.data(), nx, xc.data(), ny, yc.data(), 0, stream))) return rc;
+    // 1. gradients of the matrices straight from the operands where the shapes allow (their partial sums lie where the
+    // chunk's product will be); otherwise the chunk's product, which they are formed from
+    int wg_done = 0;
+    if (wg) {
+      VecPlan cp = sh.plan;
+      cp.E[0] = cbn;
+      std::vector<const gelib_part_desc *> gd, xd, yd;
+      for (auto &v : sh.G) gd.push_back(&gc[v.d - g]);
+      for (auto &v : sh.X) xd.push_back(&xc[v.d - x]);
+      for (auto &v : sh.Y) yd.push_back(&yc[v.d - y]);
+      if ((rc = cg_linear_wgrad(cp, gd, xd, yd, WG, sh.tau, accumulate || b0 > 0, base, pb, s, &wg_done))) return rc;
+      if (!wg_done && (rc = vec_fwd_entry(false, (int)P.size(), P.data(), nx, xc.data(), ny, yc.data(), 0, stream))) return rc;
+    }
     for (size_t k = 0; k < sh.G.size(); k++) {
       const gelib_part_desc &go = gc[sh.G[k].d - g];
       const long long rows = cbn * sh.G01 * (2 * sh.G[k].l + 1);
       const int tau = (int)sh.tau[k], n_out = sh.G[k].n;
       // 2. gradient of the matrix: first chunk straight into wg (or onto it), later chunks through the temporary
-      if (wg) {
+      if (wg && !wg_done) {
         const bool direct = b0 == 0 && !accumulate;
         rc = launch_mix_wgrad(direct ? WG[k] : wg_tmp, (const float2 *)P[k].ptr, (const float2 *)go.ptr, rows, tau, n_out,
                               tau, go.strides[3], wg_ws, wb, s);
         if (rc) return rc == 11 ? GELIB_HIP_ERR_UNSUPPORTED : rc;
         if (!direct && (rc = launch_add_into(WG[k], wg_tmp, (long long)tau * n_out, true, s))) return rc;
       }
-      // 3. gradient of the product, over the product itself
+      // 3. gradient of the product, over the product itself or the sums of 1.
       if (xg || yg) {
         rc = launch_mix((float2 *)P[k].ptr, (const float2 *)go.ptr, W[k], rows, n_out, tau, go.strides[3], tau, true, mix_ws,
                         mb, s);

@@ -233,11 +233,10 @@ uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes_shared(int nr, const gelib_p
  *     wg[k]  (+)= sum over the rows of P_l^H g_l     (the gradient of the matmul of python/src/gelib/SO3vec.py:174-177
  *                                                    with respect to the matrix; w[k] and wg[k] belong to g[k]).
  * Any of xg, yg, wg may be NULL.  Neither P nor gP is ever held at full size (25 GB each at the headline type): the
- * batch is taken in chunks whose product fits the workspace -- the forward kernels form a chunk's product there, the
- * matrix-gradient kernel reads it, gP overwrites it in place and the backward kernels read that -- so the call moves the
- * same bytes as the four separate calls and runs at their speed, in the memory of one chunk.  (One kernel that keeps the
- * product on chip throughout would be no faster on this GPU: it needs two matrix products of 12.3 MFLOP per cell and
- * three product-sized contractions on the vector unit, and for float32 the two units do not run at the same time.)
+ * batch is taken in chunks whose product fits the workspace.  For operands and product up to l = 4, at most 16 channels on
+ * every side and at least about 19 channel pairs per (l1, l2), the matrices' gradients come straight from the operands;
+ * otherwise the forward kernels form a chunk's product there and the matrix-gradient kernel reads it.  gP is formed in that
+ * memory and the backward kernels read it.
  * workspace: 256-byte aligned device memory; gelib_hip_so3vec_cg_linear_bwd_workspace_bytes(..., batch_chunk) tells the
  * bytes that let the call take batch_chunk batch entries at a time (<= 0: the whole batch at once); with less, the call
  * takes smaller chunks, and GELIB_HIP_ERR_WORKSPACE when not even one batch entry fits.  Conditions

@@ -340,3 +340,36 @@ def test_waves_that_share_a_group(cabi, B, tx, ty):
         d = np.abs((got[0][l] - got[1][l]).view(np.float32))
         bound = 4 * 2 * eps * np.repeat(S[l][..., None], 2, -1).reshape(d.shape) + 1e-7
         assert (d <= bound).all(), "l=%d: %g" % (l, float((d / bound).max()))
+
+
+@pytest.mark.parametrize("B,tx,ty,nouts", [
+    (1, {l: 16 for l in range(5)}, {l: 16 for l in range(5)}, [16] * 5),         # less than a tile of cells, whole sums
+    (133, {l: 7 for l in range(5)}, {l: 6 for l in range(5)}, [2, 16, 4, 12, 6]),  # 42 channels a pair: a part of a sum of 32
+    (41, {4: 16, 2: 4}, {0: 16, 4: 10}, [6] * 5),                                # pairs of 256, 160, 64 and 40 channels
+    (300, {2: 16}, {2: 16}, [16] * 5),                                           # one pair, two blocks of its channels
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_matrix_gradient_without_the_product(cabi, B, tx, ty, nouts, accumulate):
+    """Matrix gradients formed straight from the operands, against complex128; a sum of B (2 l + 1) terms in float32 lies
+    within 4 eps32 of the sum of their moduli (the bound of the channel-mixing tests: the matrix cores add term after term,
+    a term here being itself a sum of at most nine)."""
+    xs = [U.seeded(11 + l, B, 2 * l + 1, n) for l, n in sorted(tx.items())]
+    ys = [U.seeded(70 + l, B, 2 * l + 1, n) for l, n in sorted(ty.items())]
+    O = U.VecOracle(xs, ys, 4, False)
+    taus = [p.shape[2] for p in O.r64]
+    assert len(taus) == 5
+    ws = weights(40, taus, nouts)
+    gs = [U.seeded(140 + l, B, 2 * l + 1, nouts[l]) for l in range(5)]
+    start = [U.seeded(240 + l, taus[l], nouts[l]) for l in range(5)]
+    dwg = [U.dev(a) if accumulate else torch.full(a.shape, 9.0, dtype=torch.complex64, device="cuda") for a in start]
+    assert cabi.so3vec_cg_linear_bwd(None, None, dwg, [U.dev(a) for a in gs], [U.dev(a) for a in xs], [U.dev(a) for a in ys],
+                                     [U.dev(a) for a in ws], accumulate=accumulate)
+    torch.cuda.synchronize()
+    eps = 2.0 ** -23
+    for l in range(5):
+        P = O.r64[l].reshape(-1, taus[l])
+        G = gs[l].astype(np.complex128).reshape(-1, nouts[l])
+        want = P.conj().T @ G + (start[l] if accumulate else 0)
+        S = O.Sr[l].reshape(-1, taus[l]).T @ (np.abs(G.real) + np.abs(G.imag)) + (np.abs(start[l]) if accumulate else 0)
+        d = U.host(dwg[l]) - want
+        assert (np.maximum(np.abs(d.real), np.abs(d.imag)) <= 1e-6 + 4 * eps * S).all(), l
