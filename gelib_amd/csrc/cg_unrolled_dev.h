@@ -23,10 +23,10 @@ struct FwdArgs {
   int accumulate;
   long long tile;                  // cells per tile; the blocks of one tile are consecutive
   int blocks_per_tile;
-  int tile_per_xcd;                // consecutive blocks go round the eight XCDs; 1: blocks are numbered so that those of a
-                                   // tile run on one XCD (eight tiles at a time), 0: a tile's blocks go round all of them
   int first_block[kMaxPairs + 1];  // inside a tile, blocks [first_block[p], first_block[p+1]) work on pair p
   int cpb[kMaxPairs];              // cells per block of pair p
+  int tile_per_xcd;                // consecutive blocks go round the eight XCDs; 1: blocks are numbered so that those of a
+                                   // tile run on one XCD (eight tiles at a time), 0: a tile's blocks go round all of them
 };
 
 struct BwdArgs {

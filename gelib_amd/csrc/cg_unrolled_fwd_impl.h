@@ -143,9 +143,12 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
   int pidx = 0, first = 0;
   const int per_tile = a.blocks_per_tile;
   // (with tile_per_xcd the grid is whole groups of eight tiles; the blocks of a tile beyond the last have no cells)
-  const int seq = a.tile_per_xcd ? (int)blockIdx.x >> 3 : (int)blockIdx.x;
-  const int turn = seq / per_tile, in_tile = seq - turn * per_tile;
-  const int tile_idx = a.tile_per_xcd ? 8 * turn + ((int)blockIdx.x & 7) : turn;
+  int tile_idx = (int)blockIdx.x / per_tile, in_tile = (int)blockIdx.x - tile_idx * per_tile;
+  if (a.tile_per_xcd) {
+    const int seq = (int)blockIdx.x >> 3, turn = seq / per_tile;
+    tile_idx = 8 * turn + ((int)blockIdx.x & 7);
+    in_tile = seq - turn * per_tile;
+  }
   static_for<(LT + 1) * (LT + 1)>([&](auto k) __attribute__((always_inline)) {
     if (k.value > 0 && k.value < a.npairs && in_tile >= a.first_block[k.value]) {
       pidx = k.value;
