@@ -7,7 +7,8 @@
 // x-gradient of a part stays in registers over all l2 and the y-gradient adds into a wave-private image in LDS
 // (9 or 25 rows).  Same order of additions on every run.  Measured (one process): L=1, 64 channels, 355113 cells forward
 // 1.40 -> 0.62 ms, backward 2.29 -> 0.88 ms; L=2, 16 channels, 1M cells 2.38 -> 1.86 and 2.82 -> 2.29 ms; L=4, 64
-// channels, 131072 cells backward 7.1 -> 6.7 ms (forward the block form wins there, 5.6 against 6.8 ms, and is kept).
+// channels, 131072 cells backward 7.1 -> 6.7 ms (forward the block form wins there, 5.6 against 6.8 ms, and is kept, but for a
+// one-channel operand up to l = 2, which leaves few pairs: see diag6_vec_fwd).
 #include "cg_diag6_impl.h"
 
 namespace gelib_hip {
