@@ -17,6 +17,7 @@
 #include <cstring>
 
 #include "cg_common.h"
+#include "gather_plan.h"
 
 namespace gelib_hip {
 
@@ -27,13 +28,8 @@ constexpr int kParts = 8;   // parts of one launch; more parts take more launche
 struct GatherPart {
   float2 *r;
   const float2 *x;
-  long long ro, xo;        // strides of the outer index (complex elements)
-  long long rt, xt;        // strides of a target slice / a source slice
-  unsigned per_target;     // threads per (outer, target): slice elements / VEC
-  unsigned long long magic;  // ceil(2^64 / per_target), 0 for per_target == 1
+  GatherSlices s;
   unsigned first_block;
-  int vec;                 // complex elements per thread: 2 (16 bytes) or 1
-  long long total;         // threads
 };
 
 struct GatherVecArgs {
@@ -60,11 +56,11 @@ struct Cplx<2> {
 template <int VEC>
 __device__ __forceinline__ void gather_one(const GatherVecArgs &a, const GatherPart &p, unsigned w) {
   typedef typename Cplx<VEC>::T T;
-  const unsigned row = p.magic ? (unsigned)__umul64hi(p.magic, w) : w;   // outer * targets + t
-  const unsigned q = w - row * p.per_target;
+  const unsigned row = p.s.magic ? (unsigned)__umul64hi(p.s.magic, w) : w;   // outer * targets + t
+  const unsigned q = w - row * p.s.per_target;
   const unsigned o = row < a.targets ? 0u : row / a.targets, t = row - o * a.targets;
-  const float2 *xp = p.x + (long long)o * p.xo + q * VEC;
-  float2 *rp = p.r + (long long)o * p.ro + (long long)t * p.rt + q * VEC;
+  const float2 *xp = p.x + (long long)o * p.s.xo + gather_element(q, VEC);
+  float2 *rp = p.r + (long long)o * p.s.ro + (long long)t * p.s.rt + gather_element(q, VEC);
   const int k0 = a.row_ptr[t], k1 = a.row_ptr[t + 1];
   T acc = {};
   if (a.accumulate) acc = *(const T *)rp;
@@ -75,7 +71,7 @@ __device__ __forceinline__ void gather_one(const GatherVecArgs &a, const GatherP
 #pragma unroll
     for (int i = 0; i < 4; i++) s[i] = a.sources[k + i];
 #pragma unroll
-    for (int i = 0; i < 4; i++) v[i] = *(const T *)(xp + (long long)s[i] * p.xt);
+    for (int i = 0; i < 4; i++) v[i] = *(const T *)(xp + (long long)s[i] * p.s.xt);
 #pragma unroll
     for (int i = 0; i < 4; i++) Cplx<VEC>::add(acc, v[i]);
   }
@@ -85,7 +81,7 @@ __device__ __forceinline__ void gather_one(const GatherVecArgs &a, const GatherP
 #pragma unroll
     for (int i = 0; i < 3; i++) s[i] = a.sources[k + i < k1 ? k + i : k1 - 1];
 #pragma unroll
-    for (int i = 0; i < 3; i++) v[i] = *(const T *)(xp + (long long)s[i] * p.xt);
+    for (int i = 0; i < 3; i++) v[i] = *(const T *)(xp + (long long)s[i] * p.s.xt);
 #pragma unroll
     for (int i = 0; i < 3; i++)
       if (k + i < k1) Cplx<VEC>::add(acc, v[i]);
@@ -99,8 +95,8 @@ __global__ void __launch_bounds__(256) gather_vec_kernel(const GatherVecArgs a) 
   for (int k = 1; k < kParts; k++)
     if (k < a.nparts && blockIdx.x >= a.p[k].first_block) p = a.p[k];
   const long long w = (long long)(blockIdx.x - p.first_block) * 256 + threadIdx.x;
-  if (w >= p.total) return;
-  if (p.vec == 2) gather_one<2>(a, p, (unsigned)w);
+  if (w >= p.s.total) return;
+  if (p.s.vec == 2) gather_one<2>(a, p, (unsigned)w);
   else gather_one<1>(a, p, (unsigned)w);
 }
 
@@ -162,38 +158,6 @@ int launch_any(const GatherJob &j, int dim, const int *row_ptr, const int *sourc
   return hipGetLastError() == hipSuccess ? 0 : 10;
 }
 
-// The part as the vector kernel sees it: what follows the gathered dimension is one contiguous slice in both tensors, what
-// precedes it one index with one stride.  False: the kernel for any strides takes the part.
-bool to_slices(const GatherJob &j, int dim, GatherPart *p) {
-  long long slice = 1;
-  for (int k = 4; k > dim; k--) {
-    if (j.D[k] > 1 && (j.rs[k] != slice || j.xs[k] != slice)) return false;
-    slice *= j.D[k];
-  }
-  long long outer = 1;
-  p->ro = p->xo = 0;
-  for (int k = dim - 1; k >= 0; k--) {   // the innermost of the outer dimensions first
-    if (j.D[k] == 1) continue;
-    if (outer > 1 && (j.rs[k] != p->ro * outer || j.xs[k] != p->xo * outer)) return false;
-    if (outer == 1) p->ro = j.rs[k], p->xo = j.xs[k];
-    outer *= j.D[k];
-  }
-  p->r = j.r;
-  p->x = j.x;
-  p->rt = j.rs[dim];
-  p->xt = j.xs[dim];
-  const bool wide = slice % 2 == 0 && ((uintptr_t)j.r & 15) == 0 && ((uintptr_t)j.x & 15) == 0 && p->rt % 2 == 0 &&
-                    p->xt % 2 == 0 && p->ro % 2 == 0 && p->xo % 2 == 0;
-  p->vec = wide ? 2 : 1;
-  const long long per = slice / p->vec;
-  p->total = outer * j.D[dim] * per;
-  if (p->total >= (1LL << 32) - 256) return false;   // the kernel's thread index is 32 bits
-  p->per_target = (unsigned)per;
-  // floor(w / per) = high half of w * ceil(2^64 / per): exact for every 32-bit w
-  p->magic = per > 1 ? ~0ull / (unsigned long long)per + 1 : 0;
-  return true;
-}
-
 }  // namespace
 
 int launch_gather(const std::vector<GatherJob> &jobs, int dim, const int *row_ptr, const int *sources, bool accumulate,
@@ -214,15 +178,17 @@ int launch_gather(const std::vector<GatherJob> &jobs, int dim, const int *row_pt
   for (auto &j : jobs) {
     GatherPart p;
     int rc = 0;
-    if (!to_slices(j, dim, &p)) {
+    if (!gather_slices(j.rs, j.xs, j.D, dim, (((uintptr_t)j.r | (uintptr_t)j.x) & 15) == 0, &p.s)) {
       if ((rc = launch_any(j, dim, row_ptr, sources, accumulate, s))) return rc;
       continue;
     }
     a.targets = (unsigned)j.D[dim];   // the same for every part: the map says it
-    const unsigned nb = (unsigned)((p.total + 255) / 256);
+    const unsigned nb = (unsigned)((p.s.total + 255) / 256);
     if (a.nparts == kParts || blocks > 0x7fffffffu - nb) {
       if ((rc = flush())) return rc;
     }
+    p.r = j.r;
+    p.x = j.x;
     p.first_block = blocks;
     blocks += nb;
     a.p[a.nparts++] = p;
