@@ -23,8 +23,6 @@ namespace gelib_hip {
 
 namespace {
 
-constexpr int kParts = 8;   // parts of one launch; more parts take more launches
-
 struct GatherPart {
   float2 *r;
   const float2 *x;
@@ -33,7 +31,7 @@ struct GatherPart {
 };
 
 struct GatherVecArgs {
-  GatherPart p[kParts];
+  GatherPart p[kGatherParts];
   const int *row_ptr;      // [targets + 1]
   const int *sources;      // [row_ptr[targets]]
   unsigned targets;
@@ -92,7 +90,7 @@ __device__ __forceinline__ void gather_one(const GatherVecArgs &a, const GatherP
 __global__ void __launch_bounds__(256) gather_vec_kernel(const GatherVecArgs a) {
   GatherPart p = a.p[0];
 #pragma unroll
-  for (int k = 1; k < kParts; k++)
+  for (int k = 1; k < kGatherParts; k++)
     if (k < a.nparts && blockIdx.x >= a.p[k].first_block) p = a.p[k];
   const long long w = (long long)(blockIdx.x - p.first_block) * 256 + threadIdx.x;
   if (w >= p.s.total) return;
@@ -183,10 +181,8 @@ int launch_gather(const std::vector<GatherJob> &jobs, int dim, const int *row_pt
       continue;
     }
     a.targets = (unsigned)j.D[dim];   // the same for every part: the map says it
-    const unsigned nb = (unsigned)((p.s.total + 255) / 256);
-    if (a.nparts == kParts || blocks > 0x7fffffffu - nb) {
-      if ((rc = flush())) return rc;
-    }
+    const unsigned nb = (unsigned)gather_blocks(p.s.total);
+    if (!gather_shares_launch(a.nparts, blocks, nb) && (rc = flush())) return rc;
     p.r = j.r;
     p.x = j.x;
     p.first_block = blocks;

@@ -3,6 +3,16 @@
 
 namespace gelib_hip {
 
+// A launch holds fewer than 2^32 threads in all (gridDim.x * blockDim.x), so this many blocks of 256.
+constexpr long long kGatherMaxBlocks = (1LL << 24) - 1;
+constexpr int kGatherParts = 8;   // parts of one launch; more parts take more launches
+
+constexpr long long gather_blocks(long long threads) { return (threads + 255) / 256; }
+// Does a part of `more` blocks go into a launch that holds `parts` parts of `blocks` blocks in all?
+constexpr bool gather_shares_launch(int parts, long long blocks, long long more) {
+  return parts < kGatherParts && blocks + more <= kGatherMaxBlocks;
+}
+
 struct GatherSlices {
   long long ro, xo;          // strides of the outer index (complex elements)
   long long rt, xt;          // strides of a target slice / a source slice
@@ -40,7 +50,7 @@ inline bool gather_slices(const long long rs[5], const long long xs[5], const lo
   p->vec = wide ? 2 : 1;
   const long long per = slice / p->vec;
   p->total = outer * D[dim] * per;
-  if (p->total >= (1LL << 32) - 256) return false;   // the kernel's thread index is 32 bits
+  if (gather_blocks(p->total) > kGatherMaxBlocks) return false;   // (which also keeps the kernel's thread index below 2^32)
   p->per_target = (unsigned)per;
   // floor(w / per) = high half of w * ceil(2^64 / per): exact for every 32-bit w
   p->magic = per > 1 ? ~0ull / (unsigned long long)per + 1 : 0;
