@@ -17,6 +17,7 @@ int g_fwd_lds_bytes = 16 * 1024;     // LDS one forward block may use for its st
 int g_fwd_cell_tile = -1;            // cells per tile of the forward launch (0 = all cells in one tile, -1 = by channels)
 int g_fwd_narrow_decline = 1;  // leave products with at most four channel pairs per block to the any-l forward kernel
 int g_fwd_tile_per_xcd = -1;          // blocks of a tile on one XCD (-1 = by the alignment of the blocks, 0 no, 1 yes)
+int g_fwd_max_blocks = 0;             // most blocks of a launch (0 = what HIP allows); more take several launches
 int g_fwd_ti = 0;                    // 0 = widest tile that divides every n1, else force 1 / 2 / 4
 int g_bwd_enable = 1;
 int g_bwd_one_enable = 1; // the backward kernel for calls with one triple
@@ -384,17 +385,27 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
     lds_bytes = std::max(lds_bytes, (size_t)(cpb * op_bytes));
     a.first_block[i] = (int)nblocks;
     nblocks += (tile + cpb - 1) / cpb;
-    if (nblocks > 0x7fffffffLL) return GELIB_HIP_ERR_ARG;
+    if (nblocks >= 1LL << 24) return GELIB_HIP_ERR_ARG;   // a tile of all cells, on request
   }
   a.first_block[a.npairs] = (int)nblocks;  // blocks of one tile
   a.tile = tile;
   a.blocks_per_tile = (int)nblocks;
   a.tile_per_xcd = want_xcd ? 1 : 0;
-  const long long ntiles = (ncells + tile - 1) / tile;
-  nblocks *= a.tile_per_xcd ? (ntiles + 7) / 8 * 8 : ntiles;
-  if (nblocks > 0x7fffffffLL) return GELIB_HIP_ERR_ARG;
-  rc = launch_unrolled_fwd(a, diag, ti, ragged, lcap, lop, (int)nblocks, lds_bytes, s);
-  if (rc) return rc;
+  // A launch holds fewer than 2^32 threads, so at most 2^24 - 1 blocks; more tiles than that allows take further launches,
+  // each on the cells behind those of the last.
+  const long long unit = a.tile_per_xcd ? 8 : 1, most = g_fwd_max_blocks > 0 ? g_fwd_max_blocks : (1LL << 24) - 1;
+  const long long ntiles = (ncells + tile - 1) / tile, per_launch = std::max<long long>(unit, most / nblocks / unit * unit);
+  for (long long t0 = 0; t0 < ntiles; t0 += per_launch) {
+    const long long here = std::min(per_launch, ntiles - t0);
+    a.ncells = std::min(ncells - t0 * tile, here * tile);
+    rc = launch_unrolled_fwd(a, diag, ti, ragged, lcap, lop, (int)((here + unit - 1) / unit * unit * nblocks), lds_bytes, s);
+    if (rc) return rc;
+    for (auto *parts : {a.x, a.y})
+      for (int i = 0; i < kFastIn; i++)
+        if (parts[i].ptr) parts[i].ptr += here * tile * parts[i].sb;
+    for (auto &R : a.r)
+      if (R.ptr) R.ptr += here * tile * R.sb;
+  }
   *used = 1;
   return GELIB_HIP_OK;
 }
@@ -668,6 +679,11 @@ int unrolled_set_option(const char *name, int value) {
   if (!std::strcmp(name, "fwd_tile_per_xcd")) {
     if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
     g_fwd_tile_per_xcd = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "fwd_max_blocks")) {
+    if (value < 0 || value >= 1 << 24) return GELIB_HIP_ERR_ARG;
+    g_fwd_max_blocks = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "fwd_narrow_decline")) {

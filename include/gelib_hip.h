@@ -314,6 +314,7 @@ int gelib_hip_set_stream_workspace(void *stream, void *ptr, uint64_t bytes);
  * "bcast_reduce" (1/0): 0 sums such a destination inside the shape-agnostic kernels, one cell after the other.
  * Tuning knobs of the fast families (0 restores the built-in choice unless noted): "unrolled_fwd" / "unrolled_bwd" /
  * "staged_fwd" / "staged_bwd" / "diag6" / "onepair" (1/0: use the family), "fwd_block_bytes", "fwd_lds_bytes", "fwd_tile", "fwd_tile_per_xcd" (-1, 0, 1),
+ * "fwd_max_blocks" (blocks of one unrolled forward launch; more take several launches),
  * "diag6_tight" / "diag6_small4_fwd" (-1, 0, 1: (cell, channel) pairs without gaps / the wave-per-cell forward kernel up to l = 4),
  * "fwd_cell_tile" (cells per tile of the unrolled forward launch, 0 = one tile, -1 = chosen by the channel counts, the
  * default), "bwd_lds_target" (LDS bytes per block the unrolled backward kernels aim at when they choose their cells per

@@ -269,3 +269,39 @@ def test_tuning_options_leave_the_results_alone(cabi):
 ])
 def test_forward_with_partial_lines_and_idle_channels(cabi, case):
     run_vec(cabi, *case, False, 77, False)
+
+
+@pytest.mark.parametrize("B,tx,ty,maxl,tile", [
+    (2131, {0: 5, 1: 3, 2: 1}, {0: 3, 2: 3}, -1, -1),      # tiles of 64 cells per XCD: groups of eight tiles a launch
+    (101, {0: 16, 1: 16, 2: 16}, {0: 8, 1: 8}, 2, 16),     # tiles that go round the XCDs, a last one that is short
+    (33, {1: 8}, {2: 8}, -1, 8),
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_forward_product_in_several_launches(cabi, B, tx, ty, maxl, tile, accumulate):
+    """More blocks than a launch holds: the cells go into launches one behind the other, with the same bits; the last case's
+    second operand is shared by the batch."""
+    xs = [U.dev(U.seeded(500 + l, B, 2 * l + 1, n)) for l, n in sorted(tx.items())]
+    ys = [U.dev(U.seeded(540 + l, 1 if B == 33 else B, 2 * l + 1, n)) for l, n in sorted(ty.items())]
+    tau = cabi.so3type_product(tx, ty, maxl)
+    got = []
+    try:
+        cabi.set_option("fwd_cell_tile", tile)
+        for blocks in (0, 1, 40):
+            cabi.set_option("fwd_max_blocks", blocks)
+            rs = [torch.full((B, 2 * l + 1, n), 2.0 - 1j, dtype=torch.complex64, device="cuda") for l, n in sorted(tau.items())]
+            cabi.so3vec_fwd(rs, xs, ys, accumulate=accumulate)
+            assert cabi.last_path() == 2
+            torch.cuda.synchronize()
+            got.append([U.host(r) for r in rs])
+    finally:
+        cabi.set_option("fwd_max_blocks", 0)
+        cabi.set_option("fwd_cell_tile", -1)
+    want = got[0]
+    run = U.VecOracle([U.host(t) for t in xs], [np.broadcast_to(U.host(t), (B,) + tuple(t.shape[1:])).copy() for t in ys], maxl, False)
+    if accumulate:
+        run.check_fwd_onto(want, [np.full(r.shape, 2.0 - 1j, np.complex64) for r in want], "one launch")
+    else:
+        run.check_fwd(want, "one launch")
+    for other in got[1:]:
+        for a, b in zip(want, other):
+            assert np.array_equal(a, b)
