@@ -26,6 +26,7 @@ thread_local std::string t_last_error;
 thread_local int t_last_path = kPathNone;
 int g_force_generic = 0;
 int g_check_pointers = 1;
+int g_linear_wgrad = 1;  // gradients of the weight matrices straight from the operands, where the shapes allow
 }  // namespace
 
 int record_hip_error(hipError_t e, const char *what) {
@@ -1139,8 +1140,9 @@ int linear_fwd_entry(int nr, const gelib_part_desc *r, int nx, const gelib_part_
 // ---- backward of CGproduct followed by the weight matrices, in bounded memory ------------------------------------
 // out_l = P_l W_l with P = CGproduct(x, y):  xg, yg = the product's backward pass on gP_l = gout_l W_l^H, and
 // wg_l = sum over the rows of P_l^H gout_l.  Neither P nor gP is ever held at full size: the batch is taken in chunks
-// whose product fits the caller's workspace; a chunk's product is formed by the forward kernels, read by the
-// matrix-gradient kernel, overwritten in place by gP and read once more by the backward kernels.
+// whose product fits the caller's workspace.  The matrices' gradients of a chunk come straight from the operands where
+// cg_linear_wgrad takes them; otherwise the forward kernels form the chunk's product and the matrix-gradient kernel reads it.
+// gP is formed in the same memory and read by the backward kernels.
 struct LinBwdShape {
   std::vector<View> G, X, Y, XG, YG;
   VecPlan plan;
@@ -1285,7 +1287,7 @@ int linear_bwd_entry(const gelib_part_desc *xg, const gelib_part_desc *yg, void 
       for (auto &v : sh.G) gd.push_back(&gc[v.d - g]);
       for (auto &v : sh.X) xd.push_back(&xc[v.d - x]);
       for (auto &v : sh.Y) yd.push_back(&yc[v.d - y]);
-      if ((rc = cg_linear_wgrad(cp, gd, xd, yd, WG, sh.tau, accumulate || b0 > 0, base, pb, s, &wg_done))) return rc;
+      if (g_linear_wgrad && (rc = cg_linear_wgrad(cp, gd, xd, yd, WG, sh.tau, accumulate || b0 > 0, g_linear_wgrad >= 2, base, pb, s, &wg_done))) return rc;
       if (!wg_done && (rc = vec_fwd_entry(false, (int)P.size(), P.data(), nx, xc.data(), ny, yc.data(), 0, stream))) return rc;
     }
     for (size_t k = 0; k < sh.G.size(); k++) {
@@ -1312,6 +1314,8 @@ int linear_bwd_entry(const gelib_part_desc *xg, const gelib_part_desc *yg, void 
       rc = vec_bwd_entry(false, xg ? xgc.data() : nullptr, yg ? ygc.data() : nullptr, (int)P.size(), P.data(), nx, xc.data(),
                          ny, yc.data(), accumulate, stream);
       if (rc) return rc;
+    } else if (wg_done) {
+      t_last_path = kPathLinear;
     }
   }
   return GELIB_HIP_OK;
@@ -1761,6 +1765,10 @@ int gelib_hip_set_option(const char *name, int value) {
   if (!std::strcmp(name, "check_pointers")) {
     g_check_pointers = value;
     forget_ranges(nullptr);
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "linear_wgrad")) {
+    g_linear_wgrad = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "bcast_scratch_kb")) {  // KiB the temporary of a broadcast gradient destination may take

@@ -27,11 +27,11 @@ int cg_linear_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
                   int *used);
 
 // wg_l (+)= sum over the rows of P_l^H g_l with P never stored (cg_linear_wgrad.hip); g, wg and tau (channels of the product's
-// parts) in the same order.  *used = 0 when the shapes are not ones the kernel takes or ws has no room for the sums of one
-// range of cells (nothing has been launched then).
+// parts) in the same order.  *used = 0 when the shapes are not ones the kernel takes (force: nor ones it is fast on) or ws has
+// no room for the sums of one range of cells (nothing has been launched then).
 int cg_linear_wgrad(const VecPlan &plan, const std::vector<const gelib_part_desc *> &g,
                     const std::vector<const gelib_part_desc *> &x, const std::vector<const gelib_part_desc *> &y,
-                    const std::vector<float2 *> &wg, const std::vector<long long> &tau, bool accumulate, void *ws,
+                    const std::vector<float2 *> &wg, const std::vector<long long> &tau, bool accumulate, bool force, void *ws,
                     size_t ws_bytes, hipStream_t s, int *used);
 
 }  // namespace gelib_hip

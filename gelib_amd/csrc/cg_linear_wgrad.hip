@@ -15,11 +15,18 @@
 // operations), then one multiply-add per term and one matrix instruction per row (l, m).  The coefficients are the same for
 // all lanes: scalar loads.  The sums of the ranges go to memory and a second kernel adds them in the order of the ranges:
 // no atomics, the same bits every run.
+// Sums in two levels: the matrix instructions add the 2 (2 l + 1) terms of each of eight cells, and those sums are added to a
+// second set of registers.  One chain of matrix instructions over a range was up to twice as far from the exact result as
+// forming the product and summing it in mix.hip, whose chains are at least 128 rows long (relative error for l = 0..4, one chain /
+// two levels / mix.hip, in 1e-7: 8192 cells of 16 x 16 -> 16 channels 2.0 3.0 3.8 4.4 4.9 / 1.4 1.7 2.0 2.2 2.5 /
+// 2.3 2.3 2.3 2.4 2.6; 8 x 8 2.6 4.0 5.0 5.9 6.6 / 1.4 1.7 2.0 2.2 2.5 / 2.3 2.4 2.5 2.6 2.8; 16 cells of 16 x 16
+// 1.2 1.8 2.3 2.8 3.1 / 0.9 1.4 1.7 2.0 2.2 / 1.0 1.4 1.7 2.0 2.3).  The second set takes the kernel from three waves per
+// SIMD to two: 8192 cells of 16 x 16 channels 1755 -> 2090 us, 8 x 8 767 -> 920.
 // What bounds it: matrix instructions (64 clocks a row and 32 channels) plus vector instructions (4 clocks each, about 2600
 // a cell and 32 channels of the L = 4 product), which do not overlap within a wave; the operands come from L2.
-// Measured against forming the product, the matrix-gradient kernels of mix.hip on it and their sums (8192 cells of L = 4,
-// microseconds): 16 x 16 -> 16 channels 2975 -> 1985 (0.10 TFLOP of
-// matrix products, 52 TFLOP/s), 8 x 8 -> 16 1180 -> 722, 7 x 6 -> 12 1284 -> 716; 1000 cells, 16 x 16 514 -> 224; 64 cells 138 -> 71.
+// Measured against forming the product, the matrix-gradient kernels of mix.hip on it and their sums (L = 4, 16 outputs,
+// microseconds, in 1 GiB): 8192 cells of 16 x 16 channels 4414 -> 2091, of 8 x 8 1107 -> 917; 1024 cells 543 -> 263 and
+// 192 -> 140; 64 cells of 16 x 16 153 -> 81.
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -36,7 +43,10 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 typedef const __attribute__((address_space(4))) float *CoeffPtr;
 
 constexpr int kWNL = kLinL + 1;
-constexpr double kWgradLeast = 0.6;
+constexpr double kWgradLeast = 0.6;      // share of a sum's 32 rows that are channels
+constexpr double kWgradLeastMany = 0.39;  // share of a block's 128 channels, for more cells than
+constexpr long long kWgradFew = 2048;
+constexpr long long kWgradCells = 16;    // fewer: mix.hip's chains are shorter than those of eight cells here
 constexpr int kWPairs = kWNL * kWNL;
 constexpr int kWTile = 8;                       // cells staged at a time
 constexpr int kWRow = 16;                       // complex numbers of a staged row of g (columns beyond its channels are zero)
@@ -66,20 +76,17 @@ __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, fl
   const bool busy = c0 < nch;               // uniform for the wave; idle waves only stage
   const int c = imin(c0 + i, nch - 1), ca = c / n2, cj = c - ca * n2;
   const float sign = (h && (i & 1)) ? -1.f : 1.f;
-  f16v acc[NLP];
+  f16v acc[NLP], sum[NLP];
 #pragma unroll
   for (int k = 0; k < NLP; k++)
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[k][e] = 0.f;
+    for (int e = 0; e < 16; e++) acc[k][e] = sum[k][e] = 0.f;
 
   const long long first = (long long)range * a.cells_per_range;
   const long long last = first + a.cells_per_range < a.ncells ? first + a.cells_per_range : a.ncells;
   for (long long cell0 = first; cell0 < last; cell0 += kWTile) {
     const int cells = last - cell0 < kWTile ? (int)(last - cell0) : kWTile;
     __syncthreads();
-    // (with the divisions taken out of the loop, offsets kept in registers instead, the kernel needs 201 registers -- two
-    // waves per SIMD, 2.15 ms -- or, held to three waves, spills: 1.94 ms at 16 x 16 channels, but 0.79 at 8 x 8 where this
-    // takes 0.71)
     for (int e = tid; e < cells * R1 * n1; e += 256) {
       const int t = e / (R1 * n1), r = e - t * (R1 * n1), m = r / n1;
       xs[t * kWOp + r] = X.ptr[(cell0 + t) * X.sb + (long long)m * X.sm + (r - m * n1)];
@@ -102,8 +109,8 @@ __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, fl
     if (!busy) continue;
     for (int t = 0; t < cells; t++) {
       // opaque per cell: hoisted out of the loop the coefficients fill the scalar registers many times over and are
-      // spilled into vector-register lanes, one more vector instruction per term (8192 cells, 16 channels: 2.48 ms instead
-      // of 1.97; two cells per step sharing them: 2.07, at two waves per SIMD instead of three)
+      // spilled into vector-register lanes, one more vector instruction per term (8192 cells, 16 channels, sums in one
+      // level: 2.48 ms instead of 1.97)
       unsigned long long bank = (unsigned long long)a.bank;
       asm volatile("" : "+s"(bank));
       const CoeffPtr C = (CoeffPtr)bank;
@@ -144,6 +151,13 @@ __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, fl
         });
       });
     }
+#pragma unroll
+    for (int k = 0; k < NLP; k++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        sum[k][e] += acc[k][e];
+        acc[k][e] = 0.f;
+      }
   }
   if (!busy) return;
   // register e of a sum: channel 8 (e / 4) + 4 h + e % 4, column i
@@ -153,7 +167,7 @@ __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, fl
 #pragma unroll
     for (int e = 0; e < 16; e++) {
       const int row = 8 * (e / 4) + 4 * h + (e % 4);
-      if (c0 + row < nch) out[row * 32] = acc[dc.value][e];
+      if (c0 + row < nch) out[row * 32] = sum[dc.value][e];
     }
   });
 }
@@ -167,23 +181,28 @@ __global__ void __launch_bounds__(256, 2) linear_wgrad_kernel(const LinWgradArgs
   });
 }
 
-// one thread per complex element of the matrices' gradients
+// One channel's row of its matrix's gradient per block: 16 threads an element, each adding a sixteenth of the ranges, whose
+// sums are then added in their order (one chain over all ranges, up to 768 of them, would be the longest sum of all).
 __global__ void __launch_bounds__(256) linear_wgrad_sum_kernel(const LinWgradArgs a) {
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  const int o = (int)(idx & 15);
-  const long long ch = idx >> 4, all = a.base[kWNL];
-  if (ch >= all) return;
+  __shared__ float2 sums[16][16];
+  const int o = (int)threadIdx.x & 15, part = (int)threadIdx.x >> 4;
+  const long long ch = blockIdx.x, all = a.base[kWNL];
+  const float2 *p = (const float2 *)a.partial + ch * 16 + o;
+  float2 s = make_float2(0.f, 0.f);
+#pragma unroll 4
+  for (int r = a.nranges * part / 16; r < a.nranges * (part + 1) / 16; r++) {
+    const float2 v = p[(long long)r * all * 16];
+    s.x += v.x;
+    s.y += v.y;
+  }
+  sums[part][o] = s;
+  __syncthreads();
+  if (part != 0) return;
+#pragma unroll
+  for (int k = 1; k < 16; k++) s.x += sums[k][o].x, s.y += sums[k][o].y;
   static_for<kWNL>([&](auto lc) __attribute__((always_inline)) {
     constexpr int l = decltype(lc)::value;
     if (ch >= a.base[l] && ch < a.base[l + 1] && o < a.g[l].n) {
-      const float2 *p = (const float2 *)a.partial + ch * 16 + o;
-      float2 s = make_float2(0.f, 0.f);
-#pragma unroll 8
-      for (int r = 0; r < a.nranges; r++) {
-        const float2 v = p[(long long)r * all * 16];
-        s.x += v.x;
-        s.y += v.y;
-      }
       float2 *q = a.wg[l] + (ch - a.base[l]) * a.g[l].n + o;
       if (a.accumulate) {
         s.x += q->x;
@@ -198,7 +217,7 @@ __global__ void __launch_bounds__(256) linear_wgrad_sum_kernel(const LinWgradArg
 
 int cg_linear_wgrad(const VecPlan &plan, const std::vector<const gelib_part_desc *> &g,
                     const std::vector<const gelib_part_desc *> &x, const std::vector<const gelib_part_desc *> &y,
-                    const std::vector<float2 *> &wg, const std::vector<long long> &tau, bool accumulate, void *ws,
+                    const std::vector<float2 *> &wg, const std::vector<long long> &tau, bool accumulate, bool force, void *ws,
                     size_t ws_bytes, hipStream_t s, int *used) {
   *used = 0;
   if (plan.diag || plan.triples.empty() || ((uintptr_t)ws & 15)) return GELIB_HIP_OK;
@@ -226,7 +245,7 @@ int cg_linear_wgrad(const VecPlan &plan, const std::vector<const gelib_part_desc
   for (auto &t : plan.triples) a.offs[t.l1][t.l2][t.l] = t.offs;
   // every pair reaches every l of its range up to kLinL, as the kernel assumes, and the channels of a matrix are those the
   // pairs feed
-  double useful = 0, padded = 0;
+  double useful = 0, padded = 0, blocks = 0;
   for (auto &p : lx)
     for (auto &q : ly) {
       int have = 0;
@@ -236,21 +255,28 @@ int cg_linear_wgrad(const VecPlan &plan, const std::vector<const gelib_part_desc
       const double rows = (2.0 * p.first + 1) * (2 * q.first + 1);
       useful += rows * (double)n;
       padded += rows * (double)((n + 31) / 32 * 32);
+      blocks += rows * (double)((n + 127) / 128 * 128);
     }
-  // Channels fill the 32 rows of a sum; with fewer than 19 channels a pair half the matrix work is padding, and the product
-  // of so few channels is small enough to store (4 x 4 channels stay with the kernels of mix.hip).
-  if (useful < kWgradLeast * padded) return GELIB_HIP_OK;
+  const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
+  if (ncells < kWgradCells) return GELIB_HIP_OK;
+  // Channels fill the 32 rows of a sum and the 128 of a block; with fewer than 19 channels a pair half the matrix work is
+  // padding, and with fewer than 50 most waves of a block only stage.  The product of so few channels is small enough to store
+  // once there are cells enough to hide the launches that takes (with the gradients of x and y, product stored / not, us, 12
+  // outputs: 32 channels a pair, 256 cells 263 / 193, 1536 cells 345 / 320, 2048 365 / 361, 3072 524 / 533, 8192 1055 / 1270;
+  // 40 channels 2048 cells 468 / 450, 5000 904 / 1019; 48 channels 5000 cells 995 / 1068; 50 channels 8192 cells 2057 / 2042,
+  // 64 channels 2146 / 1938).
+  const bool few = ncells <= kWgradFew;
+  if (!force && (useful < kWgradLeast * padded || (!few && useful < kWgradLeastMany * blocks))) return GELIB_HIP_OK;
   int nwork = 0;
   for (int k = 0; k < kWPairs; k++) {
     const int l1 = kLinL - k / kWNL, l2 = kLinL - k % kWNL;
     a.first[k] = nwork;
-    if (a.x[l1].ptr && a.y[l2].ptr && l1 + l2 >= 0) nwork += (a.x[l1].n * a.y[l2].n + 127) / 128;
+    if (a.x[l1].ptr && a.y[l2].ptr) nwork += (a.x[l1].n * a.y[l2].n + 127) / 128;
   }
   a.first[kWPairs] = nwork;
-  const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
-  if (nwork == 0 || ncells == 0) return GELIB_HIP_OK;
-  // ranges of cells: three blocks per place of the GPU (two blocks a compute unit), at least two tiles of cells each, as far
-  // as the memory for their sums goes
+  if (nwork == 0) return GELIB_HIP_OK;
+  // ranges of cells: three blocks per place of the GPU (two blocks a compute unit: two waves per SIMD), at least two tiles of
+  // cells each, as far as the memory for their sums goes
   const long long fit = (long long)(ws_bytes / ((size_t)a.base[kWNL] * 32 * sizeof(float)));
   long long nranges = std::min<long long>({(1536LL + nwork - 1) / nwork, (ncells + 2 * kWTile - 1) / (2 * kWTile), fit});
   if (nranges < 1) return GELIB_HIP_OK;
@@ -264,8 +290,7 @@ int cg_linear_wgrad(const VecPlan &plan, const std::vector<const gelib_part_desc
   a.accumulate = accumulate ? 1 : 0;
   hipLaunchKernelGGL(linear_wgrad_kernel, dim3((unsigned)(nwork * nranges)), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
-  const long long threads = a.base[kWNL] * 16;
-  hipLaunchKernelGGL(linear_wgrad_sum_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(linear_wgrad_sum_kernel, dim3((unsigned)a.base[kWNL]), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   *used = 1;
   return GELIB_HIP_OK;

@@ -233,9 +233,10 @@ uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes_shared(int nr, const gelib_p
  *     wg[k]  (+)= sum over the rows of P_l^H g_l     (the gradient of the matmul of python/src/gelib/SO3vec.py:174-177
  *                                                    with respect to the matrix; w[k] and wg[k] belong to g[k]).
  * Any of xg, yg, wg may be NULL.  Neither P nor gP is ever held at full size (25 GB each at the headline type): the
- * batch is taken in chunks whose product fits the workspace.  For operands and product up to l = 4, at most 16 channels on
- * every side and at least about 19 channel pairs per (l1, l2), the matrices' gradients come straight from the operands;
- * otherwise the forward kernels form a chunk's product there and the matrix-gradient kernel reads it.  gP is formed in that
+ * batch is taken in chunks whose product fits the workspace.  For operands up to l = 4, a product with every l up
+ * to min(l1 + l2, 4), at most 16 channels on every side, at least about 19 channel pairs per (l1, l2) (50 in chunks of more than
+ * 2048 cells) and 16 cells, the matrices' gradients come straight from the operands; otherwise the forward kernels form a
+ * chunk's product there and the matrix-gradient kernel reads it.  gP is formed in that
  * memory and the backward kernels read it.
  * workspace: 256-byte aligned device memory; gelib_hip_so3vec_cg_linear_bwd_workspace_bytes(..., batch_chunk) tells the
  * bytes that let the call take batch_chunk batch entries at a time (<= 0: the whole batch at once); with less, the call
@@ -311,6 +312,8 @@ int gelib_hip_set_stream_workspace(void *stream, void *ptr, uint64_t bytes);
  * still passes until its entry is pushed out -- gelib_hip_free forgets the entry, setting the option (to any value)
  * forgets all of them, and 2 asks the driver on every call (about 30 us per call instead of 3).
  * "bcast_scratch_kb": KiB the temporary of a broadcast gradient destination may take (0 restores 64 MiB);
+ * "linear_wgrad" (1/0: gradients of the weight matrices straight from the operands where that is faster; 2: wherever it can be
+ * done);
  * "bcast_reduce" (1/0): 0 sums such a destination inside the shape-agnostic kernels, one cell after the other.
  * Tuning knobs of the fast families (0 restores the built-in choice unless noted): "unrolled_fwd" / "unrolled_bwd" /
  * "staged_fwd" / "staged_bwd" / "diag6" / "onepair" (1/0: use the family), "fwd_block_bytes", "fwd_lds_bytes", "fwd_tile", "fwd_tile_per_xcd" (-1, 0, 1),
@@ -342,7 +345,8 @@ int gelib_hip_set_stream_workspace(void *stream, void *ptr, uint64_t bytes);
  * GELIB_HIP_ERR_ARG.  Options are process-wide.
  * gelib_hip_last_path() tells which kernel family the last call of this thread used
  * (0 = none, 1 = generic, 2 = unrolled small-l kernels, 3 = staged any-l kernels, 4 = lane-per-channel Diag
- * kernels for operand l up to 6, 5 = single-pair kernels for large l, 6 = the product fused with the weight matrices).
+ * kernels for operand l up to 6, 5 = single-pair kernels for large l, 6 = the product fused with the weight matrices, or
+ * the matrices' gradients alone, straight from the operands).
  */
 int gelib_hip_set_option(const char *name, int value);
 int gelib_hip_last_path(void);
