@@ -75,7 +75,7 @@ class SO3partArr(torch.Tensor):
     def gather(self, gmap, dim=0):
         """Sums of cells along grid dimension dim: cell t of the result = sum of the cells s of self over the pairs
         (s, t) of gmap (python/src/gelib/SO3partArr.py:142-146)."""
-        return SO3partArr_GatherFn.apply(gmap, dim, self)[0]
+        return SO3partArr_GatherFn.apply(self, gmap, dim)
 
     def CGproduct(self, y, l):
         return SO3partArr_CGproductFn.apply(self, y, l)
@@ -123,36 +123,45 @@ SO3partArr_CGproductFn = _part_fn(False)
 SO3partArr_DiagCGproductFn = _part_fn(True)
 
 
+@without_torch_function
+def gathered(gmap, d, xs):
+    """The parts xs gathered along grid dimension d, each result written by the launch that sums it (one launch for all)."""
+    from gelib_amd.gather_map import gather_map
+    assert isinstance(gmap, gather_map)
+    rs = []
+    for x in xs:
+        shape = list(x.size())
+        adims = shape[1:-2]
+        assert 0 <= d < len(adims) and len(adims) <= 2, "gather runs along one of at most two grid dimensions"
+        assert adims[d] == gmap.d_in()
+        shape[1 + d] = gmap.d_out()
+        rs.append(SO3partArr(torch.empty(shape, dtype=torch.complex64, device=x.device)))
+    backend().SO3part.set_gather(rs, list(xs), gmap.obj, d, False)
+    return rs
+
+
+@without_torch_function
+def gathered_back(gmap, d, rgs):
+    """Its gradient: the map read backwards; None where there is no gradient to take in."""
+    xgs = [None] * len(rgs)
+    used = [i for i, g in enumerate(rgs) if g is not None]
+    for i in used:
+        shape = list(rgs[i].size())
+        shape[1 + d] = gmap.d_in()
+        xgs[i] = SO3partArr(torch.empty(shape, dtype=torch.complex64, device=rgs[i].device))
+    if used:
+        backend().SO3part.set_gather([xgs[i] for i in used], [rgs[i].contiguous() for i in used], gmap.obj, d, True)
+    return xgs
+
+
 class SO3partArr_GatherFn(torch.autograd.Function):
-    """python/src/gelib/SO3partArr.py:236-254: forward add_gather, backward add_gather_back with the same map; here of all
-    parts of a vector at once (SO3vecArr.gather), each result written by the launch that sums it."""
+    """python/src/gelib/SO3partArr.py:236-254: forward add_gather, backward add_gather_back with the same map."""
 
     @staticmethod
-    @without_torch_function
-    def forward(ctx, gmap, d, *xs):
-        from gelib_amd.gather_map import gather_map
-        assert isinstance(gmap, gather_map)
-        ctx.gmap, ctx.d, ctx.shapes = gmap, d, [list(x.size()) for x in xs]
-        ctx.set_materialize_grads(False)
-        rs = []
-        for x in xs:
-            shape = list(x.size())
-            adims = shape[1:-2]
-            assert 0 <= d < len(adims) and len(adims) <= 2, "gather runs along one of at most two grid dimensions"
-            assert adims[d] == gmap.d_in()
-            shape[1 + d] = gmap.d_out()
-            rs.append(SO3partArr(torch.empty(shape, dtype=torch.complex64, device=x.device)))
-        backend().SO3part.set_gather(rs, list(xs), gmap.obj, d, False)
-        return tuple(rs)
+    def forward(ctx, x, gmap, d):
+        ctx.gmap, ctx.d = gmap, d
+        return gathered(gmap, d, [x])[0]
 
     @staticmethod
-    @without_torch_function
-    def backward(ctx, *rgs):
-        used = [i for i, g in enumerate(rgs) if g is not None]
-        xgs = [None] * len(rgs)
-        for i in used:
-            shape = [rgs[i].size(0)] + ctx.shapes[i][1:]
-            xgs[i] = SO3partArr(torch.empty(shape, dtype=torch.complex64, device=rgs[i].device))
-        if used:
-            backend().SO3part.set_gather([xgs[i] for i in used], [rgs[i].contiguous() for i in used], ctx.gmap.obj, ctx.d, True)
-        return tuple([None, None] + xgs)
+    def backward(ctx, rg):
+        return gathered_back(ctx.gmap, ctx.d, [rg])[0], None, None

@@ -5,7 +5,7 @@ import torch
 
 from gelib_amd.SO3weights import mix_channels
 from gelib_amd.gelib_common import backend
-from gelib_amd.SO3partArr import SO3partArr, SO3partArr_GatherFn
+from gelib_amd.SO3partArr import SO3partArr, gathered, gathered_back
 from gelib_amd.SO3vec import _product_fn
 
 
@@ -97,7 +97,7 @@ class SO3vecArr:
         with torch._C.DisableTorchFunctionSubclass():
             alike = len({(p.requires_grad, p.device) for p in parts}) == 1
         if alike:
-            return SO3vecArr(*SO3partArr_GatherFn.apply(gmap, dim, *parts))
+            return SO3vecArr(*SO3vecArr_GatherFn.apply(gmap, dim, *parts))
         return SO3vecArr(*[SO3partArr(p).gather(gmap, dim) for p in parts])
 
     def odot(self, y):
@@ -148,3 +148,17 @@ class SO3vecArr:
 
 SO3vecArr_CGproductFn = _product_fn(False, SO3partArr, "SO3vecArr")
 SO3vecArr_DiagCGproductFn = _product_fn(True, SO3partArr, "SO3vecArr")
+
+
+class SO3vecArr_GatherFn(torch.autograd.Function):
+    """SO3partArr_GatherFn of every part of a vector, in one launch each way."""
+
+    @staticmethod
+    def forward(ctx, gmap, d, *xs):
+        ctx.gmap, ctx.d = gmap, d
+        ctx.set_materialize_grads(False)
+        return tuple(gathered(gmap, d, xs))
+
+    @staticmethod
+    def backward(ctx, *rgs):
+        return tuple([None, None] + gathered_back(ctx.gmap, ctx.d, rgs))

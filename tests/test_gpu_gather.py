@@ -171,3 +171,17 @@ def test_vec_gather_gradients_of_some_parts(G):
         for s in (0, 3, 3, 8):
             want[s] += 1
         assert torch.equal(got[1].as_subclass(torch.Tensor).real.cpu(), want.reshape(1, 9, 1, 1).expand(1, 9, 5, 4))
+
+
+def test_gather_function_of_one_part(G):
+    """The autograd function of one part takes (x, map, dimension), as the reference's does, and returns the part."""
+    from gelib_amd.SO3partArr import SO3partArr_GatherFn
+    gmap = G.gather_map.random(6, 4, 0.5, seed=11)
+    src, tgt = gmap.pairs()
+    x = cplx(2, 3, 6, 5, 4, seed=21).cuda().requires_grad_()
+    r = SO3partArr_GatherFn.apply(x, gmap, 1)
+    assert isinstance(r, G.SO3partArr) and list(r.shape) == [2, 3, 4, 5, 4]
+    assert np.array_equal(U.host(r), ora.gather(U.host(x), src, tgt, 4, 2))
+    g = cplx(2, 3, 4, 5, 4, seed=22).cuda()
+    (xg,) = torch.autograd.grad(r, x, g)
+    assert np.array_equal(U.host(xg), ora.gather(U.host(g), tgt, src, 6, 2))
