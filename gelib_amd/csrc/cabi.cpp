@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <string>
@@ -905,7 +906,9 @@ int vec_bwd_entry(bool diag, const gelib_part_desc *xg, const gelib_part_desc *y
 // kernels for those take their product as it stands, the blocks at the offsets counted here: four launches where the
 // reference has one per (mu1, mu2, mu).
 struct ParityViews {
-  std::vector<View> p[2];           // [0]: parity +1, [1]: -1, each sorted by l
+  std::vector<View> all;            // as handed in
+  std::vector<View> p[2], empty[2];  // [0]: parity +1, [1]: -1, each sorted by l; the parts without channels (empty) have no
+                                     // block in a product, and the kernels' launch shapes are not made for them
   std::vector<std::pair<int, int>> order;   // (parity index, position in p[..]) of every part by 2l + (p == -1)
 };
 
@@ -917,6 +920,7 @@ int split_parities(int n, const gelib_part_desc *parts, const int *parity, int m
     View v;
     int rc = check_desc(&parts[i], v);
     if (rc) return rc;
+    out.all.push_back(v);
     out.p[parity[i] < 0].push_back(v);
   }
   for (int q = 0; q < 2; q++) {
@@ -925,6 +929,8 @@ int split_parities(int n, const gelib_part_desc *parts, const int *parity, int m
     std::sort(L.begin(), L.end(), [](const View &a, const View &b) { return a.l < b.l; });
     for (size_t i = 1; i < L.size(); i++)
       if (L[i].l == L[i - 1].l) return GELIB_HIP_ERR_PARTS;
+    std::copy_if(L.begin(), L.end(), std::back_inserter(out.empty[q]), [](const View &v) { return v.n == 0; });
+    L.erase(std::remove_if(L.begin(), L.end(), [](const View &v) { return v.n == 0; }), L.end());
     for (size_t i = 0; i < L.size(); i++) out.order.push_back({q, (int)i});
   }
   std::sort(out.order.begin(), out.order.end(), [&](const std::pair<int, int> &a, const std::pair<int, int> &b) {
@@ -942,21 +948,32 @@ int build_parity_plans(bool diag, const ParityViews &R, const ParityViews &X, co
   }
   std::vector<long long> offset[2];
   for (int q = 0; q < 2; q++) offset[q].assign(R.p[q].size(), 0);
+  auto wanted = [&](const std::vector<View> &L, int l) { return std::any_of(L.begin(), L.end(), [&](const View &v) { return v.l == l; }); };
+  if (diag)   // the channel counts of a pair agree, none on both sides included
+    for (int k = 0; k < 4; k++)
+      for (auto *xs : {&X.p[k >> 1], &X.empty[k >> 1]})
+        for (auto *ys : {&Y.p[k & 1], &Y.empty[k & 1]})
+          for (auto &x : *xs)
+            for (auto &y : *ys)
+              for (int l = std::abs(x.l - y.l); l <= x.l + y.l && x.n != y.n; l++)
+                for (auto *rs : {&R.p[(k >> 1) ^ (k & 1)], &R.empty[(k >> 1) ^ (k & 1)]})
+                  if (wanted(*rs, l)) return GELIB_HIP_ERR_DIAG_CHANNELS;
   for (auto &ox : X.order)
     for (auto &oy : Y.order) {
       const View &x = X.p[ox.first][ox.second], &y = Y.p[oy.first][oy.second];
       if (x.l > kMaxL || y.l > kMaxL) return GELIB_HIP_ERR_PARTS;
       const int q = ox.first ^ oy.first;
-      for (int l = std::abs(x.l - y.l); l <= x.l + y.l; l++)
+      for (int l = std::abs(x.l - y.l); l <= x.l + y.l; l++) {
+        if (wanted(R.empty[q], l)) return GELIB_HIP_ERR_CHANNELS;
         for (size_t k = 0; k < R.p[q].size(); k++) {
           if (R.p[q][k].l != l) continue;
-          if (diag && x.n != y.n) return GELIB_HIP_ERR_DIAG_CHANNELS;
           const long long nout = diag ? x.n : (long long)x.n * y.n;
           if (offset[q][k] + nout > R.p[q][k].n) return GELIB_HIP_ERR_CHANNELS;
           plans[ox.first][oy.first].triples.push_back(
               {ox.second, oy.second, (int)k, x.l, y.l, l, (int)offset[q][k], (int)nout});
           offset[q][k] += nout;
         }
+      }
     }
   return GELIB_HIP_OK;
 }
@@ -964,17 +981,15 @@ int build_parity_plans(bool diag, const ParityViews &R, const ParityViews &X, co
 int reconcile_views(std::initializer_list<const ParityViews *> lists, long long E[3]) {
   std::vector<const gelib_part_desc *> all;
   for (auto *v : lists)
-    for (auto &L : v->p)
-      for (auto &w : L) all.push_back(w.d);
+    for (auto &w : v->all) all.push_back(w.d);
   return reconcile(all.data(), (int)all.size(), E);
 }
 
 int check_views(std::initializer_list<const ParityViews *> lists, bool dest) {
   int rc;
   for (auto *v : lists)
-    for (auto &L : v->p)
-      for (auto &w : L)
-        if ((rc = dest ? check_dest(w.d) : check_pointer(w.d))) return rc;
+    for (auto &w : v->all)
+      if ((rc = dest ? check_dest(w.d) : check_pointer(w.d))) return rc;
   return GELIB_HIP_OK;
 }
 
@@ -1012,12 +1027,10 @@ int o3vec_bwd_entry(bool diag, const gelib_part_desc *xg, const gelib_part_desc 
       (rc = split_parities(ny, y, yp, kMaxParts, Y)) || (xg && (rc = split_parities(nx, xg, xp, kMaxParts, XG))) ||
       (yg && (rc = split_parities(ny, yg, yp, kMaxParts, YG))))
     return rc;
-  for (int q = 0; q < 2; q++) {
-    for (size_t i = 0; i < XG.p[q].size(); i++)
-      if (XG.p[q][i].l != X.p[q][i].l || XG.p[q][i].n != X.p[q][i].n) return GELIB_HIP_ERR_PARTS;
-    for (size_t i = 0; i < YG.p[q].size(); i++)
-      if (YG.p[q][i].l != Y.p[q][i].l || YG.p[q][i].n != Y.p[q][i].n) return GELIB_HIP_ERR_PARTS;
-  }
+  for (size_t i = 0; i < XG.all.size(); i++)
+    if (XG.all[i].l != X.all[i].l || XG.all[i].n != X.all[i].n) return GELIB_HIP_ERR_PARTS;
+  for (size_t i = 0; i < YG.all.size(); i++)
+    if (YG.all[i].l != Y.all[i].l || YG.all[i].n != Y.all[i].n) return GELIB_HIP_ERR_PARTS;
   if (ng == 0 || nx == 0 || ny == 0) return GELIB_HIP_OK;
   long long E[3];
   if ((rc = reconcile_views({&G, &X, &Y, &XG, &YG}, E))) return rc;
@@ -1038,6 +1051,7 @@ int o3vec_bwd_entry(bool diag, const gelib_part_desc *xg, const gelib_part_desc 
     std::vector<int> dests;
     bool bcast = false;
     for (int i = ixg; i < (int)d.size(); i++) {
+      if (d[i].dims[4] == 0) continue;
       dests.push_back(i);
       bcast = bcast || dest_broadcasts(&d[i], E);
     }

@@ -171,3 +171,24 @@ def test_part_count_limits():
     assert L.gelib_hip_so3vec_cg_fwd(1, (cabi.PartDesc * 1)(fake(1, 1, 0, ptr=None)), 33, xs, 1, y, 1, None) in (0, 5)
     assert L.gelib_hip_part_mix_workspace_bytes(0, 10, 32, 16) >= 16 * 32 * 16
     assert L.gelib_hip_part_mix_workspace_bytes(2, 10, 32, 16) == 0
+
+
+def test_o3_parts_without_channels_take_part_in_the_checks():
+    L = cabi.lib()
+
+    def status(diag, *vecs):
+        args = [diag]
+        for parts, parities in vecs:
+            args += [len(parts), (cabi.PartDesc * len(parts))(*parts), (ctypes.c_int * len(parts))(*parities)]
+        return L.gelib_hip_o3vec_cg_fwd(*args, 0, None)
+
+
+    def vec(n, b=2):
+        d = fake(b, 1, n, ptr=0x1000 if n else 0)
+        d.strides[0] = max(1, n)          # as torch has them
+        return [d], [1]
+
+    assert status(1, vec(0), vec(0), vec(3)) == 4          # Diag: channel counts differ
+    assert status(0, vec(0), vec(2), vec(3)) == 5          # no room for the block
+    assert status(0, vec(0), vec(0), vec(0, b=3)) == 6     # batches differ
+    assert status(0, vec(0), vec(0), vec(0)) == 0 and status(1, vec(0), vec(0), vec(0)) == 0

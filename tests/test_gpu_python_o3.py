@@ -187,3 +187,33 @@ def test_o3vec_entry_points_match_part_level_calls(G, xmus, ymus, diag, accumula
     r2 = new(start)
     cabi.o3vec_fwd(r2[::-1], ps(rmus)[::-1], x[::-1], ps(xmus)[::-1], y, ps(ymus), accumulate=accumulate, diag=diag)
     assert all(torch.equal(torch.view_as_real(a), torch.view_as_real(b)) for a, b in zip(r, r2))
+
+
+@pytest.mark.parametrize("xtau,ytau", [
+    ({(0, 1): 0}, {(0, 1): 0}),                                   # nothing at all
+    ({(0, 1): 3, (1, 1): 0, (1, -1): 2}, {(0, 1): 0, (1, -1): 2}),
+    ({(1, 1): 0, (2, -1): 4}, {(1, 1): 4, (1, -1): 0}),
+])
+@pytest.mark.parametrize("shared", [False, True])
+def test_vec_product_with_parts_without_channels(G, xtau, ytau, shared):
+    """A part without channels has no block in a product, its gradient is empty, and the others are as without it."""
+    x = {mu: U.dev(U.seeded(3 + i, 3, 2 * mu[0] + 1, n)).requires_grad_() for i, (mu, n) in enumerate(xtau.items())}
+    y = {mu: U.dev(U.seeded(30 + i, 1 if shared else 3, 2 * mu[0] + 1, n)).requires_grad_() for i, (mu, n) in enumerate(ytau.items())}
+    z = G.CGproduct(G.O3vec(x), G.O3vec(y))
+    full = lambda v: {mu: p for mu, p in v.items() if p.size(-1)}
+    leaves = list(x.values()) + list(y.values())
+    gs = {mu: U.dev(U.seeded(60 + i, *p.shape)) for i, (mu, p) in enumerate(z.parts.items())}
+    grads = torch.autograd.grad(list(z.parts.values()), leaves, list(gs.values()))
+    for t, g in zip(leaves, grads):
+        assert g.shape == t.shape
+    if not full(x) or not full(y):
+        assert all(p.numel() == 0 or not p.any() for p in z.parts.values()) and not any(g.any() for g in grads)
+        return
+    w = G.CGproduct(G.O3vec(full(x)), G.O3vec(full(y)))
+    for mu, p in z.parts.items():
+        if p.size(-1):
+            assert torch.equal(torch.view_as_real(p), torch.view_as_real(w.parts[mu]))
+    some = list(full(x).values()) + list(full(y).values())
+    want = torch.autograd.grad(list(w.parts.values()), some, [gs[mu] for mu in w.parts])
+    for t, g in zip(some, want):
+        assert torch.equal(torch.view_as_real(g), torch.view_as_real(grads[[t is u for u in leaves].index(True)]))
