@@ -67,8 +67,8 @@ static void spharm(SO3part<float> &r, const at::Tensor &X, const int accumulate)
     TORCH_CHECK(X.stride(i) >= 0, "GElib: negative strides are not supported");
     strides.push_back((size_t)X.stride(i));
   }
-  StreamGuard sg(accumulate);
-  r.add_spharm(cnine::TensorView<float>(X.data_ptr<float>(), dims, cnine::GstridesB(strides), X.is_cuda() ? 1 : 0));
+  StreamGuard sg;
+  r.put_spharm(cnine::TensorView<float>(X.data_ptr<float>(), dims, cnine::GstridesB(strides), X.is_cuda() ? 1 : 0), accumulate);
 }
 
 static std::vector<gelib_part_desc> parts_on_gpu(const std::vector<at::Tensor> &v) {
@@ -171,14 +171,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       // Written into an uninitialised part (no zero-fill, no read of r); no counterpart in the reference.
       .def("set_CGproduct",
            [](SO3part<float> &r, const SO3part<float> &x, const SO3part<float> &y) {
-             StreamGuard g(0);
-             Gpart_add_CGproduct(r, x, y, 0);
+             StreamGuard g;
+             Gpart_set_CGproduct(r, x, y);
            },
            py::arg("x"), py::arg("y"))
       .def("set_DiagCGproduct",
            [](SO3part<float> &r, const SO3part<float> &x, const SO3part<float> &y) {
-             StreamGuard g(0);
-             Gpart_add_DiagCGproduct(r, x, y, 0);
+             StreamGuard g;
+             Gpart_set_DiagCGproduct(r, x, y);
            },
            py::arg("x"), py::arg("y"))
       .def("add_spharm", [](SO3part<float> &r, at::Tensor &X) { spharm(r, X, 1); }, py::arg("X"))
@@ -202,9 +202,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                     std::vector<SO3part<float>> R, X;
                     for (auto &t : r) R.push_back(SO3part<float>(view_of(t)));
                     for (auto &t : x) X.push_back(SO3part<float>(view_of(t)));
-                    gmap.device_handle();  // made on the caller's map, which the reversed copy below shares
-                    StreamGuard sg(0);
-                    SO3part<float>::gather_parts(R, X, back ? gmap.inv() : gmap, d);
+                    if (back) gmap.device_handle();  // made on the caller's map, which the reversed copy below shares
+                    StreamGuard sg;
+                    SO3part<float>::gather_parts(R, X, back ? gmap.inv() : gmap, d, 0);
                   },
                   py::arg("r"), py::arg("x"), py::arg("gmap"), py::arg("d"), py::arg("back"))
       .def("getl", &SO3part<float>::getl)
@@ -234,9 +234,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
            const std::vector<int> &xp, const std::vector<at::Tensor> &y, const std::vector<int> &yp) {
           GELIB_ASSRT(r.size() == rp.size() && x.size() == xp.size() && y.size() == yp.size());
           auto R = parts_on_gpu(r), X = parts_on_gpu(x), Y = parts_on_gpu(y);
-          StreamGuard g(0);
+          StreamGuard g;
           GElib::detail::skip_on(gelib_hip_o3vec_cg_fwd(diag, (int)R.size(), R.data(), rp.data(), (int)X.size(), X.data(), xp.data(),
-                                                 (int)Y.size(), Y.data(), yp.data(), accumulate_mode(), gelib_stream()));
+                                                 (int)Y.size(), Y.data(), yp.data(), 0, gelib_stream()));
         });
   m.def("o3vec_product_back",
         [](bool diag, const std::vector<at::Tensor> &xg, const std::vector<at::Tensor> &yg, const std::vector<at::Tensor> &gr,
@@ -245,9 +245,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           GELIB_ASSRT(gr.size() == gp.size() && x.size() == xp.size() && y.size() == yp.size() && xg.size() == x.size() &&
                       yg.size() == y.size());
           auto XG = parts_on_gpu(xg), YG = parts_on_gpu(yg), G = parts_on_gpu(gr), X = parts_on_gpu(x), Y = parts_on_gpu(y);
-          StreamGuard g(0);
+          StreamGuard g;
           GElib::detail::skip_on(gelib_hip_o3vec_cg_bwd(diag, XG.data(), YG.data(), (int)G.size(), G.data(), gp.data(), (int)X.size(),
-                                                 X.data(), xp.data(), (int)Y.size(), Y.data(), yp.data(), accumulate_mode(),
+                                                 X.data(), xp.data(), (int)Y.size(), Y.data(), yp.data(), 0,
                                                  gelib_stream()));
         });
 

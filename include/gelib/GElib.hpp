@@ -397,7 +397,9 @@ class SO3part : public cnine::BatchedTensor<std::complex<TYPE>>, public GpartBas
   }
 
   // ---- spherical harmonics (SO3/SO3part.hpp:340-403): x is (.., 3, n) real, leading dims as this part's or 1 ----
-  void add_spharm(const cnine::TensorView<float> &x) const {
+  void add_spharm(const cnine::TensorView<float> &x) const { put_spharm(x, 1); }
+  void set_spharm(const cnine::TensorView<float> &x) const { put_spharm(x, 0); }
+  void put_spharm(const cnine::TensorView<float> &x, const int accumulate) const {
     GELIB_ASSRT(x.get_dev() == dev);
     if (dev != 1) GELIB_ERROR("SO3part::add_spharm: the operands must be on GPU");
     const int d = ndims(), xd = x.ndims();
@@ -424,13 +426,14 @@ class SO3part : public cnine::BatchedTensor<std::complex<TYPE>>, public GpartBas
         xstr[1] = (int64_t)x.strides[ng];
       }
     }
-    gelib_check(gelib_hip_so3part_spharm(&R, x.arr, xdims, xstr, accumulate_mode(), gelib_stream()));
+    gelib_check(gelib_hip_so3part_spharm(&R, x.arr, xdims, xstr, accumulate, gelib_stream()));
   }
 
   // ---- sums of slices along grid dimension d (core/Gpart.hpp:556-562) ----
-  void add_gather(const SO3part &x, const cnine::GatherMapB &gmap, const int d = 0) const { gather_parts({*this}, {x}, gmap, d); }
+  void add_gather(const SO3part &x, const cnine::GatherMapB &gmap, const int d = 0) const { gather_parts({*this}, {x}, gmap, d, 1); }
   // r[i] (+)= x[i] gathered, for several parts in one call (parts of ordinary layout share a launch)
-  static void gather_parts(const std::vector<SO3part> &r, const std::vector<SO3part> &x, const cnine::GatherMapB &gmap, const int d) {
+  static void gather_parts(const std::vector<SO3part> &r, const std::vector<SO3part> &x, const cnine::GatherMapB &gmap, const int d,
+                           const int accumulate) {
     GELIB_ASSRT(r.size() == x.size());
     std::vector<gelib_part_desc> R, X;
     for (size_t i = 0; i < r.size(); i++) {
@@ -444,7 +447,7 @@ class SO3part : public cnine::BatchedTensor<std::complex<TYPE>>, public GpartBas
       X.push_back(x[i].descriptor());
     }
     gelib_check(gelib_hip_vec_gather((int)R.size(), R.data(), X.data(), gmap.device_handle(), d + 1, gmap.inverted ? 1 : 0,
-                                     accumulate_mode(), gelib_stream()));
+                                     accumulate, gelib_stream()));
   }
   void add_gather_back(const SO3part &r, const cnine::GatherMapB &gmap, const int d = 0) const {
     gmap.device_handle();  // made on the caller's map, so the reversed copy below shares it instead of uploading,
@@ -477,19 +480,22 @@ inline void skip_on(const int rc) {
 }
 }  // namespace detail
 
-#define GELIB_PART_DISPATCH(NAME, ENTRY)                                                          \
+// add: "+="; set: written into an uninitialised destination (no counterpart in the reference)
+#define GELIB_PART_DISPATCH(NAME, ENTRY, ACCUMULATE)                                              \
   template <typename GPART>                                                                       \
   void NAME(GPART dest, GPART a, GPART b, const int offs = 0) {                                   \
     detail::check_devices(dest, a, b);                                                            \
     auto D = dest.descriptor(), A = a.descriptor(), B = b.descriptor();                           \
-    detail::skip_on(ENTRY(&D, &A, &B, offs, accumulate_mode(), gelib_stream()));                         \
+    detail::skip_on(ENTRY(&D, &A, &B, offs, ACCUMULATE, gelib_stream()));                         \
   }
-GELIB_PART_DISPATCH(Gpart_add_CGproduct, gelib_hip_so3part_cg_fwd)              // (r, x, y, offs)
-GELIB_PART_DISPATCH(Gpart_add_CGproduct_back0, gelib_hip_so3part_cg_back0)      // (xg, g, y, offs)
-GELIB_PART_DISPATCH(Gpart_add_CGproduct_back1, gelib_hip_so3part_cg_back1)      // (yg, g, x, offs)
-GELIB_PART_DISPATCH(Gpart_add_DiagCGproduct, gelib_hip_so3part_diagcg_fwd)
-GELIB_PART_DISPATCH(Gpart_add_DiagCGproduct_back0, gelib_hip_so3part_diagcg_back0)
-GELIB_PART_DISPATCH(Gpart_add_DiagCGproduct_back1, gelib_hip_so3part_diagcg_back1)
+GELIB_PART_DISPATCH(Gpart_add_CGproduct, gelib_hip_so3part_cg_fwd, 1)              // (r, x, y, offs)
+GELIB_PART_DISPATCH(Gpart_add_CGproduct_back0, gelib_hip_so3part_cg_back0, 1)      // (xg, g, y, offs)
+GELIB_PART_DISPATCH(Gpart_add_CGproduct_back1, gelib_hip_so3part_cg_back1, 1)      // (yg, g, x, offs)
+GELIB_PART_DISPATCH(Gpart_add_DiagCGproduct, gelib_hip_so3part_diagcg_fwd, 1)
+GELIB_PART_DISPATCH(Gpart_add_DiagCGproduct_back0, gelib_hip_so3part_diagcg_back0, 1)
+GELIB_PART_DISPATCH(Gpart_add_DiagCGproduct_back1, gelib_hip_so3part_diagcg_back1, 1)
+GELIB_PART_DISPATCH(Gpart_set_CGproduct, gelib_hip_so3part_cg_fwd, 0)
+GELIB_PART_DISPATCH(Gpart_set_DiagCGproduct, gelib_hip_so3part_diagcg_fwd, 0)
 #undef GELIB_PART_DISPATCH
 
 template <typename GPART>

@@ -47,6 +47,19 @@ int main(int argc, char **argv) {
   for (auto &p : v.parts) dump(f, p.second);
   for (auto &p : w.parts) dump(f, p.second);
 
+  // accumulate_mode() is the vectors' business: a part-level add_ adds whatever it says
+  SO3part<float> twice = r.zeros_like(), other(r, 1);
+  accumulate_mode() = 0;
+  Gpart_add_CGproduct(twice, xd, yd);
+  Gpart_add_CGproduct(twice, xd, yd);
+  accumulate_mode() = 1;
+  Gpart_set_CGproduct(other, xd, yd);
+  {
+    TensorView<std::complex<float>> h1(r, 0), h2(twice, 0), h3(other, 0);
+    for (size_t i = 0; i < h1.asize(); i++)
+      if (std::abs(h2.arr[i] - 2.f * h1.arr[i]) > 1e-5f * (1.f + std::abs(h1.arr[i])) || h3.arr[i] != h1.arr[i]) return 8;
+  }
+
   // type arithmetic known answers (python/docs/source/abandoned/SO3type.rst:28-41)
   SO3type t1({{0, 1}, {1, 1}, {2, 1}});
   if (!(CGproduct(t1, t1) == SO3type(std::vector<int>{3, 6, 6, 3, 1}))) return 3;
