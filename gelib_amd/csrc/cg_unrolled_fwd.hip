@@ -12,8 +12,6 @@ int launch_unrolled_fwd_cg4_l4(const FwdArgs &a, int nblocks, size_t lds_bytes, 
 int launch_unrolled_fwd_cg4_l8(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s);
 int launch_unrolled_fwd_diag_l4(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s);
 int launch_unrolled_fwd_diag_l8(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s);
-int launch_unrolled_fwd_cg2_l4_ragged(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s);
-int launch_unrolled_fwd_cg2_l8_ragged(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s);
 int launch_unrolled_fwd_cg4_l4_ragged(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s);
 int launch_unrolled_fwd_cg4_l8_ragged(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s);
 int launch_unrolled_fwd_cg2_l6l(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s);
@@ -29,10 +27,8 @@ bool unrolled_fwd_takes(bool diag, int ti, int lcap, int lop) {
 int launch_unrolled_fwd(const FwdArgs &a, bool diag, int ti, bool ragged, int lcap, int lop, int nblocks, size_t lds_bytes,
                         hipStream_t s) {
   if (nblocks <= 0) return GELIB_HIP_OK;
-  if (ragged) {   // two or four channels per thread, operands up to l = 4
-    const bool small = lcap <= kLT;
-    if (ti == 4) return small ? launch_unrolled_fwd_cg4_l4_ragged(a, nblocks, lds_bytes, s) : launch_unrolled_fwd_cg4_l8_ragged(a, nblocks, lds_bytes, s);
-    return small ? launch_unrolled_fwd_cg2_l4_ragged(a, nblocks, lds_bytes, s) : launch_unrolled_fwd_cg2_l8_ragged(a, nblocks, lds_bytes, s);
+  if (ragged) {   // four channels per thread, operands up to l = 4
+    return lcap <= kLT ? launch_unrolled_fwd_cg4_l4_ragged(a, nblocks, lds_bytes, s) : launch_unrolled_fwd_cg4_l8_ragged(a, nblocks, lds_bytes, s);
   }
   if (lop > kLT) return launch_unrolled_fwd_cg2_l6l(a, nblocks, lds_bytes, s);
   const bool small = lcap <= kLT;

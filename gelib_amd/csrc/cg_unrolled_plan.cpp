@@ -317,6 +317,7 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
     }
     if (g_fwd_ti == 1 || g_fwd_ti == 2 || g_fwd_ti == 4) ti = std::min(ti, g_fwd_ti);
     for (auto &t : triples) ragged = ragged || xs[t.xi].second % ti;
+    if (ragged && ti < 4) ti = 1, ragged = false;   // fewer than four on request: counts that do not divide take one
   }
   if (lop > kLT && ti == 4) ti = 2;  // the kernel for operands above kLT is built for two channels per thread
   if (!unrolled_fwd_takes(diag, ti, lcap_all, lop) || (lop > kLT && !g_fwd_l6_enable)) return GELIB_HIP_OK;

@@ -335,3 +335,21 @@ def test_no_gradient_for_harmonics(cabi):
     both = torch.autograd.grad(list(G.CGproduct(G.SO3vec(*x), G.SO3vec(*y), 3).parts.values()), x + y, gs)
     for a, b in zip(got, both):
         assert float((a - b).abs().max()) <= 1e-6 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("B,tx,ty,maxl,diag", [t for t in TIGHT if max(t[1]) <= 4 and max(t[2]) <= 4])
+@pytest.mark.parametrize("small4", [0, 1])
+def test_forward_with_and_without_a_block_per_cell(cabi, B, tx, ty, maxl, diag, small4):
+    """The wave-per-cell forward kernel and the block form, each on everything it can be asked for."""
+    xs = [U.seeded(1500 + l, B, 2 * l + 1, n) for l, n in sorted(tx.items())]
+    ys = [U.seeded(1550 + l, B, 2 * l + 1, n) for l, n in sorted(ty.items())]
+    O = U.VecOracle(xs, ys, maxl, diag)
+    drs = [torch.full(p.shape, 7.0 + 1j, dtype=torch.complex64, device="cuda") for p in O.r32]
+    cabi.set_option("diag6_small4_fwd", small4)
+    try:
+        cabi.so3vec_fwd(drs, [U.dev(a) for a in xs], [U.dev(a) for a in ys], accumulate=False, diag=diag)
+        assert cabi.last_path() == DIAG6
+        torch.cuda.synchronize()
+    finally:
+        cabi.set_option("diag6_small4_fwd", -1)
+    O.check_fwd([U.host(a) for a in drs], "B%d %s x %s small4 %d" % (B, tx, ty, small4))

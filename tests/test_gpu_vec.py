@@ -305,3 +305,27 @@ def test_forward_product_in_several_launches(cabi, B, tx, ty, maxl, tile, accumu
     for other in got[1:]:
         for a, b in zip(want, other):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("option,values", [("fwd_tile", (1, 2, 4)), ("fwd_tile_per_xcd", (0, 1)), ("fwd_narrow_decline", (0,))])
+@pytest.mark.parametrize("B,tx,ty,maxl", [
+    (517, {0: 9, 1: 5, 2: 13}, {0: 7, 1: 9, 2: 5}, 2),      # odd counts: four channels a thread, or one
+    (1100, {0: 10, 1: 6}, {0: 7, 1: 10}, 1),                # two, or one
+    (300, {0: 16, 2: 32}, {1: 16}, -1),
+    (2500, {0: 2, 1: 1}, {0: 2, 1: 2}, -1),                 # at most four pairs a block: the any-l kernel unless told otherwise
+])
+def test_forward_options_leave_the_results_alone(cabi, option, values, B, tx, ty, maxl):
+    xs = [U.seeded(700 + l, B, 2 * l + 1, n) for l, n in sorted(tx.items())]
+    ys = [U.seeded(740 + l, B, 2 * l + 1, n) for l, n in sorted(ty.items())]
+    run = U.VecOracle(xs, ys, maxl, False)
+    dx, dy = [U.dev(a) for a in xs], [U.dev(a) for a in ys]
+    default = {"fwd_tile": 0, "fwd_tile_per_xcd": -1, "fwd_narrow_decline": 1}[option]
+    for v in values:
+        rs = [torch.full(p.shape, 9.0, dtype=torch.complex64, device="cuda") for p in run.r32]
+        cabi.set_option(option, v)
+        try:
+            cabi.so3vec_fwd(rs, dx, dy, accumulate=False)
+            torch.cuda.synchronize()
+        finally:
+            cabi.set_option(option, default)
+        run.check_fwd([U.host(r) for r in rs], "%s %d" % (option, v))
