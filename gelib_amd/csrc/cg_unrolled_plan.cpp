@@ -344,22 +344,31 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   // Measured in one process, forward pass: L=4 with 16 channels 4.41 ms at 64 cells per tile, 4.30 at 32, 4.56 at 128;
   // 8 channels 4.34 at 32 and 64, 4.89 at 4096; 4 channels (128-byte pieces per pair and row) 7.0 at 64, 6.7 at 1024,
   // 5.85 at 4096, 7.9 with all cells in one tile.
-  // Blocks of a row that are not whole 128-byte lines share a line with the next pair's: the two halves meet in one L2 cache
-  // only if both blocks run on the same XCD, and otherwise reach memory as two partial lines.  There the blocks of a tile
+  // Blocks of a row that are not whole half-lines (64 bytes) share one with the next pair's: the two pieces meet in one L2
+  // cache only if both blocks run on the same XCD, and otherwise reach memory as partial writes.  There the blocks of a tile
   // go to one XCD, eight tiles at a time, in tiles small enough that a part's neighbouring blocks are written close
-  // together in time (tiles over all XCDs / one each, microseconds: 9 channels, L=4, 16384 cells 1195 / 983; 13 x 7 uncapped
-  // 2139 / 1883; 5 channels, L=3, 100000 cells 1434 / 1110; 3 channels, 200000 cells 1622 / 977; 6 channels, L=4, 50000 cells
-  // 1944 / 1673; 6 channels, L=5, 10000 cells 846 / 709; 17 x 2 channels 526 / 541).  Whole lines go round the XCDs: 12
-  // channels, L=4 1328 / 1486, 4 channels 578 / 660.  Fewer than 32 tiles would leave XCDs without work.
-  long long auto_tile = 4096;
-  bool unaligned = false;
+  // together in time, and large enough to fill the blocks of narrow pairs: 16 cells where every pair has 64 channels, 32 where
+  // one has, otherwise 64.  Tiles over all XCDs / one each, microseconds, 1 GB of product in memory that other calls have
+  // pushed out of the caches: L=4, 9 channels 314 / 262; 13 x 7 377 / 311; L=3, 5 channels 459 / 371; L=4, 6 x 3 484 / 385;
+  // 20, 12, 9, 6, 3 x 10, 7, 6, 5 channels, every l 381 / 336; 12, 6, 3 x 6, 3, 1 485 / 447 (589 in tiles of 16).
+  // Not with fewer than seven blocks (l1, l2, l), which leave few neighbours: L=1, 10 x 10 393 / 405, 6 x 3 545 / 614,
+  // (5 channels l = 0) x (3, 3) 541 / 734; whole half-lines (6 x 4 channels, L=2 to 4) 1.0 to 1.1.
+  // Not for a product that about fills the 256 MB memory-side cache either: written again and again, it stays there, where the
+  // partial writes meet as well (300 MB, L=4, 9 channels 69 / 87, 6 channels 67 / 88; 200 MB 49 / 49 and 45 / 48; 450 MB
+  // 146 / 128 and 173 / 153).  Fewer than 32 tiles would leave XCDs without work.
+  long long auto_tile = 4096, product_bytes = 0;
+  bool any_wide = false, all_wide = true, unaligned = false;
   for (auto &p : plan->pairs) {
     const long long n = (long long)p.n1 * (diag ? 1 : p.n2);
-    if (n >= 64) auto_tile = 32;
-    unaligned = unaligned || n % 16;
+    any_wide = any_wide || n >= 64;
+    all_wide = all_wide && n >= 64;
+    unaligned = unaligned || n % 8;
   }
-  const long long xcd_tile = auto_tile == 32 ? 16 : 64;
-  const bool want_xcd = g_fwd_tile_per_xcd < 0 ? unaligned && !diag && a.npairs > 1 && ncells >= 32 * xcd_tile
+  if (any_wide) auto_tile = 32;
+  for (auto &t : triples) product_bytes += 8 * ncells * (2 * t.l + 1) * t.nout;
+  const bool cached = product_bytes > 200000000LL && product_bytes < 400000000LL;
+  const long long xcd_tile = all_wide ? 16 : (any_wide ? 32 : 64);
+  const bool want_xcd = g_fwd_tile_per_xcd < 0 ? unaligned && !diag && triples.size() >= 7 && !cached && ncells >= 32 * xcd_tile
                                                : g_fwd_tile_per_xcd == 1;
   if (want_xcd) auto_tile = xcd_tile;
   const long long want_tile = g_fwd_cell_tile < 0 ? auto_tile : g_fwd_cell_tile;

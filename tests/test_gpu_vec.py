@@ -260,9 +260,11 @@ def test_tuning_options_leave_the_results_alone(cabi):
 
 
 @pytest.mark.parametrize("case", [
-    (517, {0: 9, 1: 5, 2: 13}, {0: 7, 1: 9, 2: 5}, 2),     # four channels a thread, idle ones; tiles of 16 cells per XCD
+    (517, {0: 9, 1: 5, 2: 13}, {0: 7, 1: 9, 2: 5}, 2),     # four channels a thread, idle ones
+    (1037, {0: 9, 1: 5, 2: 13}, {0: 7, 1: 9, 2: 5}, 2),    # ... some blocks below 64 channels: tiles of 32 cells per XCD
+    (517, {0: 9, 1: 10, 2: 13}, {0: 9, 1: 9, 2: 9}, 2),    # ... none: tiles of 16
     (2131, {0: 5, 1: 3, 2: 1}, {0: 3, 2: 3}, -1),          # blocks below 64 channels: tiles of 64 cells per XCD, a last group of tiles that is short
-    (520, {0: 10, 1: 6}, {0: 7, 1: 10}, 1),                # even counts that leave partial lines
+    (520, {0: 10, 1: 6}, {0: 7, 1: 10}, 1),                # even counts that leave partial lines, too few blocks for tiles per XCD
     (511, {3: 7, 4: 11}, {4: 17}, -1),                     # one tile too few for that; l up to 8
     (70, {0: 1, 1: 1, 3: 1}, {0: 9, 1: 17}, -1),           # one channel: stays one channel a thread
     (3, {2: 63}, {1: 1, 2: 3}, 3),
