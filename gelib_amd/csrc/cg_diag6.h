@@ -48,21 +48,22 @@ struct Diag6Args {
   const float *bank;  // device, kBankFloats coefficients followed by kZeroFloats zeros
   long long nwaves;   // cells * groups, or cells / (64 >> lg_npad) rounded up
   long long ncells;
-  // tight: the (cell, channel) pairs follow each other without gaps, 64 per wave, so that a channel count that is no power
-  // of two (or no multiple of 64) leaves no lane idle; kernels of the packed form only, and no sums over the lanes of a
-  // cell (lg_npad is 0 then).  nwaves = cells * n / 64 rounded up.
-  int tight;
-  unsigned long long magic64;  // ceil(2^64 / n): quotients of pair numbers below 2^50
-  unsigned magic32;            // ceil(2^32 / n): quotients of numbers below n + 64
   int groups;         // 64-channel groups per cell (more than 32 channels)
-  int lg_npad;        // log2 of the channel count rounded up to a power of two, at most 6
+  int lg_npad;        // log2 of the channel count rounded up to a power of two, at most 6; or kDiagTight
   int n;              // channels of every part (of every part of the wider operand when xbc or ybc is set)
   int xbc, ybc;       // CGproduct with a one-channel first / second operand: every lane reads that channel
   int offs_add;
   int accumulate;
   int want_x, want_y;  // backward: which gradients are stored (the operand of an unwanted one is never read)
   int owner[kNP];      // backward: which of the block's four waves takes the pairs with this l2
+  // (last, so that the loads of the fields above are those of the launches that do not need these)
+  unsigned long long magic64;  // kDiagTight: ceil(2^64 / n), quotients of pair numbers below 2^50
+  unsigned magic32;            // kDiagTight: ceil(2^32 / n), quotients of numbers below n + 64
 };
+// lg_npad of a launch whose (cell, channel) pairs follow each other without gaps, 64 per wave, so that a channel count that is
+// no power of two (or no multiple of 64) leaves no lane idle; kernels of the packed form only, and no sums over the lanes of a
+// cell.  nwaves = cells * n / 64 rounded up.
+constexpr int kDiagTight = -1;
 
 int launch_diag6_fwd_l6(const Diag6Args &a, hipStream_t s);  // product l up to 6
 int launch_diag6_bwd_l6(const Diag6Args &a, hipStream_t s);

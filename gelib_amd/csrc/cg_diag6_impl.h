@@ -63,17 +63,18 @@ struct WavePos {
   bool live;
 };
 
+template <bool PACKED>
 __device__ __forceinline__ WavePos wave_pos(const Diag6Args &a, long long w) {
   WavePos q;
   const int lane = (int)(threadIdx.x & 63);
-  if (a.tight) {
+  if (PACKED && a.lg_npad == kDiagTight) {
     const unsigned long long first = (unsigned long long)w << 6;
     q.cell = (long long)__umul64hi(a.magic64, first);
     const unsigned at = (unsigned)(first - (unsigned long long)q.cell * (unsigned)a.n) + (unsigned)lane;
     q.cell_local = (int)__umulhi(a.magic32, at);
     q.ch = (int)at - q.cell_local * a.n;
     q.live = q.cell + q.cell_local < a.ncells;
-  } else if (a.lg_npad < 6) {
+  } else if (PACKED) {
     q.cell = w << (6 - a.lg_npad);
     q.cell_local = lane >> a.lg_npad;
     q.ch = lane & ((1 << a.lg_npad) - 1);
@@ -216,7 +217,7 @@ __global__ void __launch_bounds__(256) diag6_fwd_kernel(const Diag6Args a) {
   __shared__ float2 yimg[(LOP + 1) * (LOP + 1) * 64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const long long w = blockIdx.x;
-  const WavePos q = wave_pos(a, w);
+  const WavePos q = wave_pos<PACKED>(a, w);
   stage_operand<PACKED, LOP>(yimg, a.y, q, wave, lane, a.ybc != 0);
   __syncthreads();
   static_for<LOP + 1>([&](auto l1c) __attribute__((always_inline)) {
@@ -383,7 +384,7 @@ __global__ void __launch_bounds__(256) diag6_bwd_kernel(const Diag6Args a) {
   __shared__ float2 yimg[kYRows * 64];
   __shared__ float2 xpart[4 * kXRows * 64];  // [wave][row][lane]
   const long long w = blockIdx.x;
-  const WavePos q = wave_pos(a, w);
+  const WavePos q = wave_pos<PACKED>(a, w);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const bool accumulate = a.accumulate != 0;
   const bool wx = a.want_x != 0, wy = a.want_y != 0;
@@ -546,7 +547,7 @@ template <int LCAP, bool PACKED>
 __global__ void __launch_bounds__(256) diag6_bwd_sets_kernel(const Diag6Args a) {
   __shared__ float2 yimg[kImgRows * 64];
   __shared__ float2 xpart[4 * (2 * kL6 + 1) * 64];  // [wave][row][lane]
-  const WavePos q = wave_pos(a, blockIdx.x);
+  const WavePos q = wave_pos<PACKED>(a, blockIdx.x);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   for (int e = threadIdx.x; e < kImgRows * 64; e += 256) yimg[e] = make_float2(0.f, 0.f);
   __syncthreads();

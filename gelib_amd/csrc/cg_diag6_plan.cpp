@@ -172,6 +172,7 @@ int make_args(const VecPlan &plan, const std::vector<const gelib_part_desc *> &r
   const bool lane_sums = (xbc && xg) || (ybc && yg);
   const bool gaps = n >= 16 && (r_is_dest ? busy < 0.79 && (n % 8 == 0 || n > 64) : busy < 0.77);
   const bool want_tight = g_tight < 0 ? gaps : g_tight != 0 && busy < 1;
+  bool tight = false;
   if (want_tight && !lane_sums) {
     const long long reach = (n + 62) / n;   // cells behind the wave's first that its lanes reach
     auto fits = [&](const std::vector<FastPart> &v) {
@@ -179,10 +180,10 @@ int make_args(const VecPlan &plan, const std::vector<const gelib_part_desc *> &r
         if (p.sb < 0 || (reach * p.sb + n) * 8 >= (1LL << 31)) return false;
       return true;
     };
-    a->tight = fits(fx) && fits(fy) && fits(fr) && fits(fxg) && fits(fyg) && ncells < (1LL << 36);
+    tight = fits(fx) && fits(fy) && fits(fr) && fits(fxg) && fits(fyg) && ncells < (1LL << 36);
   }
-  if (a->tight) {
-    a->lg_npad = 0;
+  if (tight) {
+    a->lg_npad = kDiagTight;
     a->groups = 1;
     a->nwaves = (ncells * n + 63) / 64;
     a->magic64 = ~0ull / (unsigned long long)n + 1;

@@ -20,7 +20,7 @@ __global__ void __launch_bounds__(256) diag6_small_fwd_kernel(const Diag6Args a)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long long w = (long long)blockIdx.x * 4 + wave;
   if (w >= a.nwaves) return;  // uniform for the wave; the kernel has no barrier
-  const WavePos q = wave_pos(a, w);
+  const WavePos q = wave_pos<PACKED>(a, w);
   static_for<kSmallLop + 1>([&](auto l1c) __attribute__((always_inline)) {
     constexpr int L1 = decltype(l1c)::value;
     if (a.x[L1].ptr != nullptr) {
@@ -47,7 +47,7 @@ __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const long long w = (long long)blockIdx.x * 4 + wave;
   if (w >= a.nwaves) return;  // uniform for the wave; the kernel has no barrier
-  const WavePos q = wave_pos(a, w);
+  const WavePos q = wave_pos<PACKED>(a, w);
   const bool accumulate = a.accumulate != 0;
   const bool wx = a.want_x != 0, wy = WY && a.want_y != 0;
   // the wave's own image: only this wave touches it, and a wave's LDS operations execute in order
