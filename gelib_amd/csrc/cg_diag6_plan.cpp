@@ -163,14 +163,27 @@ int make_args(const VecPlan &plan, const std::vector<const gelib_part_desc *> &r
   while ((1 << lg) < n && lg < 6) lg++;
   a->lg_npad = lg;
   // Sums over the lanes of a cell (the gradient of a one-channel operand) need the cells in aligned groups of lanes.
-  // Otherwise the cells follow each other without gaps where enough lanes would idle.  Measured, aligned groups / without gaps,
-  // microseconds: features x harmonics up to l = 2, 24 channels, L = 3, 60013 cells forward 460 / 440, x-gradient 358 / 340;
-  // 48 channels, L = 2 528 / 496, 544 / 455; Diag L = 6, 72 channels, 8000 cells 2617 / 2045, 2242 / 1684; L = 4, 100 channels
-  // 1153 / 976, 943 / 909.  Forward, rows that are no multiple of 64 bytes then lie across more cache lines per store
-  // (Diag L = 6, 20 channels 1943 / 2097, 50 channels 1967 / 2795); backward that is less (1611 / 1298, 1516 / 1575).
+  // Otherwise the cells follow each other without gaps where enough lanes would idle.  Time without gaps over time in aligned
+  // groups, at 100 MB / 300 MB / 1 GB or more of operands and results, memory that other calls have pushed out of the caches:
+  // Forward, whole 64-byte pieces: Diag L = 3, 72 channels .79 .70 .63, L = 4 .85 .79 .64, L = 6 .99 .88 .82, 24 channels L = 3 1.01
+  // .96 .96, L = 6 1.00 1.00 .91, but L = 4 1.00 1.08 .98.  Rows that are no multiple of 64 bytes lie across more cache lines per store: 17
+  // channels 1.19 1.07 1.02, 1.06 1.14 1.29; above 64 channels that pays at L = 3 and 4 (65 channels .93 .83 .79, 98
+  // 1.01 .95 .87), not below (L = 1, 98 channels 1.04 1.08 1.08).  Features x harmonics up to l = 1: 24 to 48 channels 1.00 to 1.04.
+  // Backward the wave count falls with the gaps, and a launch that does not fill the GPU gains nothing for its unaligned
+  // rows: L = 4, 33 channels 1.07 (870 waves) .93 (2670) .79, 44 channels 1.04 1.07 (2000) .92 (10000); L = 6, 36 channels
+  // 1.11 (230) 1.05 (700) .90 (3400); L = 3, 48 channels 1.00 1.01 (4200) .92 (21000), 20 channels 1.02 1.07 (5000) .89
+  // (25000).  Capped products only up to 32 channels
+  // (every l: L = 4, 17 channels 1.04 1.03 1.06); harmonics of l = 0 alone 1.0 to 1.1.
   const double busy = n <= 64 ? (double)n / (1 << lg) : (double)n / (64 * ((n + 63) / 64));
   const bool lane_sums = (xbc && xg) || (ybc && yg);
-  const bool gaps = n >= 16 && (r_is_dest ? busy < 0.79 && (n % 8 == 0 || n > 64) : busy < 0.77);
+  const long long waves = lg < 6 ? ncells >> (6 - lg) : ncells * ((n + 63) / 64);   // of aligned groups
+  const int top_x = lx.back().first, top_y = ly.back().first, lop = std::max(top_x, top_y);
+  const int narrow = xbc ? top_x : (ybc ? top_y : kNP);   // largest l of a one-channel operand
+  bool gaps;
+  if (r_is_dest) gaps = busy < 0.79 && (n > 64 ? n % 8 == 0 || (n < 128 && lop >= 3 && lop <= 4)
+                                               : n >= 16 && n % 8 == 0 && lop != 4 && (narrow >= 2 || lop <= 1));
+  else gaps = n >= 16 && ((busy <= 0.63 && waves >= (lop == 3 ? 6000 : 2200)) || (busy <= 0.76 && waves >= 8192)) &&
+              (n > 32 || *lcap <= lop) && (narrow >= 1 || lop <= 1);
   const bool want_tight = g_tight < 0 ? gaps : g_tight != 0 && busy < 1;
   bool tight = false;
   if (want_tight && !lane_sums) {
@@ -237,13 +250,18 @@ int diag6_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
   if (l8 && !(lcap <= 8 && operands_up_to(a, 4) && g_l8_enable)) return GELIB_HIP_OK;
   a.accumulate = accumulate ? 1 : 0;
   // A one-channel operand up to l = 2 (harmonics) leaves few pairs per part of the other one, and the block form's staging
-  // and barrier cost more than its waves' neighbouring stores gain, from 24 channels on (block / wave form, microseconds:
-  // L = 3, 24 channels, 60013 cells 440 / 371; 40 channels 470 / 388; 64 channels 441 / 352; L = 2, 48 channels, harmonics
-  // up to l = 3 496 / 356 -- but 17 channels 319 / 399, and up to l = 4 at L = 4, 16 channels 640 / 676).
-  int narrow_l = kNP;
-  for (int l = 0; l < kNP; l++)
+  // and barrier cost more than its waves' neighbouring stores gain, from 24 channels on.  Wave / block form at 100 MB and 1 GB:
+  // harmonics of l = 0, L = 3 .45 to .76 and .38 to .66; up to l = 1, L = 3, 24 channels .87 .80, 64 .86 .81, 72 .67 .54, L = 4 .85
+  // .87, .98 .86, .66 .54; up to l = 2, L = 3 .98 .90, .93 .85, .73 .67.  Not for 17 to 23 channels (L = 4, up to l = 2: 1.01
+  // 1.25; 22 .97 1.25) and 25 to 31 (28: L = 3 1.01 1.04, L = 4 1.05 1.17), nor for harmonics up to l = 2 at L = 4 (32 channels 1.12
+  // .89, 48 1.11 .84, 96 1.08 .76) or above (L = 4, up to l = 3 1.1 to 1.5).
+  int narrow_l = kNP, wide_l = 0;
+  for (int l = 0; l < kNP; l++) {
     if ((a.xbc && a.x[l].ptr) || (a.ybc && a.y[l].ptr)) narrow_l = l;
-  const bool small4 = g_small_enable && (g_small4_fwd < 0 ? narrow_l <= 2 && a.n >= 24 : g_small4_fwd != 0);
+    if ((a.xbc && a.y[l].ptr) || (a.ybc && a.x[l].ptr)) wide_l = l;
+  }
+  const bool few_pairs = narrow_l <= 1 || (narrow_l == 2 && wide_l <= 3);
+  const bool small4 = g_small_enable && (g_small4_fwd < 0 ? few_pairs && (a.n > 32 || (a.n >= 24 && a.n % 8 == 0)) : g_small4_fwd != 0);
   if (g_small_enable && lcap <= 4 && operands_up_to(a, 2)) rc = launch_diag6_small_fwd(a, s);
   else if (small4 && lcap <= 6 && operands_up_to(a, 4)) rc = launch_diag6_small4_fwd(a, s);
   else if (hi) rc = a.lg_npad < 6 ? launch_diag6_fwd_hi_packed(a, s) : launch_diag6_fwd_hi(a, s);
