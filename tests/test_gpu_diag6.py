@@ -353,3 +353,26 @@ def test_forward_with_and_without_a_block_per_cell(cabi, B, tx, ty, maxl, diag, 
     finally:
         cabi.set_option("diag6_small4_fwd", -1)
     O.check_fwd([U.host(a) for a in drs], "B%d %s x %s small4 %d" % (B, tx, ty, small4))
+
+
+@pytest.mark.parametrize("tx,ty,maxl", [({0: 70}, {l: 1 for l in range(7)}, 0), ({0: 70, 1: 70}, {l: 1 for l in range(7)}, 1),
+                                        ({l: 1 for l in range(6)}, {0: 24, 1: 24}, 1)])
+def test_parts_above_the_cap_are_left_out(cabi, tx, ty, maxl):
+    """Harmonics that reach no part of the product: the wide operand's gradient, and both (zeros for what feeds nothing)."""
+    B = 6
+    xs = [U.seeded(1700 + l, B, 2 * l + 1, n) for l, n in sorted(tx.items())]
+    ys = [U.seeded(1750 + l, B, 2 * l + 1, n) for l, n in sorted(ty.items())]
+    O = U.VecOracle(xs, ys, maxl, False, gseed=1800)
+    dxs, dys, dgs = [U.dev(a) for a in xs], [U.dev(a) for a in ys], [U.dev(a) for a in O.gs]
+    drs = [torch.full(p.shape, 7.0 + 1j, dtype=torch.complex64, device="cuda") for p in O.r32]
+    new = lambda L: [torch.full(a.shape, 3.0 - 2j, dtype=torch.complex64, device="cuda") for a in L]
+    cabi.so3vec_fwd(drs, dxs, dys, accumulate=False)
+    assert cabi.last_path() == DIAG6
+    xg, yg, xg1, yg1 = new(xs), new(ys), new(xs), new(ys)
+    cabi.so3vec_bwd(xg, yg, dgs, dxs, dys, accumulate=False)
+    cabi.so3vec_bwd(xg1, None, dgs, dxs, dys, accumulate=False)
+    cabi.so3vec_bwd(None, yg1, dgs, dxs, dys, accumulate=False)
+    torch.cuda.synchronize()
+    O.check_fwd([U.host(a) for a in drs], "forward")
+    O.check_bwd([U.host(a) for a in xg], [U.host(a) for a in yg], "both")
+    O.check_bwd([U.host(a) for a in xg1], [U.host(a) for a in yg1], "one at a time")
