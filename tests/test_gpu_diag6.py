@@ -322,18 +322,38 @@ def test_pairs_without_gaps_and_one_gradient(cabi, B, tx, ty, maxl, diag, tight)
     O.check_bwd([U.host(a) for a in xg1], [U.host(a) for a in yg1], tag + " one at a time")
 
 
-def test_no_gradient_for_harmonics(cabi):
-    """An operand that needs no gradient gets none, and the other's is the same as with it."""
+@pytest.mark.parametrize("lead,shared,swap", [((7,), False, False), ((7,), False, True), ((7,), True, False), ((7,), True, True),
+                                              ((2, 3, 2, 2), False, False), ((2, 3, 2, 2), False, True), ((2, 3, 2, 2), True, False)])
+def test_no_gradient_for_harmonics(cabi, monkeypatch, lead, shared, swap):
+    """An operand that needs no gradient gets none -- the library is not asked for it --, and the other's is the same as with it;
+    also with the harmonics first, more than two grid dimensions, and the harmonics shared by the batch and the grid."""
     import gelib_amd as G
-    x = [U.dev(U.seeded(3 + l, 7, 2 * l + 1, 24)).requires_grad_() for l in range(4)]
-    y = [U.dev(U.seeded(30 + l, 7, 2 * l + 1, 1)) for l in range(3)]
-    out = list(G.CGproduct(G.SO3vec(*x), G.SO3vec(*y), 3).parts.values())
+    from gelib_amd.gelib_common import backend
+    vec = G.SO3vec if len(lead) == 1 else G.SO3vecArr
+    real = backend().SO3vec.setCGproduct_back
+    asked = []
+
+    def recorded(xg, yg, g, x, y):
+        asked.append([len(v.get_tau().get_parts()) for v in (xg, yg)])
+        return real(xg, yg, g, x, y)
+
+    monkeypatch.setattr(backend().SO3vec, "setCGproduct_back", staticmethod(recorded))
+    small = tuple(1 for _ in lead) if shared else lead
+    x = [U.dev(U.seeded(3 + l, *lead, 2 * l + 1, 24)).requires_grad_() for l in range(4)]
+    y = [U.dev(U.seeded(30 + l, *small, 2 * l + 1, 1)) for l in range(3)]
+    product = lambda: list((G.CGproduct(vec(*y), vec(*x), 3) if swap else G.CGproduct(vec(*x), vec(*y), 3)).parts.values())
+    out = product()
     gs = [U.dev(U.seeded(60 + i, *p.shape)) for i, p in enumerate(out)]
     got = torch.autograd.grad(out, x, gs)
     for t in y:
         t.requires_grad_()
-    both = torch.autograd.grad(list(G.CGproduct(G.SO3vec(*x), G.SO3vec(*y), 3).parts.values()), x + y, gs)
+    both = torch.autograd.grad(product(), x + y, gs)
+    assert asked == ([[0, 4], [3, 4]] if swap else [[4, 0], [4, 3]])
     for a, b in zip(got, both):
+        assert float((a - b).abs().max()) <= 1e-6 * float(b.abs().max())
+    only = torch.autograd.grad([p for p in product()], y, gs)   # every part of either operand needs one: both are formed
+    assert asked[2] == asked[1]
+    for a, b in zip(only, both[4:]):
         assert float((a - b).abs().max()) <= 1e-6 * float(b.abs().max())
 
 
