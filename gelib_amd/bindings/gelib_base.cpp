@@ -202,9 +202,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                     std::vector<SO3part<float>> R, X;
                     for (auto &t : r) R.push_back(SO3part<float>(view_of(t)));
                     for (auto &t : x) X.push_back(SO3part<float>(view_of(t)));
-                    if (back) gmap.device_handle();  // made on the caller's map, which the reversed copy below shares
                     StreamGuard sg;
-                    SO3part<float>::gather_parts(R, X, back ? gmap.inv() : gmap, d, 0);
+                    SO3part<float>::gather_parts(R, X, gmap, d, back, 0);
                   },
                   py::arg("r"), py::arg("x"), py::arg("gmap"), py::arg("d"), py::arg("back"))
       .def("getl", &SO3part<float>::getl)

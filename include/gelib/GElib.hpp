@@ -430,29 +430,28 @@ class SO3part : public cnine::BatchedTensor<std::complex<TYPE>>, public GpartBas
   }
 
   // ---- sums of slices along grid dimension d (core/Gpart.hpp:556-562) ----
-  void add_gather(const SO3part &x, const cnine::GatherMapB &gmap, const int d = 0) const { gather_parts({*this}, {x}, gmap, d, 1); }
-  // r[i] (+)= x[i] gathered, for several parts in one call (parts of ordinary layout share a launch)
+  void add_gather(const SO3part &x, const cnine::GatherMapB &gmap, const int d = 0) const { gather_parts({*this}, {x}, gmap, d, false, 1); }
+  void add_gather_back(const SO3part &r, const cnine::GatherMapB &gmap, const int d = 0) const { gather_parts({*this}, {r}, gmap, d, true, 1); }
+  // r[i] (+)= x[i] gathered, for several parts in one call (parts of ordinary layout share a launch); back: with the map read
+  // backwards.  The map is the caller's own throughout: a copy of it copies its pairs, and is without the device's copy until
+  // one is made.
   static void gather_parts(const std::vector<SO3part> &r, const std::vector<SO3part> &x, const cnine::GatherMapB &gmap, const int d,
-                           const int accumulate) {
+                           const bool back, const int accumulate) {
     GELIB_ASSRT(r.size() == x.size());
+    const int n_from = back ? gmap.d_out() : gmap.d_in(), n_to = back ? gmap.d_in() : gmap.d_out();
     std::vector<gelib_part_desc> R, X;
     for (size_t i = 0; i < r.size(); i++) {
       GELIB_ASSRT(x[i].dev == r[i].dev);
       if (r[i].dev != 1) GELIB_ERROR("SO3part::add_gather: the operands must be on GPU");
       GELIB_ASSRT(r[i].ndims() <= 5 && x[i].ndims() == r[i].ndims());
       GELIB_ASSRT(d >= 0 && d < r[i].ndims() - 3);
-      GELIB_ASSRT(gmap.d_in() == x[i].dims[d + 1]);
-      GELIB_ASSRT(gmap.d_out() == r[i].dims[d + 1]);
+      GELIB_ASSRT(n_from == x[i].dims[d + 1]);
+      GELIB_ASSRT(n_to == r[i].dims[d + 1]);
       R.push_back(r[i].descriptor());
       X.push_back(x[i].descriptor());
     }
-    gelib_check(gelib_hip_vec_gather((int)R.size(), R.data(), X.data(), gmap.device_handle(), d + 1, gmap.inverted ? 1 : 0,
+    gelib_check(gelib_hip_vec_gather((int)R.size(), R.data(), X.data(), gmap.device_handle(), d + 1, gmap.inverted != back ? 1 : 0,
                                      accumulate, gelib_stream()));
-  }
-  void add_gather_back(const SO3part &r, const cnine::GatherMapB &gmap, const int d = 0) const {
-    gmap.device_handle();  // made on the caller's map, so the reversed copy below shares it instead of uploading,
-                           // using and freeing a device copy of its own on every call
-    add_gather(r, gmap.inv(), d);
   }
 
   std::string classname() const { return "GElib::SO3part"; }

@@ -147,3 +147,32 @@ def test_recorded_calls_use_lent_scratch(cabi):
     finally:
         cabi.set_option("bcast_reduce", 1)
         cabi.set_stream_workspace(None, stream)
+
+
+def test_gather_reuses_the_maps_copy_on_the_device():
+    """A map is uploaded once, by the first call that uses it: later calls of either direction can be recorded into a graph,
+    which neither an allocation nor a copy from the host can."""
+    import gelib_amd as G
+    gmap = G.gather_map.random(40, 30, 0.2, seed=5)
+    x = G.SO3vecArr(*[U.dev(U.seeded(l, 1, 40, 2 * l + 1, 4)) for l in range(3)])
+    y = [U.dev(U.seeded(10 + l, 1, 30, 2 * l + 1, 4)) for l in range(3)]
+    for p in x.parts.values():
+        p.requires_grad_()
+
+    def step():
+        out = list(x.gather(gmap).parts.values())
+        return out + list(torch.autograd.grad(out, list(x.parts.values()), y))
+
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for turn in range(3):
+        for i, t in enumerate(list(x.parts.values()) + y):
+            t.data.copy_(U.dev(U.seeded(100 * turn + i, *t.shape)))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = bits([t.detach().as_subclass(torch.Tensor) for t in out])
+        want = bits([t.detach().as_subclass(torch.Tensor) for t in step()])
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
