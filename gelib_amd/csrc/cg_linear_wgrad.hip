@@ -18,15 +18,16 @@
 // Sums in two levels: the matrix instructions add the 2 (2 l + 1) terms of each of eight cells, and those sums are added to a
 // second set of registers.  One chain of matrix instructions over a range was up to twice as far from the exact result as
 // forming the product and summing it in mix.hip, whose chains are at least 128 rows long (relative error for l = 0..4, one chain /
-// two levels / mix.hip, in 1e-7: 8192 cells of 16 x 16 -> 16 channels 2.0 3.0 3.8 4.4 4.9 / 1.4 1.7 2.0 2.2 2.5 /
-// 2.3 2.3 2.3 2.4 2.6; 8 x 8 2.6 4.0 5.0 5.9 6.6 / 1.4 1.7 2.0 2.2 2.5 / 2.3 2.4 2.5 2.6 2.8; 16 cells of 16 x 16
+// two levels / mix.hip, in 1e-7: 8192 cells in chunks of 1024 of 16 x 16 -> 16 channels 2.0 3.0 3.8 4.4 4.9 / 1.4 1.7 2.0 2.2
+// 2.5 / 2.3 2.3 2.3 2.4 2.6, all at once - / 1.6 1.9 2.2 2.4 2.6 / 2.3 3.4 4.7 5.7 6.0; 8 x 8 2.6 4.0 5.0 5.9 6.6 /
+// 1.4 1.7 2.0 2.2 2.5 / 2.3 2.4 2.5 2.6 2.8; 16 cells of 16 x 16
 // 1.2 1.8 2.3 2.8 3.1 / 0.9 1.4 1.7 2.0 2.2 / 1.0 1.4 1.7 2.0 2.3).  The second set takes the kernel from three waves per
 // SIMD to two: 8192 cells of 16 x 16 channels 1755 -> 2090 us, 8 x 8 767 -> 920.
 // What bounds it: matrix instructions (64 clocks a row and 32 channels) plus vector instructions (4 clocks each, about 2600
 // a cell and 32 channels of the L = 4 product), which do not overlap within a wave; the operands come from L2.
 // Measured against forming the product, the matrix-gradient kernels of mix.hip on it and their sums (L = 4, 16 outputs,
-// microseconds, in 1 GiB): 8192 cells of 16 x 16 channels 4414 -> 2091, of 8 x 8 1107 -> 917; 1024 cells 543 -> 263 and
-// 192 -> 140; 64 cells of 16 x 16 153 -> 81.
+// microseconds): 8192 cells of 16 x 16 channels 2638 -> 1888 (in 1 GiB 4414 -> 2091), of 8 x 8 910 -> 885; 1024 cells
+// 543 -> 263 and 192 -> 140; 64 cells of 16 x 16 153 -> 81.
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -44,8 +45,8 @@ typedef const __attribute__((address_space(4))) float *CoeffPtr;
 
 constexpr int kWNL = kLinL + 1;
 constexpr double kWgradLeast = 0.6;      // share of a sum's 32 rows that are channels
-constexpr double kWgradLeastMany = 0.39;  // share of a block's 128 channels, for more cells than
-constexpr long long kWgradFew = 2048;
+// ... and of a block's 128, for this many cells at a time
+constexpr double least_of_block(long long ncells) { return ncells <= 2048 ? 0.0 : (ncells <= 8192 ? 0.43 : (ncells <= 16384 ? 0.62 : 0.7)); }
 constexpr long long kWgradCells = 16;    // fewer: mix.hip's chains are shorter than those of eight cells here
 constexpr int kWPairs = kWNL * kWNL;
 constexpr int kWTile = 8;                       // cells staged at a time
@@ -260,13 +261,14 @@ int cg_linear_wgrad(const VecPlan &plan, const std::vector<const gelib_part_desc
   const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
   if (ncells < kWgradCells) return GELIB_HIP_OK;
   // Channels fill the 32 rows of a sum and the 128 of a block; with fewer than 19 channels a pair half the matrix work is
-  // padding, and with fewer than 50 most waves of a block only stage.  The product of so few channels is small enough to store
-  // once there are cells enough to hide the launches that takes (with the gradients of x and y, product stored / not, us, 12
-  // outputs: 32 channels a pair, 256 cells 263 / 193, 1536 cells 345 / 320, 2048 365 / 361, 3072 524 / 533, 8192 1055 / 1270;
-  // 40 channels 2048 cells 468 / 450, 5000 904 / 1019; 48 channels 5000 cells 995 / 1068; 50 channels 8192 cells 2057 / 2042,
-  // 64 channels 2146 / 1938).
-  const bool few = ncells <= kWgradFew;
-  if (!force && (useful < kWgradLeast * padded || (!few && useful < kWgradLeastMany * blocks))) return GELIB_HIP_OK;
+  // padding, and with fewer than 128 some waves of a block only stage.  The product of few channels is small enough to store
+  // once there are cells enough to hide the launches that takes (with the gradients of x and y, 12 outputs, product stored /
+  // not, microseconds: 256 cells, 32 channels a pair 263 / 193; 2048 cells, 32 channels 365 / 361, 40 channels 468 / 450;
+  // 3072 cells, 32 channels 524 / 533; 4096 cells, 48 channels 888 / 896, 56 channels 1043 / 955; 8192 cells, 50 channels 1837 /
+  // 1906, 56 channels 1729 / 1670, 132 channels 3672 / 3700; 16384 cells, 64 channels 3105 / 3262, 80 channels 4010 / 3876, 144
+  // channels 6413 / 6908, 192 channels 8651 / 8297; 32768 cells, 80 channels 7428 / 7964, 96 channels 8905 / 8412, 156
+  // channels 15.7 / 16.2 ms, 192 channels 17.3 / 16.6).
+  if (!force && (useful < kWgradLeast * padded || useful < least_of_block(ncells) * blocks)) return GELIB_HIP_OK;
   int nwork = 0;
   for (int k = 0; k < kWPairs; k++) {
     const int l1 = kLinL - k / kWNL, l2 = kLinL - k % kWNL;

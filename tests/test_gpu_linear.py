@@ -407,7 +407,8 @@ def test_matrix_gradient_is_as_exact_as_through_the_product(cabi, B, n1, n2, nou
         assert a <= 1.03 * b, err
 
 
-@pytest.mark.parametrize("B,n1,n2,direct", [(2048, 5, 4, True), (2049, 5, 4, False), (2049, 10, 5, True), (64, 4, 4, False)])
+@pytest.mark.parametrize("B,n1,n2,direct", [(2048, 5, 4, True), (2049, 5, 4, False), (2049, 8, 7, True), (8193, 8, 7, False), (8193, 10, 8, True),
+                                              (16385, 10, 8, False), (16385, 12, 8, True), (64, 4, 4, False)])
 def test_where_matrix_gradients_come_straight_from_the_operands(cabi, B, n1, n2, direct):
     xs = [torch.zeros(B, 2 * l + 1, n1, dtype=torch.complex64, device="cuda") for l in range(5)]
     ys = [torch.zeros(B, 2 * l + 1, n2, dtype=torch.complex64, device="cuda") for l in range(5)]
@@ -417,7 +418,7 @@ def test_where_matrix_gradients_come_straight_from_the_operands(cabi, B, n1, n2,
     for option, want in ((1, direct), (0, False), (2, True)):
         cabi.set_option("linear_wgrad", option)
         try:
-            assert cabi.so3vec_cg_linear_bwd(None, None, [torch.empty_like(w) for w in ws], gs, xs, ys, ws)
+            assert cabi.so3vec_cg_linear_bwd(None, None, [torch.empty_like(w) for w in ws], gs, xs, ys, ws, workspace_bytes=16 << 30)
             assert (cabi.last_path() == 6) == want
         finally:
             cabi.set_option("linear_wgrad", 1)
