@@ -94,12 +94,14 @@ class SO3linear(torch.nn.Module):
 
 
 class CGproductLinearFn(torch.autograd.Function):
-    """CGproduct(x, y, maxl) * W with the product formed and consumed inside one kernel (forward).  The backward pass
-    forms the product again, a chunk of the batch at a time (gelib_hip_so3vec_cg_linear_bwd): the product and its gradient
-    exist only for the chunk at hand, in a workspace of at most BWD_WORKSPACE_BYTES, and nothing of the product's size is
-    kept between the two passes."""
+    """CGproduct(x, y, maxl) * W with the product formed and consumed inside one kernel (forward).  The backward pass works
+    through the batch a chunk at a time (gelib_hip_so3vec_cg_linear_bwd): the product's gradient, and the product where
+    the matrices' gradients are not formed straight from the operands, exist only for the chunk at hand, in a workspace of
+    at most BWD_WORKSPACE_BYTES, and nothing of the product's size is kept between the two passes.  The waves of a launch
+    share the channel sums of a group of cells as the launch's size allows, so the last bits of a cell's result depend on
+    the size of the batch it is in; from run to run they do not change."""
 
-    BWD_WORKSPACE_BYTES = 8 << 30   # headline type, 32768 cells: 34.6 ms with 1 GiB, 24.5 with 4, 22.0 with 8, 19.5 with 28 (one chunk)
+    BWD_WORKSPACE_BYTES = 8 << 30   # headline type, 32768 cells: 24.1 ms with 1 GiB, 19.1 with 4, 19.1 with 8, 18.5 with 28 (one chunk)
 
     @staticmethod
     def forward(ctx, k1, k2, maxl, *args):

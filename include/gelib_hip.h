@@ -210,7 +210,7 @@ int gelib_hip_o3vec_cg_bwd(int diag, const gelib_part_desc *xg, const gelib_part
  * index.  Anything else returns GELIB_HIP_ERR_UNSUPPORTED with nothing launched: the caller then forms the product with
  * gelib_hip_so3vec_cg_fwd and mixes each part with gelib_hip_part_mix_channels.  The sums over c run in a fixed order
  * (in float32 on the matrix cores: ascending c per row, or, where the workspace has room for partial sums, several such
- * sums over parts of the range of c added in a fixed order); results agree with the two-call form to rounding, not bit
+ * sums over parts of the range of c, as many as the number of cells leaves waves idle, added in a fixed order); results agree with the two-call form to rounding, not bit
  * for bit. */
 int gelib_hip_so3vec_cg_linear_fwd(int nr, const gelib_part_desc *r, int nx, const gelib_part_desc *x, int ny,
                                    const gelib_part_desc *y, const void *const *w, int accumulate, void *workspace,
@@ -221,7 +221,9 @@ int gelib_hip_so3vec_cg_linear_fwd(int nr, const gelib_part_desc *r, int nx, con
 uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes(int nr, const gelib_part_desc *r, int nx, const gelib_part_desc *x,
                                                     int ny, const gelib_part_desc *y);
 /* ... and with room for the partial sums of launches too small to fill the GPU with one wave per 32 cells (at most
- * 420 MB more; nothing more for large batches): with this much the call is up to 60 times faster on such batches. */
+ * 420 MB more; nothing more for large batches): with this much the call is up to 60 times faster on such batches.
+ * How many sums a cell's result is added from then depends on the number of cells in the call, and with it the last bits of the
+ * result (never on timing); with the workspace of the function above every call adds in ascending c, whatever its size. */
 uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes_shared(int nr, const gelib_part_desc *r, int nx,
                                                            const gelib_part_desc *x, int ny, const gelib_part_desc *y);
 
@@ -234,8 +236,8 @@ uint64_t gelib_hip_so3vec_cg_linear_workspace_bytes_shared(int nr, const gelib_p
  *                                                    with respect to the matrix; w[k] and wg[k] belong to g[k]).
  * Any of xg, yg, wg may be NULL.  Neither P nor gP is ever held at full size (25 GB each at the headline type): the
  * batch is taken in chunks whose product fits the workspace.  For operands up to l = 4, a product with every l up
- * to min(l1 + l2, 4), at most 16 channels on every side, at least about 19 channel pairs per (l1, l2) (50 in chunks of more than
- * 2048 cells) and 16 cells, the matrices' gradients come straight from the operands; otherwise the forward kernels form a
+ * to min(l1 + l2, 4), at most 16 channels on every side, at least about 19 channel pairs per (l1, l2) (more in
+ * chunks of more than 2048 cells: 55 to 90) and 16 cells, the matrices' gradients come straight from the operands; otherwise the forward kernels form a
  * chunk's product there and the matrix-gradient kernel reads it.  gP is formed in that
  * memory and the backward kernels read it.
  * workspace: 256-byte aligned device memory; gelib_hip_so3vec_cg_linear_bwd_workspace_bytes(..., batch_chunk) tells the
