@@ -53,12 +53,13 @@ struct Diag6Args {
   int n;              // channels of every part (of every part of the wider operand when xbc or ybc is set)
   int xbc, ybc;       // CGproduct with a one-channel first / second operand: every lane reads that channel
   int offs_add;
-  int accumulate;
+  int write;           // WriteMode
   int want_x, want_y;  // backward: which gradients are stored (the operand of an unwanted one is never read)
   int owner[kNP];      // backward: which of the block's four waves takes the pairs with this l2
   // (last, so that the loads of the fields above are those of the launches that do not need these)
   unsigned long long magic64;  // kDiagTight: ceil(2^64 / n), quotients of pair numbers below 2^50
   unsigned magic32;            // kDiagTight: ceil(2^32 / n), quotients of numbers below n + 64
+  int once;                    // backward (the host's choice of kernel): g is read with loads that do not keep the line
 };
 // lg_npad of a launch whose (cell, channel) pairs follow each other without gaps, 64 per wave, so that a channel count that is
 // no power of two (or no multiple of 64) leaves no lane idle; kernels of the packed form only, and no sums over the lanes of a

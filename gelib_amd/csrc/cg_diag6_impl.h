@@ -42,6 +42,14 @@ __device__ __forceinline__ float2 row_load(RowPtr row, unsigned lane_off) {
   const v2f t = *(GlobalIn)(row + lane_off);
   return make_float2(t.x, t.y);
 }
+// ... of a row of g.  ONCE: streaming loads (Diag6Args::once).
+template <bool ONCE>
+__device__ __forceinline__ float2 row_load_g(RowPtr row, unsigned lane_off) {
+  if constexpr (!ONCE) return row_load(row, lane_off);
+  asm volatile("" : "+v"(lane_off));
+  const v2f t = __builtin_nontemporal_load((GlobalIn)(row + lane_off));
+  return make_float2(t.x, t.y);
+}
 __device__ __forceinline__ void row_store(RowPtr row, unsigned lane_off, float2 v, bool accumulate) {
   v2f o = {v.x, v.y};
   if (accumulate) {
@@ -51,6 +59,13 @@ __device__ __forceinline__ void row_store(RowPtr row, unsigned lane_off, float2 
   }
   asm volatile("" : "+v"(lane_off));
   *(GlobalOut)(row + lane_off) = o;
+}
+__device__ __forceinline__ void row_store_stream(RowPtr row, unsigned lane_off, float2 v) {
+  const v2f o = {v.x, v.y};
+  asm volatile("" : "+v"(lane_off));  // (also keeps this store and the one above apart: at the head of two branches they
+                                      // would become one ordinary store)
+  __builtin_nontemporal_store(o, (GlobalOut)(row + lane_off));
+  asm volatile("");
 }
 
 // A wave covers 64 channels of one cell, or -- when a part has 32 channels or fewer -- all channels of 64 / n_pad
@@ -126,7 +141,7 @@ __device__ __forceinline__ void fwd_pair(const Diag6Args &a, const float2 (&xv)[
     constexpr int NL = LTOP - LMIN + 1;
     const OffsPtr offs = (OffsPtr)a.offs + (L1 * kNP + L2) * kNR;
     const CoeffPtr C = (CoeffPtr)a.bank;
-    const bool accumulate = a.accumulate != 0;
+    const bool accumulate = a.write == kWriteAdd, stream = a.write == kWriteStream;
     // the row of part l that the next m of that part is stored to; a triple that is not there is never stored
     RowPtr row[NL];
     unsigned lo[NL];
@@ -164,7 +179,10 @@ __device__ __forceinline__ void fwd_pair(const Diag6Args &a, const float2 (&xv)[
         constexpr int dl = decltype(dc)::value;
         constexpr int L = LMIN + dl;
         if constexpr (L >= MABS) {
-          if (present[dl] && q.live) row_store(row[dl], lo[dl], acc[dl], accumulate);
+          if (present[dl] && q.live) {
+            if (stream) row_store_stream(row[dl], lo[dl], acc[dl]);
+            else row_store(row[dl], lo[dl], acc[dl], accumulate);
+          }
           row[dl] += row_step(a.r[L]);
         }
       });
@@ -243,7 +261,7 @@ __global__ void __launch_bounds__(256) diag6_fwd_kernel(const Diag6Args a) {
 
 // One pair of the backward pass: every l of the pair together, one row number m = m1 + m2 at a time.  WY = false: the
 // y-gradient is not wanted (no sums, no image).
-template <int L1, int L2, int LCAP, bool PACKED, int LLO = 0, bool WY = true>
+template <int L1, int L2, int LCAP, bool PACKED, bool ONCE, int LLO = 0, bool WY = true>
 __device__ __forceinline__ void bwd_pair(const Diag6Args &a, const float2 (&xv)[2 * L1 + 1],
                                          const float2 (&yv)[2 * L2 + 1], float2 (&ax)[2 * L1 + 1], float2 *yimg,
                                          const WavePos q) {
@@ -278,7 +296,7 @@ __device__ __forceinline__ void bwd_pair(const Diag6Args &a, const float2 (&xv)[
       static_for<NL>([&](auto dc) __attribute__((always_inline)) {
         constexpr int dl = decltype(dc)::value;
         if constexpr (LMIN + dl >= iabs(m)) {
-          dst[dl] = row_load(row[dl], lo[dl]);
+          dst[dl] = row_load_g<ONCE>(row[dl], lo[dl]);
           row[dl] += step[dl];
         }
       });
@@ -377,7 +395,7 @@ __device__ __forceinline__ void store_rows(const float2 *v, int vstride, const F
 // Three waves per SIMD (168 registers) is what the LDS of a block lets a compute unit hold; both forms fit by
 // themselves (the packed one with a smaller row budget).  Forcing the limit with amdgpu_waves_per_eu instead changed the
 // schedule for the worse (twice as many waits).
-template <int LCAP, bool PACKED, int LOP, int LLO = 0>
+template <int LCAP, bool PACKED, int LOP, int LLO, bool ONCE>
 __global__ void __launch_bounds__(256) diag6_bwd_kernel(const Diag6Args a) {
   constexpr int kXRows = 2 * LOP + 1;
   constexpr int kYRows = (LOP + 1) * (LOP + 1);
@@ -386,7 +404,7 @@ __global__ void __launch_bounds__(256) diag6_bwd_kernel(const Diag6Args a) {
   const long long w = blockIdx.x;
   const WavePos q = wave_pos<PACKED>(a, w);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const bool accumulate = a.accumulate != 0;
+  const bool accumulate = a.write == kWriteAdd;
   const bool wx = a.want_x != 0, wy = a.want_y != 0;
   for (int e = threadIdx.x; e < kYRows * 64; e += 256) yimg[e] = make_float2(0.f, 0.f);
   __syncthreads();
@@ -416,7 +434,7 @@ __global__ void __launch_bounds__(256) diag6_bwd_kernel(const Diag6Args a) {
 #pragma unroll
               for (int m2 = 0; m2 <= 2 * L2; m2++) yv[m2] = make_float2(0.f, 0.f);
             }
-            bwd_pair<L1, L2, LCAP, PACKED, LLO>(a, xv, yv, ax, yimg, q);
+            bwd_pair<L1, L2, LCAP, PACKED, ONCE, LLO>(a, xv, yv, ax, yimg, q);
           }
         }
       });
@@ -470,13 +488,13 @@ __global__ void __launch_bounds__(256) diag6_bwd_kernel(const Diag6Args a) {
 // of the image in LDS, the x-gradient partials meet in LDS after the last pair of an l1 -- so the sums are formed in
 // the same order and the results are the same bits.  The four waves run four instantiations of the loop over l1 and
 // meet at its two barriers per l1.
-template <int LCAP, bool PACKED, int LA, int LB>
+template <int LCAP, bool PACKED, bool ONCE, int LA, int LB>
 __device__ __forceinline__ void bwd_wave_set(const Diag6Args &a, float2 *yimg, float2 *xpart, const WavePos q, int wave,
                                              int lane) {
   constexpr int kXRows = 2 * kL6 + 1;
   constexpr int RB = LB >= 0 ? 2 * LB + 1 : 1;
   constexpr int LBX = LB >= 0 ? LB : 0;
-  const bool accumulate = a.accumulate != 0;
+  const bool accumulate = a.write == kWriteAdd;
   const bool wx = a.want_x != 0, wy = a.want_y != 0;
   float2 ya[2 * LA + 1], yb[RB];
 #pragma unroll
@@ -499,8 +517,8 @@ __device__ __forceinline__ void bwd_wave_set(const Diag6Args &a, float2 *yimg, f
       }
 #pragma unroll
       for (int m1 = 0; m1 <= 2 * L1; m1++) ax[m1] = make_float2(0.f, 0.f);
-      bwd_pair<L1, LA, LCAP, PACKED>(a, xv, ya, ax, yimg, q);
-      if constexpr (LB >= 0) bwd_pair<L1, LBX, LCAP, PACKED>(a, xv, yb, ax, yimg, q);
+      bwd_pair<L1, LA, LCAP, PACKED, ONCE>(a, xv, ya, ax, yimg, q);
+      if constexpr (LB >= 0) bwd_pair<L1, LBX, LCAP, PACKED, ONCE>(a, xv, yb, ax, yimg, q);
       if (!wx) return;  // continues with the next l1; uniform for the block
       float2 *mine = xpart + wave * kXRows * 64 + lane;
 #pragma unroll
@@ -543,7 +561,7 @@ __device__ __forceinline__ void bwd_wave_set(const Diag6Args &a, float2 *yimg, f
   }
 }
 
-template <int LCAP, bool PACKED>
+template <int LCAP, bool PACKED, bool ONCE>
 __global__ void __launch_bounds__(256) diag6_bwd_sets_kernel(const Diag6Args a) {
   __shared__ float2 yimg[kImgRows * 64];
   __shared__ float2 xpart[4 * (2 * kL6 + 1) * 64];  // [wave][row][lane]
@@ -551,15 +569,16 @@ __global__ void __launch_bounds__(256) diag6_bwd_sets_kernel(const Diag6Args a) 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   for (int e = threadIdx.x; e < kImgRows * 64; e += 256) yimg[e] = make_float2(0.f, 0.f);
   __syncthreads();
-  if (wave == 0) bwd_wave_set<LCAP, PACKED, 6, -1>(a, yimg, xpart, q, wave, lane);
-  else if (wave == 1) bwd_wave_set<LCAP, PACKED, 5, 0>(a, yimg, xpart, q, wave, lane);
-  else if (wave == 2) bwd_wave_set<LCAP, PACKED, 4, 1>(a, yimg, xpart, q, wave, lane);
-  else bwd_wave_set<LCAP, PACKED, 3, 2>(a, yimg, xpart, q, wave, lane);
+  if (wave == 0) bwd_wave_set<LCAP, PACKED, ONCE, 6, -1>(a, yimg, xpart, q, wave, lane);
+  else if (wave == 1) bwd_wave_set<LCAP, PACKED, ONCE, 5, 0>(a, yimg, xpart, q, wave, lane);
+  else if (wave == 2) bwd_wave_set<LCAP, PACKED, ONCE, 4, 1>(a, yimg, xpart, q, wave, lane);
+  else bwd_wave_set<LCAP, PACKED, ONCE, 3, 2>(a, yimg, xpart, q, wave, lane);
 }
 
 template <int LCAP, bool PACKED>
 int launch_diag6_bwd_sets_variant(const Diag6Args &a, hipStream_t s) {
-  hipLaunchKernelGGL((diag6_bwd_sets_kernel<LCAP, PACKED>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
+  if (a.once) hipLaunchKernelGGL((diag6_bwd_sets_kernel<LCAP, PACKED, true>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((diag6_bwd_sets_kernel<LCAP, PACKED, false>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
 }
@@ -573,7 +592,8 @@ int launch_diag6_fwd_variant(const Diag6Args &a, hipStream_t s) {
 
 template <int LCAP, bool PACKED, int LOP = kL6, int LLO = 0>
 int launch_diag6_bwd_variant(const Diag6Args &a, hipStream_t s) {
-  hipLaunchKernelGGL((diag6_bwd_kernel<LCAP, PACKED, LOP, LLO>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
+  if (a.once) hipLaunchKernelGGL((diag6_bwd_kernel<LCAP, PACKED, LOP, LLO, true>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((diag6_bwd_kernel<LCAP, PACKED, LOP, LLO, false>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
 }

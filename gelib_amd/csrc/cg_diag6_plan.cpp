@@ -25,6 +25,8 @@ int g_small_enable = 1;  // operands up to l = 2, and backward up to l = 4: the 
 int g_hi_enable = 1;    // the kernels for the part l = 7..12 of a product by itself
 int g_tight = -1;        // (cell, channel) pairs without gaps between the cells: -1 where enough lanes would idle, 0 never, 1 always
 int g_small4_fwd = -1;   // forward, operands up to l = 4: the kernel that gives a wave a cell and channel group (-1 = by the shape)
+int g_stream = -1;       // forward: streaming stores (-1 = by the shape, 0 never, 1 always)
+int g_once = -1;         // backward: streaming loads of g (-1 = by the shape, 0 never, 1 always)
 int g_one_channel = 1;  // CGproduct with a one-channel operand runs here as the Diag product with the channel repeated
 
 int device_bank(const float **out) {
@@ -260,7 +262,6 @@ int diag6_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
   const bool hi = llo > kL6 && g_hi_enable;
   const bool l8 = lcap > kL6 && !hi;
   if (l8 && !(lcap <= 8 && operands_up_to(a, 4) && g_l8_enable)) return GELIB_HIP_OK;
-  a.accumulate = accumulate ? 1 : 0;
   // A one-channel operand up to l = 2 (harmonics) leaves few pairs per part of the other one, and the block form's staging
   // and barrier cost more than its waves' neighbouring stores gain, from 24 channels on.  Wave / block form at 100 MB and 1 GB:
   // harmonics of l = 0, L = 3 .45 to .76 and .38 to .66; up to l = 1, L = 3, 24 channels .87 .80, 64 .86 .81, 72 .67 .54, L = 4 .85
@@ -274,6 +275,14 @@ int diag6_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
   }
   const bool few_pairs = narrow_l <= 1 || (narrow_l == 2 && wide_l <= 3);
   const bool small4 = g_small_enable && (g_small4_fwd < 0 ? few_pairs && (a.n > 32 || (a.n >= 24 && a.n % 8 == 0)) : g_small4_fwd != 0);
+  // Streaming stores where rows are whole half-lines; other rows' pieces must meet in a cache before they go to memory.  Streaming /
+  // ordinary at 40, 250 and 1500 MB of product written again and again | the largest, pushed out of the caches: Diag L=6 64 channels
+  // .89 .88 .78 | .96, 24 .90 .82 .74 | .79, 17 .91 1.60 1.71 | 1.71, L=4 48 .92 .95 .75 | .98, 8 .90 .99 .79 | .96, 20 .91 1.40 1.37 |
+  // 1.41, L=2 16 .92 .80 .97 | 1.05; features x harmonics up to l = 2, L=3, 24 channels .89 .94 .75 | .90, 16 .96 .80 .63 | 1.02, 20
+  // 1.00 1.11 1.02 | .96, L=4 24 .92 .79 .56 | .97.  Not for the wave form from 32 channels on (L=3, up to l = 2, 64 channels .91 1.02
+  // .85 | 1.13), nor 8 channels with harmonics up to l = 1 (L=3 .97 .65 1.03 | 1.07).
+  const bool stream = a.n % 8 == 0 && !(small4 && a.n >= 32) && !(a.n == 8 && narrow_l <= 1 && wide_l >= 3);
+  a.write = accumulate ? kWriteAdd : ((g_stream < 0 ? stream : g_stream != 0) ? kWriteStream : kWriteOver);
   if (g_small_enable && lcap <= 4 && operands_up_to(a, 2)) rc = launch_diag6_small_fwd(a, s);
   else if (small4 && lcap <= 6 && operands_up_to(a, 4)) rc = launch_diag6_small4_fwd(a, s);
   else if (hi) rc = a.lg_npad < 6 ? launch_diag6_fwd_hi_packed(a, s) : launch_diag6_fwd_hi(a, s);
@@ -301,7 +310,20 @@ int diag6_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
   const bool hi = llo > kL6 && g_hi_enable;
   const bool l8 = lcap > kL6 && !hi;
   if (l8 && !(lcap <= 8 && operands_up_to(a, 4) && g_l8_enable >= 2)) return GELIB_HIP_OK;
-  a.accumulate = accumulate ? 1 : 0;
+  a.write = accumulate ? kWriteAdd : kWriteOver;
+  // Streaming loads of g (the line is not kept) where a block's rows are whole cache lines, or nearly (operands above l = 4): what
+  // an ordinary load leaves in the caches is never read again, and pushes out what is.  Rows that share lines with the next
+  // block's must keep them.  Streaming / ordinary, 250 MB and 1.5 GB of g that other calls have pushed out of the caches: Diag L=6
+  // 64 channels .77 .87, 24 .80 .88, 17 .82 1.27, L=4 64 .78 .96, 24 .82 1.14, 8 .92 1.28, 3 1.23 1.32, L=2 32 .78 .96, L=1 16 .92
+  // .97; features x harmonics up to l = 2, L=4 32 .64 .90, L=3 16 .65 .91, 24 .79 1.14; capped at l = 1 with harmonics above it .89
+  // 1.02, and 1.1 to 1.2 where g is still in the caches.
+  int top = 0, narrow = kNP;
+  for (int l = 0; l < kNP; l++) {
+    if (a.x[l].ptr || a.y[l].ptr) top = l;
+    if ((a.xbc && a.x[l].ptr) || (a.ybc && a.y[l].ptr)) narrow = l;
+  }
+  const bool lines = top > 4 ? a.n % 8 == 0 && a.n >= 16 : a.n % 16 == 0;
+  a.once = g_once < 0 ? lines && !(lcap <= 1 && narrow >= 2 && narrow < kNP) : g_once;
   a.want_x = xg.empty() ? 0 : 1;
   a.want_y = yg.empty() ? 0 : 1;
   bool all_y = true;
@@ -350,6 +372,16 @@ int diag6_set_option(const char *name, int value) {
   if (!std::strcmp(name, "diag6_tight")) {
     if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
     g_tight = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "diag6_stream")) {
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_stream = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "diag6_once")) {
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_once = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "diag6_small4_fwd")) {

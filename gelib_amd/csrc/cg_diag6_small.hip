@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) diag6_small_fwd_kernel(const Diag6Args a)
 
 // WY = false: only the x-gradient is wanted -- half the multiply-adds behind the contraction, and without the image of the
 // y-gradient (51 KB a block for operands up to l = 4) the registers alone say how many waves a compute unit holds.
-template <int kSmallLop, int kSmallCap, bool PACKED, int LLO, bool WY>
+template <int kSmallLop, int kSmallCap, bool PACKED, int LLO, bool WY, bool ONCE>
 __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a) {
   constexpr int kYRows = (kSmallLop + 1) * (kSmallLop + 1);
   __shared__ float2 yimg_all[WY ? 4 * kYRows * 64 : 1];  // [wave][row][lane]
@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a)
   const long long w = (long long)blockIdx.x * 4 + wave;
   if (w >= a.nwaves) return;  // uniform for the wave; the kernel has no barrier
   const WavePos q = wave_pos<PACKED>(a, w);
-  const bool accumulate = a.accumulate != 0;
+  const bool accumulate = a.write == kWriteAdd;
   const bool wx = a.want_x != 0, wy = WY && a.want_y != 0;
   // the wave's own image: only this wave touches it, and a wave's LDS operations execute in order
   float2 *yimg = yimg_all + (WY ? wave * kYRows * 64 : 0);
@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a)
 #pragma unroll
             for (int m2 = 0; m2 <= 2 * L2; m2++) yv[m2] = make_float2(0.f, 0.f);
           }
-          if constexpr (L1 + L2 >= LLO) bwd_pair<L1, L2, kSmallCap, PACKED, LLO, WY>(a, xv, yv, ax, yimg, q);
+          if constexpr (L1 + L2 >= LLO) bwd_pair<L1, L2, kSmallCap, PACKED, ONCE, LLO, WY>(a, xv, yv, ax, yimg, q);
         }
       });
       if (wx && a.xg[L1].ptr != nullptr) store_rows<L1, PACKED>(ax, 1, a.xg[L1], q, accumulate, a.xbc != 0, a.lg_npad);
@@ -95,19 +95,23 @@ __global__ void __launch_bounds__(256) diag6_small_bwd_kernel(const Diag6Args a)
   });
 }
 
-template <int LOP, int LCAP, int LLO = 0>
-int launch_small_bwd(const Diag6Args &a, hipStream_t s) {
+template <int LOP, int LCAP, int LLO, bool ONCE>
+int launch_small_bwd_g(const Diag6Args &a, hipStream_t s) {
   const unsigned nblocks = (unsigned)((a.nwaves + 3) / 4);
   const bool packed = a.lg_npad < 6;
   if (LLO == 0 && !a.want_y) {
-    if (packed) hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, true, 0, false>), dim3(nblocks), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, false, 0, false>), dim3(nblocks), dim3(256), 0, s, a);
+    if (packed) hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, true, 0, false, ONCE>), dim3(nblocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, false, 0, false, ONCE>), dim3(nblocks), dim3(256), 0, s, a);
   } else {
-    if (packed) hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, true, LLO, true>), dim3(nblocks), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, false, LLO, true>), dim3(nblocks), dim3(256), 0, s, a);
+    if (packed) hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, true, LLO, true, ONCE>), dim3(nblocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((diag6_small_bwd_kernel<LOP, LCAP, false, LLO, true, ONCE>), dim3(nblocks), dim3(256), 0, s, a);
   }
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
+}
+template <int LOP, int LCAP, int LLO = 0>
+int launch_small_bwd(const Diag6Args &a, hipStream_t s) {
+  return a.once ? launch_small_bwd_g<LOP, LCAP, LLO, true>(a, s) : launch_small_bwd_g<LOP, LCAP, LLO, false>(a, s);
 }
 
 template <int LOP, int LCAP>

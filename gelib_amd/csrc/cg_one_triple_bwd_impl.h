@@ -78,7 +78,7 @@ __device__ __forceinline__ void one_triple_cell(const BwdArgs &a, PairPtr pr, co
 #pragma unroll
     for (int r = 0; r < RL; r++) {
       if constexpr (K == 2) {
-        const v4f t = *reinterpret_cast<GlobalRows4>(gp + r * G.sm);
+        const v4f t = __builtin_nontemporal_load(reinterpret_cast<GlobalRows4>(gp + r * G.sm));
         g[0][r] = v2f{t.x, t.y};
         g[1][r] = v2f{t.z, t.w};
       } else {

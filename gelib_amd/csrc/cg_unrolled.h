@@ -19,6 +19,10 @@ constexpr int kLTMax = 6;             // ... and by the one backward kernel buil
 constexpr int kMaxDl = 2 * kLTMax + 1;  // most l values one (l1,l2) pair can produce
 constexpr int kMaxPairs = (kLTMax + 1) * (kLTMax + 1);  // most (x part, y part) pairs of one launch
 
+// How a forward kernel writes its results: over what is there, onto it, or over it with stores that leave the cache line for
+// memory at once instead of keeping it.
+enum WriteMode { kWriteOver = 0, kWriteAdd = 1, kWriteStream = 2 };
+
 struct VecTriple {
   int xi, yi, ri;  // indices into the l-sorted part lists
   int l1, l2, l;

@@ -127,7 +127,7 @@ __device__ __forceinline__ LanePos lane_pos(int run, int lane, int log2_u, int r
 // and run where 350 are needed, and 24 row loads where 9 are.)
 // LLO: the launch takes only the l from LLO up (a product that reaches above l = 6 with operands above l = 4 is taken
 // in two launches, l <= 6 and l >= 7, each reading its own parts of g; the second adds onto the first).
-template <int L1, int L2, int LCAP, bool DIAG, bool WX, bool WY, bool PAD, bool REC, int ONLY = -1, int LLO = 0>
+template <int L1, int L2, int LCAP, bool DIAG, bool WX, bool WY, bool PAD, bool REC, bool ONCE, int ONLY = -1, int LLO = 0>
 __device__ __forceinline__ void pair_bwd(const GParts<LCAP> &gp, PairPtr pr, CoeffPtr Cs, CoeffPtr Zc, GlobalRows zrows,
                                          const float2 *xs, const float2 *ys, float2 *xacc, float2 *yacc, int xsize,
                                          int ysize, long long cell0, int offs_add, const LanePos q) {
@@ -208,7 +208,8 @@ __device__ __forceinline__ void pair_bwd(const GParts<LCAP> &gp, PairPtr pr, Coe
       constexpr int dl = decltype(dl_c)::value;
       constexpr int L = LMIN + dl;
       if constexpr (L >= cabs_(m)) {
-        const v2f t = gptr[dl][(m + L) * gsm[dl]];
+        const GlobalRows at = gptr[dl] + (m + L) * gsm[dl];
+        const v2f t = ONCE ? __builtin_nontemporal_load(at) : *at;
         dst[dl] = make_float2(t.x, t.y);
       }
     });
@@ -388,7 +389,7 @@ __device__ __forceinline__ void copy_image(const FastPart (&parts)[kFastIn], con
 // LT: largest operand l of the pairs the kernel has code for.
 // The kernel for operands above kLT is asked to fit three waves per SIMD (168 registers): left alone it takes 169.
 // ONE: the call has one triple (a.only_dl says which l of its pair).
-template <int L1, int L2, int LCAP, bool DIAG, bool WX, bool WY, bool PAD>
+template <int L1, int L2, int LCAP, bool DIAG, bool WX, bool WY, bool PAD, bool ONCE>
 __device__ __forceinline__ void pair_bwd_one(int only_dl, const GParts<LCAP> &gp, PairPtr pr, CoeffPtr Cs, CoeffPtr Zc,
                                              GlobalRows zrows, const float2 *xs, const float2 *ys, float2 *xacc,
                                              float2 *yacc, int xsize, int ysize, long long cell0, int offs_add,
@@ -396,12 +397,12 @@ __device__ __forceinline__ void pair_bwd_one(int only_dl, const GParts<LCAP> &gp
   static_for<2 * cmin_(L1, L2) + 1>([&](auto dc) __attribute__((always_inline)) {
     constexpr int D = decltype(dc)::value;
     if (only_dl == D)  // uniform
-      pair_bwd<L1, L2, LCAP, DIAG, WX, WY, PAD, false, D>(gp, pr, Cs, Zc, zrows, xs, ys, xacc, yacc, xsize, ysize, cell0,
+      pair_bwd<L1, L2, LCAP, DIAG, WX, WY, PAD, false, ONCE, D>(gp, pr, Cs, Zc, zrows, xs, ys, xacc, yacc, xsize, ysize, cell0,
                                                            offs_add, q);
   });
 }
 
-template <int LCAP, bool DIAG, bool WX, bool WY, bool PAD, int LT, bool ONE, int LLO = 0>
+template <int LCAP, bool DIAG, bool WX, bool WY, bool PAD, int LT, bool ONE, int LLO, bool ONCE>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(LT > kLT ? 3 : 1)))
 unrolled_bwd_kernel(const BwdArgs a) {
   constexpr int KR = 2 * LCAP + 1;
@@ -457,10 +458,10 @@ unrolled_bwd_kernel(const BwdArgs a) {
   case A * (kLTMax + 1) + B:                                                                                  \
     if constexpr (A <= LT && B <= LT && A + B >= LLO) { /* the pair has an l the launch takes */              \
       if constexpr (ONE)                                                                                      \
-        pair_bwd_one<A, B, LCAP, DIAG, WX, WY, PAD>(only_dl, gp, p, C, Zc, zrows, xs, ys, xacc, yacc, xsize, ysize,   \
+        pair_bwd_one<A, B, LCAP, DIAG, WX, WY, PAD, ONCE>(only_dl, gp, p, C, Zc, zrows, xs, ys, xacc, yacc, xsize, ysize,   \
                                                     cell0, offs_add, q);                                      \
       else                                                                                                    \
-        pair_bwd<A, B, LCAP, DIAG, WX, WY, PAD, (LT > kLT || GELIB_BWD_RECORDS_ALL), -1, LLO>(gp, p, C, Zc, zrows, xs, ys, xacc, yacc, xsize,  \
+        pair_bwd<A, B, LCAP, DIAG, WX, WY, PAD, (LT > kLT || GELIB_BWD_RECORDS_ALL), ONCE, -1, LLO>(gp, p, C, Zc, zrows, xs, ys, xacc, yacc, xsize,  \
                                                                        ysize, cell0, offs_add, q);            \
     }                                                                                                         \
     break;
@@ -498,9 +499,9 @@ unrolled_bwd_kernel(const BwdArgs a) {
   if (WY) copy_image<false>(a.yg, a.yrows, a.ny, yacc_all, ysize, cell0, ncell, kWaves, cpb * ysize, a.accumulate != 0);
 }
 
-template <int LCAP, bool DIAG, bool WX, bool WY, bool PAD, int LT, bool ONE, int LLO>
+template <int LCAP, bool DIAG, bool WX, bool WY, bool PAD, int LT, bool ONE, int LLO, bool ONCE = false>
 int launch_variant(const BwdArgs &a, int nblocks, size_t lds, hipStream_t s) {
-  auto kern = unrolled_bwd_kernel<LCAP, DIAG, WX, WY, PAD, LT, ONE, LLO>;
+  auto kern = unrolled_bwd_kernel<LCAP, DIAG, WX, WY, PAD, LT, ONE, LLO, ONCE>;
   static bool attr_set = false;  // benign race: setting the attribute twice is harmless
   if (!attr_set) {
     GELIB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -517,6 +518,8 @@ template <int LCAP, bool DIAG, bool PAD, int LT = kLT, bool ONE = false, int LLO
 int launch_bwd_variants(const BwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s) {
   static_assert(kLTMax == 6 && LT <= kLTMax, "the case table above lists l1, l2 = 0..6");
   const bool wx = a.want_x != 0, wy = a.want_y != 0;
+  if constexpr (!DIAG)
+    if (wx && wy && a.once) return launch_variant<LCAP, DIAG, true, true, PAD, LT, ONE, LLO, true>(a, nblocks, lds_bytes, s);
   if (wx && wy) return launch_variant<LCAP, DIAG, true, true, PAD, LT, ONE, LLO>(a, nblocks, lds_bytes, s);
   if (wx) return launch_variant<LCAP, DIAG, true, false, PAD, LT, ONE, LLO>(a, nblocks, lds_bytes, s);
   return launch_variant<LCAP, DIAG, false, true, PAD, LT, ONE, LLO>(a, nblocks, lds_bytes, s);

@@ -20,7 +20,7 @@ struct FwdArgs {
   long long ncells;
   int npairs;
   int offs_add;     // extra channel offset (part-level calls)
-  int accumulate;
+  int write;        // WriteMode
   long long tile;                  // cells per tile; the blocks of one tile are consecutive
   int blocks_per_tile;
   int first_block[kMaxPairs + 1];  // inside a tile, blocks [first_block[p], first_block[p+1]) work on pair p
@@ -52,6 +52,7 @@ struct BwdArgs {
   // adds the pair_split images of a cell in their order and writes the gradients.  1: one block takes all pairs.
   int pair_split;
   float2 *part_x, *part_y;
+  int once;         // (the host's choice of kernel) both gradients: g is read with loads that do not keep the line
 };
 
 size_t unrolled_bwd_lds_bytes(int bank_len, int xsize, int ysize, int cells_per_block);

@@ -28,10 +28,11 @@ typedef __attribute__((address_space(1))) v2f *GlobalOut;  // product rows: glob
 
 // One (l1,l2,l) triple for one thread: rows m = -L..L of the block, TI channels each.
 // last: the thread's channels 0..last exist (RAGGED; otherwise all TI do).
-template <int L1, int L2, int L, int TI, bool RAGGED>
+// STREAM: the kernel can write with streaming stores (a.write says whether it does).
+template <int L1, int L2, int L, int TI, bool RAGGED, bool STREAM>
 __device__ __forceinline__ void triple_fwd(const float2 (&xv)[TI][2 * L1 + 1], const float2 (&yv)[2 * L2 + 1],
                                            CoeffPtr C, GlobalOut rp, int sm, int kstride, bool accumulate,
-                                           bool live, int last) {
+                                           bool live, int last, bool stream) {
 #pragma unroll
   for (int m = -L; m <= L; m++) {
     float2 acc[TI];
@@ -61,6 +62,11 @@ __device__ __forceinline__ void triple_fwd(const float2 (&xv)[TI][2 * L1 + 1], c
         v2f v;
         v.x = acc[k].x;
         v.y = acc[k].y;
+        if (STREAM && stream) {
+          __builtin_nontemporal_store(v, &row[k * kstride]);
+          asm volatile("");  // (two equal stores at the ends of two branches would become one ordinary store)
+          continue;
+        }
         if (accumulate) v += row[k * kstride];
         row[k * kstride] = v;
       }
@@ -75,10 +81,10 @@ struct RParts {
   FastPart R[LCAP + 1];
 };
 
-template <int L1, int L2, int LCAP, int TI, bool DIAG, bool RAGGED>
+template <int L1, int L2, int LCAP, int TI, bool DIAG, bool RAGGED, bool STREAM>
 __device__ __forceinline__ void pair_fwd(const RParts<LCAP> &rp_all, PairPtr pr, CoeffPtr Cs, const float2 *xs,
                                          const float2 *ys, int offs_add, bool accumulate, long long cell, int dc,
-                                         int u, bool live) {
+                                         int u, bool live, bool stream) {
   const __attribute__((address_space(4))) PairRec &p = *pr;
   const int N1 = p.n1, N2 = p.n2;
   int i0, j;
@@ -115,7 +121,7 @@ __device__ __forceinline__ void pair_fwd(const RParts<LCAP> &rp_all, PairPtr pr,
       if (p.ri[dl] >= 0) {
         const FastPart R = rp_all.R[L];
         GlobalOut rp = (GlobalOut)R.ptr + cell * R.sb + (p.offs[dl] + offs_add + u);
-        triple_fwd<L1, L2, L, TI, RAGGED>(xv, yv, Cs + p.cg[dl], rp, R.sm, kstride, accumulate, live, last);
+        triple_fwd<L1, L2, L, TI, RAGGED, STREAM>(xv, yv, Cs + p.cg[dl], rp, R.sm, kstride, accumulate, live, last, stream);
       }
     }
   });
@@ -170,7 +176,7 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
   RParts<LCAP> rp_all;
   static_for<LCAP + 1>([&](auto l) __attribute__((always_inline)) { rp_all.R[l.value] = a.r[l.value]; });
   const int offs_add = a.offs_add;
-  const bool accumulate = a.accumulate != 0;
+  const bool accumulate = a.write == kWriteAdd, stream = a.write == kWriteStream;
   __syncthreads();
 
   const int U = DIAG ? n1 : (RAGGED ? (n1 + TI - 1) / TI : n1 / TI) * n2;
@@ -188,7 +194,7 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
 #define GELIB_CASE(A, B)                                                                                      \
   case A * (kLTMax + 1) + B:                                                                                  \
     if constexpr (A <= LT && B <= LT)                                                                         \
-      pair_fwd<A, B, LCAP, TI, DIAG, RAGGED>(rp_all, p, C, xs, ys, offs_add, accumulate, cell, dc, u, live);          \
+      pair_fwd<A, B, LCAP, TI, DIAG, RAGGED, (LT > kLT)>(rp_all, p, C, xs, ys, offs_add, accumulate, cell, dc, u, live, stream); \
     break;
 #define GELIB_ROW(A) \
   GELIB_CASE(A, 0) GELIB_CASE(A, 1) GELIB_CASE(A, 2) GELIB_CASE(A, 3) GELIB_CASE(A, 4) GELIB_CASE(A, 5) GELIB_CASE(A, 6)

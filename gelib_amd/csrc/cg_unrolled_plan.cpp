@@ -18,6 +18,8 @@ int g_fwd_cell_tile = -1;            // cells per tile of the forward launch (0 
 int g_fwd_narrow_decline = 1;  // leave products with at most four channel pairs per block to the any-l forward kernel
 int g_fwd_tile_per_xcd = -1;          // blocks of a tile on one XCD (-1 = by the alignment of the blocks, 0 no, 1 yes)
 int g_fwd_max_blocks = 0;             // most blocks of a launch (0 = what HIP allows); more take several launches
+int g_fwd_stream = -1;               // streaming stores: -1 = by the shape, 0 never, 1 always
+int g_bwd_once = -1;                 // streaming loads of g: -1 = by the shape, 0 never, 1 always
 int g_fwd_ti = 0;                    // 0 = widest tile that divides every n1, else force 1 / 2 / 4
 int g_bwd_enable = 1;
 int g_bwd_one_enable = 1; // the backward kernel for calls with one triple
@@ -334,7 +336,14 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   a.ncells = ncells;
   a.npairs = (int)plan->pairs.size();
   a.offs_add = offs_add;
-  a.accumulate = accumulate ? 1 : 0;
+  // Streaming stores: in the kernel for operands above kLT, where every block is whole runs of 512 bytes (L=6, 8 channels, streaming
+  // / ordinary at 40, 250 and 1500 MB of product .94 .93 .79; 4 channels .92 1.25 1.07, 6 channels .91 1.65 1.63).  The kernels up to
+  // kLT keep ordinary stores: with several channels per thread a row's pieces meet in the caches (L=4 16 channels .97 1.00 .97, 8
+  // channels .96 1.08 1.05, 12 .98 1.14 1.09, 20 .97 1.18 1.26, 9 .93 1.65 1.67, 3 1.94 4.3 4.3).
+  bool lines = lop > kLT;
+  for (auto &t : triples) lines = lines && t.nout % 64 == 0;
+  const bool stream = lop > kLT && (g_fwd_stream < 0 ? lines : g_fwd_stream != 0);   // (the kernels up to kLT have no such stores)
+  a.write = accumulate ? kWriteAdd : (stream ? kWriteStream : kWriteOver);
   long long nblocks = 0;
   size_t lds_bytes = 0;
   int lcap = 0;
@@ -496,6 +505,15 @@ int run_bwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   const size_t lds = unrolled_bwd_lds_bytes(a.bank_len, a.xsize, a.ysize, cpb);
   if (lds > 150 * 1024) return GELIB_HIP_OK;
   a.cells_per_block = cpb;
+  // Streaming loads of g (the line is not kept) where every block is whole cache lines: nothing reads g again, and what an
+  // ordinary load leaves in the caches pushes out what will be.  Blocks that share lines with their neighbours' must find them there.
+  // Streaming / ordinary, g warm and pushed out of the caches, 250 MB and 1.5 GB: L=4 16 channels .96 .75 | .90 .85, 8 .97 .73 | .96 .90, 4
+  // .95 .73 | .97 .91, 20 1.03 .79 | 1.02 .94; L=6 8 channels .97 .81 | .90 .85; 8 x 2 .98 .80 | .96 .96; 3 channels 1.04 .92 | 1.11 1.13, 2
+  // 1.20 1.07 | 1.32 1.35, 1 1.70 1.82 | 2.16 2.28.  Odd counts gain in this launch and lose more in the next: 20, 12, 9, 6, 3 x 10, 7, 6, 5
+  // channels, every l, 5003 cells, backward 347 -> 319 us, the forward launch behind it 171 -> 228.
+  bool lines = !diag;
+  for (auto &t : triples) lines = lines && t.nout % 16 == 0;
+  a.once = g_bwd_once < 0 ? lines : g_bwd_once;
   a.only_dl = -1;
   if (triples.size() == 1 && !diag && !plan->padded && lop <= kLT && g_bwd_one_enable)
     a.only_dl = triples[0].l - std::abs(triples[0].l1 - triples[0].l2);
@@ -740,6 +758,16 @@ int unrolled_set_option(const char *name, int value) {
   }
   if (!std::strcmp(name, "unrolled_bwd_one_wide_cells")) {
     g_bwd_one_wide_cells = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "bwd_once")) {
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_bwd_once = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "fwd_stream")) {
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_fwd_stream = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "unrolled_bwd_one_wide")) {  // 0 off, otherwise the cells per wave of a block of that kernel
