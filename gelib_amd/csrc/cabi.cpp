@@ -708,7 +708,9 @@ int pairwise_onepair_bwd(const VecPlan &plan, const std::vector<View> &G, const 
   int rc;
   for (auto &sub : subs) {  // first pass: would every pair be taken?
     int ok = 0;
-    if ((rc = onepair_vec_bwd(sub.plan, gd, {X[sub.p].d}, {Y[sub.q].d}, {XG[sub.p].d}, {YG[sub.q].d}, true, s, &ok, true)))
+    if ((rc = onepair_mfma_vec_bwd(sub.plan, gd, {X[sub.p].d}, {Y[sub.q].d}, {XG[sub.p].d}, {YG[sub.q].d}, true, s, &ok, true)))
+      return rc;
+    if (!ok && (rc = onepair_vec_bwd(sub.plan, gd, {X[sub.p].d}, {Y[sub.q].d}, {XG[sub.p].d}, {YG[sub.q].d}, true, s, &ok, true)))
       return rc;
     if (!ok) return GELIB_HIP_OK;
   }

@@ -68,6 +68,9 @@ struct OnePairMfmaArgs {
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) v4f *GlobalIn4;
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(1))) v2f *GlobalIn2;
+typedef __attribute__((address_space(1))) v2f *GlobalOut2;
 typedef __attribute__((address_space(1))) v4f *GlobalOut4;
 typedef const __attribute__((address_space(1))) float *GlobalIn1;
 typedef __attribute__((address_space(1))) float *GlobalOut1;
@@ -104,7 +107,10 @@ struct PairShape {
   static_assert(JL == N2 || 2 * JL == N2, "a lane holds a whole row of j or half of one");
 };
 
-template <int N1, int N2>
+// PAD: the parts have n1 <= N1 and n2 <= N2 channels (a.x.n, a.y.n), or rows that are not 16-byte aligned.  The operands of the
+// channels beyond are zeros; their places in a row of g are read from the channel with 0 in place of what is beyond, whose
+// sums they share anyway (so nothing that is not a number enters a sum it does not belong to), eight bytes at a time.
+template <int N1, int N2, bool PAD>
 __global__ void __launch_bounds__((64 * PairShape<N1, N2>::W)) onepair_mfma_bwd_kernel(const OnePairMfmaArgs a) {
   using Sh = PairShape<N1, N2>;
   constexpr int T = Sh::T, JL = Sh::JL, W = Sh::W;
@@ -138,8 +144,10 @@ __global__ void __launch_bounds__((64 * PairShape<N1, N2>::W)) onepair_mfma_bwd_
     gbase[nl] = (unsigned long long)a.coef;
     growb[nl] = 0u;
   }
+  const int n1 = PAD ? a.x.n : N1, n2 = PAD ? a.y.n : N2;
   for (int e = threadIdx.x; e < r2 * N2; e += 64 * W) {
-    ys[e] = a.y.ptr[cell * a.y.sb + (long long)(e / N2) * a.y.sm + (e % N2)];
+    const int j = e % N2;
+    ys[e] = !PAD || j < n2 ? a.y.ptr[cell * a.y.sb + (long long)(e / N2) * a.y.sm + j] : make_float2(0.f, 0.f);
 #pragma unroll
     for (int k = 0; k < W * Sh::kSlots; k++) accy_all[k][e] = make_float2(0.f, 0.f);
   }
@@ -147,7 +155,7 @@ __global__ void __launch_bounds__((64 * PairShape<N1, N2>::W)) onepair_mfma_bwd_
   float2 xv[4];
 #pragma unroll
   for (int b = 0; b < 4; b++)
-    xv[b] = i < r1 ? a.x.ptr[cell * a.x.sb + (long long)i * a.x.sm + a_of(b)] : make_float2(0.f, 0.f);
+    xv[b] = i < r1 && (!PAD || a_of(b) < n1) ? a.x.ptr[cell * a.x.sb + (long long)i * a.x.sm + a_of(b)] : make_float2(0.f, 0.f);
   __syncthreads();
 
   // The steps of all m form one sequence (two values of l per step, m ascending), padded with idle steps to a multiple
@@ -194,14 +202,25 @@ __global__ void __launch_bounds__((64 * PairShape<N1, N2>::W)) onepair_mfma_bwd_
   // the lane's piece of a row: 4 T bytes, 512 bytes on for every wave; the harmless row (the coefficient table) is
   // read at the same offsets, which its idle steps at the end cover
   const unsigned lane_off = (unsigned)wave * 512u + (unsigned)i * (4u * T);
+  // PAD: byte offset of the place of channel `slot` of the N1 x N2 in a row
+  auto place = [&](int slot) __attribute__((always_inline)) {
+    const int ca = slot / N2, cj = slot % N2;
+    return (unsigned)((ca < n1 ? ca : 0) * n2 + (cj < n2 ? cj : 0)) * 8u;
+  };
+  const unsigned off0 = !PAD ? lane_off : (T == 4 ? place(wave * 64 + 2 * i) : place(i >> 1) + 4u * (unsigned)(i & 1));
+  const unsigned off1 = PAD && T == 4 ? place(wave * 64 + 2 * i + 1) : 0u;
   auto fetch = [&](const Cursor &c, GT &g, float &cf) __attribute__((always_inline)) {
     int dl = c.dlb + h;
     dl = dl < nl ? dl : nl;
     const unsigned long long base = gbase[dl];
     const unsigned rowb = growb[dl];
-    const unsigned long long addr = base + (unsigned long long)((unsigned)(c.m + lmin + dl) * rowb) + lane_off;
-    if constexpr (T == 4) g = *(GlobalIn4)addr;
-    else g = *(GlobalIn1)addr;
+    const unsigned long long addr = base + (unsigned long long)((unsigned)(c.m + lmin + dl) * rowb) + off0;
+    if constexpr (T == 4 && PAD) {
+      const v2f lo = *(GlobalIn2)addr, hi = *(GlobalIn2)(addr - off0 + off1);
+      g = v4f{lo.x, lo.y, hi.x, hi.y};
+    } else if constexpr (T == 4) g = __builtin_nontemporal_load((GlobalIn4)addr);
+    else if constexpr (PAD) g = *(GlobalIn1)addr;
+    else g = __builtin_nontemporal_load((GlobalIn1)addr);
     cf = *((GlobalIn1)a.coef + coef_at);   // the table ends with a queue's worth of idle steps
     coef_at += 64;
   };
@@ -334,6 +353,7 @@ __global__ void __launch_bounds__((64 * PairShape<N1, N2>::W)) onepair_mfma_bwd_
 #pragma unroll
     for (int b = 0; b < 4; b++) {
       if (!kHalfIsA && (b >> 1) != h) continue;  // each half stores two of the four
+      if (PAD && a_of(b) >= n1) continue;
       float2 *p = a.xg.ptr + cell * a.xg.sb + (long long)i * a.xg.sm + a_of(b);
       float2 o = ax[b];
       if (accumulate) o.x += p->x, o.y += p->y;
@@ -341,6 +361,7 @@ __global__ void __launch_bounds__((64 * PairShape<N1, N2>::W)) onepair_mfma_bwd_
     }
   }
   for (int e = threadIdx.x; e < r2 * N2; e += 64 * W) {
+    if (PAD && e % N2 >= n2) continue;
     float2 *p = a.yg.ptr + cell * a.yg.sb + (long long)(e / N2) * a.yg.sm + (e % N2);
     float2 o = accy_all[0][e];
 #pragma unroll
@@ -366,7 +387,8 @@ constexpr int kCellsF = 8;                     // cells (waves) per block of the
 // Channels: a wave's columns are the floats of 64 neighbouring channels (column i of tile t = float 4 i + t: the lane
 // forms the products of channels 2 i and 2 i + 1 = (a, j) and (a, j + 1)), or of all 16 (one tile, column i = float i:
 // the lane forms the real or the imaginary part of channel i / 2).
-template <int N1, int N2, bool ONE_ROWB>
+// PAD: as in the backward kernel; the places of the channels beyond are not stored, the others 8 bytes at a time.
+template <int N1, int N2, bool ONE_ROWB, bool PAD>
 __global__ void __launch_bounds__(64 * kCellsF) onepair_mfma_fwd_kernel(const OnePairMfmaArgs a) {
   using Sh = PairShape<N1, N2>;
   constexpr int T = Sh::T, W = Sh::W;
@@ -391,8 +413,11 @@ __global__ void __launch_bounds__(64 * kCellsF) onepair_mfma_fwd_kernel(const On
   long long cell = (long long)blockIdx.x * (kCellsF / W) + cw;
   const bool live = cell < a.ncells;  // a wave beyond the last cell repeats it and stores nothing
   cell = live ? cell : a.ncells - 1;
-  for (int e = ww * 64 + lane; e < r1 * N1; e += 64 * W) xs[e] = a.x.ptr[cell * a.x.sb + (long long)(e / N1) * a.x.sm + (e % N1)];
-  for (int e = ww * 64 + lane; e < r2 * N2; e += 64 * W) ys[e] = a.y.ptr[cell * a.y.sb + (long long)(e / N2) * a.y.sm + (e % N2)];
+  const int n1 = PAD ? a.x.n : N1, n2 = PAD ? a.y.n : N2;
+  for (int e = ww * 64 + lane; e < r1 * N1; e += 64 * W)
+    xs[e] = !PAD || e % N1 < n1 ? a.x.ptr[cell * a.x.sb + (long long)(e / N1) * a.x.sm + (e % N1)] : make_float2(0.f, 0.f);
+  for (int e = ww * 64 + lane; e < r2 * N2; e += 64 * W)
+    ys[e] = !PAD || e % N2 < n2 ? a.y.ptr[cell * a.y.sb + (long long)(e / N2) * a.y.sm + (e % N2)] : make_float2(0.f, 0.f);
   if (ww == 0) {
     if (lane < N1) xs[r1 * N1 + lane] = make_float2(0.f, 0.f);
     if (lane < N2) {
@@ -404,6 +429,10 @@ __global__ void __launch_bounds__(64 * kCellsF) onepair_mfma_fwd_kernel(const On
   // that part for the m at hand (the rows of a part start at m = -l; before that the address is not used), advanced by
   // the row length after every m.  Bit v of `there`: the part exists and the wave has a cell.
   const long long rowb = a.rowb;
+  const int chan = T == 4 ? ww * 64 + 2 * i : i >> 1;  // the lane's channel(s): (a, j), and for a wave of 64 channels (a, j + 1) as well
+  const bool mine = !PAD || (chan / N2 < n1 && chan % N2 < n2), both = T == 4 && mine && (!PAD || chan % N2 + 1 < n2);
+  const unsigned lane_off = !PAD ? (unsigned)ww * 512u + (unsigned)i * (4u * T)
+                                 : (unsigned)(chan / N2 * n2 + chan % N2) * 8u + (T == 4 ? 0u : 4u * (unsigned)(i & 1));
   unsigned long long cur[16];
   unsigned rowbv[ONE_ROWB ? 1 : 16];
   unsigned there = 0;
@@ -414,11 +443,11 @@ __global__ void __launch_bounds__(64 * kCellsF) onepair_mfma_fwd_kernel(const On
     static_for<2>([&](auto hc) __attribute__((always_inline)) {
       constexpr int dl = 8 * (v / 4) + 4 * decltype(hc)::value + (v % 4);
       if constexpr (dl < kNLm) {
-        if (hc.value == h && dl < nl && live && a.g[dl].ptr != nullptr) {
+        if (hc.value == h && dl < nl && live && mine && a.g[dl].ptr != nullptr) {
           const FastPart P = a.g[dl];
           const long long rb = ONE_ROWB ? rowb : (long long)P.sm * 8;
           cur[v] = (unsigned long long)(P.ptr + cell * P.sb + (a.offs[dl] + a.offs_add)) +
-                   (unsigned long long)((long long)(lmin + dl - lt) * rb) + (unsigned)ww * 512u + (unsigned)i * (4u * T);
+                   (unsigned long long)((long long)(lmin + dl - lt) * rb) + lane_off;
           if constexpr (!ONE_ROWB) rowbv[v] = (unsigned)rb;
           there |= 1u << v;
         }
@@ -426,8 +455,6 @@ __global__ void __launch_bounds__(64 * kCellsF) onepair_mfma_fwd_kernel(const On
     });
   });
   const int lbase = lmin + 4 * h;  // l of register v: lbase + 8 (v / 4) + v % 4
-  // the lane's channel(s): (a, j), and for a wave of 64 channels (a, j + 1) as well
-  const int chan = T == 4 ? ww * 64 + 2 * i : i >> 1;
   const char *xmine = reinterpret_cast<const char *>(xs + chan / N2);  // row r: + r * XROW bytes
   const char *ymine = reinterpret_cast<const char *>(ys + chan % N2);  // row r: + r * YROW
   const bool imag = (i & 1) != 0;  // one tile: the lane's float is the imaginary part
@@ -477,17 +504,27 @@ __global__ void __launch_bounds__(64 * kCellsF) onepair_mfma_fwd_kernel(const On
 #pragma unroll
     for (int v = 0; v < 16; v++) {
       if (((there >> v) & 1u) && lbase + (8 * (v / 4) + v % 4) >= mabs) {
-        if constexpr (T == 4) {
+        if constexpr (T == 4 && PAD) {
+          v2f lo = {D[0][v], D[1][v]}, hi = {D[2][v], D[3][v]};
+          const GlobalOut2 q = (GlobalOut2)cur[v];
+          if (accumulate) {
+            lo += q[0];
+            if (both) hi += q[1];
+          }
+          q[0] = lo;
+          if (both) q[1] = hi;
+        } else if constexpr (T == 4) {
           GlobalOut4 q = (GlobalOut4)cur[v];
           v4f o;
           o.x = D[0][v], o.y = D[1][v], o.z = D[2][v], o.w = D[3][v];
           if (accumulate) o += *q;
-          *q = o;
+          __builtin_nontemporal_store(o, q);
         } else {
           GlobalOut1 q = (GlobalOut1)cur[v];
           float o = D[0][v];
           if (accumulate) o += *q;
-          *q = o;
+          if constexpr (PAD) *q = o;
+          else __builtin_nontemporal_store(o, q);
         }
       }
       cur[v] += ONE_ROWB ? (unsigned long long)rowb : (unsigned long long)rowbv[v];
@@ -506,7 +543,7 @@ struct Tables {
 };
 std::mutex g_mutex;
 std::map<std::vector<int>, Tables> g_tables;  // (device, l1, l2, lmin, lt, nl, present...) -> device tables
-int g_enable = 1, g_enable_fwd = 1, g_paired = 1;
+int g_enable = 1, g_enable_fwd = 1, g_paired = 1, g_pad = 1;
 
 int device_tables(int l1, int l2, int lmin, int lt, int nl, const std::vector<int> &present, bool paired, Tables *out) {
   int dev = 0;
@@ -595,15 +632,40 @@ bool bwd_shape_built(int n1, int n2) {
 #undef GELIB_X
   return false;
 }
-void launch_bwd_shape(int n1, int n2, const OnePairMfmaArgs &a, hipStream_t s) {
+// The smallest built shape that holds n1 x n2 channels; places beyond the real ones cost as much as real ones.
+bool padded_shape(int n1, int n2, int *N1, int *N2) {
+  int best = 1 << 30;
+#define GELIB_X(A, B) if (n1 <= A && n2 <= B && A * B < best) best = A * B, *N1 = A, *N2 = B;
+  GELIB_ONEPAIR_SHAPES(GELIB_X)
+#undef GELIB_X
+  return best < (1 << 30);
+}
+// Backward: more than 64 lane slots (channel counts rounded up to powers of two) would go to the shape-agnostic kernels, up to
+// 64 to the LDS-column kernel, which pads the same way.  Before / padded here, l = 10 x 10, all l, microseconds: 9 x 9 channels 104
+// cells 13584 / 144, 1399 cells 14000 / 550; 12 x 6, 1574 cells 7230 / 350; 5 x 16, 1417 cells 5430 / 233; 5 x 5, 4535 cells 599 / 351;
+// 3 x 3, 12597 cells 576 / 319; 5 x 2, 11337 cells 569 / 285; 4 x 12, 2362 cells 413 / 220.  A shape of more places than that kernel's
+// slots would lose (2 x 2 in 4 x 4, 4 x 5 in 8 x 8).
+bool bwd_padded_pays(int n1, int n2, int N1, int N2) {
+  int s1 = 1, s2 = 1;
+  while (s1 < n1) s1 *= 2;
+  while (s2 < n2) s2 *= 2;
+  return s1 * s2 > 64 || s1 * s2 >= N1 * N2;
+}
+// Forward, against the any-l kernel: where more than half of the places are real (8 x 5 channels 422 -> 263 us, 4 x 12 387 -> 259, 6 x 5
+// 298 / 305, 5 x 9 385 / 392).  16 channels are stored four bytes at a time, which only launches that are over before the memory is
+// busy can afford (7 x 9, 3 x 3: 1461 cells 152 -> 82 us, 19493 cells 352 / 460).
+bool fwd_padded_pays(int n1, int n2, int N1, int N2, long long ncells) { return 2 * n1 * n2 > N1 * N2 && (N1 * N2 > 16 || ncells <= 2048); }
+void launch_bwd_shape(int n1, int n2, bool pad, const OnePairMfmaArgs &a, hipStream_t s) {
 #define GELIB_X(A, B)                                                                                                   \
-  if (n1 == A && n2 == B)                                                                                               \
-    hipLaunchKernelGGL((onepair_mfma_bwd_kernel<A, B>), dim3((unsigned)a.ncells), dim3(64 * PairShape<A, B>::W), 0, s, a);
+  if (n1 == A && n2 == B) {                                                                                             \
+    if (pad) hipLaunchKernelGGL((onepair_mfma_bwd_kernel<A, B, true>), dim3((unsigned)a.ncells), dim3(64 * PairShape<A, B>::W), 0, s, a); \
+    else hipLaunchKernelGGL((onepair_mfma_bwd_kernel<A, B, false>), dim3((unsigned)a.ncells), dim3(64 * PairShape<A, B>::W), 0, s, a); \
+  }
   GELIB_ONEPAIR_SHAPES(GELIB_X)
 #undef GELIB_X
 }
 
-template <int N1, int N2, bool ONE_ROWB>
+template <int N1, int N2, bool ONE_ROWB, bool PAD>
 int launch_fwd_one(const OnePairMfmaArgs &a, unsigned nblocks, size_t lds, hipStream_t s) {
   static std::mutex attr_mutex;
   static std::map<int, bool> attr_set;  // device -> the kernel may use 80 KB of LDS
@@ -612,18 +674,20 @@ int launch_fwd_one(const OnePairMfmaArgs &a, unsigned nblocks, size_t lds, hipSt
   {
     std::lock_guard<std::mutex> lock(attr_mutex);
     if (!attr_set[dev]) {
-      GELIB_HIP_TRY(hipFuncSetAttribute((const void *)onepair_mfma_fwd_kernel<N1, N2, ONE_ROWB>,
+      GELIB_HIP_TRY(hipFuncSetAttribute((const void *)onepair_mfma_fwd_kernel<N1, N2, ONE_ROWB, PAD>,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)(80 * 1024)));
       attr_set[dev] = true;
     }
   }
-  hipLaunchKernelGGL((onepair_mfma_fwd_kernel<N1, N2, ONE_ROWB>), dim3(nblocks), dim3(64 * kCellsF), lds, s, a);
+  hipLaunchKernelGGL((onepair_mfma_fwd_kernel<N1, N2, ONE_ROWB, PAD>), dim3(nblocks), dim3(64 * kCellsF), lds, s, a);
   return GELIB_HIP_OK;
 }
-int launch_fwd_shape(int n1, int n2, bool one_rowb, const OnePairMfmaArgs &a, unsigned nblocks, size_t lds, hipStream_t s) {
+int launch_fwd_shape(int n1, int n2, bool one_rowb, bool pad, const OnePairMfmaArgs &a, unsigned nblocks, size_t lds, hipStream_t s) {
 #define GELIB_X(A, B)                                                                     \
-  if (n1 == A && n2 == B)                                                                 \
-    return one_rowb ? launch_fwd_one<A, B, true>(a, nblocks, lds, s) : launch_fwd_one<A, B, false>(a, nblocks, lds, s);
+  if (n1 == A && n2 == B) {                                                               \
+    if (pad) return one_rowb ? launch_fwd_one<A, B, true, true>(a, nblocks, lds, s) : launch_fwd_one<A, B, false, true>(a, nblocks, lds, s); \
+    return one_rowb ? launch_fwd_one<A, B, true, false>(a, nblocks, lds, s) : launch_fwd_one<A, B, false, false>(a, nblocks, lds, s);        \
+  }
   GELIB_ONEPAIR_SHAPES(GELIB_X)
 #undef GELIB_X
   return GELIB_HIP_ERR_ARG;
@@ -636,7 +700,7 @@ int launch_fwd_shape(int n1, int n2, bool one_rowb, const OnePairMfmaArgs &a, un
 int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part_desc *> &g,
                          const std::vector<const gelib_part_desc *> &x, const std::vector<const gelib_part_desc *> &y,
                          const std::vector<const gelib_part_desc *> &xg, const std::vector<const gelib_part_desc *> &yg,
-                         bool accumulate, hipStream_t s, int *used) {
+                         bool accumulate, hipStream_t s, int *used, bool dry) {
   *used = 0;
   if (!g_enable || plan.diag || x.size() != 1 || y.size() != 1 || xg.size() != 1 || yg.size() != 1 || plan.triples.empty())
     return GELIB_HIP_OK;
@@ -647,7 +711,10 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
       !lists_to_fast(yg, plan.E, true, &fyg, nullptr))
     return GELIB_HIP_OK;
   const int l1 = lx[0].first, l2 = ly[0].first, n1 = lx[0].second, n2 = ly[0].second;
-  if (!bwd_shape_built(n1, n2) || l1 > kMaxLm || l2 > kMaxLm) return GELIB_HIP_OK;
+  int N1 = 0, N2 = 0;
+  if (!padded_shape(n1, n2, &N1, &N2) || l1 > kMaxLm || l2 > kMaxLm) return GELIB_HIP_OK;
+  bool pad = !bwd_shape_built(n1, n2);
+  if (pad && (!g_pad || l1 + l2 >= kNLm || !bwd_padded_pays(n1, n2, N1, N2))) return GELIB_HIP_OK;
   const int lmin = std::abs(l1 - l2);
   int lmax = -1;
   for (auto &t : plan.triples) lmax = std::max(lmax, t.l);
@@ -667,12 +734,15 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
     present[dl] = 1;
     // 64 channels per wave: the lane's 16 bytes of a row must be 16-byte aligned (block offset, row and cell strides
     // even); with 16 channels a lane loads single floats
-    if (n1 * n2 >= 64 && (((t.offs) & 1) || (fg[t.ri].sm & 1) || (fg[t.ri].sb & 1) || ((uintptr_t)fg[t.ri].ptr & 15)))
-      return GELIB_HIP_OK;
+    if (N1 * N2 >= 64 && (((t.offs) & 1) || (fg[t.ri].sm & 1) || (fg[t.ri].sb & 1) || ((uintptr_t)fg[t.ri].ptr & 15))) pad = true;
     if ((long long)fg[t.ri].sm * 8 * (2 * t.l + 1) >= (1LL << 32)) return GELIB_HIP_OK;  // row offsets are 32 bits
   }
   const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
   if (ncells > 0x7fffffffLL) return GELIB_HIP_OK;
+  if (dry) {
+    *used = 1;
+    return GELIB_HIP_OK;
+  }
   Tables t;
   const int lt = std::min(l1 + l2, lmax);
   const bool paired = g_paired && l1 == l2 && lt == 2 * l1;
@@ -688,7 +758,7 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
   a.lt = lt;
   a.nl = nl;
   a.accumulate = accumulate ? 1 : 0;
-  launch_bwd_shape(n1, n2, a, s);
+  launch_bwd_shape(N1, N2, pad, a, s);
   GELIB_HIP_TRY(hipGetLastError());
   *used = 1;
   return GELIB_HIP_OK;
@@ -706,7 +776,10 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
       !lists_to_fast(r, plan.E, true, &fr, &lr))
     return GELIB_HIP_OK;
   const int l1 = lx[0].first, l2 = ly[0].first, n1 = lx[0].second, n2 = ly[0].second;
-  if (!bwd_shape_built(n1, n2) || l1 > kMaxLm || l2 > kMaxLm) return GELIB_HIP_OK;
+  int N1 = 0, N2 = 0;
+  if (!padded_shape(n1, n2, &N1, &N2) || l1 > kMaxLm || l2 > kMaxLm) return GELIB_HIP_OK;
+  bool pad = !bwd_shape_built(n1, n2);
+  if (pad && (!g_pad || l1 + l2 >= kNLm || !fwd_padded_pays(n1, n2, N1, N2, plan.E[0] * plan.E[1] * plan.E[2]))) return GELIB_HIP_OK;
   const int lmin = std::abs(l1 - l2);
   int lmax = -1;
   for (auto &t : plan.triples) lmax = std::max(lmax, t.l);
@@ -726,8 +799,7 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
     present[dl] = 1;
     // 64 channels per wave: a lane stores 16 bytes at a time (block offset, row and cell strides even, base aligned);
     // with 16 channels it stores single floats
-    if (n1 * n2 >= 64 && (((t.offs) & 1) || (fr[t.ri].sm & 1) || (fr[t.ri].sb & 1) || ((uintptr_t)fr[t.ri].ptr & 15)))
-      return GELIB_HIP_OK;
+    if (N1 * N2 >= 64 && (((t.offs) & 1) || (fr[t.ri].sm & 1) || (fr[t.ri].sb & 1) || ((uintptr_t)fr[t.ri].ptr & 15))) pad = true;
     if ((long long)fr[t.ri].sm * 8 >= (1LL << 32)) return GELIB_HIP_OK;  // row lengths are 32 bits
     if (a.rowb == 0) a.rowb = (long long)fr[t.ri].sm * 8;
     if (a.rowb != (long long)fr[t.ri].sm * 8) one_rowb = false;
@@ -749,11 +821,11 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
   a.accumulate = accumulate ? 1 : 0;
   // LDS of a block: the table and its cells' operands (with their rows of zeros); two blocks per compute unit fit
   // up to 80 KB each, beyond that the any-l kernels take the pair
-  const int cells_per_block = n1 * n2 >= 64 ? kCellsF * 64 / (n1 * n2) : kCellsF;
+  const int cells_per_block = N1 * N2 >= 64 ? kCellsF * 64 / (N1 * N2) : kCellsF;
   const size_t lds = (size_t)t.nsteps_fwd * 2 * kColsF * 4 +
-                     (size_t)cells_per_block * ((size_t)(2 * l1 + 2) * n1 + (size_t)(2 * l2 + 3) * n2) * 8;
+                     (size_t)cells_per_block * ((size_t)(2 * l1 + 2) * N1 + (size_t)(2 * l2 + 3) * N2) * 8;
   if (lds > 80 * 1024) return GELIB_HIP_OK;
-  rc = launch_fwd_shape(n1, n2, one_rowb, a, (unsigned)((ncells + cells_per_block - 1) / cells_per_block), lds, s);
+  rc = launch_fwd_shape(N1, N2, one_rowb, pad, a, (unsigned)((ncells + cells_per_block - 1) / cells_per_block), lds, s);
   if (rc) return rc;
   GELIB_HIP_TRY(hipGetLastError());
   *used = 1;
@@ -763,6 +835,10 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
 int onepair_mfma_set_option(const char *name, int value) {
   if (!std::strcmp(name, "onepair_mfma_fwd")) {
     g_enable_fwd = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "onepair_mfma_pad")) {   // other channel counts than those of GELIB_ONEPAIR_SHAPES
+    g_pad = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "onepair_mfma_paired")) {

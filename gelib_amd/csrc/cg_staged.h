@@ -94,7 +94,7 @@ int onepair_set_option(const char *name, int value);
 int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part_desc *> &g,
                          const std::vector<const gelib_part_desc *> &x, const std::vector<const gelib_part_desc *> &y,
                          const std::vector<const gelib_part_desc *> &xg, const std::vector<const gelib_part_desc *> &yg,
-                         bool accumulate, hipStream_t s, int *used);
+                         bool accumulate, hipStream_t s, int *used, bool dry = false);
 // The forward pass of the same shapes on the matrix cores (the reduction over m1).
 int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *> &r,
                          const std::vector<const gelib_part_desc *> &x, const std::vector<const gelib_part_desc *> &y,

@@ -1,0 +1,84 @@
+"""The matrix-core kernels for one x part times one y part with channel counts that none of their shapes has exactly (or rows that
+are not 16-byte aligned): products and gradients against the CPU oracle, and that what is not a number stays where it belongs."""
+import numpy as np
+import pytest
+
+from tests import gpu_util as U
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+ONEPAIR = 5
+
+
+@pytest.fixture(scope="module")
+def cabi():
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    from gelib_amd import cabi as c
+    c.lib()
+    return c
+
+
+CASES = [
+    # (B, l1, n1, l2, n2, maxl): one short of a shape and one channel of it on each side, both halves and all waves of a cell
+    (5, 8, 3, 9, 3, -1), (3, 10, 5, 8, 2, -1), (2, 9, 7, 9, 7, -1), (3, 10, 3, 8, 9, -1), (2, 7, 5, 10, 16, 12),
+    (2, 10, 9, 10, 5, -1), (1, 9, 16, 9, 6, 10), (2, 8, 9, 8, 9, -1), (1, 10, 16, 10, 15, -1), (1, 10, 13, 11, 11, -1),
+    (3000, 7, 3, 9, 3, 8),    # 16 places forward: the any-l kernel from 2049 cells on
+]
+
+
+@pytest.mark.parametrize("B,l1,n1,l2,n2,maxl", CASES)
+def test_padded_shapes(cabi, B, l1, n1, l2, n2, maxl):
+    xs, ys = [U.seeded(1 + B, B, 2 * l1 + 1, n1)], [U.seeded(2 + B, B, 2 * l2 + 1, n2)]
+    O = U.VecOracle(xs, ys, maxl, False, gseed=100 + B)
+    dx, dy, dg = [U.dev(a) for a in xs], [U.dev(a) for a in ys], [U.dev(a) for a in O.gs]
+    dr = [torch.full(p.shape, 5.0, dtype=torch.complex64, device="cuda") for p in O.r32]
+    cabi.so3vec_fwd(dr, dx, dy, accumulate=False)
+    N = min(a * b for a, b in [(8, 8), (4, 4), (8, 16), (16, 16), (16, 8), (4, 16), (8, 2)] if n1 <= a and n2 <= b)
+    assert (cabi.last_path() == ONEPAIR) == (2 * n1 * n2 > N and (N > 16 or B <= 2048))
+    dxg, dyg = [torch.full_like(t, 3.0 - 2j) for t in dx], [torch.full_like(t, 3.0 - 2j) for t in dy]
+    cabi.so3vec_bwd(dxg, dyg, dg, dx, dy, accumulate=False)
+    assert cabi.last_path() == ONEPAIR
+    torch.cuda.synchronize()
+    O.check_fwd([U.host(t) for t in dr], "forward")
+    O.check_bwd([U.host(dxg[0])], [U.host(dyg[0])], "backward")
+    ax, ay = [t.clone() for t in dxg], [t.clone() for t in dyg]
+    cabi.so3vec_bwd(ax, ay, dg, dx, dy, accumulate=True)
+    torch.cuda.synchronize()
+    O.check_bwd_onto([U.host(t) for t in ax], [U.host(t) for t in ay], [U.host(t) for t in dxg], [U.host(t) for t in dyg], "added")
+
+
+def test_rows_that_are_not_aligned(cabi):
+    """8 x 8 channels in parts of 65 channels (an odd row length): eight bytes at a time, the same bits as from aligned rows."""
+    B, l = 3, 9
+    x, y = U.dev(U.seeded(1, B, 2 * l + 1, 8)), U.dev(U.seeded(2, B, 2 * l + 1, 8))
+    tau = cabi.so3type_product({l: 8}, {l: 8}, -1)
+    ref = [torch.empty(B, 2 * k + 1, n, dtype=torch.complex64, device="cuda") for k, n in tau.items()]
+    wide = [torch.full((B, 2 * k + 1, n + 1), 7.0, dtype=torch.complex64, device="cuda") for k, n in tau.items()]
+    cabi.so3vec_fwd(ref, [x], [y], accumulate=False)
+    cabi.so3vec_fwd([w[..., :64] for w in wide], [x], [y], accumulate=False)
+    assert cabi.last_path() == ONEPAIR
+    assert all(torch.equal(w[..., :64], r) and bool((w[..., 64] == 7).all()) for w, r in zip(wide, ref))
+    got = []
+    for g in (ref, [w[..., :64] for w in wide]):
+        xg, yg = [torch.empty_like(x)], [torch.empty_like(y)]
+        cabi.so3vec_bwd(xg, yg, g, [x], [y], accumulate=False)
+        assert cabi.last_path() == ONEPAIR
+        got.append(xg + yg)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def test_not_a_number_stays_with_its_channels(cabi):
+    """One element of g that is not a number reaches the gradients of its own channels of x and y and no other."""
+    B, l, n1, n2 = 2, 8, 5, 6
+    x, y = U.dev(U.seeded(1, B, 2 * l + 1, n1)), U.dev(U.seeded(2, B, 2 * l + 1, n2))
+    tau = cabi.so3type_product({l: n1}, {l: n2}, -1)
+    for a, j in ((0, 0), (0, 5), (4, 0), (4, 5), (2, 3)):
+        g = [U.dev(U.seeded(9 + k, B, 2 * k + 1, n)) for k, n in tau.items()]
+        g[6][1, 3, a * n2 + j] = complex(float("nan"), 0.0)
+        xg, yg = [torch.empty_like(x)], [torch.empty_like(y)]
+        cabi.so3vec_bwd(xg, yg, g, [x], [y], accumulate=False)
+        assert cabi.last_path() == ONEPAIR
+        bad_x, bad_y = torch.isnan(torch.view_as_real(xg[0])).any(-1).any(1), torch.isnan(torch.view_as_real(yg[0])).any(-1).any(1)
+        assert bad_x.nonzero().tolist() == [[1, a]] and bad_y.nonzero().tolist() == [[1, j]]
