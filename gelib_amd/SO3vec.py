@@ -3,7 +3,7 @@ of python/src/gelib/SO3vec.py:22-309 for the CG product path.  The products are 
 forward writes into uninitialised parts and the backward computes both gradients from a single pass over g."""
 import torch
 
-from gelib_amd.SO3weights import mix_channels
+from gelib_amd.SO3weights import mix_parts
 from gelib_amd.gelib_common import backend, common_batch, without_torch_function
 from gelib_amd.SO3part import SO3part
 
@@ -86,7 +86,7 @@ class SO3vec:
 
     def __mul__(self, y):
         """Multiply every part by the matching weight matrix of an SO3weights (python/src/gelib/SO3vec.py:174-177)."""
-        return SO3vec(*[mix_channels(p, w) for p, w in zip(self.parts.values(), y.parts)])
+        return SO3vec(*mix_parts(list(self.parts.values()), list(y.parts)))
 
     def CGproduct(self, y, maxl=-1):
         xparts = list(self.parts.values())
@@ -154,18 +154,19 @@ def _product_fn(diag, part_cls=SO3part, prefix="SO3vec"):
 
         @staticmethod
         def backward(ctx, *gargs):
-            k1, k2 = ctx.k1, ctx.k2
-            saved = ctx.saved_tensors
+            return tuple([None, None, None] + Fn.grads(ctx.k1, ctx.k2, ctx.saved_tensors, gargs, ctx.needs_input_grad[3:]))
+
+        @staticmethod
+        def grads(k1, k2, saved, gargs, need):
             # An operand none of whose parts needs a gradient (harmonics of edge directions, say) gets none where the kernels
             # gain by that: products without sums over channels of operands up to l = 6.  The kernels for large l compute
             # both gradients faster than one.
-            need = ctx.needs_input_grad[3:]
             want = [True] * len(saved)
             if diag or all(t.size(-1) == 1 for t in saved[:k1]) != all(t.size(-1) == 1 for t in saved[k1:]):
                 if max(t.size(-2) for t in saved) <= 13:
-                    want = [any(need[:k1])] * k1 + [any(need[k1:])] * k2
-            grads = [torch.empty_like(t, memory_format=torch.contiguous_format) if w else None for t, w in zip(saved, want)]
-            return tuple([None, None, None] + Fn.fill(k1, k2, saved, grads, gargs))
+                    want = [any(need[:k1])] * k1 + [any(need[k1:k1 + k2])] * k2
+            out = [torch.empty_like(t, memory_format=torch.contiguous_format) if w else None for t, w in zip(saved, want)]
+            return Fn.fill(k1, k2, saved, out, gargs)
 
         @staticmethod
         @without_torch_function

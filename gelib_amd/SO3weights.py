@@ -50,6 +50,67 @@ def mix_channels(x, w):
     return torch.matmul(x, w)
 
 
+class MixPartsFn(torch.autograd.Function):
+    """x_k w_k for all parts of a vector in one call, any channel counts; contiguous complex64 GPU tensors.  classes: what the
+    results are (torch.matmul gives a part of an odd number of channels its class back)."""
+
+    @staticmethod
+    def forward(ctx, k, classes, *args):
+        from gelib_amd import cabi
+        xs, ws = list(args[:k]), list(args[k:])
+        ctx.k = k
+        ctx.save_for_backward(*args)
+        rs = [torch.empty(x.shape[:-1] + w.shape[1:], dtype=x.dtype, device=x.device) for x, w in zip(xs, ws)]
+        cabi.vec_mix_channels(rs, xs, ws, 0)
+        return tuple(r if c is torch.Tensor else r.as_subclass(c) for r, c in zip(rs, classes))
+
+    @staticmethod
+    def backward(ctx, *gs):
+        from gelib_amd import cabi
+        k = ctx.k
+        xs, ws = ctx.saved_tensors[:k], ctx.saved_tensors[k:]
+        need = ctx.needs_input_grad[2:]
+        gs = [g.as_subclass(torch.Tensor).contiguous() for g in gs]
+        gx, gw = [None] * k, [None] * k
+        if torch.is_grad_enabled():   # a graph of the gradients is wanted: torch's own operations
+            for i, (x, w, g) in enumerate(zip(xs, ws, gs)):
+                if need[i]:
+                    gx[i] = torch.matmul(g, w.conj().transpose(0, 1))
+                if need[k + i]:
+                    gw[i] = torch.matmul(x.reshape(-1, x.shape[-1]).conj().transpose(0, 1), g.reshape(-1, g.shape[-1]))
+            return tuple([None, None] + gx + gw)
+        todo = [i for i in range(k) if need[i]]
+        if todo:
+            for i in todo:
+                gx[i] = torch.empty_like(xs[i])
+            cabi.vec_mix_channels([gx[i] for i in todo], [gs[i] for i in todo], [ws[i] for i in todo], 1)
+        todo = [i for i in range(k) if need[k + i]]
+        if todo:
+            for i in todo:
+                gw[i] = torch.empty_like(ws[i])
+            cabi.vec_mix_channels([gw[i] for i in todo], [xs[i] for i in todo], [gs[i] for i in todo], 2)
+        return tuple([None, None] + gx + gw)
+
+
+def plain_autograd():
+    """False inside forward-mode derivatives and function transforms, which only torch's own operations support."""
+    return torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+
+
+def mix_parts(xs, ws):
+    """[torch.matmul(x, w) for x, w in zip(xs, ws)], on the GPU in one call of the library."""
+    pairs = list(zip(xs, ws))
+    if pairs and plain_autograd() and all(
+            x.is_cuda and w.is_cuda and x.device == w.device == xs[0].device and x.dtype == w.dtype == torch.complex64 and w.dim() == 2 and
+            x.numel() > 0 and w.numel() > 0 and x.shape[-1] == w.shape[0] for x, w in pairs):
+        odd = [x.shape[-1] % 2 != 0 for x, _ in pairs]
+        classes = [type(x) if o else torch.Tensor for (x, _), o in zip(pairs, odd)]
+        xp = [x.as_subclass(torch.Tensor).contiguous() for x, _ in pairs]
+        wp = [w.as_subclass(torch.Tensor).contiguous() for _, w in pairs]
+        return list(MixPartsFn.apply(len(pairs), classes, *(xp + wp)))
+    return [mix_channels(x, w) for x, w in pairs]
+
+
 class SO3weights:
 
     def __init__(self, *args):
@@ -132,14 +193,74 @@ class CGproductLinearFn(torch.autograd.Function):
                                      workspace_bytes=CGproductLinearFn.BWD_WORKSPACE_BYTES):
             grads = (xg or [None] * k1) + (yg or [None] * k2) + (wg or [None] * len(ws))
             return tuple([None, None, None] + [g if n else None for g, n in zip(grads, need)])
-        leaves = [t.detach().requires_grad_() for t in saved]
-        with torch.enable_grad():
-            x, y = SO3vec(*leaves[0:k1]), SO3vec(*leaves[k1:k1 + k2])
-            out = x.CGproduct(y, ctx.maxl) * SO3weights(*leaves[k1 + k2:])
-            outs = list(out.parts.values())
-        wanted = [t for t, need in zip(leaves, ctx.needs_input_grad[3:]) if need]
-        got = iter(torch.autograd.grad(outs, wanted, [g.contiguous() for g in gargs]))
-        return tuple([None, None, None] + [next(got) if need else None for need in ctx.needs_input_grad[3:]])
+        if not torch.is_grad_enabled():
+            # shapes that call does not take (odd channel counts): the product again, and the kernels for any counts
+            from gelib_amd.SO3vec import SO3vec
+            with torch._C.DisableTorchFunctionSubclass():
+                P = list(SO3vec(*xs).CGproduct(SO3vec(*ys), ctx.maxl).parts.values())
+                return tuple([None, None, None] + _mixed_product_grads(k1, k2, xs, ys, ws, [p.as_subclass(torch.Tensor) for p in P], gs, need))
+        return tuple([None, None, None] + _two_step_grads(k1, k2, ctx.maxl, saved, gs, need))
+
+
+def _two_step_grads(k1, k2, maxl, saved, gs, need):
+    """Gradients of the product followed by its matrices through the two separate autograd functions."""
+    from gelib_amd.SO3vec import SO3vec
+    leaves = [t.detach().requires_grad_() for t in saved]
+    with torch.enable_grad():
+        x, y = SO3vec(*leaves[0:k1]), SO3vec(*leaves[k1:k1 + k2])
+        out = x.CGproduct(y, maxl) * SO3weights(*leaves[k1 + k2:])
+        outs = list(out.parts.values())
+    wanted = [t for t, n in zip(leaves, need) if n]
+    got = iter(torch.autograd.grad(outs, wanted, gs))
+    return [next(got) if n else None for n in need]
+
+
+def _mixed_product_grads(k1, k2, xs, ys, ws, P, gs, need):
+    """Gradients of P_l W_l with P = CGproduct(x, y) at hand: the matrices' in one call, the product's in one, and the product's
+    backward pass."""
+    from gelib_amd import cabi
+    from gelib_amd.SO3vec import SO3vec_CGproductFn
+    wg = [None] * len(ws)
+    if any(need[k1 + k2:]):
+        wg = [torch.empty_like(w) for w in ws]
+        cabi.vec_mix_channels(wg, P, gs, 2)
+    xyg = [None] * (k1 + k2)
+    if any(need[0:k1 + k2]):
+        gP = [torch.empty_like(p) for p in P]
+        cabi.vec_mix_channels(gP, gs, ws, 1)
+        xyg = SO3vec_CGproductFn.grads(k1, k2, xs + ys, gP, need)
+    return [g if n else None for g, n in zip(list(xyg) + wg, need)]
+
+
+class CGproductMixFn(torch.autograd.Function):
+    """CGproduct(x, y, maxl) * W for the shapes the fused kernel does not take: the product is formed and kept, as the two
+    separate functions keep it, but all its parts are mixed in one call, forward and backward."""
+
+    @staticmethod
+    def forward(ctx, k1, k2, maxl, *args):
+        from gelib_amd import cabi
+        from gelib_amd.SO3part import SO3part
+        from gelib_amd.SO3vec import SO3vec
+        xs, ys, ws = list(args[0:k1]), list(args[k1:k1 + k2]), list(args[k1 + k2:])
+        ctx.k1, ctx.k2, ctx.maxl = k1, k2, maxl
+        P = [p.as_subclass(torch.Tensor) for p in SO3vec(*xs).CGproduct(SO3vec(*ys), maxl).parts.values()]
+        out = [torch.empty(p.shape[:-1] + w.shape[1:], dtype=p.dtype, device=p.device) for p, w in zip(P, ws)]
+        cabi.vec_mix_channels(out, P, ws, 0)
+        ctx.save_for_backward(*args, *P)
+        return tuple(r.as_subclass(SO3part) if p.shape[-1] % 2 else r for r, p in zip(out, P))
+
+    @staticmethod
+    def backward(ctx, *gargs):
+        k1, k2 = ctx.k1, ctx.k2
+        saved = ctx.saved_tensors
+        need = ctx.needs_input_grad[3:]
+        args, P = list(saved[:len(need)]), list(saved[len(need):])
+        gs = [g.as_subclass(torch.Tensor).contiguous() for g in gargs]
+        if torch.is_grad_enabled():   # a graph of the gradients is wanted
+            grads = _two_step_grads(k1, k2, ctx.maxl, args, gs, need)
+        else:
+            grads = _mixed_product_grads(k1, k2, args[0:k1], args[k1:k1 + k2], args[k1 + k2:], P, gs, need)
+        return tuple([None, None, None] + grads)
 
 
 def fused_linear_ok(x, y, W, maxl):
@@ -161,14 +282,40 @@ def fused_linear_ok(x, y, W, maxl):
     return all(w.dim() == 2 and w.shape[0] == taus[l] and 1 <= w.shape[1] <= 16 for l, w in enumerate(ws))
 
 
+def mixed_product_ok(x, y, W, maxl):
+    """True when CGproductMixFn takes CGproduct(x, y, maxl) * W: complex64 parts on one GPU, contiguous, the same leading
+    dimensions, one matrix for every part of the product, and nothing that only torch's own operations support (forward-mode
+    derivatives, function transforms)."""
+    xs, ys, ws = list(x.parts.values()), list(y.parts.values()), list(W.parts)
+    ts = xs + ys + ws
+    if not xs or not ys or not ws or not all(t.is_cuda and t.dtype == torch.complex64 and t.is_contiguous() and
+                                             t.device == ts[0].device and t.numel() > 0 for t in ts):
+        return False
+    if any(t.shape[:-2] != xs[0].shape[:-2] for t in xs + ys) or any(w.dim() != 2 for w in ws):
+        return False
+    if not plain_autograd():
+        return False
+    from gelib_amd import cabi
+    from gelib_amd.SO3vec import _one_channel_side
+    if _one_channel_side(xs, ys) is not None and max(t.shape[-1] for t in xs + ys) > 64:
+        return False   # (SO3vec.CGproduct repeats the channel there, and its backward pass is that of the Diag product)
+    taus = cabi.so3type_product(x.tau(), y.tau(), maxl)
+    return [w.shape[0] for w in ws] == list(taus.values())
+
+
 def CGproduct_linear(x, y, W, maxl=-1):
     """x.CGproduct(y, maxl) * W (python/src/gelib/SO3vec.py:174-177 applied to the result of SO3vec.CGproduct).  On the GPU,
     for the shapes fused_linear_ok accepts, one kernel forms the product and multiplies it by the matrices without
-    storing it; every other case runs the two steps one after the other."""
+    storing it; other shapes keep the product, and mix all its parts in one call.  What neither takes runs the two steps one after
+    the other."""
     from gelib_amd.SO3vec import SO3vec
     if fused_linear_ok(x, y, W, maxl):
-        xs = [p.as_subclass(torch.Tensor) for p in x.parts.values()]
-        ys = [p.as_subclass(torch.Tensor) for p in y.parts.values()]
-        ws = [w.as_subclass(torch.Tensor) for w in W.parts]
-        return SO3vec(*CGproductLinearFn.apply(len(xs), len(ys), maxl, *(xs + ys + ws)))
-    return x.CGproduct(y, maxl) * W
+        fn = CGproductLinearFn
+    elif mixed_product_ok(x, y, W, maxl):
+        fn = CGproductMixFn
+    else:
+        return x.CGproduct(y, maxl) * W
+    xs = [p.as_subclass(torch.Tensor) for p in x.parts.values()]
+    ys = [p.as_subclass(torch.Tensor) for p in y.parts.values()]
+    ws = [w.as_subclass(torch.Tensor) for w in W.parts]
+    return SO3vec(*fn.apply(len(xs), len(ys), maxl, *(xs + ys + ws)))

@@ -19,6 +19,7 @@ SYMBOLS = [
     "gelib_hip_so3vec_diagcg_bwd", "gelib_hip_so3part_spharm", "gelib_hip_gather_map_create",
     "gelib_hip_gather_map_destroy", "gelib_hip_part_gather", "gelib_hip_part_mix_channels",
     "gelib_hip_part_mix_channels_static", "gelib_hip_part_mix_channels_wgrad", "gelib_hip_part_mix_workspace_bytes",
+    "gelib_hip_vec_mix_channels", "gelib_hip_vec_mix_workspace_bytes",
     "gelib_hip_so3vec_cg_linear_fwd", "gelib_hip_so3vec_cg_linear_workspace_bytes",
     "gelib_hip_so3vec_cg_linear_workspace_bytes_shared", "gelib_hip_vec_gather",
     "gelib_hip_o3vec_cg_fwd", "gelib_hip_o3vec_cg_bwd",
@@ -104,6 +105,10 @@ def lib():
             getattr(L, name).argtypes = [ctypes.c_int, P, ctypes.c_int, P, ctypes.c_int, P]
         L.gelib_hip_part_mix_workspace_bytes.restype = ctypes.c_uint64
         L.gelib_hip_part_mix_workspace_bytes.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+        L.gelib_hip_vec_mix_workspace_bytes.restype = ctypes.c_uint64
+        L.gelib_hip_vec_mix_workspace_bytes.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 3 + [ctypes.c_int]
+        L.gelib_hip_vec_mix_channels.argtypes = ([ctypes.c_int] + [ctypes.c_void_p] * 6 + [ctypes.c_int, ctypes.c_void_p,
+                                                 ctypes.c_uint64, ctypes.c_void_p])
         L.gelib_hip_set_option.argtypes = [ctypes.c_char_p, ctypes.c_int]
         L.gelib_hip_set_stream_workspace.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint64]
         _lib = L
@@ -378,6 +383,35 @@ def part_mix_channels_wgrad(wg, x, g):
     ws, nbytes = mix_workspace(1, rows, n_in, n_out, wg.device)
     check(lib().gelib_hip_part_mix_channels_wgrad(wg.data_ptr(), x.data_ptr(), g.data_ptr(), rows, n_in, n_out, n_in,
                                                   n_out, ws.data_ptr(), nbytes, _stream(wg)))
+
+
+def vec_mix_channels(rs, xs, ws, kind):
+    """Channel mixing of all parts of a vector in one call, any channel counts (contiguous complex64 tensors).  kind 0:
+    r[..., o] = sum_c x[..., c] w[c, o]; kind 1: r[..., c] = sum_o x[..., o] conj(w[c, o]), the gradient of that with respect
+    to the part; kind 2: r[c, o] = sum over the leading indices of conj(x[..., c]) w[..., o], the gradient with respect to
+    the matrix (w: the gradient of the result)."""
+    import torch
+    k = len(rs)
+    n_in = [x.shape[-1] for x in xs]
+    n_out = [r.shape[-1] for r in rs]
+    for r, x, w, i, o in zip(rs, xs, ws, n_in, n_out):
+        fit = (tuple(w.shape) == (i, o) and r.shape[:-1] == x.shape[:-1] if kind == 0 else
+               tuple(w.shape) == (o, i) and r.shape[:-1] == x.shape[:-1] if kind == 1 else
+               tuple(r.shape) == (i, o) and w.shape[:-1] == x.shape[:-1] and w.shape[-1] == o)
+        if not fit:
+            raise ValueError("shapes of r, x and w do not fit")
+        if not (r.is_contiguous() and x.is_contiguous() and w.is_contiguous()):
+            raise ValueError("contiguous tensors are needed")
+    if k == 0:
+        return
+    P = ctypes.c_void_p * k
+    rows = (ctypes.c_int64 * k)(*[x.numel() // i if i else 0 for x, i in zip(xs, n_in)])
+    ci, co = (ctypes.c_int * k)(*n_in), (ctypes.c_int * k)(*n_out)
+    nbytes = int(lib().gelib_hip_vec_mix_workspace_bytes(k, rows, ci, co, kind))
+    ws_t = torch.empty(nbytes, dtype=torch.uint8, device=rs[0].device) if nbytes else None
+    check(lib().gelib_hip_vec_mix_channels(k, P(*[t.data_ptr() for t in rs]), P(*[t.data_ptr() for t in xs]),
+                                           P(*[t.data_ptr() for t in ws]), rows, ci, co, kind,
+                                           ws_t.data_ptr() if nbytes else None, nbytes, _stream(rs[0])))
 
 
 def set_option(name, value):

@@ -15,6 +15,7 @@
 
 #include "cg_common.h"
 #include "cg_linear.h"
+#include "mix_vec.h"
 #include "cg_staged.h"
 #include "cg_unrolled.h"
 
@@ -1153,6 +1154,87 @@ int linear_fwd_entry(int nr, const gelib_part_desc *r, int nx, const gelib_part_
 }
 
 
+// ---- channel mixing of all parts of a vector ------------------------------------------------------------------------
+int g_vec_mix = -1;   // kernels of mix_vec.hip: -1 by the shape, 0 only where mix.hip's do not take a part, 1 always
+
+// Is the part one for mix.hip's matrix-core kernels?
+bool matrix_part(int kind, long long rows, int n_in, int n_out) {
+  if ((n_in & 1) || rows > (1LL << 38) || g_vec_mix == 1) return false;
+  if (g_vec_mix == 0) return true;
+  // Gradients of matrices with even channel counts stay with mix.hip's kernel: the backward pass of the fused layer forms the
+  // same sums with it, and the two give the same bits.
+  if (kind == kVMGrad) return true;
+  // The launches for mix.hip's kernels cost about 20 us a part more, and its forward kernels for long rows walk a row at 1 us
+  // every 64 channels; beyond about this many multiply-adds its matrix instructions win.  Both, all parts, microseconds:
+  // forward L=3 16 x 16 -> 16 channels, 1024 cells 364 / 151, 4096 cells 425 / 546, L=4 8 x 8 -> 16, 4096 cells 281 / 321, -> 32
+  // 638 / 508; gradient of the product L=3 16 x 16 -> 16, 1024 cells 156 / 108, 4096 cells 376 / 425, L=4 8 x 8 -> 32, 4096
+  // cells 377 / 409.
+  const double madds = (double)rows * n_in * n_out;
+  return madds >= (kind == kVMForward ? (n_out > 16 ? 2e9 : 2.6e8) : 5e8);
+}
+
+struct VecMixSets {
+  std::vector<int> matrix;              // parts for mix.hip, one after the other
+  std::vector<VecMixPart> rest, all;    // parts of one launch, and every part as one
+  size_t matrix_bytes = 0;
+};
+VecMixSets vec_mix_sets(int nparts, void *const *r, const void *const *x, const void *const *w, const int64_t *rows,
+                        const int *n_in, const int *n_out, int kind) {
+  VecMixSets v;
+  for (int k = 0; k < nparts; k++) {
+    if (rows[k] == 0 || n_out[k] == 0) continue;
+    VecMixPart p;
+    p.a = x ? (const float2 *)x[k] : nullptr;
+    p.b = w ? (const float2 *)w[k] : nullptr;
+    p.c = r ? (float2 *)r[k] : nullptr;
+    p.m = kind == kVMGrad ? n_in[k] : rows[k];
+    p.n = n_out[k];
+    p.k = kind == kVMGrad ? rows[k] : n_in[k];
+    v.all.push_back(p);
+    if (matrix_part(kind, rows[k], n_in[k], n_out[k])) {
+      v.matrix.push_back(k);
+      v.matrix_bytes = std::max(v.matrix_bytes, kind == kVMGrad ? mix_wgrad_workspace_bytes(rows[k], n_in[k], n_out[k])
+                                                               : mix_workspace_bytes(n_in[k], n_out[k]));
+    } else {
+      v.rest.push_back(p);
+    }
+  }
+  return v;
+}
+int vec_mix_args(int nparts, const int64_t *rows, const int *n_in, const int *n_out, int kind) {
+  if (nparts < 0 || kind < 0 || kind > 2) return GELIB_HIP_ERR_ARG;
+  if (nparts > 0 && (!rows || !n_in || !n_out)) return GELIB_HIP_ERR_NULL;
+  for (int k = 0; k < nparts; k++)
+    if (rows[k] < 0 || n_out[k] < 0 || n_in[k] < 1 || rows[k] > (1LL << 38) || (kind == kVMGrad && rows[k] == 0)) return GELIB_HIP_ERR_ARG;
+  return GELIB_HIP_OK;
+}
+
+size_t vec_mix_bytes(const VecMixSets &v) {
+  // (a part for mix.hip whose memory is not aligned for it takes all parts to the one launch)
+  return std::max({v.matrix_bytes, vec_mix_workspace_bytes(v.rest), vec_mix_workspace_bytes(v.all)});
+}
+
+// r_k = x_k w_k and its gradients for all parts, shapes and pointers checked by the caller
+int vec_mix_run(int nparts, void *const *r, const void *const *x, const void *const *w, const int64_t *rows, const int *n_in,
+                const int *n_out, int kind, void *ws, size_t ws_bytes, hipStream_t s) {
+  const VecMixSets v = vec_mix_sets(nparts, r, x, w, rows, n_in, n_out, kind);
+  bool aligned = true;
+  for (int k : v.matrix) aligned = aligned && ((uintptr_t)x[k] & 15) == 0;
+  int rc;
+  if (aligned)
+    for (int k : v.matrix) {
+      if (kind == kVMGrad)
+        rc = launch_mix_wgrad((float2 *)r[k], (const float2 *)x[k], (const float2 *)w[k], rows[k], n_in[k], n_out[k], n_in[k],
+                              n_out[k], (float *)ws, ws_bytes, s);
+      else
+        rc = launch_mix((float2 *)r[k], (const float2 *)x[k], (const float2 *)w[k], rows[k], n_in[k], n_out[k], n_in[k],
+                        n_out[k], kind == kVMAdjoint, (float *)ws, ws_bytes, s);
+      if (rc) return rc == 11 ? GELIB_HIP_ERR_ARG : rc;
+    }
+  rc = launch_vec_mix(aligned ? v.rest : v.all, kind, ws, ws_bytes, s);
+  return rc == 11 ? GELIB_HIP_ERR_ARG : rc;
+}
+
 // ---- backward of CGproduct followed by the weight matrices, in bounded memory ------------------------------------
 // out_l = P_l W_l with P = CGproduct(x, y):  xg, yg = the product's backward pass on gP_l = gout_l W_l^H, and
 // wg_l = sum over the rows of P_l^H gout_l.  Neither P nor gP is ever held at full size: the batch is taken in chunks
@@ -1176,6 +1258,13 @@ size_t lin_bwd_bytes(const LinBwdShape &sh, long long cb, size_t *p_bytes, size_
     mb = std::max(mb, mix_workspace_bytes(sh.G[k].n, (int)sh.tau[k]));
     wb = std::max(wb, mix_wgrad_workspace_bytes(rows, (int)sh.tau[k], sh.G[k].n));
     tb = std::max(tb, (size_t)sh.tau[k] * sh.G[k].n * sizeof(float2));
+  }
+  {
+    const int n = (int)sh.G.size();
+    std::vector<int64_t> rows(n);
+    std::vector<int> tau(n), nout(n);
+    for (int k = 0; k < n; k++) rows[k] = cb * sh.G01 * (2 * sh.G[k].l + 1), tau[k] = (int)sh.tau[k], nout[k] = sh.G[k].n;
+    mb = std::max(mb, vec_mix_bytes(vec_mix_sets(n, nullptr, nullptr, nullptr, rows.data(), nout.data(), tau.data(), kVMAdjoint)));
   }
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   if (p_bytes) *p_bytes = pb;
@@ -1306,22 +1395,37 @@ int linear_bwd_entry(const gelib_part_desc *xg, const gelib_part_desc *yg, void 
       if (g_linear_wgrad && (rc = cg_linear_wgrad(cp, gd, xd, yd, WG, sh.tau, accumulate || b0 > 0, g_linear_wgrad >= 2, base, pb, s, &wg_done))) return rc;
       if (!wg_done && (rc = vec_fwd_entry(false, (int)P.size(), P.data(), nx, xc.data(), ny, yc.data(), 0, stream))) return rc;
     }
-    for (size_t k = 0; k < sh.G.size(); k++) {
+    // 2. gradients of the matrices: first chunk straight into wg, later chunks (and gradients that are added to) through the
+    // temporary;  3. gradient of the product, over the product itself or the sums of 1., all parts in one call where the rows
+    // of g are packed
+    const int np = (int)sh.G.size();
+    std::vector<int64_t> rows(np);
+    std::vector<int> tau(np), nout(np);
+    std::vector<void *> pp(np);
+    std::vector<const void *> gp(np), wp(np);
+    bool packed = true;
+    for (int k = 0; k < np; k++) {
       const gelib_part_desc &go = gc[sh.G[k].d - g];
-      const long long rows = cbn * sh.G01 * (2 * sh.G[k].l + 1);
-      const int tau = (int)sh.tau[k], n_out = sh.G[k].n;
-      // 2. gradient of the matrix: first chunk straight into wg (or onto it), later chunks through the temporary
-      if (wg && !wg_done) {
-        const bool direct = b0 == 0 && !accumulate;
-        rc = launch_mix_wgrad(direct ? WG[k] : wg_tmp, (const float2 *)P[k].ptr, (const float2 *)go.ptr, rows, tau, n_out,
-                              tau, go.strides[3], wg_ws, wb, s);
+      rows[k] = cbn * sh.G01 * (2 * sh.G[k].l + 1), tau[k] = (int)sh.tau[k], nout[k] = sh.G[k].n;
+      pp[k] = P[k].ptr, gp[k] = go.ptr, wp[k] = W[k];
+      packed = packed && go.strides[3] == nout[k];
+    }
+    const bool direct = b0 == 0 && !accumulate;
+    if (wg && !wg_done) {
+      for (int k = 0; k < np; k++) {
+        rc = launch_mix_wgrad(direct ? WG[k] : wg_tmp, (const float2 *)pp[k], (const float2 *)gp[k], rows[k], tau[k], nout[k], tau[k],
+                              gc[sh.G[k].d - g].strides[3], wg_ws, wb, s);
         if (rc) return rc == 11 ? GELIB_HIP_ERR_UNSUPPORTED : rc;
-        if (!direct && (rc = launch_add_into(WG[k], wg_tmp, (long long)tau * n_out, true, s))) return rc;
+        if (!direct && (rc = launch_add_into(WG[k], wg_tmp, (long long)tau[k] * nout[k], true, s))) return rc;
       }
-      // 3. gradient of the product, over the product itself or the sums of 1.
-      if (xg || yg) {
-        rc = launch_mix((float2 *)P[k].ptr, (const float2 *)go.ptr, W[k], rows, n_out, tau, go.strides[3], tau, true, mix_ws,
-                        mb, s);
+    }
+    if ((xg || yg) && packed) {
+      rc = vec_mix_run(np, pp.data(), gp.data(), wp.data(), rows.data(), nout.data(), tau.data(), kVMAdjoint, mix_ws, mb, s);
+      if (rc) return rc;
+    } else if (xg || yg) {
+      for (int k = 0; k < np; k++) {
+        rc = launch_mix((float2 *)pp[k], (const float2 *)gp[k], W[k], rows[k], nout[k], tau[k], gc[sh.G[k].d - g].strides[3], tau[k], true,
+                        mix_ws, mb, s);
         if (rc) return rc == 11 ? GELIB_HIP_ERR_UNSUPPORTED : rc;
       }
     }
@@ -1713,6 +1817,37 @@ uint64_t gelib_hip_part_mix_workspace_bytes(int kind, int64_t rows, int n_in, in
   return 0;
 }
 
+uint64_t gelib_hip_vec_mix_workspace_bytes(int nparts, const int64_t *rows, const int *n_in, const int *n_out, int kind) {
+  if (vec_mix_args(nparts, rows, n_in, n_out, kind)) return 0;
+  return vec_mix_bytes(vec_mix_sets(nparts, nullptr, nullptr, nullptr, rows, n_in, n_out, kind));
+}
+
+int gelib_hip_vec_mix_channels(int nparts, void *const *r, const void *const *x, const void *const *w, const int64_t *rows,
+                               const int *n_in, const int *n_out, int kind, void *workspace, uint64_t workspace_bytes,
+                               void *stream) {
+  t_last_path = kPathNone;
+  int rc = vec_mix_args(nparts, rows, n_in, n_out, kind);
+  if (rc) return rc;
+  if (nparts > 0 && (!r || !x || !w)) return GELIB_HIP_ERR_NULL;
+  auto whole = [&](const void *p, long long a, long long b) {
+    const int64_t d[5] = {a, 1, 1, 1, b}, st[5] = {b, 0, 0, 0, 1};
+    return check_range(p, d, st, 2 * sizeof(float));
+  };
+  for (int k = 0; k < nparts; k++) {
+    if (rows[k] == 0 || n_out[k] == 0) continue;
+    if (!r[k] || !x[k] || !w[k]) return GELIB_HIP_ERR_NULL;
+    if ((rc = whole(x[k], rows[k], n_in[k]))) return rc;
+    if ((rc = whole(w[k], kind == kVMForward ? n_in[k] : (kind == kVMAdjoint ? n_out[k] : rows[k]),
+                    kind == kVMAdjoint ? n_in[k] : n_out[k])))
+      return rc;
+    if ((rc = whole(r[k], kind == kVMGrad ? n_in[k] : rows[k], n_out[k]))) return rc;
+  }
+  const int64_t sd[5] = {(int64_t)workspace_bytes, 1, 1, 1, 1}, sst[5] = {1, 0, 0, 0, 0};
+  if (workspace && workspace_bytes && (rc = check_range(workspace, sd, sst, 1))) return rc;
+  t_last_path = kPathGeneric;
+  return vec_mix_run(nparts, r, x, w, rows, n_in, n_out, kind, workspace, (size_t)workspace_bytes, (hipStream_t)stream);
+}
+
 int gelib_hip_set_stream_workspace(void *stream, void *ptr, uint64_t bytes) {
   int dev = 0;
   GELIB_HIP_TRY(hipGetDevice(&dev));
@@ -1781,6 +1916,11 @@ int gelib_hip_set_option(const char *name, int value) {
   if (!std::strcmp(name, "check_pointers")) {
     g_check_pointers = value;
     forget_ranges(nullptr);
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "vec_mix")) {
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_vec_mix = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "linear_wgrad")) {

@@ -184,6 +184,16 @@ int gelib_hip_part_mix_channels_wgrad(void *wg, const void *x, const void *g, in
 /* Bytes of workspace the two calls above need: kind 0 for gelib_hip_part_mix_channels (either value of adjoint; n_in and
  * n_out as passed to that call), kind 1 for gelib_hip_part_mix_channels_wgrad.  0 for empty shapes or an unknown kind. */
 uint64_t gelib_hip_part_mix_workspace_bytes(int kind, int64_t rows, int n_in, int n_out);
+/* The same for all parts of a vector in one call, packed arrays of any channel counts and any 8-byte alignment; part k has
+ * rows[k] rows, n_in[k] channels of x[k] and n_out[k] of the result.  kind 0: r_k = x_k w_k, w_k (n_in, n_out).  kind 1:
+ * r_k = x_k w_k^H, w_k (n_out, n_in), the gradient with respect to the part.  kind 2: r_k = x_k^H w_k, w_k (rows, n_out), r_k
+ * (n_in, n_out), the gradient with respect to the matrix.  Parts without rows or results are left alone (kind 2 without rows:
+ * GELIB_HIP_ERR_ARG).  Results overwrite; fixed orders of summation.  workspace: at least
+ * gelib_hip_vec_mix_workspace_bytes(...) bytes (0: none needed), 16-byte aligned, rules as above. */
+int gelib_hip_vec_mix_channels(int nparts, void *const *r, const void *const *x, const void *const *w, const int64_t *rows,
+                               const int *n_in, const int *n_out, int kind, void *workspace, uint64_t workspace_bytes,
+                               void *stream);
+uint64_t gelib_hip_vec_mix_workspace_bytes(int nparts, const int64_t *rows, const int *n_in, const int *n_out, int kind);
 
 /* ---- vectors with two parts per l, told apart by a parity (O(3)) ------------------------------------------------------------
  * The product (diag: the Diag product) of vectors whose parts carry a label (l, p), p = +1 or -1, given in rp / xp / yp; a

@@ -1,0 +1,128 @@
+"""Channel mixing of all parts of a vector in one call (any channel counts) against numpy's complex128 matmul, and the layer
+built on it against the two separate steps.  Tolerance: that of test_gpu_mix.py, 1e-6 + 4 eps32 times the sum of the moduli
+of an element's terms (16 terms are added at a time here, so the chains are shorter than there)."""
+import numpy as np
+import pytest
+
+from tests import gpu_util as U
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def cabi():
+    assert torch.cuda.is_available()
+    from gelib_amd import cabi as c
+    c.lib()
+    return c
+
+
+def rand(shape, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.view_as_complex(torch.randn(*shape, 2, device="cuda", generator=g))
+
+
+# (rows, n_in, n_out) per part: edges of the tiles (4, 8, 16, 32 columns; 64 and 128 rows; 16 terms a step), one of everything,
+# sums long enough to be cut into pieces, parts of different sizes in one call, and more parts than a launch takes
+CASES = [
+    [(1, 1, 1)],
+    [(129, 15, 4), (7, 17, 3)],
+    [(128, 16, 8), (64, 33, 5), (3, 1, 7)],
+    [(65, 31, 16), (63, 300, 9)],
+    [(64, 2001, 32), (5, 7, 33), (1, 5, 70)],
+    [(40000, 3, 3), (13, 4097, 2)],
+    [(k + 1, 2 * k + 1, 3) for k in range(19)],
+]
+
+
+@pytest.mark.parametrize("mode", [-1, 0, 1])
+@pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("case", CASES, ids=[str(i) for i in range(len(CASES))])
+def test_vec_mix(cabi, case, kind, mode):
+    xs = [rand((rows, n_in), 1 + k) for k, (rows, n_in, _) in enumerate(case)]
+    ws = [rand({0: (i, o), 1: (o, i), 2: (rows, o)}[kind], 50 + k) for k, (rows, i, o) in enumerate(case)]
+    rs = [torch.full((i, o) if kind == 2 else (rows, o), float("nan"), dtype=torch.complex64, device="cuda") for rows, i, o in case]
+    cabi.set_option("vec_mix", mode)   # -1 by the shape, 0 the matrix-core kernels wherever they can, 1 never
+    try:
+        cabi.vec_mix_channels(rs, xs, ws, kind)
+    finally:
+        cabi.set_option("vec_mix", -1)
+    for r, x, w in zip(rs, xs, ws):
+        hx, hw = U.host(x).astype(np.complex128), U.host(w).astype(np.complex128)
+        a = hx.conj().T if kind == 2 else hx
+        b = hw.conj().T if kind == 1 else hw
+        tol = 1e-6 + 4 * np.finfo(np.float32).eps * (np.abs(a) @ np.abs(b))
+        err = np.abs(U.host(r) - a @ b)
+        assert (err <= tol).all(), "kind %d %s x %s: worst error / tolerance %.2f" % (kind, x.shape, w.shape, (err / tol).max())
+
+
+def test_vec_mix_refuses(cabi):
+    x, w, r = rand((5, 3), 1), rand((3, 2), 2), rand((5, 2), 3)
+    with pytest.raises(ValueError):
+        cabi.vec_mix_channels([r], [x], [rand((4, 2), 2)], 0)
+    with pytest.raises(cabi.GelibHipError):   # a sum long enough to be cut, and no workspace
+        import ctypes
+        a, b, c = rand((4, 4096), 1), rand((4096, 2), 2), rand((4, 2), 3)
+        P = ctypes.c_void_p * 1
+        cabi.check(cabi.lib().gelib_hip_vec_mix_channels(1, P(c.data_ptr()), P(a.data_ptr()), P(b.data_ptr()),
+                                                         (ctypes.c_int64 * 1)(4), (ctypes.c_int * 1)(4096), (ctypes.c_int * 1)(2),
+                                                         0, None, 0, None))
+
+
+@pytest.mark.parametrize("lx,ly,maxl,n1,n2,out,b", [(2, 2, 2, 4, 2, 5, 33), (3, 3, 3, 3, 3, 3, 130), (4, 4, 4, 3, 1, 3, 70),
+                                                   (2, 1, -1, 2, 3, 8, 5), (4, 4, 4, 13, 6, 13, 22), (3, 3, 3, 16, 8, 20, 300)])
+def test_layer_matches_the_two_steps(cabi, lx, ly, maxl, n1, n2, out, b):
+    """Values and all gradients of CGproduct_linear where the fused kernels do not take it (l other than 0..4, odd counts),
+    against the product and torch's matmul in complex128; a second pass gives the same bits."""
+    import gelib_amd as gelib
+    xs = [rand((b, 2 * l + 1, n1), l).requires_grad_() for l in range(lx + 1)]
+    ys = [rand((b, 2 * l + 1, n2), 10 + l).requires_grad_() for l in range(ly + 1)]
+    tau = cabi.so3type_product({l: n1 for l in range(lx + 1)}, {l: n2 for l in range(ly + 1)}, maxl)
+    ws = [(rand((n, out), 20 + l) / np.sqrt(n)).requires_grad_() for l, n in tau.items()]
+    gs = [rand((b, 2 * l + 1, out), 40 + l) for l in tau]
+
+    def run():
+        r = gelib.CGproduct_linear(gelib.SO3vec(*xs), gelib.SO3vec(*ys), gelib.SO3weights(*ws), maxl)
+        rs = list(r.parts.values())
+        return rs + list(torch.autograd.grad(rs, xs + ys + ws, gs))
+
+    got, again = run(), run()
+    assert all(torch.equal(a, c) for a, c in zip(got, again))
+    P = [p.detach() for p in gelib.SO3vec(*xs).CGproduct(gelib.SO3vec(*ys), maxl).parts.values()]
+    P64 = [p.as_subclass(torch.Tensor).cpu().to(torch.complex128) for p in P]
+    w64, g64 = [w.detach().cpu().to(torch.complex128) for w in ws], [g.cpu().to(torch.complex128) for g in gs]
+    want = [torch.matmul(p, w) for p, w in zip(P64, w64)]
+    gP = [torch.matmul(g, w.conj().T).to(torch.complex64).cuda() for g, w in zip(g64, w64)]
+    xg, yg = [torch.empty_like(x) for x in xs], [torch.empty_like(y) for y in ys]
+    cabi.so3vec_bwd(xg, yg, gP, [x.detach() for x in xs], [y.detach() for y in ys], accumulate=False)
+    want += [t.cpu() for t in xg + yg]
+    want += [torch.matmul(p.reshape(-1, p.shape[-1]).conj().T, g.reshape(-1, out)) for p, g in zip(P64, g64)]
+    for k, (a, c) in enumerate(zip(got, want)):
+        c = c.to(torch.complex128)
+        d = (a.detach().cpu().to(torch.complex128) - c).norm() / c.norm()
+        assert d < 2e-6, "output %d: relative error %.2g" % (k, d)   # sums of up to 3000 float32 terms, rounded randomly
+
+
+@pytest.mark.parametrize("nout", [16, 5])
+def test_matrix_gradient_from_strided_parts(cabi, nout):
+    """Matrix gradients straight from operands whose cells and rows do not follow each other in memory: the bits of packed ones."""
+    B, n1, n2 = 43, 8, 16
+    xs, ys = [rand((B, 2 * l + 1, n1), l) for l in range(5)], [rand((B, 2 * l + 1, n2), 10 + l) for l in range(5)]
+    tau = cabi.so3type_product({l: n1 for l in range(5)}, {l: n2 for l in range(5)}, 4)
+    ws, gs = [rand((n, 16), 20 + l) for l, n in tau.items()], [rand((B, 2 * l + 1, 16), 40 + l) for l in tau]
+    if nout != 16:   # even, as the call wants it, and less than the columns of a tile
+        nout += 1
+        ws, gs = [w[:, :nout].contiguous() for w in ws], [g[..., :nout].contiguous() for g in gs]
+    def strided(t):
+        w = torch.zeros(t.shape[0], t.shape[1], t.shape[2] + 3, dtype=t.dtype, device=t.device)
+        w[..., :t.shape[2]] = t
+        return w[..., :t.shape[2]]
+    out = []
+    for px in (xs, [strided(t) for t in xs]):
+        wg = [torch.full_like(w, float("nan")) for w in ws]
+        assert cabi.so3vec_cg_linear_bwd(None, None, wg, gs, px, ys, ws, accumulate=False)
+        assert cabi.last_path() == 6
+        out.append(wg)
+    assert all(torch.equal(a, b) for a, b in zip(*out))
