@@ -24,9 +24,11 @@
 // 1.2 1.8 2.3 2.8 3.1 / 0.9 1.4 1.7 2.0 2.2 / 1.0 1.4 1.7 2.0 2.3).  The second set takes the kernel from three waves per
 // SIMD to two: 8192 cells of 16 x 16 channels 1755 -> 2090 us, 8 x 8 767 -> 920.
 // What bounds it: matrix instructions (64 clocks a row and 32 channels) plus vector instructions (4 clocks each, about 2600
-// a cell and 32 channels of the L = 4 product), which do not overlap within a wave; the operands come from L2.
+// a cell and 32 channels of the L = 4 product), which do not overlap within a wave; the operands come from L2.  Packed parts are
+// staged as they lie, 16 bytes a thread: with a quotient by the row length and one by the channel count for every element
+// staging was a third of the vector instructions (8192 cells of 16 x 16 channels 2000 -> 1665 us).
 // Measured against forming the product, the matrix-gradient kernels of mix.hip on it and their sums (L = 4, 16 outputs,
-// microseconds): 8192 cells of 16 x 16 channels 2638 -> 1888 (in 1 GiB 4414 -> 2091), of 8 x 8 910 -> 885; 1024 cells
+// microseconds, before that): 8192 cells of 16 x 16 channels 2638 -> 1888 (in 1 GiB 4414 -> 2091), of 8 x 8 910 -> 885; 1024 cells
 // 543 -> 263 and 192 -> 140; 64 cells of 16 x 16 153 -> 81.
 #include <algorithm>
 #include <cstring>
@@ -66,10 +68,18 @@ struct LinWgradArgs {
                                        // channels first[k] .. first[k + 1]
 };
 
-template <int L1, int L2>
+// n complex numbers that follow each other, 16 bytes a thread
+__device__ __forceinline__ void stage_packed(float2 *dst, const float2 *src, int n, int tid) {
+#pragma unroll 2
+  for (int e = tid; e < n / 2; e += 256) ((float4 *)dst)[e] = ((const float4 *)src)[e];
+  if ((n & 1) && tid == 0) dst[n - 1] = src[n - 1];
+}
+
+// LDS: x and y as in memory, [cell of the tile][row][channel]; g per l, [l][cell of the tile][row][16 columns].
+template <int L1, int L2, bool PACKED>
 __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, float2 *ys, float2 *gs, int group, int range) {
   constexpr int lmin = iabs(L1 - L2), lmax = imin(L1 + L2, kLinL), NLP = lmax - lmin + 1;
-  constexpr int R1 = 2 * L1 + 1, R2 = 2 * L2 + 1, RG = (lmax + 1) * (lmax + 1) - lmin * lmin;
+  constexpr int R1 = 2 * L1 + 1, R2 = 2 * L2 + 1;
   const FastPart X = a.x[L1], Y = a.y[L2];
   const int n1 = X.n, n2 = Y.n, nch = n1 * n2;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = tid & 31, h = (tid >> 5) & 1;
@@ -88,23 +98,42 @@ __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, fl
   for (long long cell0 = first; cell0 < last; cell0 += kWTile) {
     const int cells = last - cell0 < kWTile ? (int)(last - cell0) : kWTile;
     __syncthreads();
-    for (int e = tid; e < cells * R1 * n1; e += 256) {
-      const int t = e / (R1 * n1), r = e - t * (R1 * n1), m = r / n1;
-      xs[t * kWOp + r] = X.ptr[(cell0 + t) * X.sb + (long long)m * X.sm + (r - m * n1)];
-    }
-    for (int e = tid; e < cells * R2 * n2; e += 256) {
-      const int t = e / (R2 * n2), r = e - t * (R2 * n2), m = r / n2;
-      ys[t * kWOp + r] = Y.ptr[(cell0 + t) * Y.sb + (long long)m * Y.sm + (r - m * n2)];
-    }
-    for (int e = tid; e < cells * RG * kWRow; e += 256) {
-      const int o = e & (kWRow - 1), tr = e / kWRow, t = tr / RG, row = tr - t * RG + lmin * lmin;
-      float2 v = make_float2(0.f, 0.f);
+    if constexpr (PACKED) {
+      stage_packed(xs, X.ptr + cell0 * (R1 * n1), cells * R1 * n1, tid);
+      stage_packed(ys, Y.ptr + cell0 * (R2 * n2), cells * R2 * n2, tid);
       static_for<NLP>([&](auto dc) __attribute__((always_inline)) {
-        constexpr int l = lmin + decltype(dc)::value;
-        if (row >= l * l && row < (l + 1) * (l + 1) && o < a.g[l].n)
-          v = a.g[l].ptr[(cell0 + t) * a.g[l].sb + (long long)(row - l * l) * a.g[l].sm + o];
+        constexpr int l = lmin + decltype(dc)::value, first_row = kWTile * (l * l - lmin * lmin);
+        const FastPart G = a.g[l];
+        float2 *dst = gs + first_row * kWRow;
+        const float2 *src = G.ptr + cell0 * ((2 * l + 1) * G.n);
+        const int rows = cells * (2 * l + 1);
+        if (G.n == kWRow) {
+          stage_packed(dst, src, rows * kWRow, tid);
+        } else {
+#pragma unroll 2
+          for (int e = tid; e < rows * kWRow; e += 256) {
+            const int o = e & (kWRow - 1);
+            dst[e] = o < G.n ? src[(e / kWRow) * G.n + o] : make_float2(0.f, 0.f);
+          }
+        }
       });
-      gs[tr * kWRow + o] = v;
+    } else {
+      for (int e = tid; e < cells * R1 * n1; e += 256) {
+        const int t = e / (R1 * n1), r = e - t * (R1 * n1), m = r / n1;
+        xs[e] = X.ptr[(cell0 + t) * X.sb + (long long)m * X.sm + (r - m * n1)];
+      }
+      for (int e = tid; e < cells * R2 * n2; e += 256) {
+        const int t = e / (R2 * n2), r = e - t * (R2 * n2), m = r / n2;
+        ys[e] = Y.ptr[(cell0 + t) * Y.sb + (long long)m * Y.sm + (r - m * n2)];
+      }
+      static_for<NLP>([&](auto dc) __attribute__((always_inline)) {
+        constexpr int l = lmin + decltype(dc)::value, first_row = kWTile * (l * l - lmin * lmin);
+        const FastPart G = a.g[l];
+        for (int e = tid; e < cells * (2 * l + 1) * kWRow; e += 256) {
+          const int o = e & (kWRow - 1), tr = e / kWRow, t = tr / (2 * l + 1), m = tr - t * (2 * l + 1);
+          gs[first_row * kWRow + e] = o < G.n ? G.ptr[(cell0 + t) * G.sb + (long long)m * G.sm + o] : make_float2(0.f, 0.f);
+        }
+      });
     }
     __syncthreads();
     if (!busy) continue;
@@ -119,13 +148,13 @@ __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, fl
       float2 yv[R2];
 #pragma unroll
       for (int k = 0; k < R1; k++) {
-        const float2 x = xs[t * kWOp + k * n1 + ca];
+        const float2 x = xs[(t * R1 + k) * n1 + ca];
         u[k] = h ? x.y : x.x;
         v[k] = h ? x.x : -x.y;
       }
 #pragma unroll
-      for (int k = 0; k < R2; k++) yv[k] = ys[t * kWOp + k * n2 + cj];
-      const float *gp = (const float *)(gs + t * RG * kWRow) + (i ^ h);
+      for (int k = 0; k < R2; k++) yv[k] = ys[(t * R2 + k) * n2 + cj];
+      const float *gp = (const float *)gs + (i ^ h);
       static_for<2 * lmax + 1>([&](auto mc) __attribute__((always_inline)) {
         constexpr int m = decltype(mc)::value - lmax;
         float q[R1];
@@ -146,7 +175,7 @@ __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, fl
                 start = false;
               }
             });
-            const float B = sign * gp[(l * l + l + m - lmin * lmin) * 2 * kWRow];
+            const float B = sign * gp[(kWTile * (l * l - lmin * lmin) + t * (2 * l + 1) + l + m) * 2 * kWRow];
             acc[dc.value] = __builtin_amdgcn_mfma_f32_32x32x2f32(P, B, acc[dc.value], 0, 0, 0);
           }
         });
@@ -173,12 +202,14 @@ __device__ __forceinline__ void wgrad_pair(const LinWgradArgs &a, float2 *xs, fl
   });
 }
 
+// PACKED: every part is packed, so a tile of cells is one piece of memory, and 16-byte aligned.
+template <bool PACKED>
 __global__ void __launch_bounds__(256, 2) linear_wgrad_kernel(const LinWgradArgs a) {
-  __shared__ float2 xs[kWTile * kWOp], ys[kWTile * kWOp], gs[kWTile * kWPairs * kWRow];
+  __shared__ __align__(16) float2 xs[kWTile * kWOp], ys[kWTile * kWOp], gs[kWTile * kWPairs * kWRow];
   const int work = (int)blockIdx.x / a.nranges, range = (int)blockIdx.x - work * a.nranges;
   static_for<kWPairs>([&](auto kc) __attribute__((always_inline)) {
     constexpr int k = decltype(kc)::value, L1 = kLinL - k / kWNL, L2 = kLinL - k % kWNL;
-    if (work >= a.first[k] && work < a.first[k + 1]) wgrad_pair<L1, L2>(a, xs, ys, gs, work - a.first[k], range);
+    if (work >= a.first[k] && work < a.first[k + 1]) wgrad_pair<L1, L2, PACKED>(a, xs, ys, gs, work - a.first[k], range);
   });
 }
 
@@ -287,10 +318,17 @@ int cg_linear_wgrad(const VecPlan &plan, const std::vector<const gelib_part_desc
   int rc = cg_table_bank(&a.bank);
   if (rc) return rc;
   a.partial = (float *)ws;
+  bool all_packed = true;
+  auto packed = [&](const std::vector<FastPart> &v, const std::vector<std::pair<int, int>> &ln) {
+    for (size_t k = 0; k < v.size(); k++)
+      if (v[k].sm != ln[k].second || v[k].sb != (long long)(2 * ln[k].first + 1) * ln[k].second || ((uintptr_t)v[k].ptr & 15)) all_packed = false;
+  };
+  packed(fx, lx), packed(fy, ly), packed(fg, lg);
   a.ncells = ncells;
   a.nranges = (int)nranges;
   a.accumulate = accumulate ? 1 : 0;
-  hipLaunchKernelGGL(linear_wgrad_kernel, dim3((unsigned)(nwork * nranges)), dim3(256), 0, s, a);
+  if (all_packed) hipLaunchKernelGGL(linear_wgrad_kernel<true>, dim3((unsigned)(nwork * nranges)), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(linear_wgrad_kernel<false>, dim3((unsigned)(nwork * nranges)), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(linear_wgrad_sum_kernel, dim3((unsigned)a.base[kWNL]), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
