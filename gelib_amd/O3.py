@@ -8,6 +8,8 @@ sorted by the index 2l + (p == -1) (O3/O3index.hpp:28-31), then l ascending, eac
 of its output part (core/Gvec.hpp:311-321) -- which the library does (gelib_hip_o3vec_cg_fwd / _bwd): one launch of the
 fused kernels per pair of parities.
 """
+import functools
+
 import torch
 
 from gelib_amd.gelib_common import backend, common_batch, without_torch_function
@@ -55,21 +57,29 @@ class O3irrep:
         return D * det if self.p == -1 else D
 
 
+@functools.lru_cache(maxsize=256)
+def _product_type(x, y, maxl, diag):
+    """The parts of a product of types (as tuples of items), in order.  Kept for the last 256 pairs of types: counting the pairs of
+    parts of two vectors with six parts each takes 35 us, and a product asked for it twice."""
+    x, y = dict(x), dict(y)
+    out = {}
+    for mu1 in sorted(x, key=_index):
+        for mu2 in sorted(y, key=_index):
+            if diag:
+                assert x[mu1] == y[mu2], "DiagCGproduct needs equal multiplicities"
+            for l in range(abs(mu1[0] - mu2[0]), mu1[0] + mu2[0] + 1):
+                if maxl >= 0 and l > maxl:
+                    continue
+                mu = (l, mu1[1] * mu2[1])
+                out[mu] = out.get(mu, 0) + (x[mu1] if diag else x[mu1] * y[mu2])
+    return tuple((mu, out[mu]) for mu in sorted(out, key=_index))
+
+
 class O3type(dict):
     """{(l, p): multiplicity}; product rules of core/Gtype.hpp:115-138 with O3group's components."""
 
     def _product(self, y, maxl, diag):
-        out = {}
-        for mu1 in sorted(self, key=_index):
-            for mu2 in sorted(y, key=_index):
-                if diag:
-                    assert self[mu1] == y[mu2], "DiagCGproduct needs equal multiplicities"
-                for l in range(abs(mu1[0] - mu2[0]), mu1[0] + mu2[0] + 1):
-                    if maxl >= 0 and l > maxl:
-                        continue
-                    mu = (l, mu1[1] * mu2[1])
-                    out[mu] = out.get(mu, 0) + (self[mu1] if diag else self[mu1] * y[mu2])
-        return O3type({mu: out[mu] for mu in sorted(out, key=_index)})
+        return O3type(_product_type(tuple(self.items()), tuple(y.items()), maxl, diag))
 
     def CGproduct(self, y, maxl=-1):
         return self._product(y, maxl, False)

@@ -2,7 +2,7 @@
 complex64 -- the class and autograd functions of python/src/gelib/SO3part.py:22-220 for the CG product path."""
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch, output
+from gelib_amd.gelib_common import backend, common_batch, output, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 
 
@@ -77,6 +77,7 @@ def _view(t):
 class SO3part_CGproductFn(torch.autograd.Function):
 
     @staticmethod
+    @without_torch_function
     def forward(ctx, x, y, l):
         ctx.l = l
         ctx.save_for_backward(x, y)
@@ -103,6 +104,7 @@ class SO3part_CGproductFn(torch.autograd.Function):
 class SO3part_DiagCGproductFn(torch.autograd.Function):
 
     @staticmethod
+    @without_torch_function
     def forward(ctx, x, y, l):
         ctx.l = l
         ctx.save_for_backward(x, y)
