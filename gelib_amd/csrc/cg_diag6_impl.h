@@ -62,10 +62,8 @@ __device__ __forceinline__ void row_store(RowPtr row, unsigned lane_off, float2 
 }
 __device__ __forceinline__ void row_store_stream(RowPtr row, unsigned lane_off, float2 v) {
   const v2f o = {v.x, v.y};
-  asm volatile("" : "+v"(lane_off));  // (also keeps this store and the one above apart: at the head of two branches they
-                                      // would become one ordinary store)
+  asm volatile("" : "+v"(lane_off));
   __builtin_nontemporal_store(o, (GlobalOut)(row + lane_off));
-  asm volatile("");
 }
 
 // A wave covers 64 channels of one cell, or -- when a part has 32 channels or fewer -- all channels of 64 / n_pad
@@ -132,7 +130,9 @@ __device__ __forceinline__ void load_rows(float2 (&v)[2 * L + 1], const FastPart
 }
 
 // LLO: the launch takes only the l from LLO up (the part of a product above l = 6 is a launch of its own).
-template <int L1, int L2, int LCAP, bool PACKED, int LLO = 0>
+// STREAM: streaming stores over what is there (kernels of their own: a second kind of store in the code of a row costs narrow parts 5 to
+// 20 % even where it never runs: 1 to 3 channels, L=3 to 6, 4 to 60 MB).
+template <int L1, int L2, int LCAP, bool PACKED, bool STREAM, int LLO = 0>
 __device__ __forceinline__ void fwd_pair(const Diag6Args &a, const float2 (&xv)[2 * L1 + 1],
                                          const float2 (&yv)[2 * L2 + 1], const WavePos q) {
   constexpr int LMIN = imax(iabs(L1 - L2), LLO);
@@ -141,7 +141,7 @@ __device__ __forceinline__ void fwd_pair(const Diag6Args &a, const float2 (&xv)[
     constexpr int NL = LTOP - LMIN + 1;
     const OffsPtr offs = (OffsPtr)a.offs + (L1 * kNP + L2) * kNR;
     const CoeffPtr C = (CoeffPtr)a.bank;
-    const bool accumulate = a.write == kWriteAdd, stream = a.write == kWriteStream;
+    const bool accumulate = a.write == kWriteAdd;
     // the row of part l that the next m of that part is stored to; a triple that is not there is never stored
     RowPtr row[NL];
     unsigned lo[NL];
@@ -180,7 +180,7 @@ __device__ __forceinline__ void fwd_pair(const Diag6Args &a, const float2 (&xv)[
         constexpr int L = LMIN + dl;
         if constexpr (L >= MABS) {
           if (present[dl] && q.live) {
-            if (stream) row_store_stream(row[dl], lo[dl], acc[dl]);
+            if (STREAM) row_store_stream(row[dl], lo[dl], acc[dl]);
             else row_store(row[dl], lo[dl], acc[dl], accumulate);
           }
           row[dl] += row_step(a.r[L]);
@@ -230,7 +230,7 @@ __device__ __forceinline__ void read_rows(float2 (&v)[2 * L + 1], const float2 *
 // leave room for three blocks per compute unit instead of five, and the store stream needs the waves (measured on
 // L = 6, 64 channels, 131072 cells: no image 18.2 - 20.2 ms, y alone 16.6 - 17.4 ms, both 29.7 ms).
 // LOP: the largest l of an operand part the kernel has code for.
-template <int LCAP, bool PACKED, int LOP, int LLO = 0>
+template <int LCAP, bool PACKED, bool STREAM, int LOP, int LLO = 0>
 __global__ void __launch_bounds__(256) diag6_fwd_kernel(const Diag6Args a) {
   __shared__ float2 yimg[(LOP + 1) * (LOP + 1) * 64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -250,7 +250,7 @@ __global__ void __launch_bounds__(256) diag6_fwd_kernel(const Diag6Args a) {
             if (((L1 * kNP + L2) & 3) == wave && a.y[L2].ptr != nullptr) {
               float2 yv[2 * L2 + 1];
               read_rows<L2>(yv, yimg, lane);
-              fwd_pair<L1, L2, LCAP, PACKED, LLO>(a, xv, yv, q);
+              fwd_pair<L1, L2, LCAP, PACKED, STREAM, LLO>(a, xv, yv, q);
             }
           }
         });
@@ -585,7 +585,8 @@ int launch_diag6_bwd_sets_variant(const Diag6Args &a, hipStream_t s) {
 
 template <int LCAP, bool PACKED, int LOP = kL6, int LLO = 0>
 int launch_diag6_fwd_variant(const Diag6Args &a, hipStream_t s) {
-  hipLaunchKernelGGL((diag6_fwd_kernel<LCAP, PACKED, LOP, LLO>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
+  if (a.write == kWriteStream) hipLaunchKernelGGL((diag6_fwd_kernel<LCAP, PACKED, true, LOP, LLO>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((diag6_fwd_kernel<LCAP, PACKED, false, LOP, LLO>), dim3((unsigned)a.nwaves), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
 }

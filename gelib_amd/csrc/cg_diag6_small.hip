@@ -15,7 +15,7 @@ namespace gelib_hip {
 
 namespace {
 
-template <int kSmallLop, int kSmallCap, bool PACKED>
+template <int kSmallLop, int kSmallCap, bool PACKED, bool STREAM>
 __global__ void __launch_bounds__(256) diag6_small_fwd_kernel(const Diag6Args a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long long w = (long long)blockIdx.x * 4 + wave;
@@ -31,7 +31,7 @@ __global__ void __launch_bounds__(256) diag6_small_fwd_kernel(const Diag6Args a)
         if (a.y[L2].ptr != nullptr) {
           float2 yv[2 * L2 + 1];
           load_rows<L2, PACKED>(yv, a.y[L2], q, a.ybc != 0);
-          fwd_pair<L1, L2, kSmallCap, PACKED>(a, xv, yv, q);
+          fwd_pair<L1, L2, kSmallCap, PACKED, STREAM>(a, xv, yv, q);
         }
       });
     }
@@ -114,13 +114,18 @@ int launch_small_bwd(const Diag6Args &a, hipStream_t s) {
   return a.once ? launch_small_bwd_g<LOP, LCAP, LLO, true>(a, s) : launch_small_bwd_g<LOP, LCAP, LLO, false>(a, s);
 }
 
-template <int LOP, int LCAP>
-int launch_small_fwd(const Diag6Args &a, hipStream_t s) {
+template <int LOP, int LCAP, bool STREAM>
+int launch_small_fwd_as(const Diag6Args &a, hipStream_t s) {
   const unsigned nblocks = (unsigned)((a.nwaves + 3) / 4);
-  if (a.lg_npad < 6) hipLaunchKernelGGL((diag6_small_fwd_kernel<LOP, LCAP, true>), dim3(nblocks), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((diag6_small_fwd_kernel<LOP, LCAP, false>), dim3(nblocks), dim3(256), 0, s, a);
+  if (a.lg_npad < 6) hipLaunchKernelGGL((diag6_small_fwd_kernel<LOP, LCAP, true, STREAM>), dim3(nblocks), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((diag6_small_fwd_kernel<LOP, LCAP, false, STREAM>), dim3(nblocks), dim3(256), 0, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
+}
+
+template <int LOP, int LCAP>
+int launch_small_fwd(const Diag6Args &a, hipStream_t s) {
+  return a.write == kWriteStream ? launch_small_fwd_as<LOP, LCAP, true>(a, s) : launch_small_fwd_as<LOP, LCAP, false>(a, s);
 }
 
 }  // namespace
