@@ -551,13 +551,18 @@ int fwd_dispatch(const VecPlan &plan, const std::vector<View> &R, const std::vec
     }
     {
       // A CGproduct of operands above l = 4 that reaches above l = 6 (the API default is uncapped): the unrolled kernel
-      // built for such operands takes the triples up to l = 6, the any-l kernels the rest (different product parts).
+      // built for such operands takes the triples up to l = 6, another launch (unrolled or any-l) the rest (different product parts).
       int lop = 0;
       for (auto &v : X) lop = std::max(lop, v.l);
       for (auto &v : Y) lop = std::max(lop, v.l);
       VecPlan A, B;
       std::vector<View> RA, RB;
-      if (!plan.diag && lop > 4 && lop <= 6 && split_at_l6(plan, R, A, B, RA, RB)) {
+      // Few pairs with an odd channel count stay with the any-l kernels, whose one launch is faster than two where they are small: (5) x
+      // (4), 3 channels, 4 MB 63 / 37 us, (6) x L=2, 5 channels, 4 to 1500 MB 1.71 1.50 1.09 1.08.
+      bool odd = false;
+      for (auto &v : X) odd = odd || v.n % 2;
+      const bool few = odd && X.size() * Y.size() <= 4;
+      if (!plan.diag && lop > 4 && lop <= 6 && !few && split_at_l6(plan, R, A, B, RA, RB)) {
         std::vector<const gelib_part_desc *> ra;
         for (auto &v : RA) ra.push_back(v.d);
         rc = unrolled_vec_fwd(A, ra, xd, yd, accumulate != 0, s, &used);

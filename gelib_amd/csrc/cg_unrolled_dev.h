@@ -99,7 +99,7 @@ __device__ __forceinline__ int pick_int(const int (&arr)[N], int i) {
 
 // ti: channels of the first operand handled per thread (1, 2 or 4); divides every n1 unless ragged.
 // lop: largest l of an operand (above kLT: the kernel for l up to kLTMax -- unrolled_fwd_takes says when it exists)
-bool unrolled_fwd_takes(bool diag, int ti, int lcap, int lop);
+bool unrolled_fwd_takes(bool diag, int ti, int lcap, int lop, int llo);
 int launch_unrolled_fwd(const FwdArgs &a, bool diag, int ti, bool ragged, int lcap, int lop, int nblocks, size_t lds_bytes, hipStream_t s);
 // lcap: largest l present in the gradient; lop: largest l of an operand (above kLT: the kernel for l up to kLTMax, which
 // exists for CGproduct with power-of-two channel counts and lcap <= kLTMax only -- unrolled_bwd_takes says so)

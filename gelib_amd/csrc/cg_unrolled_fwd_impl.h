@@ -1,4 +1,4 @@
-// Forward CG / DiagCG product for l1, l2 <= kLT, all (l1,l2,l) triples of an SO3vec product in one launch.
+// Forward CG / DiagCG product for l1, l2 <= kLT (CGproduct: kLTMax), all (l1,l2,l) triples of an SO3vec product in one launch.
 //
 // Work split: a block owns one (x part, y part) pair and a run of cells.  It first copies the two operand parts
 // of its cells into LDS (the only loads from memory it ever waits for); after that its 256 threads sweep the
@@ -28,11 +28,12 @@ typedef __attribute__((address_space(1))) v2f *GlobalOut;  // product rows: glob
 
 // One (l1,l2,l) triple for one thread: rows m = -L..L of the block, TI channels each.
 // last: the thread's channels 0..last exist (RAGGED; otherwise all TI do).
-// STREAM: the kernel can write with streaming stores (a.write says whether it does).
+// STREAM: streaming stores over what is there (kernels of their own: a second kind of store in the code of a row costs 2 to 7 % even
+// where it never runs).
 template <int L1, int L2, int L, int TI, bool RAGGED, bool STREAM>
 __device__ __forceinline__ void triple_fwd(const float2 (&xv)[TI][2 * L1 + 1], const float2 (&yv)[2 * L2 + 1],
                                            CoeffPtr C, GlobalOut rp, int sm, int kstride, bool accumulate,
-                                           bool live, int last, bool stream) {
+                                           bool live, int last) {
 #pragma unroll
   for (int m = -L; m <= L; m++) {
     float2 acc[TI];
@@ -62,9 +63,8 @@ __device__ __forceinline__ void triple_fwd(const float2 (&xv)[TI][2 * L1 + 1], c
         v2f v;
         v.x = acc[k].x;
         v.y = acc[k].y;
-        if (STREAM && stream) {
+        if (STREAM) {
           __builtin_nontemporal_store(v, &row[k * kstride]);
-          asm volatile("");  // (two equal stores at the ends of two branches would become one ordinary store)
           continue;
         }
         if (accumulate) v += row[k * kstride];
@@ -76,15 +76,16 @@ __device__ __forceinline__ void triple_fwd(const float2 (&xv)[TI][2 * L1 + 1], c
 
 // The product parts, indexed by their l (the host fills FwdArgs::r that way), copied out of the kernel arguments
 // once so that the unrolled code can name them with compile-time indices.
-template <int LCAP>
+// LLO..LCAP: the l that the kernel has code for.
+template <int LCAP, int LLO>
 struct RParts {
-  FastPart R[LCAP + 1];
+  FastPart R[LCAP - LLO + 1];
 };
 
-template <int L1, int L2, int LCAP, int TI, bool DIAG, bool RAGGED, bool STREAM>
-__device__ __forceinline__ void pair_fwd(const RParts<LCAP> &rp_all, PairPtr pr, CoeffPtr Cs, const float2 *xs,
+template <int L1, int L2, int LCAP, int LLO, int TI, bool DIAG, bool RAGGED, bool STREAM>
+__device__ __forceinline__ void pair_fwd(const RParts<LCAP, LLO> &rp_all, PairPtr pr, CoeffPtr Cs, const float2 *xs,
                                          const float2 *ys, int offs_add, bool accumulate, long long cell, int dc,
-                                         int u, bool live, bool stream) {
+                                         int u, bool live) {
   const __attribute__((address_space(4))) PairRec &p = *pr;
   const int N1 = p.n1, N2 = p.n2;
   int i0, j;
@@ -117,11 +118,11 @@ __device__ __forceinline__ void pair_fwd(const RParts<LCAP> &rp_all, PairPtr pr,
   static_for<NL>([&](auto dl_c) __attribute__((always_inline)) {
     constexpr int dl = decltype(dl_c)::value;
     constexpr int L = LMIN + dl;
-    if constexpr (L <= LCAP) {
+    if constexpr (L <= LCAP && L >= LLO) {
       if (p.ri[dl] >= 0) {
-        const FastPart R = rp_all.R[L];
+        const FastPart R = rp_all.R[L - LLO];
         GlobalOut rp = (GlobalOut)R.ptr + cell * R.sb + (p.offs[dl] + offs_add + u);
-        triple_fwd<L1, L2, L, TI, RAGGED, STREAM>(xv, yv, Cs + p.cg[dl], rp, R.sm, kstride, accumulate, live, last, stream);
+        triple_fwd<L1, L2, L, TI, RAGGED, STREAM>(xv, yv, Cs + p.cg[dl], rp, R.sm, kstride, accumulate, live, last);
       }
     }
   });
@@ -143,7 +144,7 @@ __device__ __forceinline__ void stage_part(float2 *dst, const FastPart P, int ro
 
 // LT: largest operand l of the pairs the kernel has code for.  RAGGED: channel counts of x that TI does not divide -- the
 // slots then are ceil(n1 / TI) * n2, and the threads of the last channels leave out those beyond n1.
-template <int LCAP, bool DIAG, int TI, int LT, bool RAGGED>
+template <int LCAP, bool DIAG, int TI, int LT, bool RAGGED, int LLO, bool STREAM>
 __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
   extern __shared__ float2 lds_ops[];
   int pidx = 0, first = 0;
@@ -173,10 +174,10 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
   float2 *ys = xs + cpb * (2 * l1 + 1) * n1;
   stage_part(xs, pick_part(a.x, p->xi), 2 * l1 + 1, cell0, ncell);
   stage_part(ys, pick_part(a.y, p->yi), 2 * l2 + 1, cell0, ncell);
-  RParts<LCAP> rp_all;
-  static_for<LCAP + 1>([&](auto l) __attribute__((always_inline)) { rp_all.R[l.value] = a.r[l.value]; });
+  RParts<LCAP, LLO> rp_all;
+  static_for<LCAP - LLO + 1>([&](auto l) __attribute__((always_inline)) { rp_all.R[l.value] = a.r[LLO + l.value]; });
   const int offs_add = a.offs_add;
-  const bool accumulate = a.write == kWriteAdd, stream = a.write == kWriteStream;
+  const bool accumulate = a.write == kWriteAdd;
   __syncthreads();
 
   const int U = DIAG ? n1 : (RAGGED ? (n1 + TI - 1) / TI : n1 / TI) * n2;
@@ -193,8 +194,8 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
     switch (code) {
 #define GELIB_CASE(A, B)                                                                                      \
   case A * (kLTMax + 1) + B:                                                                                  \
-    if constexpr (A <= LT && B <= LT)                                                                         \
-      pair_fwd<A, B, LCAP, TI, DIAG, RAGGED, (LT > kLT)>(rp_all, p, C, xs, ys, offs_add, accumulate, cell, dc, u, live, stream); \
+    if constexpr (A <= LT && B <= LT && A + B >= LLO)                                                         \
+      pair_fwd<A, B, LCAP, LLO, TI, DIAG, RAGGED, STREAM>(rp_all, p, C, xs, ys, offs_add, accumulate, cell, dc, u, live); \
     break;
 #define GELIB_ROW(A) \
   GELIB_CASE(A, 0) GELIB_CASE(A, 1) GELIB_CASE(A, 2) GELIB_CASE(A, 3) GELIB_CASE(A, 4) GELIB_CASE(A, 5) GELIB_CASE(A, 6)
@@ -206,10 +207,10 @@ __global__ void __launch_bounds__(kBlock) unrolled_fwd_kernel(const FwdArgs a) {
   }
 }
 
-template <int LCAP, bool DIAG, int TI, int LT = kLT, bool RAGGED = false>
+template <int LCAP, bool DIAG, int TI, int LT = kLT, bool RAGGED = false, int LLO = 0, bool STREAM = false>
 int launch_fwd_variant(const FwdArgs &a, int nblocks, size_t lds_bytes, hipStream_t s) {
   static_assert(kLTMax == 6 && LT <= kLTMax, "the case table above lists l1, l2 = 0..6");
-  hipLaunchKernelGGL((unrolled_fwd_kernel<LCAP, DIAG, TI, LT, RAGGED>), dim3(nblocks), dim3(kBlock), lds_bytes, s, a);
+  hipLaunchKernelGGL((unrolled_fwd_kernel<LCAP, DIAG, TI, LT, RAGGED, LLO, STREAM>), dim3(nblocks), dim3(kBlock), lds_bytes, s, a);
   GELIB_HIP_TRY(hipGetLastError());
   return GELIB_HIP_OK;
 }

@@ -267,6 +267,36 @@ struct FastLists {
   std::vector<FastPart> x, y, r, xg, yg;
 };
 
+// Operands above kLT: odd channel counts, and what lies above l = kLTMax, here or in the any-l kernels.  Time here / there in
+// vectors with 4, 60, 600 and 1500 MB of product:
+//   odd counts, capped: L=6 3 channels .18 .26 .61 .65, 7 .21 .27 .61 .72; L=5 5 channels .17 .32 .60 .69; (5) x (5) .73 .72 .78 .79;
+//   uncapped (both launches): L=6 5 channels .40 .43 .65 .66, 8 .81 .67 .97 .90, 12 .69 .51 .86 .94; L=5 4 channels .67 .61 .89 .85;
+//   L=6 8 channels x (1) .72 .74 .84 .86; (6) x (2) .90 .86 .65 .62; (1,2) x L=6 .62 .60 .76 .91.
+// Above kLTMax the pairs with a short side (l up to 3) must be more than half: two long ones, whose sums are long, only gain
+// in small launches ((5,6) x (5,6), 8 channels .84 .80 1.08 1.13, (6) x (6) 1.15 1.14 .85 .93).
+// One triple by itself, 4, 60 and 600 MB, odd counts: (5,2)->4 3 x 3 channels .20 .49 .44, 7 x 20 .70 .73 .89, 31 x 32 .83 .85 .93;
+// (6,6)->6 9 x 9 .49 .57 .65; but short results of many channels (6,6)->0 7 x 20 .89 1.28 1.44, 17 x 3 1.34 1.32 1.47, ->1 7 x 20
+// .68 1.00 1.17, 31 x 32 1.35 1.05 .93 (9 x 9 .58 .69 .71).  Above kLTMax: (6,6)->12 8 x 8 .46 .50 .81, 16 x 16 .32 .38 .81, (5,5)->10 16 x 16
+// .65 .71 1.11, (3,6)->8 64 x 48 .61 .63 1.14, odd counts .20 to .97 throughout.
+bool l6_pays(const std::vector<VecTriple> &triples, const std::vector<std::pair<int, int>> &xs,
+             const std::vector<std::pair<int, int>> &ys, int lcap, bool ragged, long long ncells) {
+  if (triples.size() == 1) {
+    const VecTriple &t = triples[0];
+    const long long nout = (long long)xs[t.xi].second * ys[t.yi].second;
+    if (ragged) return t.l > 2 || nout <= (t.l == 0 ? 32 : 128);
+    if (lcap <= kLTMax) return true;
+    return 8 * ncells * (2 * t.l + 1) * nout < 256000000LL || (std::min(t.l1, t.l2) <= 3 && nout < 1024);
+  }
+  if (lcap <= kLTMax) return true;
+  std::vector<std::pair<int, int>> pairs;
+  for (auto &t : triples) pairs.push_back({t.xi, t.yi});
+  std::sort(pairs.begin(), pairs.end());
+  pairs.erase(std::unique(pairs.begin(), pairs.end()), pairs.end());
+  size_t narrow = 0;
+  for (auto &p : pairs) narrow += std::min(xs[p.first].first, ys[p.second].first) <= 3;
+  return 2 * narrow > pairs.size();
+}
+
 int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<std::pair<int, int>> &xs,
             const std::vector<std::pair<int, int>> &ys, const std::vector<int> &rls, const FastLists &f,
             long long ncells, int offs_add, bool accumulate, hipStream_t s, int *used) {
@@ -287,8 +317,8 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   }
   // which kernel would run is decided from the type alone, before any table is built: a product this family declines
   // (e.g. operands of l = 6 uncapped) must not cost a device allocation, and its l range does not fit a PairRec
-  int lcap_all = 0, lop = 0;
-  for (auto &t : triples) lcap_all = std::max(lcap_all, t.l), lop = std::max(lop, std::max(t.l1, t.l2));
+  int lcap_all = 0, lop = 0, llo = 1 << 30;
+  for (auto &t : triples) lcap_all = std::max(lcap_all, t.l), llo = std::min(llo, t.l), lop = std::max(lop, std::max(t.l1, t.l2));
   int ti = 1;
   bool ragged = false;
   if (!diag) {
@@ -321,8 +351,12 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
     for (auto &t : triples) ragged = ragged || xs[t.xi].second % ti;
     if (ragged && ti < 4) ti = 1, ragged = false;   // fewer than four on request: counts that do not divide take one
   }
-  if (lop > kLT && ti == 4) ti = 2;  // the kernel for operands above kLT is built for two channels per thread
-  if (!unrolled_fwd_takes(diag, ti, lcap_all, lop) || (lop > kLT && !g_fwd_l6_enable)) return GELIB_HIP_OK;
+  if (lop > kLT && !diag) {   // the kernels for operands above kLT are built for two channels per thread, an odd last one left out
+    if (ti == 4) ti = 2;
+    if (ti == 1 && g_fwd_ti != 1) ti = 2, ragged = true;
+  }
+  if (!unrolled_fwd_takes(diag, ti, lcap_all, lop, llo) || (lop > kLT && !g_fwd_l6_enable)) return GELIB_HIP_OK;
+  if (lop > kLT && !l6_pays(triples, xs, ys, lcap_all, ragged, ncells)) return GELIB_HIP_OK;
   const DevicePlan *plan = nullptr;
   int rc = get_plan(diag, triples, xs, ys, rls, &plan);
   if (rc) return rc;
