@@ -642,7 +642,7 @@ bool padded_shape(int n1, int n2, int *N1, int *N2) {
 }
 // Backward: more than 64 lane slots (channel counts rounded up to powers of two) would go to the shape-agnostic kernels, up to
 // 64 to the LDS-column kernel, which pads the same way.  Before / padded here, l = 10 x 10, all l, microseconds: 9 x 9 channels 104
-// cells 13584 / 144, 1399 cells 14000 / 550; 12 x 6, 1574 cells 7230 / 350; 5 x 16, 1417 cells 5430 / 233; 5 x 5, 4535 cells 599 / 351;
+// cells 13584 / 144, 1399 cells 14000 / 400; 12 x 6, 1574 cells 7230 / 295; 5 x 16, 1417 cells 5430 / 233; 5 x 5, 4535 cells 599 / 351;
 // 3 x 3, 12597 cells 576 / 319; 5 x 2, 11337 cells 569 / 285; 4 x 12, 2362 cells 413 / 220.  A shape of more places than that kernel's
 // slots would lose (2 x 2 in 4 x 4, 4 x 5 in 8 x 8).
 bool bwd_padded_pays(int n1, int n2, int N1, int N2) {
@@ -696,7 +696,7 @@ int launch_fwd_shape(int n1, int n2, bool one_rowb, bool pad, const OnePairMfmaA
 }  // namespace
 
 // Both gradients of a non-Diag product of one x part with one y part, l1, l2 <= 15, for the channel counts listed in
-// GELIB_ONEPAIR_SHAPES.  *used = 1 if the launch was made; anything else is left to the other kernels.
+// GELIB_ONEPAIR_SHAPES and, where that pays, others up to 16 x 16 in the next larger of them.  *used = 1 if the launch was made; anything else is left to the other kernels.
 int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part_desc *> &g,
                          const std::vector<const gelib_part_desc *> &x, const std::vector<const gelib_part_desc *> &y,
                          const std::vector<const gelib_part_desc *> &xg, const std::vector<const gelib_part_desc *> &yg,
