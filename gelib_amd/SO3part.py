@@ -2,7 +2,7 @@
 complex64 -- the class and autograd functions of python/src/gelib/SO3part.py:22-220 for the CG product path."""
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch, output, without_torch_function
+from gelib_amd.gelib_common import backend, common_batch, output, packed, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 
 
@@ -89,7 +89,7 @@ class SO3part_CGproductFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         x, y = ctx.saved_tensors
-        g = g.contiguous()
+        g = packed(g)
         # both gradients from ONE pass over g (the vector-level backward on one-part vectors); the reference makes two
         # calls, each of which reads g.  An operand shared by the batch (extent 1) gets the sum over the batch, formed
         # inside the library in a fixed order.
@@ -117,7 +117,7 @@ class SO3part_DiagCGproductFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         x, y = ctx.saved_tensors
-        g = g.contiguous()
+        g = packed(g)
         xg = torch.zeros_like(x)
         yg = torch.zeros_like(y)
         _view(xg).add_DiagCGproduct_back0(_view(g), _view(y))

@@ -3,7 +3,7 @@ of python/src/gelib/SO3partArr.py:18-234 for the CG product path.  The grid dime
 as the grid dimensions of the part descriptor (core/Gpart.hpp:416-432, 495-531); nothing is reshaped or copied."""
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch, output, without_torch_function
+from gelib_amd.gelib_common import backend, common_batch, output, packed, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 from gelib_amd.SO3part import SO3part
 
@@ -108,7 +108,7 @@ def _part_fn(diag):
         @staticmethod
         def backward(ctx, g):
             x, y = ctx.saved_tensors
-            g = g.contiguous()
+            g = packed(g)
             xg = torch.zeros_like(x)
             yg = torch.zeros_like(y)
             getattr(_view(xg), "add_%s_back0" % name)(_view(g), _view(y))
@@ -150,7 +150,7 @@ def gathered_back(gmap, d, rgs):
         shape[1 + d] = gmap.d_in()
         xgs[i] = SO3partArr(torch.empty(shape, dtype=torch.complex64, device=rgs[i].device))
     if used:
-        backend().SO3part.set_gather([xgs[i] for i in used], [rgs[i].contiguous() for i in used], gmap.obj, d, True)
+        backend().SO3part.set_gather([xgs[i] for i in used], [packed(rgs[i]) for i in used], gmap.obj, d, True)
     return xgs
 
 

@@ -7,6 +7,7 @@ matrix; tensors on the host stay with torch."""
 import torch
 
 from gelib_amd.SO3type import SO3type
+from gelib_amd.gelib_common import packed
 
 
 class MixChannelsFn(torch.autograd.Function):
@@ -25,7 +26,7 @@ class MixChannelsFn(torch.autograd.Function):
         from gelib_amd import cabi
         x, w = ctx.saved_tensors
         gx = gw = None
-        g = g.contiguous()
+        g = packed(g)
         if ctx.needs_input_grad[0]:
             if cabi.mix_channels_ok(g):
                 gx = torch.empty_like(x)
@@ -43,8 +44,8 @@ def mix_channels(x, w):
     when the part is complex64 with an even number of channels, else torch's own matmul."""
     if x.is_cuda and x.dtype == torch.complex64 and w.dtype == torch.complex64 and w.dim() == 2 and x.numel() > 0:
         from gelib_amd import cabi
-        xp = x.as_subclass(torch.Tensor).contiguous()
-        wp = w.as_subclass(torch.Tensor).contiguous()
+        xp = packed(x.as_subclass(torch.Tensor))
+        wp = packed(w.as_subclass(torch.Tensor))
         if cabi.mix_channels_ok(xp):
             return MixChannelsFn.apply(xp, wp)
     return torch.matmul(x, w)
@@ -70,7 +71,7 @@ class MixPartsFn(torch.autograd.Function):
         k = ctx.k
         xs, ws = ctx.saved_tensors[:k], ctx.saved_tensors[k:]
         need = ctx.needs_input_grad[2:]
-        gs = [g.as_subclass(torch.Tensor).contiguous() for g in gs]
+        gs = [packed(g.as_subclass(torch.Tensor)) for g in gs]
         gx, gw = [None] * k, [None] * k
         if torch.is_grad_enabled():   # a graph of the gradients is wanted: torch's own operations
             for i, (x, w, g) in enumerate(zip(xs, ws, gs)):
@@ -105,8 +106,8 @@ def mix_parts(xs, ws):
             x.numel() > 0 and w.numel() > 0 and x.shape[-1] == w.shape[0] for x, w in pairs):
         odd = [x.shape[-1] % 2 != 0 for x, _ in pairs]
         classes = [type(x) if o else torch.Tensor for (x, _), o in zip(pairs, odd)]
-        xp = [x.as_subclass(torch.Tensor).contiguous() for x, _ in pairs]
-        wp = [w.as_subclass(torch.Tensor).contiguous() for _, w in pairs]
+        xp = [packed(x.as_subclass(torch.Tensor)) for x, _ in pairs]
+        wp = [packed(w.as_subclass(torch.Tensor)) for _, w in pairs]
         return list(MixPartsFn.apply(len(pairs), classes, *(xp + wp)))
     return [mix_channels(x, w) for x, w in pairs]
 
@@ -185,7 +186,7 @@ class CGproductLinearFn(torch.autograd.Function):
         saved = ctx.saved_tensors
         xs, ys, ws = list(saved[0:k1]), list(saved[k1:k1 + k2]), list(saved[k1 + k2:])
         need = ctx.needs_input_grad[3:]
-        gs = [g.contiguous() for g in gargs]
+        gs = [packed(g) for g in gargs]
         xg = [torch.empty_like(t, memory_format=torch.contiguous_format) for t in xs] if any(need[0:k1]) else None
         yg = [torch.empty_like(t, memory_format=torch.contiguous_format) for t in ys] if any(need[k1:k1 + k2]) else None
         wg = [torch.empty_like(t, memory_format=torch.contiguous_format) for t in ws] if any(need[k1 + k2:]) else None
@@ -255,7 +256,7 @@ class CGproductMixFn(torch.autograd.Function):
         saved = ctx.saved_tensors
         need = ctx.needs_input_grad[3:]
         args, P = list(saved[:len(need)]), list(saved[len(need):])
-        gs = [g.as_subclass(torch.Tensor).contiguous() for g in gargs]
+        gs = [packed(g.as_subclass(torch.Tensor)) for g in gargs]
         if torch.is_grad_enabled():   # a graph of the gradients is wanted
             grads = _two_step_grads(k1, k2, ctx.maxl, args, gs, need)
         else:
@@ -289,7 +290,7 @@ def mixed_product_ok(x, y, W, maxl):
     xs, ys, ws = list(x.parts.values()), list(y.parts.values()), list(W.parts)
     ts = xs + ys + ws
     if not xs or not ys or not ws or not all(t.is_cuda and t.dtype == torch.complex64 and t.is_contiguous() and
-                                             t.device == ts[0].device and t.numel() > 0 for t in ts):
+                                             not t.is_conj() and not t.is_neg() and t.device == ts[0].device and t.numel() > 0 for t in ts):
         return False
     if any(t.shape[:-2] != xs[0].shape[:-2] for t in xs + ys) or any(w.dim() != 2 for w in ws):
         return False

@@ -23,6 +23,14 @@ def output(shape, x, y):
     return make(shape, dtype=torch.complex64, device=x.device)
 
 
+def packed(t):
+    """t with its elements in memory as they read: contiguous, and no view that torch conjugates (or negates) on reading only, which
+    contiguous() leaves as it is (the gradient of out.conj().sum() is one)."""
+    if t.is_conj() or t.is_neg():
+        t = t.resolve_conj().resolve_neg()
+    return t.contiguous()
+
+
 def common_batch(x, y):
     assert x.dim() >= 1
     assert y.dim() >= 1

@@ -126,3 +126,32 @@ def test_matrix_gradient_from_strided_parts(cabi, nout):
         assert cabi.last_path() == 6
         out.append(wg)
     assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+def layer(cabi, n1, n2, out, b, L=2):
+    xs = [rand((b, 2 * l + 1, n1), l).requires_grad_() for l in range(L + 1)]
+    ys = [rand((b, 2 * l + 1, n2), 10 + l).requires_grad_() for l in range(L + 1)]
+    tau = cabi.so3type_product({l: n1 for l in range(L + 1)}, {l: n2 for l in range(L + 1)}, L)
+    return xs, ys, [(rand((n, out), 20 + l) / np.sqrt(n)).requires_grad_() for l, n in tau.items()]
+
+
+def near(got, want):
+    for a, c in zip(got, want):
+        a, c = a.detach().cpu().to(torch.complex128), c.detach().cpu().to(torch.complex128)
+        assert (a - c).norm() <= 2e-6 * c.norm()   # sums of up to a few hundred float32 terms, as above
+
+
+@pytest.mark.parametrize("n1,n2", [(3, 3), (4, 2)])
+def test_conjugate_views(cabi, n1, n2):
+    """Parts, matrices and gradients that torch conjugates on reading only: as their copies."""
+    import gelib_amd as gelib
+    xs, ys, ws = layer(cabi, n1, n2, 5, 20)
+
+    def run(conj):
+        out = gelib.CGproduct_linear(gelib.SO3vec(*xs), gelib.SO3vec(*ys), gelib.SO3weights(*[conj(w) for w in ws]), 2).parts.values()
+        mixed = (gelib.SO3vec(*[conj(x) for x in xs]) * gelib.SO3weights(*[conj(w)[:n1].contiguous() for w in ws])).parts.values()
+        rs = list(out) + list(mixed)
+        gs = [conj(rand(tuple(r.shape), 60 + k)) for k, r in enumerate(rs)]
+        return rs + list(torch.autograd.grad(rs, xs + ys + ws, gs))
+
+    near(run(lambda t: t.conj()), run(lambda t: t.conj().resolve_conj()))
