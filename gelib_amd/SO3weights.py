@@ -203,16 +203,18 @@ class CGproductLinearFn(torch.autograd.Function):
         return tuple([None, None, None] + _two_step_grads(k1, k2, ctx.maxl, saved, gs, need))
 
 
-def _two_step_grads(k1, k2, maxl, saved, gs, need):
-    """Gradients of the product followed by its matrices through the two separate autograd functions."""
+def _two_step_grads(k1, k2, maxl, saved, gs, need, graph=False):
+    """Gradients of the product followed by its matrices through the two separate autograd functions; graph: a graph of the
+    gradients themselves is wanted, back to the saved tensors and gs."""
     from gelib_amd.SO3vec import SO3vec
-    leaves = [t.detach().requires_grad_() for t in saved]
     with torch.enable_grad():
+        # (views, so that a tensor which is both operands has a gradient for each)
+        leaves = [t.view_as(t) if graph else t.detach().requires_grad_() for t in saved]
         x, y = SO3vec(*leaves[0:k1]), SO3vec(*leaves[k1:k1 + k2])
         out = x.CGproduct(y, maxl) * SO3weights(*leaves[k1 + k2:])
         outs = list(out.parts.values())
     wanted = [t for t, n in zip(leaves, need) if n]
-    got = iter(torch.autograd.grad(outs, wanted, gs))
+    got = iter(torch.autograd.grad(outs, wanted, gs, create_graph=graph))
     return [next(got) if n else None for n in need]
 
 
@@ -258,7 +260,7 @@ class CGproductMixFn(torch.autograd.Function):
         args, P = list(saved[:len(need)]), list(saved[len(need):])
         gs = [packed(g.as_subclass(torch.Tensor)) for g in gargs]
         if torch.is_grad_enabled():   # a graph of the gradients is wanted
-            grads = _two_step_grads(k1, k2, ctx.maxl, args, gs, need)
+            grads = _two_step_grads(k1, k2, ctx.maxl, args, gs, need, graph=True)
         else:
             grads = _mixed_product_grads(k1, k2, args[0:k1], args[k1:k1 + k2], args[k1 + k2:], P, gs, need)
         return tuple([None, None, None] + grads)

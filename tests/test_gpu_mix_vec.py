@@ -155,3 +155,22 @@ def test_conjugate_views(cabi, n1, n2):
         return rs + list(torch.autograd.grad(rs, xs + ys + ws, gs))
 
     near(run(lambda t: t.conj()), run(lambda t: t.conj().resolve_conj()))
+
+
+def test_graph_of_the_gradients(cabi):
+    """A function of the matrices' gradients is differentiated back to the operands and to the gradient of the result; one
+    vector is both operands."""
+    import gelib_amd as gelib
+    xs, _, _ = layer(cabi, 3, 3, 5, 20)
+    _, _, ws = layer(cabi, 3, 3, 5, 1)
+    gs = [rand((20, 2 * l + 1, 5), 40 + l).requires_grad_() for l in range(3)]
+    vs = [rand(tuple(w.shape), 70 + l) for l, w in enumerate(ws)]
+
+    def run(step):
+        rs = step(gelib.SO3vec(*xs))
+        first = torch.autograd.grad(rs, xs + ws, gs, create_graph=True)
+        return list(first) + list(torch.autograd.grad(first[3:], xs + gs, vs))
+
+    mixed = run(lambda x: list(gelib.CGproduct_linear(x, x, gelib.SO3weights(*ws), 2).parts.values()))
+    plain = run(lambda x: [torch.matmul(p.as_subclass(torch.Tensor), w) for p, w in zip(x.CGproduct(x, 2).parts.values(), ws)])
+    near(mixed, plain)
