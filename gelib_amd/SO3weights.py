@@ -94,8 +94,17 @@ class MixPartsFn(torch.autograd.Function):
 
 
 def plain_autograd():
-    """False inside forward-mode derivatives and function transforms, which only torch's own operations support."""
-    return torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+    """False inside forward-mode derivatives, function transforms, tracing and dispatch modes (shapes without data, counters of
+    operations), which only torch's own operations support."""
+    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and
+            torch._C._len_torch_dispatch_stack() == 0 and torch._C._get_tracing_state() is None and
+            not torch.compiler.is_compiling())
+
+
+def one_launch_holds(xs, ws):
+    """Do the tiles of all parts fit a launch of vec_mix_channels, in either direction (2^24 blocks of at least 64 rows and 32
+    columns)?  Rows beyond that stay with torch's product."""
+    return sum((x.numel() // w.shape[0] + 64) * (max(w.shape) // 32 + 1) for x, w in zip(xs, ws)) <= 1 << 30
 
 
 def mix_parts(xs, ws):
@@ -103,7 +112,7 @@ def mix_parts(xs, ws):
     pairs = list(zip(xs, ws))
     if pairs and plain_autograd() and all(
             x.is_cuda and w.is_cuda and x.device == w.device == xs[0].device and x.dtype == w.dtype == torch.complex64 and w.dim() == 2 and
-            x.numel() > 0 and w.numel() > 0 and x.shape[-1] == w.shape[0] for x, w in pairs):
+            x.numel() > 0 and w.numel() > 0 and x.shape[-1] == w.shape[0] for x, w in pairs) and one_launch_holds(xs, ws):
         odd = [x.shape[-1] % 2 != 0 for x, _ in pairs]
         classes = [type(x) if o else torch.Tensor for (x, _), o in zip(pairs, odd)]
         xp = [packed(x.as_subclass(torch.Tensor)) for x, _ in pairs]
@@ -303,7 +312,10 @@ def mixed_product_ok(x, y, W, maxl):
     if _one_channel_side(xs, ys) is not None and max(t.shape[-1] for t in xs + ys) > 64:
         return False   # (SO3vec.CGproduct repeats the channel there, and its backward pass is that of the Diag product)
     taus = cabi.so3type_product(x.tau(), y.tau(), maxl)
-    return [w.shape[0] for w in ws] == list(taus.values())
+    if [w.shape[0] for w in ws] != list(taus.values()):
+        return False
+    cells = xs[0].numel() // (xs[0].shape[-1] * xs[0].shape[-2])
+    return sum((cells * (2 * l + 1) + 64) * (max(w.shape) // 32 + 1) for l, w in zip(taus, ws)) <= 1 << 30   # one_launch_holds
 
 
 def CGproduct_linear(x, y, W, maxl=-1):

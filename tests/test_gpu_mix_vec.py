@@ -174,3 +174,15 @@ def test_graph_of_the_gradients(cabi):
     mixed = run(lambda x: list(gelib.CGproduct_linear(x, x, gelib.SO3weights(*ws), 2).parts.values()))
     plain = run(lambda x: [torch.matmul(p.as_subclass(torch.Tensor), w) for p, w in zip(x.CGproduct(x, 2).parts.values(), ws)])
     near(mixed, plain)
+
+
+def test_dispatch_modes_see_the_products(cabi):
+    """Counters of operations are shown torch's own products, with the same values."""
+    import gelib_amd as gelib
+    from torch.utils.flop_counter import FlopCounterMode
+    x, w = rand((6, 3, 5), 1), rand((5, 3), 2)
+    want = list((gelib.SO3vec(x) * gelib.SO3weights(w)).parts.values())
+    with FlopCounterMode(display=False) as counter:
+        got = list((gelib.SO3vec(x) * gelib.SO3weights(w)).parts.values())
+    assert counter.get_total_flops() > 0
+    near(got, want)
