@@ -702,7 +702,7 @@ __global__ void __launch_bounds__(256) wgrad_sum_kernel(const float *part, float
 namespace {
 struct WgradPlan {
   int ew, jt, u, tiles, jt_total, kgroups;
-  long long nranges, rows_per_range, pitch;
+  long long nranges, most_ranges, rows_per_range, pitch;
 };
 WgradPlan plan_wgrad(long long rows, int n_in, int n_out) {
   WgradPlan p;
@@ -716,7 +716,7 @@ WgradPlan plan_wgrad(long long rows, int n_in, int n_out) {
   // enough waves to fill the chip a few times over, every range a whole number of steps and not empty
   const long long waves_per_range = (long long)p.kgroups * (p.jt_total / p.jt);
   long long nranges = std::max<long long>(1, std::min<long long>(4096 / waves_per_range, rows / (8LL * p.u)));
-  nranges = std::min<long long>(nranges, 256);
+  nranges = p.most_ranges = std::min<long long>(nranges, 256);
   p.rows_per_range = ((rows + nranges - 1) / nranges + 2 * p.u - 1) / (2 * p.u) * (2 * p.u);
   p.nranges = (rows + p.rows_per_range - 1) / p.rows_per_range;
   p.pitch = 32LL * p.jt_total;
@@ -732,7 +732,9 @@ __global__ void zero_fill_kernel(float2 *p, long long n) {
 size_t mix_wgrad_workspace_bytes(long long rows, int n_in, int n_out) {
   if (rows <= 0 || n_in <= 0 || n_out <= 0) return 0;
   const WgradPlan p = plan_wgrad(rows, n_in, n_out);
-  return sizeof(float) * (size_t)(p.nranges * 2 * n_in * p.pitch);
+  // (for the number of ranges aimed at: whole steps can make more rows fewer ranges, 16384 rows 256 and 16385 rows 205, and memory
+  // for more rows has to do for fewer -- the last chunk of a batch)
+  return sizeof(float) * (size_t)(p.most_ranges * 2 * n_in * p.pitch);
 }
 
 // 0, 10, 11 or 13 as launch_mix; the workspace (mix_wgrad_workspace_bytes) holds the partial sums of the row ranges

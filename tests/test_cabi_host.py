@@ -192,3 +192,20 @@ def test_o3_parts_without_channels_take_part_in_the_checks():
     assert status(0, vec(0), vec(2), vec(3)) == 5          # no room for the block
     assert status(0, vec(0), vec(0), vec(0, b=3)) == 6     # batches differ
     assert status(0, vec(0), vec(0), vec(0)) == 0 and status(1, vec(0), vec(0), vec(0)) == 0
+
+
+def test_less_work_asks_for_no_more_workspace():
+    """The last chunk of a batch runs in the memory that was asked for a full one."""
+    L = cabi.lib()
+    A = cabi.PartDesc * 1
+    for nout, chunks in ((4, (16000, 16384, 16385)),):
+        n = 16 if nout == 8192 else 2
+        x, y, g = A(fake(1 << 20, 1, 2)), A(fake(1 << 20, 1, n)), A(fake(1 << 20, 1, nout))
+        need = [L.gelib_hip_so3vec_cg_linear_bwd_workspace_bytes(1, g, 1, x, 1, y, c) for c in chunks]
+        assert need[0] > 0 and need == sorted(need), (nout, need)
+
+
+@pytest.mark.parametrize("n_in,n_out", [(2, 2), (4, 16), (32, 20), (128, 128)])
+def test_fewer_rows_ask_for_no_more_workspace(n_in, n_out):
+    need = [cabi.lib().gelib_hip_part_mix_workspace_bytes(1, rows, n_in, n_out) for rows in range(1, 40000, 7)]
+    assert need == sorted(need)

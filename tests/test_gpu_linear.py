@@ -423,3 +423,29 @@ def test_where_matrix_gradients_come_straight_from_the_operands(cabi, B, n1, n2,
         finally:
             cabi.set_option("linear_wgrad", 1)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("cb,nout", [(16385, 4)])
+def test_last_chunk_is_a_little_shorter(cabi, cb, nout):
+    """Two chunks of the batch whose second is one entry shorter than the workspace was asked for, where one entry less means more
+    pieces of the sums over the rows: the call goes through, writing and adding."""
+    import ctypes
+    B = 2 * cb - 1
+    gen = torch.Generator(device="cuda").manual_seed(cb)
+    rand = lambda *shape: torch.view_as_complex(torch.randn(*shape, 2, device="cuda", generator=gen))
+    x, y, w, g = rand(B, 1, 2), rand(B, 1, 2), rand(4, nout), rand(B, 1, nout)
+    need = int(cabi.lib().gelib_hip_so3vec_cg_linear_bwd_workspace_bytes(1, cabi._arr([g]), 1, cabi._arr([x]), 1, cabi._arr([y]), cb))
+    whole = int(cabi.lib().gelib_hip_so3vec_cg_linear_bwd_workspace_bytes(1, cabi._arr([g]), 1, cabi._arr([x]), 1, cabi._arr([y]), 0))
+    assert need < whole
+    x8, y8, w8, g8 = (t.to(torch.complex128) for t in (x[:, 0], y[:, 0], w, g[:, 0]))
+    P = (x8[:, :, None] * y8[:, None, :]).reshape(B, 4)
+    gP = torch.matmul(g8, w8.conj().T).reshape(B, 2, 2)
+    want = [(gP * y8.conj()[:, None, :]).sum(2), (gP * x8.conj()[:, :, None]).sum(1), torch.matmul(P.conj().T, g8)]
+    start = [rand(B, 1, 2), rand(B, 1, 2), rand(4, nout)]
+    for add in (False, True):
+        got = [t.clone() for t in start]
+        assert cabi.so3vec_cg_linear_bwd([got[0]], [got[1]], [got[2]], [g], [x], [y], [w], accumulate=add, workspace_bytes=need)
+        for a, s, e in zip(got, start, want):
+            d = a.to(torch.complex128) - (s.to(torch.complex128) if add else 0)
+            # sums of at most 65537 float32 terms in ranges of a few hundred, rounded randomly: a missing range is 1e-2
+            assert (d.reshape(e.shape) - e).norm() <= 4e-6 * e.norm() + (1e-7 * s.norm() if add else 0)
