@@ -1219,9 +1219,10 @@ size_t vec_mix_bytes(const VecMixSets &v) {
   return std::max({v.matrix_bytes, vec_mix_workspace_bytes(v.rest), vec_mix_workspace_bytes(v.all)});
 }
 
-// r_k = x_k w_k and its gradients for all parts, shapes and pointers checked by the caller
+// r_k = x_k w_k and its gradients for all parts, shapes and pointers checked by the caller.  fit: as in launch_vec_mix (what mix.hip's
+// kernels need does not depend on the rows).
 int vec_mix_run(int nparts, void *const *r, const void *const *x, const void *const *w, const int64_t *rows, const int *n_in,
-                const int *n_out, int kind, void *ws, size_t ws_bytes, hipStream_t s) {
+                const int *n_out, int kind, void *ws, size_t ws_bytes, bool fit, hipStream_t s) {
   const VecMixSets v = vec_mix_sets(nparts, r, x, w, rows, n_in, n_out, kind);
   bool aligned = true;
   for (int k : v.matrix) aligned = aligned && ((uintptr_t)x[k] & 15) == 0;
@@ -1236,7 +1237,7 @@ int vec_mix_run(int nparts, void *const *r, const void *const *x, const void *co
                         n_out[k], kind == kVMAdjoint, (float *)ws, ws_bytes, s);
       if (rc) return rc == 11 ? GELIB_HIP_ERR_ARG : rc;
     }
-  rc = launch_vec_mix(aligned ? v.rest : v.all, kind, ws, ws_bytes, s);
+  rc = launch_vec_mix(aligned ? v.rest : v.all, kind, ws, ws_bytes, fit, s);
   return rc == 11 ? GELIB_HIP_ERR_ARG : rc;
 }
 
@@ -1263,13 +1264,6 @@ size_t lin_bwd_bytes(const LinBwdShape &sh, long long cb, size_t *p_bytes, size_
     mb = std::max(mb, mix_workspace_bytes(sh.G[k].n, (int)sh.tau[k]));
     wb = std::max(wb, mix_wgrad_workspace_bytes(rows, (int)sh.tau[k], sh.G[k].n));
     tb = std::max(tb, (size_t)sh.tau[k] * sh.G[k].n * sizeof(float2));
-  }
-  {
-    const int n = (int)sh.G.size();
-    std::vector<int64_t> rows(n);
-    std::vector<int> tau(n), nout(n);
-    for (int k = 0; k < n; k++) rows[k] = cb * sh.G01 * (2 * sh.G[k].l + 1), tau[k] = (int)sh.tau[k], nout[k] = sh.G[k].n;
-    mb = std::max(mb, vec_mix_bytes(vec_mix_sets(n, nullptr, nullptr, nullptr, rows.data(), nout.data(), tau.data(), kVMAdjoint)));
   }
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   if (p_bytes) *p_bytes = pb;
@@ -1425,7 +1419,7 @@ int linear_bwd_entry(const gelib_part_desc *xg, const gelib_part_desc *yg, void 
       }
     }
     if ((xg || yg) && packed) {
-      rc = vec_mix_run(np, pp.data(), gp.data(), wp.data(), rows.data(), nout.data(), tau.data(), kVMAdjoint, mix_ws, mb, s);
+      rc = vec_mix_run(np, pp.data(), gp.data(), wp.data(), rows.data(), nout.data(), tau.data(), kVMAdjoint, mix_ws, mb, true, s);
       if (rc) return rc;
     } else if (xg || yg) {
       for (int k = 0; k < np; k++) {
@@ -1850,7 +1844,7 @@ int gelib_hip_vec_mix_channels(int nparts, void *const *r, const void *const *x,
   const int64_t sd[5] = {(int64_t)workspace_bytes, 1, 1, 1, 1}, sst[5] = {1, 0, 0, 0, 0};
   if (workspace && workspace_bytes && (rc = check_range(workspace, sd, sst, 1))) return rc;
   t_last_path = kPathGeneric;
-  return vec_mix_run(nparts, r, x, w, rows, n_in, n_out, kind, workspace, (size_t)workspace_bytes, (hipStream_t)stream);
+  return vec_mix_run(nparts, r, x, w, rows, n_in, n_out, kind, workspace, (size_t)workspace_bytes, false, (hipStream_t)stream);
 }
 
 int gelib_hip_set_stream_workspace(void *stream, void *ptr, uint64_t bytes) {

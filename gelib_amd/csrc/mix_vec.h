@@ -18,9 +18,11 @@ struct VecMixPart {
   long long m, n, k;
 };
 
-// Bytes for the partial results of parts with few tiles (pointers are not looked at).
+// Bytes for the partial results of parts with few tiles (pointers are not looked at).  Fewer rows can need more: fewer tiles are cut
+// into more pieces.
 size_t vec_mix_workspace_bytes(const std::vector<VecMixPart> &parts);
-// 0, 10, 11 (more tiles than a launch holds) or 13 (workspace).  Parts with k = 0 are left to the caller.
-int launch_vec_mix(const std::vector<VecMixPart> &parts, int mode, void *ws, size_t ws_bytes, hipStream_t s);
+// 0, 10, 11 (more tiles than a launch holds) or 13 (workspace).  Parts with k = 0 are left to the caller.  fit: no more pieces than
+// ws_bytes has room for, so that any size will do.
+int launch_vec_mix(const std::vector<VecMixPart> &parts, int mode, void *ws, size_t ws_bytes, bool fit, hipStream_t s);
 
 }  // namespace gelib_hip

@@ -14,6 +14,7 @@
 // What bounds it: small calls the latency of the steps (about 1 us each), large ones the vector unit at a third of its rate
 // (LDS reads and the address arithmetic beside the multiply-adds), the gradient of the product the stores.
 #include <algorithm>
+#include <cstdint>
 #include <cstring>
 #include <vector>
 
@@ -190,8 +191,8 @@ VMShape shape_of(const std::vector<VecMixPart> &parts) {
   return {16, 2, 4};
 }
 
-// the launch's blocks and the pieces of k of every part; false: too many blocks
-bool plan(const std::vector<VecMixPart> &parts, const VMShape &sh, std::vector<VMPart> *out, long long *blocks, size_t *bytes) {
+// the launch's blocks and the pieces of k of every part, as many as their partial results have room for; false: too many blocks
+bool plan(const std::vector<VecMixPart> &parts, const VMShape &sh, size_t room, std::vector<VMPart> *out, long long *blocks, size_t *bytes) {
   out->clear();
   long long tiles = 0;
   for (auto &p : parts) {
@@ -210,7 +211,9 @@ bool plan(const std::vector<VecMixPart> &parts, const VMShape &sh, std::vector<V
   size_t off = 0;
   for (auto &q : *out) {
     const long long want = std::max<long long>(1, kVMBlocks / std::max<long long>(1, tiles));
-    long long s = std::max<long long>(1, std::min<long long>({want, q.k / (8 * kVMK), (long long)kVMSplits}));
+    const size_t piece = (size_t)q.m * q.n * sizeof(float2);
+    const long long fit = (long long)(((room - off) & ~(size_t)255) / piece);
+    long long s = std::max<long long>(1, std::min<long long>({want, q.k / (8 * kVMK), (long long)kVMSplits, fit}));
     q.per = ((q.k + s - 1) / s + kVMK - 1) / kVMK * kVMK;
     s = (q.k + q.per - 1) / q.per;
     q.splits = (int)s;
@@ -218,7 +221,7 @@ bool plan(const std::vector<VecMixPart> &parts, const VMShape &sh, std::vector<V
     first += (long long)q.mtiles * q.ntiles * s;
     if (s > 1) {
       q.part = (float2 *)off;   // the offset for now
-      off += ((size_t)s * q.m * q.n * sizeof(float2) + 255) & ~(size_t)255;
+      off += (s * piece + 255) & ~(size_t)255;
     }
   }
   *blocks = first;
@@ -254,19 +257,19 @@ size_t vec_mix_workspace_bytes(const std::vector<VecMixPart> &parts) {
     std::vector<VMPart> q;
     long long blocks = 0;
     size_t bytes = 0;
-    plan(g, shape_of(g), &q, &blocks, &bytes);
+    plan(g, shape_of(g), SIZE_MAX, &q, &blocks, &bytes);
     most = std::max(most, bytes);
   }
   return most;
 }
 
-int launch_vec_mix(const std::vector<VecMixPart> &parts, int mode, void *ws, size_t ws_bytes, hipStream_t s) {
+int launch_vec_mix(const std::vector<VecMixPart> &parts, int mode, void *ws, size_t ws_bytes, bool fit, hipStream_t s) {
   for (auto &g : groups_of(parts)) {
     const VMShape sh = shape_of(g);
     std::vector<VMPart> q;
     long long blocks = 0;
     size_t bytes = 0;
-    if (!plan(g, sh, &q, &blocks, &bytes)) return 11;
+    if (!plan(g, sh, fit ? ws_bytes : SIZE_MAX, &q, &blocks, &bytes)) return 11;
     if (bytes && (!ws || ((uintptr_t)ws & 15) || ws_bytes < bytes)) return 13;
     VMArgs a;
     std::memset(&a, 0, sizeof(a));

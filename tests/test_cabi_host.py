@@ -198,7 +198,7 @@ def test_less_work_asks_for_no_more_workspace():
     """The last chunk of a batch runs in the memory that was asked for a full one."""
     L = cabi.lib()
     A = cabi.PartDesc * 1
-    for nout, chunks in ((4, (16000, 16384, 16385)),):
+    for nout, chunks in ((256, (100, 65536, 65537)), (4, (16000, 16384, 16385)), (8192, (512, 2048, 32768, 65536))):
         n = 16 if nout == 8192 else 2
         x, y, g = A(fake(1 << 20, 1, 2)), A(fake(1 << 20, 1, n)), A(fake(1 << 20, 1, nout))
         need = [L.gelib_hip_so3vec_cg_linear_bwd_workspace_bytes(1, g, 1, x, 1, y, c) for c in chunks]

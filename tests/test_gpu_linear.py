@@ -425,10 +425,10 @@ def test_where_matrix_gradients_come_straight_from_the_operands(cabi, B, n1, n2,
     torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("cb,nout", [(16385, 4)])
+@pytest.mark.parametrize("cb,nout", [(65537, 256), (16385, 4)])
 def test_last_chunk_is_a_little_shorter(cabi, cb, nout):
     """Two chunks of the batch whose second is one entry shorter than the workspace was asked for, where one entry less means more
-    pieces of the sums over the rows: the call goes through, writing and adding."""
+    pieces of the sums over the outputs (256) and of those over the rows (4): the call goes through, writing and adding."""
     import ctypes
     B = 2 * cb - 1
     gen = torch.Generator(device="cuda").manual_seed(cb)
