@@ -12,7 +12,7 @@ import functools
 
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch, packed, without_torch_function
+from gelib_amd.gelib_common import backend, common_batch, packed, resolved, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 
 
@@ -174,6 +174,7 @@ def _vec_fn(diag):
         def forward(ctx, xmus, ymus, maxl, *args):
             gb = backend()
             k1 = len(xmus)
+            args = resolved(*args)
             xs, ys = args[:k1], args[k1:]
             tau = getattr(O3type({mu: t.size(-1) for mu, t in zip(xmus, xs)}), name)(
                 O3type({mu: t.size(-1) for mu, t in zip(ymus, ys)}), maxl)

@@ -2,7 +2,7 @@
 complex64 -- the class and autograd functions of python/src/gelib/SO3part.py:22-220 for the CG product path."""
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch, output, packed, without_torch_function
+from gelib_amd.gelib_common import backend, common_batch, output, packed, resolved, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 
 
@@ -21,6 +21,7 @@ class SO3part(torch.Tensor):
         """Spherical harmonics of the vectors (x, y, z) in X, shaped (b, 3, n) float32
         (python/src/gelib/SO3part.py:55-62)."""
         assert X.dim() == 3
+        X, = resolved(X)
         R = SO3part(torch.empty([X.size(0), 2 * l + 1, X.size(2)], dtype=torch.complex64, device=X.device))
         R.backend().set_spharm(X)
         return R
@@ -80,6 +81,7 @@ class SO3part_CGproductFn(torch.autograd.Function):
     @without_torch_function
     def forward(ctx, x, y, l):
         ctx.l = l
+        x, y = resolved(x, y)
         ctx.save_for_backward(x, y)
         b = common_batch(x, y)
         r = SO3part(output([b, 2 * l + 1, x.size(-1) * y.size(-1)], x, y))
@@ -107,6 +109,7 @@ class SO3part_DiagCGproductFn(torch.autograd.Function):
     @without_torch_function
     def forward(ctx, x, y, l):
         ctx.l = l
+        x, y = resolved(x, y)
         ctx.save_for_backward(x, y)
         b = common_batch(x, y)
         assert x.size(-1) == y.size(-1)

@@ -3,7 +3,7 @@ of python/src/gelib/SO3partArr.py:18-234 for the CG product path.  The grid dime
 as the grid dimensions of the part descriptor (core/Gpart.hpp:416-432, 495-531); nothing is reshaped or copied."""
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch, output, packed, without_torch_function
+from gelib_amd.gelib_common import backend, common_batch, output, packed, resolved, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 from gelib_amd.SO3part import SO3part
 
@@ -27,6 +27,7 @@ class SO3partArr(torch.Tensor):
         """Spherical harmonics of the vectors (x, y, z) in X, shaped (b, a_1..a_k, 3, n) float32
         (python/src/gelib/SO3partArr.py:59-67)."""
         assert X.size(-2) == 3
+        X, = resolved(X)
         R = SO3partArr.zeros(X.size(0), list(X.size())[1:X.dim() - 2], l, X.size(-1), device=X.device)
         R.backend().add_spharm(X)
         return R
@@ -94,11 +95,13 @@ def _part_fn(diag):
     class Fn(torch.autograd.Function):
 
         @staticmethod
+        @without_torch_function
         def forward(ctx, x, y, l):
             ctx.l = l
+            x, y = resolved(x, y)
             ctx.save_for_backward(x, y)
             b = common_batch(x, y)
-            a = x.get_adims() if isinstance(x, SO3partArr) else list(x.size()[1:x.dim() - 2])
+            a = list(x.size()[1:x.dim() - 2])
             if diag:
                 assert x.size(-1) == y.size(-1)
             r = SO3partArr(output([b] + list(a) + [2 * l + 1, x.size(-1) if diag else x.size(-1) * y.size(-1)], x, y))
@@ -136,7 +139,7 @@ def gathered(gmap, d, xs):
         assert adims[d] == gmap.d_in()
         shape[1 + d] = gmap.d_out()
         rs.append(SO3partArr(torch.empty(shape, dtype=torch.complex64, device=x.device)))
-    backend().SO3part.set_gather(rs, list(xs), gmap.obj, d, False)
+    backend().SO3part.set_gather(rs, list(resolved(*xs)), gmap.obj, d, False)
     return rs
 
 

@@ -4,7 +4,7 @@ forward writes into uninitialised parts and the backward computes both gradients
 import torch
 
 from gelib_amd.SO3weights import mix_parts
-from gelib_amd.gelib_common import backend, common_batch, packed, without_torch_function
+from gelib_amd.gelib_common import backend, common_batch, packed, resolved, without_torch_function
 from gelib_amd.SO3part import SO3part
 
 
@@ -139,6 +139,7 @@ def _product_fn(diag, part_cls=SO3part, prefix="SO3vec"):
         def forward(ctx, k1, k2, maxl, *args):
             gb = backend()
             ctx.k1, ctx.k2 = k1, k2
+            args = resolved(*args)
             ctx.save_for_backward(*args)
             x = gb.SO3vec.view(list(args[0:k1]))
             y = gb.SO3vec.view(list(args[k1:k1 + k2]))

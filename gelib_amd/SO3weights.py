@@ -7,7 +7,7 @@ matrix; tensors on the host stay with torch."""
 import torch
 
 from gelib_amd.SO3type import SO3type
-from gelib_amd.gelib_common import packed
+from gelib_amd.gelib_common import packed, resolved
 
 
 class MixChannelsFn(torch.autograd.Function):
@@ -301,7 +301,7 @@ def mixed_product_ok(x, y, W, maxl):
     xs, ys, ws = list(x.parts.values()), list(y.parts.values()), list(W.parts)
     ts = xs + ys + ws
     if not xs or not ys or not ws or not all(t.is_cuda and t.dtype == torch.complex64 and t.is_contiguous() and
-                                             not t.is_conj() and not t.is_neg() and t.device == ts[0].device and t.numel() > 0 for t in ts):
+                                             t.device == ts[0].device and t.numel() > 0 for t in ts):
         return False
     if any(t.shape[:-2] != xs[0].shape[:-2] for t in xs + ys) or any(w.dim() != 2 for w in ws):
         return False
@@ -330,7 +330,5 @@ def CGproduct_linear(x, y, W, maxl=-1):
         fn = CGproductMixFn
     else:
         return x.CGproduct(y, maxl) * W
-    xs = [p.as_subclass(torch.Tensor) for p in x.parts.values()]
-    ys = [p.as_subclass(torch.Tensor) for p in y.parts.values()]
-    ws = [w.as_subclass(torch.Tensor) for w in W.parts]
-    return SO3vec(*fn.apply(len(xs), len(ys), maxl, *(xs + ys + ws)))
+    ts = resolved(*[t.as_subclass(torch.Tensor) for t in (*x.parts.values(), *y.parts.values(), *W.parts)])
+    return SO3vec(*fn.apply(len(x.parts), len(y.parts), maxl, *ts))

@@ -15,8 +15,14 @@ using namespace GElib;
 
 typedef cnine::TensorView<std::complex<float>> tensorc;
 
+// The kernels read the memory behind a tensor, so a view that torch conjugates or negates on reading only is refused.
+static void check_in_memory(const at::Tensor &x) {
+  TORCH_CHECK(!x.is_conj() && !x.is_neg(), "GElib: a view that is conjugated or negated on reading: resolve_conj() / resolve_neg() first");
+}
+
 // zero-copy view of a complex64 tensor; dev 0 = host, 1 = GPU
 static tensorc view_of(const at::Tensor &x) {
+  check_in_memory(x);
   TORCH_CHECK(x.scalar_type() == at::kComplexFloat, "GElib: SO3parts are complex64 tensors");
   cnine::Gdims dims;
   std::vector<size_t> strides;
@@ -59,6 +65,7 @@ static SO3vec<float> vec_of(const std::vector<at::Tensor> &parts) {
 }
 
 static void spharm(SO3part<float> &r, const at::Tensor &X, const int accumulate) {
+  check_in_memory(X);
   TORCH_CHECK(X.scalar_type() == at::kFloat, "GElib: add_spharm takes a float32 tensor of (x, y, z) vectors");
   cnine::Gdims dims;
   std::vector<size_t> strides;
@@ -213,7 +220,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def("__repr__", &SO3part<float>::repr);
 
   // value-returning product of two parts; the result is a fresh torch tensor
-  m.def("CGproduct", [](at::Tensor &x, at::Tensor &y, const int l) {
+  m.def("CGproduct", [](const at::Tensor &x_, const at::Tensor &y_, const int l) {
+    const at::Tensor x = x_.resolve_conj().resolve_neg(), y = y_.resolve_conj().resolve_neg();
     SO3part<float> X(view_of(x)), Y(view_of(y));
     GELIB_ASSRT(SO3group::CGmultiplicity(X.getl(), Y.getl(), l) > 0);
     std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());

@@ -124,23 +124,28 @@ def check(status):
         raise GelibHipError(status, msg)
 
 
+def _in_memory(*ts):
+    """Refuses views that torch conjugates or negates on reading only: the library reads the memory behind them."""
+    for t in ts:
+        if t.is_conj() or t.is_neg():
+            raise ValueError("a view that is conjugated or negated on reading: resolve_conj() / resolve_neg() first")
+
+
 def desc(t):
     """5-D descriptor of a complex64 tensor shaped (b, [g0, [g1]], 2l+1, n)."""
     import torch
+    if t.is_conj() or t.is_neg():
+        _in_memory(t)
     if t.dtype != torch.complex64:
         raise TypeError("SO3parts are complex64 tensors")
-    if t.dim() < 3 or t.dim() > 5:
+    shape, strides = tuple(t.shape), t.stride()
+    k = len(shape) - 3
+    if k < 0 or k > 2:
         raise ValueError("an SO3part view has 3 to 5 dimensions (batch, [grid], 2l+1, channels)")
     d = PartDesc()
     d.ptr = t.data_ptr() if t.numel() > 0 else None
-    shape = list(t.shape)
-    strides = list(t.stride())
-    k = t.dim() - 3
-    dims = [shape[0]] + shape[1:1 + k] + [1] * (2 - k) + shape[-2:]
-    strs = [strides[0]] + strides[1:1 + k] + [0] * (2 - k) + strides[-2:]
-    for i in range(5):
-        d.dims[i] = dims[i]
-        d.strides[i] = strs[i]
+    d.dims[:] = shape[:1 + k] + (1, 1)[k:] + shape[-2:]
+    d.strides[:] = strides[:1 + k] + (0, 0)[k:] + strides[-2:]
     return d
 
 
@@ -248,6 +253,7 @@ def so3vec_cg_linear_fwd(rparts, xparts, yparts, wparts, accumulate=False):
     if nbytes == 0:
         return False
     ws = torch.empty(nbytes, dtype=torch.uint8, device=rparts[0].device)
+    _in_memory(*wparts)
     wp = (ctypes.c_void_p * len(wparts))(*[w.data_ptr() for w in wparts])
     rc = L.gelib_hip_so3vec_cg_linear_fwd(len(rparts), ra, len(xparts), xa, len(yparts), ya, wp, int(accumulate),
                                           ctypes.c_void_p(ws.data_ptr()), nbytes, _stream(rparts[0]))
@@ -274,6 +280,7 @@ def so3vec_cg_linear_bwd(xgparts, ygparts, wgparts, gparts, xparts, yparts, wpar
     nbytes = whole if whole <= workspace_bytes else max(one, workspace_bytes)
     ws = torch.empty(nbytes + 256, dtype=torch.uint8, device=gparts[0].device)
     base = (ws.data_ptr() + 255) & ~255
+    _in_memory(*wparts, *(wgparts or ()))
     wp = (ctypes.c_void_p * len(wparts))(*[w.data_ptr() for w in wparts])
     wgp = (ctypes.c_void_p * len(wgparts))(*[w.data_ptr() for w in wgparts]) if wgparts is not None else None
     rc = L.gelib_hip_so3vec_cg_linear_bwd(_arr(xgparts), _arr(ygparts), wgp, len(gparts), ga, len(xparts), xa, len(yparts),
@@ -301,6 +308,7 @@ def set_stream_workspace(buf, stream=None):
 def so3part_spharm(r, x, accumulate=True):
     """r (b, [grid], 2l+1, n) complex64 (+)= spherical harmonics of the float32 vectors x (b or 1, [grid], 3, n)."""
     import torch
+    _in_memory(x)
     if x.dtype != torch.float32:
         raise TypeError("the vectors are float32")
     if x.dim() != r.dim() or x.size(-2) != 3:
@@ -361,6 +369,7 @@ def mix_workspace(kind, rows, n_in, n_out, device):
 def part_mix_channels(r, x, w, adjoint=False):
     """r[..., o] = sum_c x[..., c] V[c, o] with V = w (n_in, n_out), or V = w^H for w (n_out, n_in) when adjoint.
     r and x are contiguous complex64 tensors that differ only in their last extent."""
+    _in_memory(r, x, w)
     n_in, n_out = x.shape[-1], r.shape[-1]
     if tuple(w.shape) != ((n_out, n_in) if adjoint else (n_in, n_out)) or r.shape[:-1] != x.shape[:-1]:
         raise ValueError("shapes of r, x and w do not fit")
@@ -374,6 +383,7 @@ def part_mix_channels(r, x, w, adjoint=False):
 
 def part_mix_channels_wgrad(wg, x, g):
     """wg (n_in, n_out) = sum over the leading indices of conj(x[..., c]) g[..., o] for contiguous complex64 tensors."""
+    _in_memory(wg, x, g)
     n_in, n_out = x.shape[-1], g.shape[-1]
     if tuple(wg.shape) != (n_in, n_out) or g.shape[:-1] != x.shape[:-1]:
         raise ValueError("shapes of wg, x and g do not fit")
@@ -391,6 +401,7 @@ def vec_mix_channels(rs, xs, ws, kind):
     to the part; kind 2: r[c, o] = sum over the leading indices of conj(x[..., c]) w[..., o], the gradient with respect to
     the matrix (w: the gradient of the result)."""
     import torch
+    _in_memory(*rs, *xs, *ws)
     k = len(rs)
     n_in = [x.shape[-1] for x in xs]
     n_out = [r.shape[-1] for r in rs]

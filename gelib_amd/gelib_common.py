@@ -31,6 +31,15 @@ def packed(t):
     return t.contiguous()
 
 
+def resolved(*ts):
+    """ts with copies in place of views that torch conjugates (or negates) on reading only: kernels read memory.  (Called with the
+    __torch_function__ hooks off, or on plain tensors.)"""
+    for t in ts:
+        if t.is_conj() or t.is_neg():
+            return tuple(t.resolve_conj().resolve_neg() for t in ts)
+    return ts
+
+
 def common_batch(x, y):
     assert x.dim() >= 1
     assert y.dim() >= 1
