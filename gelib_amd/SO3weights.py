@@ -60,6 +60,7 @@ class MixPartsFn(torch.autograd.Function):
         from gelib_amd import cabi
         xs, ws = list(args[:k]), list(args[k:])
         ctx.k = k
+        ctx.set_materialize_grads(False)   # parts that a loss does not use get no gradients
         ctx.save_for_backward(*args)
         rs = [torch.empty(x.shape[:-1] + w.shape[1:], dtype=x.dtype, device=x.device) for x, w in zip(xs, ws)]
         cabi.vec_mix_channels(rs, xs, ws, 0)
@@ -71,21 +72,23 @@ class MixPartsFn(torch.autograd.Function):
         k = ctx.k
         xs, ws = ctx.saved_tensors[:k], ctx.saved_tensors[k:]
         need = ctx.needs_input_grad[2:]
-        gs = [packed(g.as_subclass(torch.Tensor)) for g in gs]
+        gs = [None if g is None else packed(g.as_subclass(torch.Tensor)) for g in gs]
         gx, gw = [None] * k, [None] * k
         if torch.is_grad_enabled():   # a graph of the gradients is wanted: torch's own operations
             for i, (x, w, g) in enumerate(zip(xs, ws, gs)):
+                if g is None:
+                    continue
                 if need[i]:
                     gx[i] = torch.matmul(g, w.conj().transpose(0, 1))
                 if need[k + i]:
                     gw[i] = torch.matmul(x.reshape(-1, x.shape[-1]).conj().transpose(0, 1), g.reshape(-1, g.shape[-1]))
             return tuple([None, None] + gx + gw)
-        todo = [i for i in range(k) if need[i]]
+        todo = [i for i in range(k) if need[i] and gs[i] is not None]
         if todo:
             for i in todo:
                 gx[i] = torch.empty_like(xs[i])
             cabi.vec_mix_channels([gx[i] for i in todo], [gs[i] for i in todo], [ws[i] for i in todo], 1)
-        todo = [i for i in range(k) if need[k + i]]
+        todo = [i for i in range(k) if need[k + i] and gs[i] is not None]
         if todo:
             for i in todo:
                 gw[i] = torch.empty_like(ws[i])
@@ -213,33 +216,36 @@ class CGproductLinearFn(torch.autograd.Function):
 
 
 def _two_step_grads(k1, k2, maxl, saved, gs, need, graph=False):
-    """Gradients of the product followed by its matrices through the two separate autograd functions; graph: a graph of the
-    gradients themselves is wanted, back to the saved tensors and gs."""
+    """Gradients of the product followed by its matrices through the two separate autograd functions; gs: None for a result that is
+    not used; graph: a graph of the gradients themselves is wanted, back to the saved tensors and gs."""
     from gelib_amd.SO3vec import SO3vec
     with torch.enable_grad():
         # (views, so that a tensor which is both operands has a gradient for each)
         leaves = [t.view_as(t) if graph else t.detach().requires_grad_() for t in saved]
         x, y = SO3vec(*leaves[0:k1]), SO3vec(*leaves[k1:k1 + k2])
         out = x.CGproduct(y, maxl) * SO3weights(*leaves[k1 + k2:])
-        outs = list(out.parts.values())
+        outs = [(o, g) for o, g in zip(out.parts.values(), gs) if g is not None]
     wanted = [t for t, n in zip(leaves, need) if n]
-    got = iter(torch.autograd.grad(outs, wanted, gs, create_graph=graph))
+    got = iter(torch.autograd.grad([o for o, _ in outs], wanted, [g for _, g in outs], create_graph=graph, allow_unused=True))
     return [next(got) if n else None for n in need]
 
 
 def _mixed_product_grads(k1, k2, xs, ys, ws, P, gs, need):
     """Gradients of P_l W_l with P = CGproduct(x, y) at hand: the matrices' in one call, the product's in one, and the product's
-    backward pass."""
+    backward pass.  gs: None for a result that is not used, whose matrix gets no gradient and whose part of the product a zero one."""
     from gelib_amd import cabi
     from gelib_amd.SO3vec import SO3vec_CGproductFn
+    used = [i for i, g in enumerate(gs) if g is not None]
     wg = [None] * len(ws)
-    if any(need[k1 + k2:]):
-        wg = [torch.empty_like(w) for w in ws]
-        cabi.vec_mix_channels(wg, P, gs, 2)
+    todo = [i for i in used if need[k1 + k2 + i]]
+    if todo:
+        for i in todo:
+            wg[i] = torch.empty_like(ws[i])
+        cabi.vec_mix_channels([wg[i] for i in todo], [P[i] for i in todo], [gs[i] for i in todo], 2)
     xyg = [None] * (k1 + k2)
     if any(need[0:k1 + k2]):
-        gP = [torch.empty_like(p) for p in P]
-        cabi.vec_mix_channels(gP, gs, ws, 1)
+        gP = [torch.zeros_like(p) if g is None else torch.empty_like(p) for p, g in zip(P, gs)]
+        cabi.vec_mix_channels([gP[i] for i in used], [gs[i] for i in used], [ws[i] for i in used], 1)
         xyg = SO3vec_CGproductFn.grads(k1, k2, xs + ys, gP, need)
     return [g if n else None for g, n in zip(list(xyg) + wg, need)]
 
@@ -255,6 +261,7 @@ class CGproductMixFn(torch.autograd.Function):
         from gelib_amd.SO3vec import SO3vec
         xs, ys, ws = list(args[0:k1]), list(args[k1:k1 + k2]), list(args[k1 + k2:])
         ctx.k1, ctx.k2, ctx.maxl = k1, k2, maxl
+        ctx.set_materialize_grads(False)   # a matrix whose result a loss does not use gets no gradient
         P = [p.as_subclass(torch.Tensor) for p in SO3vec(*xs).CGproduct(SO3vec(*ys), maxl).parts.values()]
         out = [torch.empty(p.shape[:-1] + w.shape[1:], dtype=p.dtype, device=p.device) for p, w in zip(P, ws)]
         cabi.vec_mix_channels(out, P, ws, 0)
@@ -267,8 +274,10 @@ class CGproductMixFn(torch.autograd.Function):
         saved = ctx.saved_tensors
         need = ctx.needs_input_grad[3:]
         args, P = list(saved[:len(need)]), list(saved[len(need):])
-        gs = [packed(g.as_subclass(torch.Tensor)) for g in gargs]
-        if torch.is_grad_enabled():   # a graph of the gradients is wanted
+        gs = [None if g is None else packed(g.as_subclass(torch.Tensor)) for g in gargs]
+        if all(g is None for g in gs):
+            grads = [None] * len(need)
+        elif torch.is_grad_enabled():   # a graph of the gradients is wanted
             grads = _two_step_grads(k1, k2, ctx.maxl, args, gs, need, graph=True)
         else:
             grads = _mixed_product_grads(k1, k2, args[0:k1], args[k1:k1 + k2], args[k1 + k2:], P, gs, need)

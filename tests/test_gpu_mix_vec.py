@@ -186,3 +186,38 @@ def test_dispatch_modes_see_the_products(cabi):
         got = list((gelib.SO3vec(x) * gelib.SO3weights(w)).parts.values())
     assert counter.get_total_flops() > 0
     near(got, want)
+
+
+# ---- what torch's products part by part give as well ------------------------------------------------------------------
+
+
+@pytest.mark.parametrize("n", [3, 4])
+def test_mixed_parts_without_a_gradient(cabi, n):
+    """A loss of one part of x * W: the other parts and matrices get no gradient, whatever values they hold."""
+    import gelib_amd as gelib
+    xs, ws = [rand((6, 2 * l + 1, n), l) for l in range(3)], [rand((n, 5), 10 + l).requires_grad_() for l in range(3)]
+    xs[2][1, 2, 0] = float("nan")
+    xs = [x.requires_grad_() for x in xs]
+    g = rand((6, 3, 5), 20)
+    for graph in (False, True):
+        rs = list((gelib.SO3vec(*xs) * gelib.SO3weights(*ws)).parts.values())
+        got = torch.autograd.grad(rs[1], xs + ws, g, allow_unused=True, create_graph=graph)
+        assert [t is None for t in got] == [True, False, True] * 2
+        near([got[1], got[4]], torch.autograd.grad(torch.matmul(xs[1], ws[1]), [xs[1], ws[1]], g))
+
+
+@pytest.mark.parametrize("n1,n2", [(3, 3), (4, 2)])
+def test_layer_outputs_without_a_gradient(cabi, n1, n2):
+    """The same for a layer: the matrices of unused results get none, and what they hold reaches no operand's gradient."""
+    import gelib_amd as gelib
+    xs, ys, ws = layer(cabi, n1, n2, 5, 20)
+    with torch.no_grad():
+        ws[2][0, 1] = float("nan")
+    g = rand((20, 3, 5), 20)
+    P = gelib.SO3vec(*xs).CGproduct(gelib.SO3vec(*ys), 2).parts[1].as_subclass(torch.Tensor)
+    want = torch.autograd.grad(torch.matmul(P, ws[1]), xs + ys + [ws[1]], g)
+    for graph in (False, True):
+        out = gelib.CGproduct_linear(gelib.SO3vec(*xs), gelib.SO3vec(*ys), gelib.SO3weights(*ws), 2)
+        got = torch.autograd.grad(out.parts[1], xs + ys + ws, g, allow_unused=True, create_graph=graph)
+        assert [t is None for t in got] == [False] * 6 + [True, False, True]
+        near(list(got[:6]) + [got[7]], want)
