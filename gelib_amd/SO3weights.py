@@ -53,7 +53,7 @@ def mix_channels(x, w):
 
 class MixPartsFn(torch.autograd.Function):
     """x_k w_k for all parts of a vector in one call, any channel counts; contiguous complex64 GPU tensors.  classes: what the
-    results are (torch.matmul gives a part of an odd number of channels its class back)."""
+    results are (mix_channels gives tensors, torch.matmul of a part with an odd number of channels its class)."""
 
     @staticmethod
     def forward(ctx, k, classes, *args):
@@ -110,17 +110,29 @@ def one_launch_holds(xs, ws):
     return sum((x.numel() // w.shape[0] + 64) * (max(w.shape) // 32 + 1) for x, w in zip(xs, ws)) <= 1 << 30
 
 
+def matmul_class(x, w):
+    """The class of torch.matmul(x, w); None where only torch can tell (classes with hooks of their own, or two that know nothing of
+    each other).  A parameter is as a tensor there."""
+    kinds = {type(t) for t in (x, w)} - {torch.Tensor, torch.nn.Parameter}
+    if not kinds:
+        return torch.Tensor
+    c = kinds.pop()
+    hook = getattr(c.__torch_function__, "__func__", None)
+    return c if not kinds and hook is torch.Tensor.__torch_function__.__func__ else None
+
+
 def mix_parts(xs, ws):
     """[torch.matmul(x, w) for x, w in zip(xs, ws)], on the GPU in one call of the library."""
     pairs = list(zip(xs, ws))
     if pairs and plain_autograd() and all(
             x.is_cuda and w.is_cuda and x.device == w.device == xs[0].device and x.dtype == w.dtype == torch.complex64 and w.dim() == 2 and
             x.numel() > 0 and w.numel() > 0 and x.shape[-1] == w.shape[0] for x, w in pairs) and one_launch_holds(xs, ws):
-        odd = [x.shape[-1] % 2 != 0 for x, _ in pairs]
-        classes = [type(x) if o else torch.Tensor for (x, _), o in zip(pairs, odd)]
+        from gelib_amd import cabi
         xp = [packed(x.as_subclass(torch.Tensor)) for x, _ in pairs]
-        wp = [packed(w.as_subclass(torch.Tensor)) for _, w in pairs]
-        return list(MixPartsFn.apply(len(pairs), classes, *(xp + wp)))
+        classes = [torch.Tensor if cabi.mix_channels_ok(p) else matmul_class(x, w) for p, (x, w) in zip(xp, pairs)]
+        if None not in classes:
+            wp = [packed(w.as_subclass(torch.Tensor)) for _, w in pairs]
+            return list(MixPartsFn.apply(len(pairs), classes, *(xp + wp)))
     return [mix_channels(x, w) for x, w in pairs]
 
 

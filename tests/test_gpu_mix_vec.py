@@ -221,3 +221,24 @@ def test_layer_outputs_without_a_gradient(cabi, n1, n2):
         got = torch.autograd.grad(out.parts[1], xs + ys + ws, g, allow_unused=True, create_graph=graph)
         assert [t is None for t in got] == [False] * 6 + [True, False, True]
         near(list(got[:6]) + [got[7]], want)
+
+
+@pytest.mark.parametrize("n", [3, 4])
+def test_classes_of_mixed_parts(cabi, n):
+    """Odd counts: the class that torch.matmul gives; even ones: a tensor."""
+    import gelib_amd as gelib
+    make = [lambda t: t, torch.nn.Parameter, lambda t: t.as_subclass(gelib.SO3part), lambda t: t.as_subclass(gelib.SO3partArr)]
+    for i, cx in enumerate(make):
+        for cw in make[:3]:
+            x, w = cx(rand((4, 3, n), 1)), cw(rand((n, 5), 2))
+            try:
+                want = torch.matmul(x, w)
+            except TypeError:   # two classes that know nothing of each other
+                if n % 2:
+                    with pytest.raises(TypeError):
+                        gelib.SO3vec(x) * gelib.SO3weights(w)
+                continue
+            got = (gelib.SO3vec(x) * gelib.SO3weights(w)).parts[1]
+            assert type(got) is (type(want) if n % 2 else torch.Tensor)
+            assert got.requires_grad == want.requires_grad and got.is_leaf == want.is_leaf
+            near([got], [want])
