@@ -4,6 +4,8 @@
 the GPU the product of a part with its matrix and the gradient with respect to the part run on the library's
 matrix-core kernels for tall, skinny complex matrices (mix_channels below), as does the gradient with respect to the
 matrix; tensors on the host stay with torch."""
+import functools
+
 import torch
 
 from gelib_amd.SO3type import SO3type
@@ -264,12 +266,12 @@ def _mixed_product_grads(k1, k2, xs, ys, ws, P, gs, need):
 
 class CGproductMixFn(torch.autograd.Function):
     """CGproduct(x, y, maxl) * W for the shapes the fused kernel does not take: the product is formed and kept, as the two
-    separate functions keep it, but all its parts are mixed in one call, forward and backward."""
+    separate functions keep it, but all its parts are mixed in one call, forward and backward.  part_cls: the class of the
+    product's parts, which mixed parts of an odd number of channels have as well (torch.matmul's rule)."""
 
     @staticmethod
-    def forward(ctx, k1, k2, maxl, *args):
+    def forward(ctx, part_cls, k1, k2, maxl, *args):
         from gelib_amd import cabi
-        from gelib_amd.SO3part import SO3part
         from gelib_amd.SO3vec import SO3vec
         xs, ys, ws = list(args[0:k1]), list(args[k1:k1 + k2]), list(args[k1 + k2:])
         ctx.k1, ctx.k2, ctx.maxl = k1, k2, maxl
@@ -278,13 +280,13 @@ class CGproductMixFn(torch.autograd.Function):
         out = [torch.empty(p.shape[:-1] + w.shape[1:], dtype=p.dtype, device=p.device) for p, w in zip(P, ws)]
         cabi.vec_mix_channels(out, P, ws, 0)
         ctx.save_for_backward(*args, *P)
-        return tuple(r.as_subclass(SO3part) if p.shape[-1] % 2 else r for r, p in zip(out, P))
+        return tuple(r.as_subclass(part_cls) if p.shape[-1] % 2 else r for r, p in zip(out, P))
 
     @staticmethod
     def backward(ctx, *gargs):
         k1, k2 = ctx.k1, ctx.k2
         saved = ctx.saved_tensors
-        need = ctx.needs_input_grad[3:]
+        need = ctx.needs_input_grad[4:]
         args, P = list(saved[:len(need)]), list(saved[len(need):])
         gs = [None if g is None else packed(g.as_subclass(torch.Tensor)) for g in gargs]
         if all(g is None for g in gs):
@@ -293,7 +295,7 @@ class CGproductMixFn(torch.autograd.Function):
             grads = _two_step_grads(k1, k2, ctx.maxl, args, gs, need, graph=True)
         else:
             grads = _mixed_product_grads(k1, k2, args[0:k1], args[k1:k1 + k2], args[k1 + k2:], P, gs, need)
-        return tuple([None, None, None] + grads)
+        return tuple([None, None, None, None] + grads)
 
 
 def fused_linear_ok(x, y, W, maxl):
@@ -316,9 +318,13 @@ def fused_linear_ok(x, y, W, maxl):
 
 
 def mixed_product_ok(x, y, W, maxl):
-    """True when CGproductMixFn takes CGproduct(x, y, maxl) * W: complex64 parts on one GPU, contiguous, the same leading
-    dimensions, one matrix for every part of the product, and nothing that only torch's own operations support (forward-mode
-    derivatives, function transforms)."""
+    """True when CGproductMixFn takes CGproduct(x, y, maxl) * W: two vectors or two arrays of vectors of complex64 parts on one GPU,
+    contiguous, the same leading dimensions, one matrix (a tensor or parameter) for every part of the product, and nothing that
+    only torch's own operations support (forward-mode derivatives, function transforms)."""
+    from gelib_amd.SO3vec import SO3vec
+    from gelib_amd.SO3vecArr import SO3vecArr
+    if type(x) is not type(y) or type(x) not in (SO3vec, SO3vecArr) or any(type(w) not in (torch.Tensor, torch.nn.Parameter) for w in W.parts):
+        return False
     xs, ys, ws = list(x.parts.values()), list(y.parts.values()), list(W.parts)
     ts = xs + ys + ws
     if not xs or not ys or not ws or not all(t.is_cuda and t.dtype == torch.complex64 and t.is_contiguous() and
@@ -343,13 +349,19 @@ def CGproduct_linear(x, y, W, maxl=-1):
     """x.CGproduct(y, maxl) * W (python/src/gelib/SO3vec.py:174-177 applied to the result of SO3vec.CGproduct).  On the GPU,
     for the shapes fused_linear_ok accepts, one kernel forms the product and multiplies it by the matrices without
     storing it; other shapes keep the product, and mix all its parts in one call.  What neither takes runs the two steps one after
-    the other."""
+    the other.  A vector of the class that the two steps give."""
+    from gelib_amd.SO3partArr import SO3partArr
+    from gelib_amd.SO3part import SO3part
     from gelib_amd.SO3vec import SO3vec
+    from gelib_amd.SO3vecArr import SO3vecArr
+    arrays = isinstance(x, SO3vecArr) and isinstance(y, SO3vecArr)
+    if arrays and maxl is None:
+        maxl = -1
     if fused_linear_ok(x, y, W, maxl):
-        fn = CGproductLinearFn
+        fn = CGproductLinearFn.apply
     elif mixed_product_ok(x, y, W, maxl):
-        fn = CGproductMixFn
+        fn = functools.partial(CGproductMixFn.apply, SO3partArr if arrays else SO3part)
     else:
         return x.CGproduct(y, maxl) * W
     ts = resolved(*[t.as_subclass(torch.Tensor) for t in (*x.parts.values(), *y.parts.values(), *W.parts)])
-    return SO3vec(*fn.apply(len(x.parts), len(y.parts), maxl, *ts))
+    return (SO3vecArr if arrays else SO3vec)(*fn(len(x.parts), len(y.parts), maxl, *ts))

@@ -242,3 +242,30 @@ def test_classes_of_mixed_parts(cabi, n):
             assert type(got) is (type(want) if n % 2 else torch.Tensor)
             assert got.requires_grad == want.requires_grad and got.is_leaf == want.is_leaf
             near([got], [want])
+
+
+@pytest.mark.parametrize("L,n,out", [(2, 3, 5), (2, 4, 6), (4, 2, 4), (5, 2, 3)])
+def test_layer_of_arrays(cabi, L, n, out):
+    """A layer of arrays of vectors is an array of vectors, with parts of the class that the two steps give."""
+    import gelib_amd as gelib
+    xs, ys = [rand((2, 3, 2 * l + 1, n), l) for l in range(L + 1)], [rand((2, 3, 2 * l + 1, n), 10 + l) for l in range(L + 1)]
+    tau = {l: n for l in range(L + 1)}
+    for maxl in (L, None):
+        ws = [rand((c, out), 20 + l) for l, c in cabi.so3type_product(tau, tau, -1 if maxl is None else maxl).items()]
+        x, y, W = gelib.SO3vecArr(*xs), gelib.SO3vecArr(*ys), gelib.SO3weights(*ws)
+        two = x.CGproduct(y, maxl) * W
+        got = gelib.CGproduct_linear(x, y, W, maxl)
+        assert type(got) is gelib.SO3vecArr and got.get_adims() == [3]
+        if len(ws) != 5:   # (the kernel of products with the parts l = 0..4 gives tensors)
+            assert [type(p) for p in got.parts.values()] == [type(p) for p in two.parts.values()]
+        near(got.parts.values(), two.parts.values())
+
+
+def test_layer_of_an_array_and_a_vector(cabi):
+    """Refused, as the product of the two is."""
+    import gelib_amd as gelib
+    xs, ys, ws = [rand((2, 1, 2 * l + 1, 3), l) for l in range(2)], [rand((2, 1, 2 * l + 1, 3), 9 + l) for l in range(2)], []
+    tau = cabi.so3type_product({0: 3, 1: 3}, {0: 3, 1: 3}, 1)
+    ws = [rand((c, 5), 20 + l) for l, c in tau.items()]
+    with pytest.raises(AssertionError):
+        gelib.CGproduct_linear(gelib.SO3vecArr(*xs), gelib.SO3vec(*ys), gelib.SO3weights(*ws), 1)
