@@ -63,7 +63,8 @@ class MixPartsFn(torch.autograd.Function):
         xs, ws = list(args[:k]), list(args[k:])
         ctx.k = k
         ctx.set_materialize_grads(False)   # parts that a loss does not use get no gradients
-        ctx.save_for_backward(*args)
+        need = ctx.needs_input_grad[2:]    # a part is kept for the gradient of its matrix, a matrix for that of its part
+        ctx.save_for_backward(*[t if n else None for t, n in zip(args, need[k:] + need[:k])])
         rs = [torch.empty(x.shape[:-1] + w.shape[1:], dtype=x.dtype, device=x.device) for x, w in zip(xs, ws)]
         cabi.vec_mix_channels(rs, xs, ws, 0)
         return tuple(r if c is torch.Tensor else r.as_subclass(c) for r, c in zip(rs, classes))
@@ -88,12 +89,12 @@ class MixPartsFn(torch.autograd.Function):
         todo = [i for i in range(k) if need[i] and gs[i] is not None]
         if todo:
             for i in todo:
-                gx[i] = torch.empty_like(xs[i])
+                gx[i] = torch.empty(gs[i].shape[:-1] + ws[i].shape[:1], dtype=gs[i].dtype, device=gs[i].device)
             cabi.vec_mix_channels([gx[i] for i in todo], [gs[i] for i in todo], [ws[i] for i in todo], 1)
         todo = [i for i in range(k) if need[k + i] and gs[i] is not None]
         if todo:
             for i in todo:
-                gw[i] = torch.empty_like(ws[i])
+                gw[i] = torch.empty(xs[i].shape[-1:] + gs[i].shape[-1:], dtype=gs[i].dtype, device=gs[i].device)
             cabi.vec_mix_channels([gw[i] for i in todo], [xs[i] for i in todo], [gs[i] for i in todo], 2)
         return tuple([None, None] + gx + gw)
 
@@ -225,7 +226,8 @@ class CGproductLinearFn(torch.autograd.Function):
             from gelib_amd.SO3vec import SO3vec
             with torch._C.DisableTorchFunctionSubclass():
                 P = list(SO3vec(*xs).CGproduct(SO3vec(*ys), ctx.maxl).parts.values())
-                return tuple([None, None, None] + _mixed_product_grads(k1, k2, xs, ys, ws, [p.as_subclass(torch.Tensor) for p in P], gs, need))
+                return tuple([None, None, None] + _mixed_product_grads(k1, k2, xs, ys, ws, [p.as_subclass(torch.Tensor) for p in P], gs, need,
+                                                                               [p.shape for p in P]))
         return tuple([None, None, None] + _two_step_grads(k1, k2, ctx.maxl, saved, gs, need))
 
 
@@ -244,9 +246,10 @@ def _two_step_grads(k1, k2, maxl, saved, gs, need, graph=False):
     return [next(got) if n else None for n in need]
 
 
-def _mixed_product_grads(k1, k2, xs, ys, ws, P, gs, need):
-    """Gradients of P_l W_l with P = CGproduct(x, y) at hand: the matrices' in one call, the product's in one, and the product's
-    backward pass.  gs: None for a result that is not used, whose matrix gets no gradient and whose part of the product a zero one."""
+def _mixed_product_grads(k1, k2, xs, ys, ws, P, gs, need, shapes):
+    """Gradients of P_l W_l with P = CGproduct(x, y), of these shapes, at hand where a matrix needs a gradient: the
+    matrices' in one call, the product's in one, and the product's backward pass.  gs: None for a result that is not used, whose
+    matrix gets no gradient and whose part of the product a zero one."""
     from gelib_amd import cabi
     from gelib_amd.SO3vec import SO3vec_CGproductFn
     used = [i for i, g in enumerate(gs) if g is not None]
@@ -258,7 +261,7 @@ def _mixed_product_grads(k1, k2, xs, ys, ws, P, gs, need):
         cabi.vec_mix_channels([wg[i] for i in todo], [P[i] for i in todo], [gs[i] for i in todo], 2)
     xyg = [None] * (k1 + k2)
     if any(need[0:k1 + k2]):
-        gP = [torch.zeros_like(p) if g is None else torch.empty_like(p) for p, g in zip(P, gs)]
+        gP = [(torch.zeros if g is None else torch.empty)(s, dtype=xs[0].dtype, device=xs[0].device) for s, g in zip(shapes, gs)]
         cabi.vec_mix_channels([gP[i] for i in used], [gs[i] for i in used], [ws[i] for i in used], 1)
         xyg = SO3vec_CGproductFn.grads(k1, k2, xs + ys, gP, need)
     return [g if n else None for g, n in zip(list(xyg) + wg, need)]
@@ -279,7 +282,9 @@ class CGproductMixFn(torch.autograd.Function):
         P = [p.as_subclass(torch.Tensor) for p in SO3vec(*xs).CGproduct(SO3vec(*ys), maxl).parts.values()]
         out = [torch.empty(p.shape[:-1] + w.shape[1:], dtype=p.dtype, device=p.device) for p, w in zip(P, ws)]
         cabi.vec_mix_channels(out, P, ws, 0)
-        ctx.save_for_backward(*args, *P)
+        ctx.shapes = [p.shape for p in P]
+        # the product is kept for the gradients of the matrices
+        ctx.save_for_backward(*args, *[p if n else None for p, n in zip(P, ctx.needs_input_grad[4 + k1 + k2:])])
         return tuple(r.as_subclass(part_cls) if p.shape[-1] % 2 else r for r, p in zip(out, P))
 
     @staticmethod
@@ -294,7 +299,7 @@ class CGproductMixFn(torch.autograd.Function):
         elif torch.is_grad_enabled():   # a graph of the gradients is wanted
             grads = _two_step_grads(k1, k2, ctx.maxl, args, gs, need, graph=True)
         else:
-            grads = _mixed_product_grads(k1, k2, args[0:k1], args[k1:k1 + k2], args[k1 + k2:], P, gs, need)
+            grads = _mixed_product_grads(k1, k2, args[0:k1], args[k1:k1 + k2], args[k1 + k2:], P, gs, need, ctx.shapes)
         return tuple([None, None, None, None] + grads)
 
 

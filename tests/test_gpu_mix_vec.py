@@ -269,3 +269,29 @@ def test_layer_of_an_array_and_a_vector(cabi):
     ws = [rand((c, 5), 20 + l) for l, c in tau.items()]
     with pytest.raises(AssertionError):
         gelib.CGproduct_linear(gelib.SO3vecArr(*xs), gelib.SO3vec(*ys), gelib.SO3weights(*ws), 1)
+
+
+def test_frozen_matrices_keep_no_product(cabi):
+    """Where the matrices learn nothing, the tensors that only their gradients would read are not kept."""
+    import gelib_amd as gelib
+    xs, ys, ws = layer(cabi, 3, 3, 5, 20)
+
+    def kept(f):
+        seen = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(tuple(t.shape)) or t, lambda t: t):
+            rs = f()
+        return rs, seen
+    frozen = [w.detach() for w in ws]
+    rs, seen = kept(lambda: list(gelib.CGproduct_linear(gelib.SO3vec(*xs), gelib.SO3vec(*ys), gelib.SO3weights(*frozen), 2).parts.values()))
+    assert not [s for s in seen if s in [(20, 2 * l + 1, w.shape[0]) for l, w in enumerate(ws)]]
+    P = gelib.SO3vec(*xs).CGproduct(gelib.SO3vec(*ys), 2).parts.values()
+    gs = [rand(tuple(r.shape), 30 + k) for k, r in enumerate(rs)]
+    near(torch.autograd.grad(rs, xs + ys, gs), torch.autograd.grad([torch.matmul(p.as_subclass(torch.Tensor), w) for p, w in zip(P, frozen)], xs + ys, gs))
+    w = [rand((3, 5), 40 + l) for l in range(3)]
+    rs, seen = kept(lambda: list((gelib.SO3vec(*xs) * gelib.SO3weights(*w)).parts.values()))
+    assert seen and all(s == (3, 5) for s in seen)
+    near(torch.autograd.grad(rs, xs, gs), torch.autograd.grad([torch.matmul(x, v) for x, v in zip(xs, w)], xs, gs))
+    fixed, learn = [x.detach() for x in xs], [v.requires_grad_() for v in w]
+    rs, seen = kept(lambda: list((gelib.SO3vec(*fixed) * gelib.SO3weights(*learn)).parts.values()))
+    assert (3, 5) not in seen
+    near(torch.autograd.grad(rs, learn, gs), torch.autograd.grad([torch.matmul(x, v) for x, v in zip(fixed, learn)], learn, gs))
