@@ -127,7 +127,8 @@ def matmul_class(x, w):
 def mix_parts(xs, ws):
     """[torch.matmul(x, w) for x, w in zip(xs, ws)], on the GPU in one call of the library."""
     pairs = list(zip(xs, ws))
-    if pairs and plain_autograd() and all(
+    # (the library's launches go to the current device)
+    if pairs and plain_autograd() and xs[0].is_cuda and xs[0].get_device() == torch.cuda.current_device() and all(
             x.is_cuda and w.is_cuda and x.device == w.device == xs[0].device and x.dtype == w.dtype == torch.complex64 and w.dim() == 2 and
             x.numel() > 0 and w.numel() > 0 and x.shape[-1] == w.shape[0] for x, w in pairs) and one_launch_holds(xs, ws):
         from gelib_amd import cabi

@@ -295,3 +295,16 @@ def test_frozen_matrices_keep_no_product(cabi):
     rs, seen = kept(lambda: list((gelib.SO3vec(*fixed) * gelib.SO3weights(*learn)).parts.values()))
     assert (3, 5) not in seen
     near(torch.autograd.grad(rs, learn, gs), torch.autograd.grad([torch.matmul(x, v) for x, v in zip(fixed, learn)], learn, gs))
+
+
+def test_parts_on_another_device(cabi, monkeypatch):
+    """Parts that are not on the current device, whose stream the library's launches go to, stay with torch's product."""
+    import gelib_amd as gelib
+    x, w = rand((4, 3, 3), 1), rand((3, 5), 2)
+    called = []
+    monkeypatch.setattr(cabi, "vec_mix_channels", lambda *a: called.append(a))
+    with monkeypatch.context() as m:
+        m.setattr(torch.cuda, "current_device", lambda: 1)
+        got = (gelib.SO3vec(x) * gelib.SO3weights(w)).parts[1]
+    assert not called
+    near([got], [torch.matmul(x, w)])
