@@ -583,7 +583,9 @@ int fwd_dispatch(const VecPlan &plan, const std::vector<View> &R, const std::vec
     {
       // Vectors of several parts with l above 7: one launch of the matrix-core single-pair kernel per (x part, y part)
       // pair (every pair writes channel blocks of its own); a pair that kernel does not take goes through this
-      // dispatch by itself.
+      // dispatch by itself.  First pairs of padded channel counts leave the vector to the any-l kernels' one launch (pair by pair / whole:
+      // l = 8, 9 x 4, 5, 7 channels 1 to 60 MB 1.5, 400 MB .97, x 8, 9, 5 and 7 channels 1.5 to 1.9, .85; 8, 10 x 3, 5, 12 and 6 channels 1.2 to
+      // 1.45; 3 channels, 8 to 11 x 8 to 10, capped at 8, 1.7).
       int lop = 0;
       for (auto &v : X) lop = std::max(lop, v.l);
       for (auto &v : Y) lop = std::max(lop, v.l);
@@ -600,7 +602,7 @@ int fwd_dispatch(const VecPlan &plan, const std::vector<View> &R, const std::vec
                 sub.triples.push_back(t);
               }
             if (sub.triples.empty()) continue;
-            rc = onepair_mfma_vec_fwd(sub, rd, {X[p].d}, {Y[q].d}, accumulate != 0, s, &used);
+            rc = onepair_mfma_vec_fwd(sub, rd, {X[p].d}, {Y[q].d}, accumulate != 0, s, &used, true);
             if (rc) return rc;
             if (used) any = true;
             else if (!any) goto whole;  // not even the first pair: the vector stays in one piece

@@ -651,10 +651,23 @@ bool bwd_padded_pays(int n1, int n2, int N1, int N2) {
   while (s2 < n2) s2 *= 2;
   return s1 * s2 > 64 || s1 * s2 >= N1 * N2;
 }
-// Forward, against the any-l kernel: where more than half of the places are real (8 x 5 channels 422 -> 263 us, 4 x 12 387 -> 259, 6 x 5
-// 298 / 305, 5 x 9 385 / 392).  16 channels are stored four bytes at a time, which only launches that are over before the memory is
-// busy can afford (7 x 9, 3 x 3: 1461 cells 152 -> 82 us, 19493 cells 352 / 460).
-bool fwd_padded_pays(int n1, int n2, int N1, int N2, long long ncells) { return 2 * n1 * n2 > N1 * N2 && (N1 * N2 > 16 || ncells <= 2048); }
+// Forward, against the any-l kernel, more than half of the places real.  What this kernel pays for is values of l (32 columns of the
+// matrix instructions, whatever their number) and idle places; the any-l kernel pays for terms, and is bound by its stores where there
+// are few.  Padded / any-l, product 1 to 30 MB | 100 to 400 MB: 16 places .34 to .71 up to 2048 cells (7 x 9, 3 x 3; 19493
+// cells 1.3: stored four bytes at a time); 5 values of l (2 x 7 to 2 x 15) .67 to .94 | 1.07 to 1.98; 7 of them .60 to .78 | .72 to 1.63; 9, 256 places
+// .65 to .76 | .79 to 1.18, 64 and 128 .94 to 1.10 | .79 to 1.30; 4 to 9 values of a product capped below l1 + l2 .67 to 1.33 | .82 to
+// 3.8; 10 and more .42 to .95 (11 x 10, 3 x 13: 1.13) | .38 to .95, but two fifths of the places idle and a count n1 that the any-l kernel takes four
+// at a time, 12 x 6: 10 x 5 1.15, 7 x 7 1.06, 12 x 9 .92.
+// The same line for the shapes themselves in rows that are not aligned (8 x 8 in 65 channels): 5 and 7 values of l .72 to 1.00 | 1.00 to 1.16, 4
+// capped 1.24 | 1.9, 15 .84 | .97, 19 and more .48 to .90 | .37 to .65, except 64 places, which the any-l kernel takes better below about
+// a thousand cells (l = 8 x 8 to 12 x 9, 3 to 320 cells 1.07 to 1.5, 640 .94 to 1.08, 1300 .64).
+bool fwd_padded_pays(int n1, int n2, int N1, int N2, int nl, bool every_l, long long ncells, long long bytes) {
+  if (2 * n1 * n2 <= N1 * N2) return false;
+  if (N1 * N2 == 16) return ncells <= 2048;
+  if (n1 == N1 && n2 == N2 && n1 * n2 == 64 && nl >= 17 && ncells < 1024) return false;
+  if (nl >= 10) return nl >= 17 || n1 % 4 || 5 * n1 * n2 >= 3 * N1 * N2;
+  return bytes < 32000000LL && every_l && (nl <= 7 || N1 * N2 == 256);
+}
 void launch_bwd_shape(int n1, int n2, bool pad, const OnePairMfmaArgs &a, hipStream_t s) {
 #define GELIB_X(A, B)                                                                                                   \
   if (n1 == A && n2 == B) {                                                                                             \
@@ -735,6 +748,7 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
     // 64 channels per wave: the lane's 16 bytes of a row must be 16-byte aligned (block offset, row and cell strides
     // even); with 16 channels a lane loads single floats
     if (N1 * N2 >= 64 && (((t.offs) & 1) || (fg[t.ri].sm & 1) || (fg[t.ri].sb & 1) || ((uintptr_t)fg[t.ri].ptr & 15))) pad = true;
+    if (pad && !g_pad) return GELIB_HIP_OK;
     if ((long long)fg[t.ri].sm * 8 * (2 * t.l + 1) >= (1LL << 32)) return GELIB_HIP_OK;  // row offsets are 32 bits
   }
   const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
@@ -764,10 +778,11 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
   return GELIB_HIP_OK;
 }
 
-// The product itself for the same shapes (non-Diag, l1, l2 <= 15, 4 to 22 values of l).
+// The product itself for the same shapes (non-Diag, l1, l2 <= 15, 4 to 22 values of l).  exact: only at the channel counts the kernels are
+// built for, in aligned rows.
 int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *> &r,
                          const std::vector<const gelib_part_desc *> &x, const std::vector<const gelib_part_desc *> &y,
-                         bool accumulate, hipStream_t s, int *used) {
+                         bool accumulate, hipStream_t s, int *used, bool exact) {
   *used = 0;
   if (!g_enable_fwd || plan.diag || x.size() != 1 || y.size() != 1 || plan.triples.empty()) return GELIB_HIP_OK;
   std::vector<FastPart> fx, fy, fr;
@@ -779,7 +794,7 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
   int N1 = 0, N2 = 0;
   if (!padded_shape(n1, n2, &N1, &N2) || l1 > kMaxLm || l2 > kMaxLm) return GELIB_HIP_OK;
   bool pad = !bwd_shape_built(n1, n2);
-  if (pad && (!g_pad || l1 + l2 >= kNLm || !fwd_padded_pays(n1, n2, N1, N2, plan.E[0] * plan.E[1] * plan.E[2]))) return GELIB_HIP_OK;
+  if (pad && l1 + l2 >= kNLm) return GELIB_HIP_OK;
   const int lmin = std::abs(l1 - l2);
   int lmax = -1;
   for (auto &t : plan.triples) lmax = std::max(lmax, t.l);
@@ -792,6 +807,8 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
   a.y = fy[0];
   std::vector<int> present(nl, 0);
   bool one_rowb = true;
+  const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
+  long long bytes = 0;
   for (auto &t : plan.triples) {
     const int dl = t.l - lmin;
     a.g[dl] = fr[t.ri];
@@ -800,12 +817,13 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
     // 64 channels per wave: a lane stores 16 bytes at a time (block offset, row and cell strides even, base aligned);
     // with 16 channels it stores single floats
     if (N1 * N2 >= 64 && (((t.offs) & 1) || (fr[t.ri].sm & 1) || (fr[t.ri].sb & 1) || ((uintptr_t)fr[t.ri].ptr & 15))) pad = true;
+    bytes += 8 * ncells * (2 * t.l + 1) * n1 * n2;
     if ((long long)fr[t.ri].sm * 8 >= (1LL << 32)) return GELIB_HIP_OK;  // row lengths are 32 bits
     if (a.rowb == 0) a.rowb = (long long)fr[t.ri].sm * 8;
     if (a.rowb != (long long)fr[t.ri].sm * 8) one_rowb = false;
   }
-  const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
   if (ncells > 0x7fffffffLL) return GELIB_HIP_OK;
+  if (pad && (exact || !g_pad || !fwd_padded_pays(n1, n2, N1, N2, nl, lmax == l1 + l2, ncells, bytes))) return GELIB_HIP_OK;
   Tables t;
   const int lt = std::min(l1 + l2, lmax);
   int rc = device_tables(l1, l2, lmin, lt, nl, present, false, &t);

@@ -98,7 +98,7 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
 // The forward pass of the same shapes on the matrix cores (the reduction over m1).
 int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *> &r,
                          const std::vector<const gelib_part_desc *> &x, const std::vector<const gelib_part_desc *> &y,
-                         bool accumulate, hipStream_t s, int *used);
+                         bool accumulate, hipStream_t s, int *used, bool exact = false);
 int onepair_mfma_set_option(const char *name, int value);  // "onepair_mfma", "onepair_mfma_fwd": 0 switches the kernel off
 
 }  // namespace gelib_hip

@@ -49,9 +49,48 @@ def test_padded_shapes(cabi, B, l1, n1, l2, n2, maxl):
     O.check_bwd_onto([U.host(t) for t in ax], [U.host(t) for t in ay], [U.host(t) for t in dxg], [U.host(t) for t in dyg], "added")
 
 
+ROUTES = [
+    # (B, l1, n1, l2, n2, maxl, extra channels of the result, taken here?): both sides of the lines that the product is taken along
+    (2048, 7, 3, 2, 3, -1, 0, True), (2049, 7, 3, 2, 3, -1, 0, False),                                      # 16 places
+    (100, 7, 7, 2, 8, -1, 0, True), (3500, 7, 7, 2, 8, -1, 0, False), (100, 7, 7, 7, 8, 7, 0, False),     # few values of l: small, large, capped
+    (20, 4, 15, 8, 15, -1, 0, True), (200, 4, 4, 8, 15, -1, 0, False),                                    # 9 of them: 256 places, 64
+    (9, 10, 5, 5, 8, -1, 0, True), (9, 10, 12, 5, 6, -1, 0, False), (9, 8, 12, 8, 6, -1, 0, True),        # more: idle places
+    (100, 8, 8, 8, 8, -1, 1, False), (1024, 8, 8, 8, 8, -1, 1, True), (9, 8, 8, 8, 8, -1, 0, True),       # rows that are not aligned
+    (9, 8, 16, 8, 8, -1, 1, True), (700, 8, 8, 8, 8, 3, 1, False),
+]
+
+
+@pytest.mark.parametrize("B,l1,n1,l2,n2,maxl,extra,here", ROUTES)
+def test_which_products_are_padded(cabi, B, l1, n1, l2, n2, maxl, extra, here):
+    """Where the any-l kernel is faster the product stays with it; the two agree to the rounding of sums of at most 31 terms."""
+    x, y = U.dev(U.seeded(1, B, 2 * l1 + 1, n1)), U.dev(U.seeded(2, B, 2 * l2 + 1, n2))
+    r = [[torch.zeros(B, 2 * l + 1, n + extra, dtype=torch.complex64, device="cuda")[..., :n]
+          for l, n in cabi.so3type_product({l1: n1}, {l2: n2}, maxl).items()] for _ in range(2)]
+    cabi.so3vec_fwd(r[0], [x], [y], accumulate=False)
+    assert (cabi.last_path() == ONEPAIR) == here
+    try:
+        cabi.set_option("onepair_mfma_fwd", 0)
+        cabi.so3vec_fwd(r[1], [x], [y], accumulate=False)
+    finally:
+        cabi.set_option("onepair_mfma_fwd", 1)
+    assert cabi.last_path() != ONEPAIR
+    # a term is at most |x| |y|, the squares of a row of coefficients add up to at most 1, and each order of the sum rounds by 31 * 2^-24
+    assert all((a - b).norm() <= 2 * 31 * 2.0 ** -24 * 31 ** 0.5 * b.norm() for a, b in zip(*r))
+
+
+def test_several_parts_stay_in_one_launch_unless_their_counts_are_built(cabi):
+    """A vector whose first pair of parts would be padded goes to the any-l kernels as a whole."""
+    for n, path in ((7, False), (8, True)):
+        xs, ys = [U.dev(U.seeded(l, 5, 2 * l + 1, n)) for l in (8, 9)], [U.dev(U.seeded(l, 5, 2 * l + 1, n)) for l in (4, 5)]
+        r = [torch.zeros(5, 2 * l + 1, c, dtype=torch.complex64, device="cuda") for l, c in cabi.so3type_product({8: n, 9: n}, {4: n, 5: n}, -1).items()]
+        cabi.so3vec_fwd(r, xs, ys, accumulate=False)
+        assert (cabi.last_path() == ONEPAIR) == path
+
+
 def test_rows_that_are_not_aligned(cabi):
-    """8 x 8 channels in parts of 65 channels (an odd row length): eight bytes at a time, the same bits as from aligned rows."""
-    B, l = 3, 9
+    """8 x 8 channels in parts of 65 channels (an odd row length): eight bytes at a time, the same bits as from aligned rows.  (Enough cells
+    for the product of such parts to be taken here.)"""
+    B, l = 1027, 9
     x, y = U.dev(U.seeded(1, B, 2 * l + 1, 8)), U.dev(U.seeded(2, B, 2 * l + 1, 8))
     tau = cabi.so3type_product({l: 8}, {l: 8}, -1)
     ref = [torch.empty(B, 2 * k + 1, n, dtype=torch.complex64, device="cuda") for k, n in tau.items()]
