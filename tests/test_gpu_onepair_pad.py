@@ -49,6 +49,44 @@ def test_padded_shapes(cabi, B, l1, n1, l2, n2, maxl):
     O.check_bwd_onto([U.host(t) for t in ax], [U.host(t) for t in ay], [U.host(t) for t in dxg], [U.host(t) for t in dyg], "added")
 
 
+@pytest.mark.parametrize("B,l1,n1,l2,n2,maxl,extra", [(3, 10, 7, 8, 7, -1, 0), (2, 9, 12, 9, 7, 9, 3), (3, 8, 3, 9, 3, -1, 1), (2, 7, 16, 8, 15, 10, 1),
+                                                      (2, 9, 16, 8, 8, -1, 1)])
+def test_products_added_onto_values(cabi, B, l1, n1, l2, n2, maxl, extra):
+    """Adding stores at every width of a row's last piece, and in parts of more channels, which keep what they hold."""
+    xs, ys = [U.seeded(1 + B, B, 2 * l1 + 1, n1)], [U.seeded(2 + B, B, 2 * l2 + 1, n2)]
+    O = U.VecOracle(xs, ys, maxl, False, gseed=100 + B)
+    start = [U.seeded(50 + k, B, p.shape[1], p.shape[2] + extra) for k, p in enumerate(O.r32)]
+    r = [U.dev(s) for s in start]
+    cabi.so3vec_fwd([t[..., :n1 * n2] for t in r], [U.dev(a) for a in xs], [U.dev(a) for a in ys], accumulate=True)
+    assert cabi.last_path() == ONEPAIR
+    torch.cuda.synchronize()
+    got = [U.host(t) for t in r]
+    assert all(np.array_equal(a[..., n1 * n2:], s[..., n1 * n2:]) for a, s in zip(got, start))
+    O.check_fwd_onto([a[..., :n1 * n2] for a in got], [s[..., :n1 * n2] for s in start], "added")
+
+
+@pytest.mark.parametrize("nx,ny", [((5, 7), (7, 5)), ((9, 3), (5, 6))])
+def test_vectors_of_several_parts(cabi, nx, ny):
+    """Pairs of parts one launch each: blocks at odd channels of parts with row lengths of their own, gradients added up."""
+    B = 3
+    xs, ys = [U.seeded(k, B, 2 * l + 1, n) for k, (l, n) in enumerate(zip((9, 10), nx))], [U.seeded(5 + k, B, 2 * l + 1, n) for k, (l, n) in enumerate(zip((8, 9), ny))]
+    O = U.VecOracle(xs, ys, -1, False, gseed=7)
+    assert len({p.shape[2] for p in O.r32}) > 2 and any(p.shape[2] % 2 for p in O.r32)
+    dx, dy, dg = [U.dev(a) for a in xs], [U.dev(a) for a in ys], [U.dev(a) for a in O.gs]
+    dr = [torch.full(p.shape, 5.0, dtype=torch.complex64, device="cuda") for p in O.r32]
+    cabi.so3vec_fwd(dr, dx, dy, accumulate=False)
+    dxg, dyg = [torch.full_like(t, 3.0 - 2j) for t in dx], [torch.full_like(t, 3.0 - 2j) for t in dy]
+    cabi.so3vec_bwd(dxg, dyg, dg, dx, dy, accumulate=False)
+    assert cabi.last_path() == ONEPAIR
+    torch.cuda.synchronize()
+    O.check_fwd([U.host(t) for t in dr], "forward")
+    O.check_bwd([U.host(t) for t in dxg], [U.host(t) for t in dyg], "backward")
+    start = [U.host(t) for t in dr]
+    cabi.so3vec_fwd(dr, dx, dy, accumulate=True)
+    torch.cuda.synchronize()
+    O.check_fwd_onto([U.host(t) for t in dr], start, "added")
+
+
 ROUTES = [
     # (B, l1, n1, l2, n2, maxl, extra channels of the result, taken here?): both sides of the lines that the product is taken along
     (2048, 7, 3, 2, 3, -1, 0, True), (2049, 7, 3, 2, 3, -1, 0, False),                                      # 16 places
