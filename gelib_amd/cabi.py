@@ -25,7 +25,7 @@ SYMBOLS = [
     "gelib_hip_o3vec_cg_fwd", "gelib_hip_o3vec_cg_bwd",
     "gelib_hip_so3vec_cg_linear_bwd", "gelib_hip_so3vec_cg_linear_bwd_workspace_bytes",
     "gelib_hip_set_option", "gelib_hip_set_stream_workspace",
-    "gelib_hip_last_path",
+    "gelib_hip_last_path", "gelib_hip_last_streaming",
     "gelib_hip_malloc", "gelib_hip_free", "gelib_hip_memcpy", "gelib_hip_memset", "gelib_hip_synchronize",
 ]
 
@@ -431,3 +431,8 @@ def set_option(name, value):
 
 def last_path():
     return lib().gelib_hip_last_path()
+
+
+def last_streaming():
+    """1: the last product of this thread was written with streaming stores, 2: its gradient read with streaming loads, 0: neither."""
+    return lib().gelib_hip_last_streaming()

@@ -23,6 +23,8 @@ using namespace gelib_hip;
 
 namespace gelib_hip {
 
+thread_local int t_streaming = 0;
+
 namespace {
 thread_local std::string t_last_error;
 thread_local int t_last_path = kPathNone;
@@ -659,6 +661,7 @@ int fwd_planned(const VecPlan &plan, const std::vector<View> &R, const std::vect
 int vec_fwd_entry(bool diag, int nr, const gelib_part_desc *r, int nx, const gelib_part_desc *x, int ny,
                   const gelib_part_desc *y, int accumulate, void *stream) {
   t_last_path = kPathNone;
+  t_streaming = 0;
   std::vector<View> R, X, Y;
   int rc;
   if ((rc = sort_parts(nr, r, kMaxOutParts, R)) || (rc = sort_parts(nx, x, kMaxParts, X)) ||
@@ -848,6 +851,7 @@ int bwd_planned(const VecPlan &plan, const std::vector<View> &G, const std::vect
 int vec_bwd_entry(bool diag, const gelib_part_desc *xg, const gelib_part_desc *yg, int ng, const gelib_part_desc *g,
                   int nx, const gelib_part_desc *x, int ny, const gelib_part_desc *y, int accumulate, void *stream) {
   t_last_path = kPathNone;
+  t_streaming = 0;
   if (!xg && !yg) return GELIB_HIP_OK;
   std::vector<View> G, X, Y, XG, YG;
   int rc;
@@ -1945,5 +1949,7 @@ int gelib_hip_set_option(const char *name, int value) {
 }
 
 int gelib_hip_last_path(void) { return t_last_path; }
+
+int gelib_hip_last_streaming(void) { return gelib_hip::t_streaming; }
 
 }  // extern "C"

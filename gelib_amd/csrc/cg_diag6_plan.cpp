@@ -280,9 +280,18 @@ int diag6_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
   // .89 .88 .78 | .96, 24 .90 .82 .74 | .79, 17 .91 1.60 1.71 | 1.71, L=4 48 .92 .95 .75 | .98, 8 .90 .99 .79 | .96, 20 .91 1.40 1.37 |
   // 1.41, L=2 16 .92 .80 .97 | 1.05; features x harmonics up to l = 2, L=3, 24 channels .89 .94 .75 | .90, 16 .96 .80 .63 | 1.02, 20
   // 1.00 1.11 1.02 | .96, L=4 24 .92 .79 .56 | .97.  Not for the wave form from 32 channels on (L=3, up to l = 2, 64 channels .91 1.02
-  // .85 | 1.13), nor 8 channels with harmonics up to l = 1 (L=3 .97 .65 1.03 | 1.07).
-  const bool stream = a.n % 8 == 0 && !(small4 && a.n >= 32) && !(a.n == 8 && narrow_l <= 1 && wide_l >= 3);
+  // .85 | 1.13), nor 8 channels with harmonics up to l = 1 (L=3 .97 .65 1.03 | 1.07).  The rows have to start at half-lines, too: in parts
+  // of 4 channels more, 1 more and 16 more from the second on, 1.2 GB: 64 channels L=6 .97 1.10 1.18, 24 1.33 1.50 1.55, L=4 48 1.12 1.27
+  // 1.28, 16 1.52 1.91 1.88, 8 1.67 1.97 1.88, L=2 16 1.38 1.67 1.58; of 8 more .83 to 1.03.  Nor products that fit the memory-side cache.
+  bool rows = true;
+  long long bytes = 0;
+  for (auto &t : plan.triples) {
+    rows = rows && pieces_aligned(a.r[t.l], t.offs + a.offs_add, 8);
+    bytes += 8 * a.ncells * (2 * t.l + 1) * a.n;
+  }
+  const bool stream = a.n % 8 == 0 && rows && bytes > kMemoryCache && !(small4 && a.n >= 32) && !(a.n == 8 && narrow_l <= 1 && wide_l >= 3);
   a.write = accumulate ? kWriteAdd : ((g_stream < 0 ? stream : g_stream != 0) ? kWriteStream : kWriteOver);
+  t_streaming |= a.write == kWriteStream ? 1 : 0;
   if (g_small_enable && lcap <= 4 && operands_up_to(a, 2)) rc = launch_diag6_small_fwd(a, s);
   else if (small4 && lcap <= 6 && operands_up_to(a, 4)) rc = launch_diag6_small4_fwd(a, s);
   else if (hi) rc = a.lg_npad < 6 ? launch_diag6_fwd_hi_packed(a, s) : launch_diag6_fwd_hi(a, s);
@@ -316,14 +325,19 @@ int diag6_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
   // block's must keep them.  Streaming / ordinary, 250 MB and 1.5 GB of g that other calls have pushed out of the caches: Diag L=6
   // 64 channels .77 .87, 24 .80 .88, 17 .82 1.27, L=4 64 .78 .96, 24 .82 1.14, 8 .92 1.28, 3 1.23 1.32, L=2 32 .78 .96, L=1 16 .92
   // .97; features x harmonics up to l = 2, L=4 32 .64 .90, L=3 16 .65 .91, 24 .79 1.14; capped at l = 1 with harmonics above it .89
-  // 1.02, and 1.1 to 1.2 where g is still in the caches.
+  // 1.02, and 1.1 to 1.2 where g is still in the caches.  Written just before, 40 to 200 MB .94 to 1.05, 400 MB and more .93 to .99.  Operands
+  // up to l = 4 want the rows to start at lines (1.2 GB, half a line and 8 bytes off: L=4 48 channels 1.14 1.14, 16 1.23 1.23, L=2
+  // 16 1.32 1.31, x harmonics up to l = 2 L=3 16 1.36 1.36; 300 MB .86 to 1.12), those above do not mind (64 channels .92, 24 .95 1.01).
   int top = 0, narrow = kNP;
   for (int l = 0; l < kNP; l++) {
     if (a.x[l].ptr || a.y[l].ptr) top = l;
     if ((a.xbc && a.x[l].ptr) || (a.ybc && a.y[l].ptr)) narrow = l;
   }
-  const bool lines = top > 4 ? a.n % 8 == 0 && a.n >= 16 : a.n % 16 == 0;
+  bool lines = top > 4 ? a.n % 8 == 0 && a.n >= 16 : a.n % 16 == 0;
+  if (top <= 4)
+    for (auto &t : plan.triples) lines = lines && pieces_aligned(a.r[t.l], t.offs + a.offs_add, 16);
   a.once = g_once < 0 ? lines && !(lcap <= 1 && narrow >= 2 && narrow < kNP) : g_once;
+  t_streaming |= a.once ? 2 : 0;
   a.want_x = xg.empty() ? 0 : 1;
   a.want_y = yg.empty() ? 0 : 1;
   bool all_y = true;

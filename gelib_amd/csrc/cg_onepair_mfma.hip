@@ -110,7 +110,8 @@ struct PairShape {
 // PAD: the parts have n1 <= N1 and n2 <= N2 channels (a.x.n, a.y.n), or rows that are not 16-byte aligned.  The operands of the
 // channels beyond are zeros; their places in a row of g are read from the channel with 0 in place of what is beyond, whose
 // sums they share anyway (so nothing that is not a number enters a sum it does not belong to), eight bytes at a time.
-template <int N1, int N2, bool PAD>
+// ONCE: streaming loads of g.
+template <int N1, int N2, bool PAD, bool ONCE>
 __global__ void __launch_bounds__((64 * PairShape<N1, N2>::W)) onepair_mfma_bwd_kernel(const OnePairMfmaArgs a) {
   using Sh = PairShape<N1, N2>;
   constexpr int T = Sh::T, JL = Sh::JL, W = Sh::W;
@@ -218,9 +219,8 @@ __global__ void __launch_bounds__((64 * PairShape<N1, N2>::W)) onepair_mfma_bwd_
     if constexpr (T == 4 && PAD) {
       const v2f lo = *(GlobalIn2)addr, hi = *(GlobalIn2)(addr - off0 + off1);
       g = v4f{lo.x, lo.y, hi.x, hi.y};
-    } else if constexpr (T == 4) g = __builtin_nontemporal_load((GlobalIn4)addr);
-    else if constexpr (PAD) g = *(GlobalIn1)addr;
-    else g = __builtin_nontemporal_load((GlobalIn1)addr);
+    } else if constexpr (T == 4) g = ONCE ? __builtin_nontemporal_load((GlobalIn4)addr) : *(GlobalIn4)addr;
+    else g = ONCE ? __builtin_nontemporal_load((GlobalIn1)addr) : *(GlobalIn1)addr;
     cf = *((GlobalIn1)a.coef + coef_at);   // the table ends with a queue's worth of idle steps
     coef_at += 64;
   };
@@ -388,7 +388,8 @@ constexpr int kCellsF = 8;                     // cells (waves) per block of the
 // forms the products of channels 2 i and 2 i + 1 = (a, j) and (a, j + 1)), or of all 16 (one tile, column i = float i:
 // the lane forms the real or the imaginary part of channel i / 2).
 // PAD: as in the backward kernel; the places of the channels beyond are not stored, the others 8 bytes at a time.
-template <int N1, int N2, bool ONE_ROWB, bool PAD>
+// STREAM: streaming stores (kernels of their own, as in cg_diag6_impl.h).
+template <int N1, int N2, bool ONE_ROWB, bool PAD, bool STREAM>
 __global__ void __launch_bounds__(64 * kCellsF) onepair_mfma_fwd_kernel(const OnePairMfmaArgs a) {
   using Sh = PairShape<N1, N2>;
   constexpr int T = Sh::T, W = Sh::W;
@@ -518,13 +519,14 @@ __global__ void __launch_bounds__(64 * kCellsF) onepair_mfma_fwd_kernel(const On
           v4f o;
           o.x = D[0][v], o.y = D[1][v], o.z = D[2][v], o.w = D[3][v];
           if (accumulate) o += *q;
-          __builtin_nontemporal_store(o, q);
+          if constexpr (STREAM) __builtin_nontemporal_store(o, q);
+          else *q = o;
         } else {
           GlobalOut1 q = (GlobalOut1)cur[v];
           float o = D[0][v];
           if (accumulate) o += *q;
-          if constexpr (PAD) *q = o;
-          else __builtin_nontemporal_store(o, q);
+          if constexpr (STREAM) __builtin_nontemporal_store(o, q);
+          else *q = o;
         }
       }
       cur[v] += ONE_ROWB ? (unsigned long long)rowb : (unsigned long long)rowbv[v];
@@ -543,7 +545,7 @@ struct Tables {
 };
 std::mutex g_mutex;
 std::map<std::vector<int>, Tables> g_tables;  // (device, l1, l2, lmin, lt, nl, present...) -> device tables
-int g_enable = 1, g_enable_fwd = 1, g_paired = 1, g_pad = 1;
+int g_enable = 1, g_enable_fwd = 1, g_paired = 1, g_pad = 1, g_stream = -1, g_once = -1;
 
 int device_tables(int l1, int l2, int lmin, int lt, int nl, const std::vector<int> &present, bool paired, Tables *out) {
   int dev = 0;
@@ -668,17 +670,20 @@ bool fwd_padded_pays(int n1, int n2, int N1, int N2, int nl, bool every_l, long 
   if (nl >= 10) return nl >= 17 || n1 % 4 || 5 * n1 * n2 >= 3 * N1 * N2;
   return bytes < 32000000LL && every_l && (nl <= 7 || N1 * N2 == 256);
 }
-void launch_bwd_shape(int n1, int n2, bool pad, const OnePairMfmaArgs &a, hipStream_t s) {
-#define GELIB_X(A, B)                                                                                                   \
-  if (n1 == A && n2 == B) {                                                                                             \
-    if (pad) hipLaunchKernelGGL((onepair_mfma_bwd_kernel<A, B, true>), dim3((unsigned)a.ncells), dim3(64 * PairShape<A, B>::W), 0, s, a); \
-    else hipLaunchKernelGGL((onepair_mfma_bwd_kernel<A, B, false>), dim3((unsigned)a.ncells), dim3(64 * PairShape<A, B>::W), 0, s, a); \
-  }
+template <int N1, int N2>
+void launch_bwd_as(bool pad, bool once, const OnePairMfmaArgs &a, hipStream_t s) {
+  const dim3 grid((unsigned)a.ncells), block(64 * PairShape<N1, N2>::W);
+  if (pad) hipLaunchKernelGGL((onepair_mfma_bwd_kernel<N1, N2, true, false>), grid, block, 0, s, a);
+  else if (once) hipLaunchKernelGGL((onepair_mfma_bwd_kernel<N1, N2, false, true>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((onepair_mfma_bwd_kernel<N1, N2, false, false>), grid, block, 0, s, a);
+}
+void launch_bwd_shape(int n1, int n2, bool pad, bool once, const OnePairMfmaArgs &a, hipStream_t s) {
+#define GELIB_X(A, B) if (n1 == A && n2 == B) launch_bwd_as<A, B>(pad, once, a, s);
   GELIB_ONEPAIR_SHAPES(GELIB_X)
 #undef GELIB_X
 }
 
-template <int N1, int N2, bool ONE_ROWB, bool PAD>
+template <int N1, int N2, bool ONE_ROWB, bool PAD, bool STREAM>
 int launch_fwd_one(const OnePairMfmaArgs &a, unsigned nblocks, size_t lds, hipStream_t s) {
   static std::mutex attr_mutex;
   static std::map<int, bool> attr_set;  // device -> the kernel may use 80 KB of LDS
@@ -687,19 +692,20 @@ int launch_fwd_one(const OnePairMfmaArgs &a, unsigned nblocks, size_t lds, hipSt
   {
     std::lock_guard<std::mutex> lock(attr_mutex);
     if (!attr_set[dev]) {
-      GELIB_HIP_TRY(hipFuncSetAttribute((const void *)onepair_mfma_fwd_kernel<N1, N2, ONE_ROWB, PAD>,
+      GELIB_HIP_TRY(hipFuncSetAttribute((const void *)onepair_mfma_fwd_kernel<N1, N2, ONE_ROWB, PAD, STREAM>,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)(80 * 1024)));
       attr_set[dev] = true;
     }
   }
-  hipLaunchKernelGGL((onepair_mfma_fwd_kernel<N1, N2, ONE_ROWB, PAD>), dim3(nblocks), dim3(64 * kCellsF), lds, s, a);
+  hipLaunchKernelGGL((onepair_mfma_fwd_kernel<N1, N2, ONE_ROWB, PAD, STREAM>), dim3(nblocks), dim3(64 * kCellsF), lds, s, a);
   return GELIB_HIP_OK;
 }
-int launch_fwd_shape(int n1, int n2, bool one_rowb, bool pad, const OnePairMfmaArgs &a, unsigned nblocks, size_t lds, hipStream_t s) {
-#define GELIB_X(A, B)                                                                     \
-  if (n1 == A && n2 == B) {                                                               \
-    if (pad) return one_rowb ? launch_fwd_one<A, B, true, true>(a, nblocks, lds, s) : launch_fwd_one<A, B, false, true>(a, nblocks, lds, s); \
-    return one_rowb ? launch_fwd_one<A, B, true, false>(a, nblocks, lds, s) : launch_fwd_one<A, B, false, false>(a, nblocks, lds, s);        \
+int launch_fwd_shape(int n1, int n2, bool one_rowb, bool pad, bool stream, const OnePairMfmaArgs &a, unsigned nblocks, size_t lds, hipStream_t s) {
+#define GELIB_X(A, B)                                                                                            \
+  if (n1 == A && n2 == B) {                                                                                      \
+    if (pad) return one_rowb ? launch_fwd_one<A, B, true, true, false>(a, nblocks, lds, s) : launch_fwd_one<A, B, false, true, false>(a, nblocks, lds, s);      \
+    if (stream) return one_rowb ? launch_fwd_one<A, B, true, false, true>(a, nblocks, lds, s) : launch_fwd_one<A, B, false, false, true>(a, nblocks, lds, s);   \
+    return one_rowb ? launch_fwd_one<A, B, true, false, false>(a, nblocks, lds, s) : launch_fwd_one<A, B, false, false, false>(a, nblocks, lds, s);             \
   }
   GELIB_ONEPAIR_SHAPES(GELIB_X)
 #undef GELIB_X
@@ -740,6 +746,7 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
   a.xg = fxg[0];
   a.yg = fyg[0];
   std::vector<int> present(nl, 0);
+  bool lines = true;
   for (auto &t : plan.triples) {
     const int dl = t.l - lmin;
     a.g[dl] = fg[t.ri];
@@ -749,6 +756,7 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
     // even); with 16 channels a lane loads single floats
     if (N1 * N2 >= 64 && (((t.offs) & 1) || (fg[t.ri].sm & 1) || (fg[t.ri].sb & 1) || ((uintptr_t)fg[t.ri].ptr & 15))) pad = true;
     if (pad && !g_pad) return GELIB_HIP_OK;
+    lines = lines && pieces_aligned(fg[t.ri], t.offs, 16);
     if ((long long)fg[t.ri].sm * 8 * (2 * t.l + 1) >= (1LL << 32)) return GELIB_HIP_OK;  // row offsets are 32 bits
   }
   const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
@@ -772,7 +780,11 @@ int onepair_mfma_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part
   a.lt = lt;
   a.nl = nl;
   a.accumulate = accumulate ? 1 : 0;
-  launch_bwd_shape(N1, N2, pad, a, s);
+  // Streaming loads: g 400 MB and 1 GB .85 to 1.0 of the time, written just before .96 to 1.0.  Not for rows of one line that lie across two
+  // (16 channels in parts of one more, 1 GB 1.06 to 1.11; from 64 channels on .95 to 1.0).
+  const bool once = !pad && (g_once < 0 ? lines || n1 * n2 >= 64 : g_once != 0);
+  t_streaming |= once ? 2 : 0;
+  launch_bwd_shape(N1, N2, pad, once, a, s);
   GELIB_HIP_TRY(hipGetLastError());
   *used = 1;
   return GELIB_HIP_OK;
@@ -806,7 +818,7 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
   a.x = fx[0];
   a.y = fy[0];
   std::vector<int> present(nl, 0);
-  bool one_rowb = true;
+  bool one_rowb = true, aligned = true;
   const long long ncells = plan.E[0] * plan.E[1] * plan.E[2];
   long long bytes = 0;
   for (auto &t : plan.triples) {
@@ -818,6 +830,7 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
     // with 16 channels it stores single floats
     if (N1 * N2 >= 64 && (((t.offs) & 1) || (fr[t.ri].sm & 1) || (fr[t.ri].sb & 1) || ((uintptr_t)fr[t.ri].ptr & 15))) pad = true;
     bytes += 8 * ncells * (2 * t.l + 1) * n1 * n2;
+    aligned = aligned && pieces_aligned(fr[t.ri], t.offs, 8);
     if ((long long)fr[t.ri].sm * 8 >= (1LL << 32)) return GELIB_HIP_OK;  // row lengths are 32 bits
     if (a.rowb == 0) a.rowb = (long long)fr[t.ri].sm * 8;
     if (a.rowb != (long long)fr[t.ri].sm * 8) one_rowb = false;
@@ -843,7 +856,11 @@ int onepair_mfma_vec_fwd(const VecPlan &plan, const std::vector<const gelib_part
   const size_t lds = (size_t)t.nsteps_fwd * 2 * kColsF * 4 +
                      (size_t)cells_per_block * ((size_t)(2 * l1 + 2) * N1 + (size_t)(2 * l2 + 3) * N2) * 8;
   if (lds > 80 * 1024) return GELIB_HIP_OK;
-  rc = launch_fwd_shape(N1, N2, one_rowb, pad, a, (unsigned)((ncells + cells_per_block - 1) / cells_per_block), lds, s);
+  // Streaming / ordinary stores, rows at whole half-lines, 400 MB and 1 GB of product .94 to 1.02, .91 to 1.0 with the next pass over it (5
+  // to 21 values of l); 100 MB .95 to .99, but 1.05 to 1.16 with it.  In parts of a channel more 1.07 to 1.3 from 64 channels on, 1.4 to 1.8 at 16.
+  const bool stream = !pad && !accumulate && (g_stream < 0 ? aligned && bytes > kMemoryCache : g_stream != 0);
+  t_streaming |= stream ? 1 : 0;
+  rc = launch_fwd_shape(N1, N2, one_rowb, pad, stream, a, (unsigned)((ncells + cells_per_block - 1) / cells_per_block), lds, s);
   if (rc) return rc;
   GELIB_HIP_TRY(hipGetLastError());
   *used = 1;
@@ -857,6 +874,16 @@ int onepair_mfma_set_option(const char *name, int value) {
   }
   if (!std::strcmp(name, "onepair_mfma_pad")) {   // other channel counts than those of GELIB_ONEPAIR_SHAPES
     g_pad = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "onepair_mfma_stream")) {   // streaming stores: -1 by the shape, 0 never, 1 always
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_stream = value;
+    return GELIB_HIP_OK;
+  }
+  if (!std::strcmp(name, "onepair_mfma_once")) {     // streaming loads of the gradient: the same values
+    if (value < -1 || value > 1) return GELIB_HIP_ERR_ARG;
+    g_once = value;
     return GELIB_HIP_OK;
   }
   if (!std::strcmp(name, "onepair_mfma_paired")) {

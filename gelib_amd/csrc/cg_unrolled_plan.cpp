@@ -373,11 +373,19 @@ int run_fwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   // Streaming stores: in the kernel for operands above kLT, where every block is whole runs of 512 bytes (L=6, 8 channels, streaming
   // / ordinary at 40, 250 and 1500 MB of product .94 .93 .79; 4 channels .92 1.25 1.07, 6 channels .91 1.65 1.63).  The kernels up to
   // kLT keep ordinary stores: with several channels per thread a row's pieces meet in the caches (L=4 16 channels .97 1.00 .97, 8
-  // channels .96 1.08 1.05, 12 .98 1.14 1.09, 20 .97 1.18 1.26, 9 .93 1.65 1.67, 3 1.94 4.3 4.3).
+  // channels .96 1.08 1.05, 12 .98 1.14 1.09, 20 .97 1.18 1.26, 9 .93 1.65 1.67, 3 1.94 4.3 4.3).  Rows at half-lines (L=6, 8 channels, parts of 8
+  // channels more .84, of 4 more, 1 more and from the second of 16 more on 1.16 1.28 1.24, 1.2 GB), and not a product that fits the
+  // memory-side cache.
   bool lines = lop > kLT;
-  for (auto &t : triples) lines = lines && t.nout % 64 == 0;
-  const bool stream = lop > kLT && (g_fwd_stream < 0 ? lines : g_fwd_stream != 0);   // (the kernels up to kLT have no such stores)
+  long long bytes = 0;
+  for (auto &t : triples) {
+    lines = lines && t.nout % 64 == 0 && pieces_aligned(f.r[t.ri], t.offs + offs_add, 8);
+    bytes += 8 * ncells * (2 * t.l + 1) * t.nout;
+  }
+  // (the kernels up to kLT have no such stores, nor those that leave an odd last channel out)
+  const bool stream = lop > kLT && !ragged && (g_fwd_stream < 0 ? lines && bytes > kMemoryCache : g_fwd_stream != 0);
   a.write = accumulate ? kWriteAdd : (stream ? kWriteStream : kWriteOver);
+  t_streaming |= a.write == kWriteStream ? 1 : 0;
   long long nblocks = 0;
   size_t lds_bytes = 0;
   int lcap = 0;
@@ -544,10 +552,13 @@ int run_bwd(bool diag, const std::vector<VecTriple> &triples, const std::vector<
   // Streaming / ordinary, g warm and pushed out of the caches, 250 MB and 1.5 GB: L=4 16 channels .96 .75 | .90 .85, 8 .97 .73 | .96 .90, 4
   // .95 .73 | .97 .91, 20 1.03 .79 | 1.02 .94; L=6 8 channels .97 .81 | .90 .85; 8 x 2 .98 .80 | .96 .96; 3 channels 1.04 .92 | 1.11 1.13, 2
   // 1.20 1.07 | 1.32 1.35, 1 1.70 1.82 | 2.16 2.28.  Odd counts gain in this launch and lose more in the next: 20, 12, 9, 6, 3 x 10, 7, 6, 5
-  // channels, every l, 5003 cells, backward 347 -> 319 us, the forward launch behind it 171 -> 228.
+  // channels, every l, 5003 cells, backward 347 -> 319 us, the forward launch behind it 171 -> 228.  Written just before, 40 to 200 MB .96 to
+  // 1.06, more .94 to .99.  Blocks of one or two lines have to start at lines (4 x 4 channels, 300 MB and 1.2 GB, half a line off: L=4 .87
+  // 1.15, L=2 .95 1.06, L=1 .91 1.07); 12 x 4 .87 .98, 16 x 16 .74 .84 and operands above l = 4 (6 x 4 x 4 .90 .97) do not mind.
   bool lines = !diag;
-  for (auto &t : triples) lines = lines && t.nout % 16 == 0;
+  for (auto &t : triples) lines = lines && t.nout % 16 == 0 && (t.nout >= 48 || lop > kLT || pieces_aligned(f.r[t.ri], t.offs + offs_add, 16));
   a.once = g_bwd_once < 0 ? lines : g_bwd_once;
+  t_streaming |= a.once && a.want_x && a.want_y && !diag ? 2 : 0;   // (kernels of both gradients)
   a.only_dl = -1;
   if (triples.size() == 1 && !diag && !plan->padded && lop <= kLT && g_bwd_one_enable)
     a.only_dl = triples[0].l - std::abs(triples[0].l1 - triples[0].l2);

@@ -334,9 +334,10 @@ int gelib_hip_set_stream_workspace(void *stream, void *ptr, uint64_t bytes);
  * "fwd_cell_tile" (cells per tile of the unrolled forward launch, 0 = one tile, -1 = chosen by the channel counts, the
  * default), "bwd_lds_target" (LDS bytes per block the unrolled backward kernels aim at when they choose their cells per
  * block), "bwd_min_runs" (runs of 64 lane slots such a block should have at least, 0 = no such rule), "unrolled_bwd_l6" / "unrolled_fwd_l6" (1/0: the backward / forward kernels for operands up to l = 6),
- * "fwd_stream" / "diag6_stream" / "bwd_once" / "diag6_once" (-1, 0, 1: streaming stores of a product / streaming loads of its gradient),
- * "vec_mix" (1/0: all parts of a vector mixed in one launch), "onepair_mfma_pad" (1/0: the matrix-core single-pair kernels at other channel
- * counts up to 16 x 16 than those they are built for),
+ * "fwd_stream" / "diag6_stream" / "onepair_mfma_stream" (streaming stores of a product) and "bwd_once" / "diag6_once" / "onepair_mfma_once" (streaming
+ * loads of its gradient; -1 by the shape, the default, 0 never, 1 always), "vec_mix" (the one launch that mixes all parts of a vector: -1 by the
+ * shape, the default, 0 only for parts that the matrix-core kernels do not take, 1 always), "onepair_mfma_pad" (1/0: the matrix-core
+ * single-pair kernels at other channel counts up to 16 x 16 than those they are built for, and in rows that are not 16-byte aligned),
  * "staged_fwd_tile" (1, 2, 4), "staged_fwd_threads", "staged_fwd_coeffs_lds" (1/0), "staged_fwd_lds_target",
  * "staged_bwd_lds_target", "staged_bwd_threads" (256, 512, 1024), "staged_bwd_stripes" (0 never, otherwise wherever they
  * apply), "staged_bwd_atomic" (1/0: allow the single-pass backward kernels that add with LDS float atomics; off by
@@ -365,6 +366,8 @@ int gelib_hip_set_stream_workspace(void *stream, void *ptr, uint64_t bytes);
  */
 int gelib_hip_set_option(const char *name, int value);
 int gelib_hip_last_path(void);
+/* 1: the last product of this thread was written with streaming stores; 2: its gradient was read with streaming loads; 0: neither. */
+int gelib_hip_last_streaming(void);
 
 #ifdef __cplusplus
 }
