@@ -325,7 +325,7 @@ int diag6_vec_bwd(const VecPlan &plan, const std::vector<const gelib_part_desc *
   // block's must keep them.  Streaming / ordinary, 250 MB and 1.5 GB of g that other calls have pushed out of the caches: Diag L=6
   // 64 channels .77 .87, 24 .80 .88, 17 .82 1.27, L=4 64 .78 .96, 24 .82 1.14, 8 .92 1.28, 3 1.23 1.32, L=2 32 .78 .96, L=1 16 .92
   // .97; features x harmonics up to l = 2, L=4 32 .64 .90, L=3 16 .65 .91, 24 .79 1.14; capped at l = 1 with harmonics above it .89
-  // 1.02, and 1.1 to 1.2 where g is still in the caches.  Written just before, 40 to 200 MB .94 to 1.05, 400 MB and more .93 to .99.  Operands
+  // 1.02, and 1.1 to 1.2 where g is still in the caches.  Written just before, 40 to 200 MB .94 to 1.09, 400 MB and more .89 to .99.  Operands
   // up to l = 4 want the rows to start at lines (1.2 GB, half a line and 8 bytes off: L=4 48 channels 1.14 1.14, 16 1.23 1.23, L=2
   // 16 1.32 1.31, x harmonics up to l = 2 L=3 16 1.36 1.36; 300 MB .86 to 1.12), those above do not mind (64 channels .92, 24 .95 1.01).
   int top = 0, narrow = kNP;
