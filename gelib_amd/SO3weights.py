@@ -124,20 +124,57 @@ def matmul_class(x, w):
     return c if not kinds and hook is torch.Tensor.__torch_function__.__func__ else None
 
 
+def torch_is_faster(x, w):
+    """Is torch's product of a part with an odd number of channels over before the call of the library is made?  All parts of a vector in
+    one call / part by part, forward and backward, 1 to 101 channels, 5 and 24 outputs: one part, 4 to 512 rows 1.7 to 1.9, 1024 1.11, 2048
+    .58; up to l = 1, 384 rows 1.45, 1536 .72; l = 2, 640 1.28, 2560 .41; l = 4, 288 1.17, 1152 .73; l = 6, 416 1.08, 1664 .5 (torch's
+    gradient of a matrix takes .3 ms from about a thousand rows on, and a millisecond every eight thousand).  Without that gradient: 1.7
+    for one part, 1.4, 1.25, 1.07, .98 for two to seven, below about 20 MB of parts (l = 2, 18 MB 1.0, 37 MB .65; l = 4, 13 MB 1.07, 25 MB .8)."""
+    if w.numel() >= LARGE_MATRIX:
+        return False
+    if torch.is_grad_enabled() and w.requires_grad:
+        return x.numel() <= 1024 * x.shape[-1]
+    return x.numel() < 2500000
+
+
+# Elements of a matrix from which on mix.hip's kernels for long rows lose to the one call, also with one part of an even number of
+# channels (one call / part by part, 4 to 8192 rows: 64 x 64 1.0, 512 x 6 1.07 to 1.17, 512 x 24 .73 to .95, 2048 x 6 .75 to .92, 2048 x 24 .3 to .6).
+LARGE_MATRIX = 8192
+
+
+def parts_of_one_call(pairs):
+    """The parts that are mixed in one call of the library: even numbers of channels from two parts on (one part 1.03 to 1.13, two .96,
+    three .9, five .84, seven .8 of the time part by part), odd ones where torch's product takes its time, and then all."""
+    even, large = [], False
+    for k, (x, w) in enumerate(pairs):
+        if x.shape[-1] % 2 == 0:
+            even.append(k)
+            large = large or w.numel() >= LARGE_MATRIX
+        elif not torch_is_faster(x, w):
+            return list(range(len(pairs)))
+    return even if large or len(even) > 1 else []
+
+
 def mix_parts(xs, ws):
-    """[torch.matmul(x, w) for x, w in zip(xs, ws)], on the GPU in one call of the library."""
+    """[torch.matmul(x, w) for x, w in zip(xs, ws)], on the GPU in one call of the library where that pays."""
     pairs = list(zip(xs, ws))
-    # (the library's launches go to the current device)
-    if pairs and plain_autograd() and xs[0].is_cuda and xs[0].get_device() == torch.cuda.current_device() and all(
-            x.is_cuda and w.is_cuda and x.device == w.device == xs[0].device and x.dtype == w.dtype == torch.complex64 and w.dim() == 2 and
-            x.numel() > 0 and w.numel() > 0 and x.shape[-1] == w.shape[0] for x, w in pairs) and one_launch_holds(xs, ws):
-        from gelib_amd import cabi
-        xp = [packed(x.as_subclass(torch.Tensor)) for x, _ in pairs]
-        classes = [torch.Tensor if cabi.mix_channels_ok(p) else matmul_class(x, w) for p, (x, w) in zip(xp, pairs)]
-        if None not in classes:
-            wp = [packed(w.as_subclass(torch.Tensor)) for _, w in pairs]
-            return list(MixPartsFn.apply(len(pairs), classes, *(xp + wp)))
-    return [mix_channels(x, w) for x, w in pairs]
+    with torch._C.DisableTorchFunctionSubclass():
+        together = parts_of_one_call(pairs) if pairs and xs[0].is_cuda else []
+        # (the library's launches go to the current device)
+        if together and plain_autograd() and xs[0].get_device() == torch.cuda.current_device() and all(
+                x.is_cuda and w.is_cuda and x.device == w.device == xs[0].device and x.dtype == w.dtype == torch.complex64 and w.dim() == 2 and
+                x.numel() > 0 and w.numel() > 0 and x.shape[-1] == w.shape[0] for x, w in pairs) and one_launch_holds(xs, ws):
+            from gelib_amd import cabi
+            xp = [packed(pairs[k][0].as_subclass(torch.Tensor)) for k in together]
+            classes = [torch.Tensor if cabi.mix_channels_ok(p) else matmul_class(*pairs[k]) for p, k in zip(xp, together)]
+            if None in classes:
+                together = []
+        else:
+            together = []
+        if together:
+            wp = [packed(pairs[k][1].as_subclass(torch.Tensor)) for k in together]
+            mixed = dict(zip(together, MixPartsFn.apply(len(together), classes, *(xp + wp))))
+    return [mixed[k] if k in together else mix_channels(*pairs[k]) for k in range(len(pairs))]
 
 
 class SO3weights:
@@ -331,6 +368,8 @@ def mixed_product_ok(x, y, W, maxl):
     from gelib_amd.SO3vecArr import SO3vecArr
     if type(x) is not type(y) or type(x) not in (SO3vec, SO3vecArr) or any(type(w) not in (torch.Tensor, torch.nn.Parameter) for w in W.parts):
         return False
+    if len(W.parts) == 1:
+        return False   # (the two steps: even counts 1.06, odd ones up to 512 rows 1.17 to 1.25 of their time here; two parts .91 to .99)
     xs, ys, ws = list(x.parts.values()), list(y.parts.values()), list(W.parts)
     ts = xs + ys + ws
     if not xs or not ys or not ws or not all(t.is_cuda and t.dtype == torch.complex64 and t.is_contiguous() and

@@ -191,14 +191,14 @@ def test_dispatch_modes_see_the_products(cabi):
 # ---- what torch's products part by part give as well ------------------------------------------------------------------
 
 
-@pytest.mark.parametrize("n", [3, 4])
-def test_mixed_parts_without_a_gradient(cabi, n):
+@pytest.mark.parametrize("n,b", [(3, 6), (3, 1100), (4, 6)])
+def test_mixed_parts_without_a_gradient(cabi, n, b):
     """A loss of one part of x * W: the other parts and matrices get no gradient, whatever values they hold."""
     import gelib_amd as gelib
-    xs, ws = [rand((6, 2 * l + 1, n), l) for l in range(3)], [rand((n, 5), 10 + l).requires_grad_() for l in range(3)]
+    xs, ws = [rand((b, 2 * l + 1, n), l) for l in range(3)], [rand((n, 5), 10 + l).requires_grad_() for l in range(3)]
     xs[2][1, 2, 0] = float("nan")
     xs = [x.requires_grad_() for x in xs]
-    g = rand((6, 3, 5), 20)
+    g = rand((b, 3, 5), 20)
     for graph in (False, True):
         rs = list((gelib.SO3vec(*xs) * gelib.SO3weights(*ws)).parts.values())
         got = torch.autograd.grad(rs[1], xs + ws, g, allow_unused=True, create_graph=graph)
@@ -223,14 +223,14 @@ def test_layer_outputs_without_a_gradient(cabi, n1, n2):
         near(list(got[:6]) + [got[7]], want)
 
 
-@pytest.mark.parametrize("n", [3, 4])
-def test_classes_of_mixed_parts(cabi, n):
+@pytest.mark.parametrize("n,b", [(3, 4), (3, 400), (4, 4)])
+def test_classes_of_mixed_parts(cabi, n, b):
     """Odd counts: the class that torch.matmul gives; even ones: a tensor."""
     import gelib_amd as gelib
     make = [lambda t: t, torch.nn.Parameter, lambda t: t.as_subclass(gelib.SO3part), lambda t: t.as_subclass(gelib.SO3partArr)]
     for i, cx in enumerate(make):
         for cw in make[:3]:
-            x, w = cx(rand((4, 3, n), 1)), cw(rand((n, 5), 2))
+            x, w = cx(rand((b, 3, n), 1)), cw(rand((n, 5), 2))
             try:
                 want = torch.matmul(x, w)
             except TypeError:   # two classes that know nothing of each other
@@ -287,24 +287,44 @@ def test_frozen_matrices_keep_no_product(cabi):
     P = gelib.SO3vec(*xs).CGproduct(gelib.SO3vec(*ys), 2).parts.values()
     gs = [rand(tuple(r.shape), 30 + k) for k, r in enumerate(rs)]
     near(torch.autograd.grad(rs, xs + ys, gs), torch.autograd.grad([torch.matmul(p.as_subclass(torch.Tensor), w) for p, w in zip(P, frozen)], xs + ys, gs))
-    w = [rand((3, 5), 40 + l) for l in range(3)]
+    xs, w = [rand((20, 2 * l + 1, 4), 50 + l).requires_grad_() for l in range(3)], [rand((4, 5), 40 + l) for l in range(3)]
     rs, seen = kept(lambda: list((gelib.SO3vec(*xs) * gelib.SO3weights(*w)).parts.values()))
-    assert seen and all(s == (3, 5) for s in seen)
+    assert seen and all(s == (4, 5) for s in seen)
     near(torch.autograd.grad(rs, xs, gs), torch.autograd.grad([torch.matmul(x, v) for x, v in zip(xs, w)], xs, gs))
     fixed, learn = [x.detach() for x in xs], [v.requires_grad_() for v in w]
     rs, seen = kept(lambda: list((gelib.SO3vec(*fixed) * gelib.SO3weights(*learn)).parts.values()))
-    assert (3, 5) not in seen
+    assert (4, 5) not in seen
     near(torch.autograd.grad(rs, learn, gs), torch.autograd.grad([torch.matmul(x, v) for x, v in zip(fixed, learn)], learn, gs))
 
 
 def test_parts_on_another_device(cabi, monkeypatch):
     """Parts that are not on the current device, whose stream the library's launches go to, stay with torch's product."""
     import gelib_amd as gelib
-    x, w = rand((4, 3, 3), 1), rand((3, 5), 2)
+    xs, ws = [rand((4, 2 * l + 1, 4), 1 + l) for l in range(2)], [rand((4, 5), 3 + l) for l in range(2)]
     called = []
     monkeypatch.setattr(cabi, "vec_mix_channels", lambda *a: called.append(a))
     with monkeypatch.context() as m:
         m.setattr(torch.cuda, "current_device", lambda: 1)
-        got = (gelib.SO3vec(x) * gelib.SO3weights(w)).parts[1]
+        got = (gelib.SO3vec(*xs) * gelib.SO3weights(*ws)).parts.values()
     assert not called
-    near([got], [torch.matmul(x, w)])
+    near(list(got), [torch.matmul(x, w) for x, w in zip(xs, ws)])
+
+
+@pytest.mark.parametrize("counts,b,out,learn,together", [
+    ((4,), 50, 5, True, 0), ((2048,), 5, 4, True, 1), ((4, 4), 50, 5, True, 2), ((3, 4, 4), 50, 5, True, 2), ((3, 4), 50, 5, True, 0),
+    ((3,), 1024, 5, True, 0), ((3,), 1025, 5, True, 1), ((3, 4), 1025, 5, True, 2), ((3, 3, 3), 204, 5, True, 0), ((3, 3, 3), 205, 5, True, 3),
+    ((3, 3, 3), 3000, 5, False, 0), ((501, 3), 4991, 5, False, 2), ((2049,), 4, 4, False, 1)])
+def test_which_parts_are_mixed_in_one_call(cabi, monkeypatch, counts, b, out, learn, together):
+    """Where the one call takes longer than the parts one after the other they stay apart; the values are the same either way."""
+    import gelib_amd as gelib
+    xs = [rand((b, 2 * l + 1, n), l).requires_grad_(learn) for l, n in enumerate(counts)]
+    ws = [rand((n, out), 10 + l).requires_grad_(learn) for l, n in enumerate(counts)]
+    inner, taken = cabi.vec_mix_channels, []
+    monkeypatch.setattr(cabi, "vec_mix_channels", lambda rs, *a: (taken.append(len(rs)), inner(rs, *a)))
+    got = list((gelib.SO3vec(*xs) * gelib.SO3weights(*ws)).parts.values())
+    assert taken == ([together] if together else [])
+    want = [torch.matmul(x, w) for x, w in zip(xs, ws)]
+    near(got, want)
+    if learn:
+        gs = [rand(tuple(r.shape), 20 + k) for k, r in enumerate(got)]
+        near(torch.autograd.grad(got, xs + ws, gs), torch.autograd.grad(want, xs + ws, gs))
