@@ -12,7 +12,7 @@ import functools
 
 import torch
 
-from gelib_amd.gelib_common import backend, common_batch, packed, resolved, without_torch_function
+from gelib_amd.gelib_common import backend, common_batch, resolved, without_torch_function
 from gelib_amd.SO3element import SO3element, SO3irrep
 
 
@@ -199,7 +199,7 @@ def _vec_fn(diag):
             xgs = [make(t, memory_format=torch.contiguous_format) for t in xs]
             ygs = [make(t, memory_format=torch.contiguous_format) for t in ys]
             gp, xp, yp = ctx.ps
-            gb.o3vec_product_back(diag, xgs, ygs, [packed(g) for g in gs], gp, list(xs), xp, list(ys), yp)
+            gb.o3vec_product_back(diag, xgs, ygs, [g.contiguous() for g in resolved(*gs)], gp, list(xs), xp, list(ys), yp)
             return tuple([None, None, None] + xgs + ygs)
 
     Fn.__name__ = "O3vec_%sFn" % name

@@ -4,7 +4,7 @@ forward writes into uninitialised parts and the backward computes both gradients
 import torch
 
 from gelib_amd.SO3weights import mix_parts
-from gelib_amd.gelib_common import backend, common_batch, packed, resolved, without_torch_function
+from gelib_amd.gelib_common import backend, common_batch, resolved, without_torch_function
 from gelib_amd.SO3part import SO3part
 
 
@@ -175,7 +175,7 @@ def _product_fn(diag, part_cls=SO3part, prefix="SO3vec"):
             gb = backend()
             x = gb.SO3vec.view(list(saved[0:k1]))
             y = gb.SO3vec.view(list(saved[k1:k1 + k2]))
-            g = gb.SO3vec.view([packed(t) for t in gargs])
+            g = gb.SO3vec.view([t.contiguous() for t in resolved(*gargs)])
             xg = gb.SO3vec.view([t for t in grads[0:k1] if t is not None])
             yg = gb.SO3vec.view([t for t in grads[k1:k1 + k2] if t is not None])
             lead = gargs[0].shape[:-2]

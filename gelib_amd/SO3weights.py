@@ -364,12 +364,12 @@ def mixed_product_ok(x, y, W, maxl):
     """True when CGproductMixFn takes CGproduct(x, y, maxl) * W: two vectors or two arrays of vectors of complex64 parts on one GPU,
     contiguous, the same leading dimensions, one matrix (a tensor or parameter) for every part of the product, and nothing that
     only torch's own operations support (forward-mode derivatives, function transforms)."""
+    if len(W.parts) == 1:
+        return False   # (the two steps: even counts 1.06, odd ones up to 512 rows 1.17 to 1.25 of their time here; two parts .91 to .99)
     from gelib_amd.SO3vec import SO3vec
     from gelib_amd.SO3vecArr import SO3vecArr
     if type(x) is not type(y) or type(x) not in (SO3vec, SO3vecArr) or any(type(w) not in (torch.Tensor, torch.nn.Parameter) for w in W.parts):
         return False
-    if len(W.parts) == 1:
-        return False   # (the two steps: even counts 1.06, odd ones up to 512 rows 1.17 to 1.25 of their time here; two parts .91 to .99)
     xs, ys, ws = list(x.parts.values()), list(y.parts.values()), list(W.parts)
     ts = xs + ys + ws
     if not xs or not ys or not ws or not all(t.is_cuda and t.dtype == torch.complex64 and t.is_contiguous() and
@@ -395,18 +395,17 @@ def CGproduct_linear(x, y, W, maxl=-1):
     for the shapes fused_linear_ok accepts, one kernel forms the product and multiplies it by the matrices without
     storing it; other shapes keep the product, and mix all its parts in one call.  What neither takes runs the two steps one after
     the other.  A vector of the class that the two steps give."""
-    from gelib_amd.SO3partArr import SO3partArr
-    from gelib_amd.SO3part import SO3part
-    from gelib_amd.SO3vec import SO3vec
-    from gelib_amd.SO3vecArr import SO3vecArr
+    from gelib_amd.SO3vecArr import SO3partArr, SO3vecArr
     arrays = isinstance(x, SO3vecArr) and isinstance(y, SO3vecArr)
     if arrays and maxl is None:
         maxl = -1
     if fused_linear_ok(x, y, W, maxl):
         fn = CGproductLinearFn.apply
     elif mixed_product_ok(x, y, W, maxl):
+        from gelib_amd.SO3part import SO3part
         fn = functools.partial(CGproductMixFn.apply, SO3partArr if arrays else SO3part)
     else:
         return x.CGproduct(y, maxl) * W
+    from gelib_amd.SO3vec import SO3vec
     ts = resolved(*[t.as_subclass(torch.Tensor) for t in (*x.parts.values(), *y.parts.values(), *W.parts)])
     return (SO3vecArr if arrays else SO3vec)(*fn(len(x.parts), len(y.parts), maxl, *ts))

@@ -91,6 +91,14 @@ static std::vector<gelib_part_desc> parts_on_gpu(const std::vector<at::Tensor> &
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("version", []() { return std::string(_GELIB_VERSION); });
 
+  m.def("in_memory", [](const py::args &ts) {
+    for (const py::handle t : ts) {
+      const at::Tensor &x = THPVariable_Unpack(t.ptr());
+      if (x.is_conj() || x.is_neg()) return false;
+    }
+    return true;
+  }, "Does the memory of every one of these tensors hold what it reads as (no view that is conjugated or negated on reading)?");
+
   py::class_<SO3type>(m, "SO3type", "Class to store the type of an SO3-vector")
       .def(py::init<>())
       .def(py::init<std::vector<int>>())

@@ -23,21 +23,18 @@ def output(shape, x, y):
     return make(shape, dtype=torch.complex64, device=x.device)
 
 
+def resolved(*ts):
+    """ts with copies in place of views that torch conjugates (or negates) on reading only: kernels read memory.  (Asked in one call of
+    the extension: two methods of each of ten tensors are 4 us.)"""
+    if backend().in_memory(*ts):
+        return ts
+    return tuple(t.resolve_conj().resolve_neg() for t in ts)
+
+
 def packed(t):
     """t with its elements in memory as they read: contiguous, and no view that torch conjugates (or negates) on reading only, which
     contiguous() leaves as it is (the gradient of out.conj().sum() is one)."""
-    if t.is_conj() or t.is_neg():
-        t = t.resolve_conj().resolve_neg()
-    return t.contiguous()
-
-
-def resolved(*ts):
-    """ts with copies in place of views that torch conjugates (or negates) on reading only: kernels read memory.  (Called with the
-    __torch_function__ hooks off, or on plain tensors.)"""
-    for t in ts:
-        if t.is_conj() or t.is_neg():
-            return tuple(t.resolve_conj().resolve_neg() for t in ts)
-    return ts
+    return resolved(t)[0].contiguous()
 
 
 def common_batch(x, y):
@@ -48,6 +45,7 @@ def common_batch(x, y):
     return max(x.size(0), y.size(0))
 
 
+@functools.lru_cache(maxsize=None)
 def backend():
     """The compiled extension; importing it fails loudly if it has not been built."""
     from gelib_amd import gelib_base
