@@ -93,11 +93,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
 
   m.def("in_memory", [](const py::args &ts) {
     for (const py::handle t : ts) {
+      if (!THPVariable_Check(t.ptr())) return false;
       const at::Tensor &x = THPVariable_Unpack(t.ptr());
       if (x.is_conj() || x.is_neg()) return false;
     }
     return true;
-  }, "Does the memory of every one of these tensors hold what it reads as (no view that is conjugated or negated on reading)?");
+  }, "Is every one of these a tensor whose memory holds what it reads as (no view that is conjugated or negated on reading)?");
 
   py::class_<SO3type>(m, "SO3type", "Class to store the type of an SO3-vector")
       .def(py::init<>())

@@ -52,6 +52,20 @@ def test_host_tensors_are_refused():
         G.CGproduct(u, u)
 
 
+def test_which_tensors_hold_what_they_read_as():
+    """Views that are conjugated or negated on reading do not; what is no tensor is left to the caller's own error."""
+    from gelib_amd import gelib_base as gb
+    from gelib_amd.gelib_common import packed, resolved
+    t = torch.randn(2, 3, 4, dtype=torch.complex64)
+    assert gb.in_memory() and gb.in_memory(t, t[:, 1:], torch.ones(2)) and gb.in_memory(t.conj().resolve_conj())
+    assert not any(gb.in_memory(t, x) for x in (t.conj(), torch._neg_view(t), None, 3))
+    for view in (t.conj(), torch._neg_view(t), torch._neg_view(t.conj())):
+        a, b = resolved(view, t)
+        assert gb.in_memory(a, b, packed(view[:, 1:])) and torch.equal(a, view) and b is not None and torch.equal(b, t)
+    with pytest.raises(AttributeError):
+        resolved(t, None)
+
+
 def test_wigner_helper():
     import gelib_amd as G
     R1, R2 = G.SO3element.random(), G.SO3element.random()
